@@ -1,9 +1,9 @@
 // Kernels of the reference's bandwidth U-Net (scripts/main.py:83-118) on gfx950.
 //
 //   uconv3x3<SRC, CA, CB, CO, EPI>  3x3 'same' convolution as an implicit GEMM on
-//     v_mfma_f32_32x32x16_bf16 (M = 32 px of a row, N = 32 output channels per N-tile, K = 16
-//     input channels per chunk) over concat[a (CA ch), b (CB ch)] staged in LDS with zero padding
-//     to whole K chunks; 16x32-px tiles, every A fragment feeds up to three output rows. Forward
+//     v_mfma_f32_32x32x16_bf16 (M = 32 output channels per channel tile, N = 32 px of a row, K = 16
+//     input channels per chunk) over concat[a (CA ch), b (CB ch)] staged in LDS; 16x32-px tiles,
+//     every B fragment feeds up to three output rows. Forward
 //     (bias + ReLU -> bf16) and data gradient (flipped, transposed fragments; ReLU-masked, or
 //     plain for concat and pooled inputs). Channel counts are the stored ones (8, 16, 24, 32, 48).
 //   uwgrad<SRC, CA, CB, CO, MT>  weight gradient over 8x32-px strips, operands from pixel-major
@@ -67,23 +67,61 @@ static_assert(sizeof(UcBatch) <= 4096, "kernel argument too large");
 
 constexpr int UT_W = 32, UT_H = 16;
 
+// Raw buffer accesses with 32-bit offsets from a tile's first row: a load at kUOob returns zero and a
+// store there is dropped, so image borders and partial tiles need no branch and all loads of a
+// staging are in flight together.
+typedef __amdgpu_buffer_rsrc_t u_rsrc;
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+typedef __attribute__((ext_vector_type(3))) unsigned int u32x3;
+constexpr uint32_t kUOob = 0xFFFFFFF0u;
+__device__ __forceinline__ u_rsrc u_buf(const void *p, size_t off, size_t bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(p) + off), (short)0, (int)(uint32_t)bytes,
+                                             0x00020000);
+}
+// Two floats -> packed bf16 {a, b}, round to nearest even (one v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint32_t u_cvt2(float a, float b)
+{
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+
+// The kernel fragments are the MFMA A operand (M = output channels) and 32 pixels of a row the B
+// operand, so a lane ends with 4 of every 8 output channels of one pixel, c = 8j + 4h + 0..3, and the
+// epilogue works in registers: bias, ReLU or mask, one conversion per channel pair, a permlane32 swap
+// per two groups of 8 channels and whole-pixel 16-B (or 8-B) stores. With the pixels on the A side a
+// lane held one channel of 16 pixels: at 8 channels three quarters of the lanes converted padding and
+// the tile went back through LDS in 2-byte writes. Only the CI real channels are staged, in pixels of
+// an odd number of 16-B units (conflict-free b128 reads); the upper half of an odd last K chunk is
+// masked to zero as it is read. Bound by HBM at 8 output channels (1920x1080, before -> now: 8 -> 8
+// 28.3 -> 19.5 us for 66 MB, images -> 8 38.7 -> 34.0 us for 158 MB), by staging latency and MFMA issue
+// elsewhere (48 -> 16 at half resolution 37.7 -> 20.4 us); registers for four waves per SIMD with one K
+// chunk, three with two, two with three chunks or two channel tiles.
 template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
-__global__ __launch_bounds__(256, (CB == 0 && CA <= 16 && CO <= 24) ? 4 : 1) void uconv3x3(UcBatch b)
+__global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 3 : 4)) void uconv3x3(UcBatch b)
 {
     static_assert(!HEAD || (CO == 8 && EPI == UC_EPI_RELU), "the head follows the 8-channel ReLU layer");
-    constexpr int CI = SRC == UC_SRC_IMAGES ? 15 : CA + CB;
-    constexpr int KC = (CI + 15) / 16, CIP = KC * 16, PS = CIP + 8;
-    constexpr int NT = (CO + 31) / 32;
-    constexpr int LW = UT_W + 2, LH = UT_H + 2;
-    constexpr int OS = CO + 8;  // epilogue pixel stride (bf16)
-    constexpr int IN_ELEMS = LH * LW * PS, OUT_ELEMS = UT_H * UT_W * OS;
-    __shared__ __attribute__((aligned(16))) uint16_t lds[IN_ELEMS > OUT_ELEMS ? IN_ELEMS : OUT_ELEMS];
+    constexpr int CI = SRC == UC_SRC_IMAGES ? 16 : CA + CB;
+    constexpr int KC = (CI + 15) / 16, QL = CI / 8, PS = 8 * (QL | 1);
+    constexpr int NT = (CO + 31) / 32, NG = CO / 8;
+    constexpr int LW = UT_W + 2, LH = UT_H + 2, NPX = LW * LH;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[NPX * PS];
+    __shared__ float hws[HEAD ? 54 : 1];  // head weights [8][6] and bias [6], read behind the MFMAs
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, px = lane & 31, h = lane >> 5;
     const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
     const UcFrame &F = b.f[L.f];
     const int H = F.H, W = F.W;
     const int x0 = L.tx * UT_W, y0 = L.ty * UT_H;
-    // kernel fragments and bias first: their loads are in flight together with the tile's
+    const int yb = max(0, y0 - 1);                                  // first staged image row
+    const size_t row0 = (size_t)yb * W, npx = (size_t)(min(H, y0 + UT_H + 1) - yb) * W;
+    // offset of a staged pixel from row yb (in pixels), or kUOob
+    auto pixel = [&](int pix) -> uint32_t {
+        const int ly = pix / LW, lx = pix - ly * LW;
+        const int gy = y0 + ly - 1, gx = x0 + lx - 1;
+        return pix < NPX && gy >= 0 && gy < H && gx >= 0 && gx < W ? (uint32_t)(gy - yb) * (uint32_t)W + (uint32_t)gx : kUOob;
+    };
+    // kernel fragments first: their loads are in flight together with the tile's
     u32x4 wf[9][KC][NT];
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -92,56 +130,91 @@ __global__ __launch_bounds__(256, (CB == 0 && CA <= 16 && CO <= 24) ? 4 : 1) voi
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
                 wf[t][kc][nt] = static_cast<const u32x4 *>(F.wfrag)[((t * KC + kc) * NT + nt) * 64 + lane];
-    float bias[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) bias[nt] = EPI == UC_EPI_RELU ? F.bias[nt * 32 + px] : 0.f;
+    if constexpr (HEAD)
+        if (tid < 54) hws[tid] = F.head_w[tid];
     if constexpr (SRC == UC_SRC_BF16)
     {
-        constexpr int QA = CA / 8, QB = CB / 8, QP = CIP / 8;
-        for (int i = tid; i < LH * LW * QP; i += 256)
+        constexpr int QA = CA / 8, QB = CB / 8;
+        constexpr int NA = (NPX * QA + 255) / 256, NB = QB ? (NPX * QB + 255) / 256 : 0;
+        const u_rsrc ra = u_buf(F.a, row0 * (CA * 2), npx * (CA * 2));
+        u32x4 va[NA];
+        u32x4 vb[NB ? NB : 1];
+#pragma unroll
+        for (int u = 0; u < NA; ++u)
         {
-            const int pix = i / QP, q = i - pix * QP;
-            const int ly = pix / LW, lx = pix - ly * LW;
-            const int gy = y0 + ly - 1, gx = x0 + lx - 1;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if (gy >= 0 && gy < H && gx >= 0 && gx < W)
-            {
-                const size_t p = (size_t)gy * W + gx;
-                if (q < QA)
-                    v = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.a) + p * CA + q * 8);
-                else if (q < QA + QB)
-                    v = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.b) + p * CB + (q - QA) * 8);
-            }
-            *reinterpret_cast<u32x4 *>(&lds[pix * PS + q * 8]) = v;
+            const int i = tid + 256 * u;
+            const uint32_t p = pixel(i / QA);
+            va[u] = __builtin_amdgcn_raw_buffer_load_b128(ra, p == kUOob ? kUOob : p * (CA * 2) + (i % QA) * 16, 0, 0);
         }
+        if constexpr (QB > 0)
+        {
+            const u_rsrc rb = u_buf(F.b, row0 * (CB * 2), npx * (CB * 2));
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+            {
+                const int i = tid + 256 * u;
+                const uint32_t p = pixel(i / QB);
+                vb[u] = __builtin_amdgcn_raw_buffer_load_b128(rb, p == kUOob ? kUOob : p * (CB * 2) + (i % QB) * 16, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NA; ++u)
+        {
+            const int i = tid + 256 * u;
+            if (i < NPX * QA) *reinterpret_cast<u32x4 *>(&lds[(i / QA) * PS + (i % QA) * 8]) = va[u];
+        }
+        if constexpr (QB > 0)
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+            {
+                const int i = tid + 256 * u;
+                if (i < NPX * QB) *reinterpret_cast<u32x4 *>(&lds[(i / QB) * PS + CA + (i % QB) * 8]) = vb[u];
+            }
     }
     else
     {
-        for (int pix = tid; pix < LH * LW; pix += 256)
+        constexpr int NP = (NPX + 255) / 256;
+        u32x3 v[NP][5];
+#pragma unroll
+        for (int im = 0; im < 5; ++im)
         {
-            const int ly = pix / LW, lx = pix - ly * LW;
-            const int gy = y0 + ly - 1, gx = x0 + lx - 1;
-            float v[16];
+            const u_rsrc r = u_buf(F.img[im], row0 * 12, npx * 12);
 #pragma unroll
-            for (int k = 0; k < 16; ++k) v[k] = 0.f;
-            if (gy >= 0 && gy < H && gx >= 0 && gx < W)
+            for (int u = 0; u < NP; ++u)
             {
-                const size_t p = (size_t)gy * W + gx;
-#pragma unroll
-                for (int im = 0; im < 5; ++im)
-                {
-                    const float *s = F.img[im] + 3 * p;
-                    v[3 * im] = s[0]; v[3 * im + 1] = s[1]; v[3 * im + 2] = s[2];
-                }
+                const uint32_t p = pixel(tid + 256 * u);
+                v[u][im] = __builtin_amdgcn_raw_buffer_load_b96(r, p == kUOob ? kUOob : p * 12, 0, 0);
             }
-            u32x4 a, c;
-            a.x = u_pack2(v[0], v[1]); a.y = u_pack2(v[2], v[3]); a.z = u_pack2(v[4], v[5]); a.w = u_pack2(v[6], v[7]);
-            c.x = u_pack2(v[8], v[9]); c.y = u_pack2(v[10], v[11]); c.z = u_pack2(v[12], v[13]);
-            c.w = u_pack2(v[14], v[15]);
-            *reinterpret_cast<u32x4 *>(&lds[pix * PS]) = a;
-            *reinterpret_cast<u32x4 *>(&lds[pix * PS + 8]) = c;
+        }
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+        {
+            const int pix = tid + 256 * u;
+            if (pix >= NPX) continue;
+            float f[16];
+#pragma unroll
+            for (int im = 0; im < 5; ++im)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) f[3 * im + k] = __uint_as_float(v[u][im][k]);
+            f[15] = 0.f;
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                *reinterpret_cast<u32x4 *>(&lds[pix * PS + 8 * q]) =
+                    u32x4{u_cvt2(f[8 * q], f[8 * q + 1]), u_cvt2(f[8 * q + 2], f[8 * q + 3]),
+                          u_cvt2(f[8 * q + 4], f[8 * q + 5]), u_cvt2(f[8 * q + 6], f[8 * q + 7])};
         }
     }
+    // the lane's output pixel of tile row 4 wv + orow, in pixels from row y0 (kUOob outside the image)
+    const size_t orow0 = (size_t)y0 * W, onpx = (size_t)(min(H, y0 + UT_H) - y0) * W;
+    auto opixel = [&](int orow) -> uint32_t {
+        const int r = 4 * wv + orow;
+        return y0 + r < H && x0 + px < W ? (uint32_t)r * (uint32_t)W + (uint32_t)(x0 + px) : kUOob;
+    };
+    const u_rsrc ro = u_buf(F.out, orow0 * (CO * 2), onpx * (CO * 2));
+    float4 bias[EPI == UC_EPI_RELU ? NG : 1];  // channels 8j + 4h + 0..3
+    if constexpr (EPI == UC_EPI_RELU)
+#pragma unroll
+        for (int j = 0; j < NG; ++j) bias[j] = *reinterpret_cast<const float4 *>(F.bias + 8 * j + 4 * h);
     __syncthreads();
 
     f32x16 acc[4][NT];
@@ -151,6 +224,7 @@ __global__ __launch_bounds__(256, (CB == 0 && CA <= 16 && CO <= 24) ? 4 : 1) voi
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int k = 0; k < 16; ++k) acc[r][nt][k] = 0.f;
+    const uint32_t hi0 = h ? 0u : 0xFFFFFFFFu;  // zeroes the upper half of an odd last K chunk
 #pragma unroll
     for (int ir = 0; ir < 6; ++ir)
 #pragma unroll
@@ -158,72 +232,102 @@ __global__ __launch_bounds__(256, (CB == 0 && CA <= 16 && CO <= 24) ? 4 : 1) voi
 #pragma unroll
             for (int kc = 0; kc < KC; ++kc)
             {
-                const u32x4 a = *reinterpret_cast<const u32x4 *>(&lds[((4 * wv + ir) * LW + px + dx) * PS + kc * 16 + 8 * h]);
+                const bool odd = (QL & 1) && kc == KC - 1;
+                u32x4 a = *reinterpret_cast<const u32x4 *>(
+                    &lds[((4 * wv + ir) * LW + px + dx) * PS + kc * 16 + (odd ? 0 : 8 * h)]);
+                if (odd) a &= u32x4{hi0, hi0, hi0, hi0};
 #pragma unroll
                 for (int orow = 0; orow < 4; ++orow)
                 {
                     const int dy = ir - orow;
                     if (dy < 0 || dy > 2) continue;
 #pragma unroll
-                    for (int nt = 0; nt < NT; ++nt) acc[orow][nt] = u_mfma(a, wf[dy * 3 + dx][kc][nt], acc[orow][nt]);
+                    for (int nt = 0; nt < NT; ++nt) acc[orow][nt] = u_mfma(wf[dy * 3 + dx][kc][nt], a, acc[orow][nt]);
                 }
             }
 
-    // epilogue: lane owns output channel nt*32 + px of 16 pixels x = 8(k/4) + 4h + k%4 per row;
-    // through LDS to 16-byte stores of whole pixels
+    // head: output channels 3h .. 3h + 2 of the lane's pixel
+    float hw[HEAD ? 24 : 1], hb[3] = {0.f, 0.f, 0.f};
+    if constexpr (HEAD)
     {
-        __syncthreads();  // the input tile is dead
 #pragma unroll
-        for (int orow = 0; orow < 4; ++orow)
+        for (int c = 0; c < 8; ++c)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-            {
-                const int n = nt * 32 + px;
-                if (n >= CO) continue;
+            for (int k = 0; k < 3; ++k) hw[c * 3 + k] = hws[c * 6 + 3 * h + k];
 #pragma unroll
-                for (int k = 0; k < 16; ++k)
-                {
-                    const int x = 8 * (k >> 2) + 4 * h + (k & 3);
-                    const float v = acc[orow][nt][k];
-                    lds[((4 * wv + orow) * UT_W + x) * OS + n] =
-                        (uint16_t)u_f2bf(EPI == UC_EPI_RELU ? fmaxf(v + bias[nt], 0.f) : v);
-                }
-            }
-        __syncthreads();
-        // head weights [8][6] + bias [6], read once (the stores below could alias them)
-        float hw[HEAD ? 54 : 1];
-        if constexpr (HEAD)
+        for (int k = 0; k < 3; ++k) hb[k] = hws[48 + 3 * h + k];
+    }
 #pragma unroll
-            for (int j = 0; j < 54; ++j) hw[j] = F.head_w[j];
-        constexpr int QO = CO / 8;
-        for (int i = tid; i < UT_H * UT_W * QO; i += 256)
+    for (int orow = 0; orow < 4; ++orow)
+    {
+        const uint32_t p = opixel(orow);
+        const bool in = p != kUOob;
+        uint32_t d[2 * NG];  // d[2j + e] = channels 8j + 4h + 2e, +1
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
         {
-            const int pix = i / QO, q = i - pix * QO;
-            const int gy = y0 + pix / UT_W, gx = x0 + (pix & (UT_W - 1));
-            if (gy >= H || gx >= W) continue;
-            u32x4 v = *reinterpret_cast<const u32x4 *>(&lds[pix * OS + q * 8]);
-            const size_t o = ((size_t)gy * W + gx) * CO + q * 8;
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[k] = acc[orow][j / 4][4 * (j & 3) + k];
+            if constexpr (EPI == UC_EPI_RELU)
+            {
+                v[0] = fmaxf(v[0] + bias[j].x, 0.f); v[1] = fmaxf(v[1] + bias[j].y, 0.f);
+                v[2] = fmaxf(v[2] + bias[j].z, 0.f); v[3] = fmaxf(v[3] + bias[j].w, 0.f);
+            }
+            d[2 * j] = u_cvt2(v[0], v[1]);
+            d[2 * j + 1] = u_cvt2(v[2], v[3]);
+        }
+        // two groups of 8 channels: each half-wave gathers one whole group of its pixels
+#pragma unroll
+        for (int g = 0; g < NG / 2; ++g)
+        {
+            u32x4 v;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+            {
+                const auto sw = __builtin_amdgcn_permlane32_swap(d[4 * g + e], d[4 * g + 2 + e], false, false);
+                v[e] = (uint32_t)sw[0];
+                v[2 + e] = (uint32_t)sw[1];
+            }
+            const uint32_t o = in ? p * (CO * 2) + 32 * g + 16 * h : kUOob;
             if constexpr (EPI == UC_EPI_MASK)
             {
-                const u32x4 m = *reinterpret_cast<const u32x4 *>(F.mask + o);
+                const u_rsrc rm = u_buf(F.mask, orow0 * (CO * 2), onpx * (CO * 2));
+                const u32x4 m = __builtin_amdgcn_raw_buffer_load_b128(rm, o, 0, 0);
                 v.x = u_keep(m.x, v.x); v.y = u_keep(m.y, v.y); v.z = u_keep(m.z, v.z); v.w = u_keep(m.w, v.w);
             }
-            *reinterpret_cast<u32x4 *>(static_cast<uint16_t *>(F.out) + o) = v;
-            if constexpr (HEAD)
+            __builtin_amdgcn_raw_buffer_store_b128(v, ro, o, 0, 0);
+        }
+        if constexpr (NG & 1)
+        {
+            u32x2 v = {d[2 * NG - 2], d[2 * NG - 1]};
+            const uint32_t o = in ? p * (CO * 2) + 16 * (NG - 1) + 8 * h : kUOob;
+            if constexpr (EPI == UC_EPI_MASK)
             {
-                // the head on the stored bf16 activation: bias, then the 8 inputs in order
-                const float in[8] = {u_lo(v.x), u_hi(v.x), u_lo(v.y), u_hi(v.y),
-                                     u_lo(v.z), u_hi(v.z), u_lo(v.w), u_hi(v.w)};
-                float *po = F.head_out + ((size_t)gy * W + gx) * 6;
-#pragma unroll
-                for (int k = 0; k < 6; ++k)
-                {
-                    float sum = hw[48 + k];
-#pragma unroll
-                    for (int c = 0; c < 8; ++c) sum += in[c] * hw[c * 6 + k];
-                    po[k] = sum;
-                }
+                const u_rsrc rm = u_buf(F.mask, orow0 * (CO * 2), onpx * (CO * 2));
+                const u32x2 m = __builtin_amdgcn_raw_buffer_load_b64(rm, o, 0, 0);
+                v.x = u_keep(m.x, v.x); v.y = u_keep(m.y, v.y);
             }
+            __builtin_amdgcn_raw_buffer_store_b64(v, ro, o, 0, 0);
+        }
+        if constexpr (HEAD)
+        {
+            // the head on the stored bf16 activation: bias, then the 8 inputs in order
+            const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[0], false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[1], false, false);
+            const uint32_t w4[4] = {(uint32_t)s0[0], (uint32_t)s1[0], (uint32_t)s0[1], (uint32_t)s1[1]};
+            float sum[3] = {hb[0], hb[1], hb[2]};
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+            {
+                const float in_c = (c & 1) ? u_hi(w4[c / 2]) : u_lo(w4[c / 2]);
+#pragma unroll
+                for (int k = 0; k < 3; ++k) sum[k] += in_c * hw[c * 3 + k];
+            }
+            const u_rsrc rh = u_buf(F.head_out, orow0 * 24, onpx * 24);
+            __builtin_amdgcn_raw_buffer_store_b96(
+                u32x3{__float_as_uint(sum[0]), __float_as_uint(sum[1]), __float_as_uint(sum[2])}, rh,
+                in ? p * 24 + 12 * h : kUOob, 0, 0);
         }
     }
 }
