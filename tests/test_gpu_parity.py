@@ -498,3 +498,35 @@ def test_empty_batch(ops, dev):
         assert rc == 0, lib.xdn_last_error().decode()
         torch.cuda.synchronize()
         assert torch.count_nonzero(grad).item() == 0
+
+
+@pytest.mark.parametrize("H,W", [(16, 64), (21, 67)])
+def test_reproject_validity_at_the_thresholds(ops, dev, H, W):
+    """Depth and normal differences within a few ulp of the validity thresholds, zero and negative
+    widths, infinities and NaN: the mask equals the dividing oracle bit for bit (every pixel whose
+    bilinear taps fail goes through the 3x3 fallback)."""
+    r = np.random.default_rng(H)
+    sh = (1, H, W)
+    fw = r.uniform(0, 0.5, sh).astype(np.float32)
+    fwn = r.uniform(0, 0.05, sh).astype(np.float32)
+    fw[0, 2], fwn[0, 3] = -0.01, -0.02
+    lz, plz = np.zeros(sh + (3,), np.float32), np.zeros(sh + (3,), np.float32)
+    lz[..., 1] = fw
+    edge = (np.float32(10.0) * (fw + np.float32(1e-2))).astype(np.float32)
+    plz[..., 0] = (edge.view(np.int32) + r.integers(-2, 3, sh)).astype(np.int32).view(np.float32)
+    n, pn = np.zeros(sh + (3,), np.float32), np.zeros(sh + (3,), np.float32)
+    nedge = (4.0 * (fwn.astype(np.float64) + 1e-2)).astype(np.float32)
+    pn[..., 0] = (nedge.view(np.int32) + r.integers(-2, 3, sh)).astype(np.int32).view(np.float32)
+    plz[0, 5, ::7, 0], plz[0, 6, ::7, 0] = np.inf, np.nan
+    pn[0, 7, ::7, 0], pn[0, 8, ::7, 0] = np.inf, np.nan
+    pfw = np.zeros(sh + (3,), np.float32)
+    pfw[..., 1] = fwn
+    one = np.ones(sh + (1,), np.float32)
+    ins = [r.uniform(0, 2, sh + (3,)).astype(np.float32) for _ in range(3)]
+    args = (np.zeros(sh + (3,), np.float32), ins, lz, plz, n, pn, pfw, one, one)
+    s_ref, o_ref = O.reproject(*args)
+    s, outs = ops.Reproject(to_dev(args[0], dev), [to_dev(a, dev) for a in ins], *[to_dev(a, dev) for a in args[2:]])
+    assert 0 < s_ref.sum() < s_ref.size
+    assert np.array_equal(to_np(s), s_ref)
+    for g, rr in zip(outs, o_ref):
+        assert rel_l2(to_np(g), rr) <= 1e-6
