@@ -15,7 +15,7 @@
 //                    d loss / d network output                                  VALU-bound
 //   sf_grad_inputs   gradient w.r.t. the four images, gather form (no atomics): every pixel
 //                    collects its own-center term and the terms of all centers whose (mirrored)
-//                    window contains it
+//                    window contains it, both from one pass over its window; two threads a pixel
 //   sf_generic       any window size, direct loads (forward / grad)
 #include "xdn_common.h"
 #include "xdn_kernels.h"
@@ -367,125 +367,189 @@ __global__ __launch_bounds__(256) void sf_generic(SfBatch b)
 //              dq += -2 b_q u (c_q - c_i)  (per image and band)
 //   tap terms  (q as the tap of center p, mirror(p+d) = q):
 //              dq += w g_p (direct, colour images only) + 2 b_p u_pq (c_p - c_q)
-// The centers p whose mirrored window contains q are enumerated per dimension: p = x - d for
-// x in {q, -q (q > 0), 2n-2-q (q <= n-2)} with 0 <= p < n.
-// LDS: the tile plus halo of every per-pixel quantity (25 floats), 26x26 pixels for win 11.
+// For a neighbour r of q inside the image both terms run over the same pair (q, r): r is a tap of q and
+// q a tap of r at the same distances, so one pass over the window computes each pair's four distances
+// once and adds both terms with one coefficient per image,
+//   dq += -2 (b_q u_qr + b_r u_rq) (c_q - c_r) + w_rq g_r,
+// 79 FMA-class instructions and four exponentials a pair instead of about 120 and the index work of a
+// tap-by-tap enumeration. Pixels within
+// HALF of an image edge are also reached through the reflection: with q' = -q or 2n - 2 - q along an
+// axis, they are taps of the centers p around q' too, at the distances of (p, q) and the pixel
+// distance of p - q'; those pairs are a second loop that only blocks at an edge run.
+// LDS: the tile plus halo of every per-pixel quantity (25 floats), 26x26 pixels for win 11: 67.6 KB, two
+// blocks per CU, so a pixel's window rows are split over two threads (rows dy <= 0 and dy > 0, joined
+// through LDS) for four waves per SIMD instead of two. VALU-bound: 512x512, win 11: 247 -> 102 us
+// (128 us with one thread per pixel).
 // ---------------------------------------------------------------------------------------------
+struct Yes {
+    static constexpr bool value = true;
+};
+struct No {
+    static constexpr bool value = false;
+};
+
 template <int HALF>
-__global__ __launch_bounds__(256) void sf_grad_inputs_tile(SfBatch b)
+__global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
 {
     constexpr int E = SF_T + 2 * HALF;
-    constexpr int NQ = 7;  // float4 per pixel
-    // per pixel: (A.xyz, B.x) (B.yz, alb.xy) (alb.z, n.xyz) (b0..b3) (b4, gA.xyz) (hA, gB.xyz) (hB, -, -, -)
-    __shared__ float4 s[NQ][E * E];
+    constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
+    // per pixel: (A.xyz, B.x) (B.yz, alb.xy) (alb.z, n.xyz) (k0..k3) (k4, gA.xyz) (hA, gB.xyz) (hB) with
+    // k = -log2e * band, k4 divided by HALF^2
+    __shared__ float4 s[6][E * E];
+    __shared__ float shB[E * E];
     const int tile = xcd_tile(blockIdx.x, b.map.total);
     const TileLoc L = locate(b.map, tile);
     const SfFrame &F = b.f[L.f];
     const int H = F.H, W = F.W;
     const int x0 = L.tx * SF_T, y0 = L.ty * SF_T;
-    for (int i = threadIdx.x; i < E * E; i += 256)
+    for (int i = threadIdx.x; i < E * E; i += 512)
     {
         const int ly = i / E, lx = i - ly * E;
         const int gy = mirror(min(y0 + ly - HALF, H - 1 + HALF), H), gx = mirror(min(x0 + lx - HALF, W - 1 + HALF), W);
         const size_t p = (size_t)gy * W + gx;
         const float3 a = ld3(F.ia, p), bb = ld3(F.ib, p), al = ld3(F.alb, p), n = ld3(F.nrm, p);
-        const float *bd = F.band + 5 * p;
-        const float3 gA = ld3(F.gaccA, p), gB = ld3(F.gaccB, p);
+        SfCenter C;
+        sf_center_bands(C, F.band, p, HALF);
+        float3 gA = ld3(F.gaccA, p), gB = ld3(F.gaccB, p);
+        float hA = F.gwA[p], hB = F.gwB[p];
+        // a window position outside the image is a tap (of the mirrored pixel's values) but no center:
+        // its weights are exp2(-inf) = 0 and its upstream gradients zero
+        const int ux = x0 + lx - HALF, uy = y0 + ly - HALF;
+        if (ux < 0 || uy < 0 || ux >= W || uy >= H)
+        {
+            C.k0 = C.k1 = C.k2 = C.k3 = hA = hB = 0.f;
+            C.k4 = -__builtin_inff();
+            gA = gB = make_float3(0.f, 0.f, 0.f);
+        }
         s[0][i] = make_float4(a.x, a.y, a.z, bb.x);
         s[1][i] = make_float4(bb.y, bb.z, al.x, al.y);
         s[2][i] = make_float4(al.z, n.x, n.y, n.z);
-        s[3][i] = make_float4(bd[0], bd[1], bd[2], bd[3]);
-        s[4][i] = make_float4(bd[4], gA.x, gA.y, gA.z);
-        s[5][i] = make_float4(F.gwA[p], gB.x, gB.y, gB.z);
-        s[6][i] = make_float4(F.gwB[p], 0.f, 0.f, 0.f);
+        s[3][i] = make_float4(C.k0, C.k1, C.k2, C.k3);
+        s[4][i] = make_float4(C.k4, gA.x, gA.y, gA.z);
+        s[5][i] = make_float4(hA, gB.x, gB.y, gB.z);
+        shB[i] = hB;
     }
     __syncthreads();
-    const int lx = threadIdx.x & (SF_T - 1), ly = threadIdx.x / SF_T;
+    const int t = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int lx = t & (SF_T - 1), ly = t / SF_T;
     const int qx = x0 + lx, qy = y0 + ly;
-    if (qx >= W || qy >= H) return;
+    const bool live = qx < W && qy < H;
     const int q0 = (ly + HALF) * E + lx + HALF;
-    auto unpack = [&](int k, float3 &cA, float3 &cB, float3 &ca, float3 &cn) {
-        const float4 P0 = s[0][k], P1 = s[1][k], P2 = s[2][k];
-        cA = make_float3(P0.x, P0.y, P0.z);
-        cB = make_float3(P0.w, P1.x, P1.y);
-        ca = make_float3(P1.z, P1.w, P2.x);
-        cn = make_float3(P2.y, P2.z, P2.w);
+    struct Px {
+        float3 A, B, al, n;
     };
-    float3 qA, qB, qa, qn;
-    unpack(q0, qA, qB, qa, qn);
-    const float4 qb03 = s[3][q0], qb4g = s[4][q0], qhg = s[5][q0];
-    const float qhB = s[6][q0].x;
-    const float3 qgA = make_float3(qb4g.y, qb4g.z, qb4g.w), qgB = make_float3(qhg.y, qhg.z, qhg.w);
-    const float qhA = qhg.x;
-    float3 dA = make_float3(0.f, 0.f, 0.f), dB = dA, da = dA, dn = dA;
-    const float inv_h2 = 1.f / (float)(HALF * HALF);
-    for (int dy = -HALF; dy <= HALF; ++dy)
-    {
-        int pys[3], npy = 0;
+    auto image = [&](int k) {
+        const float4 P0 = s[0][k], P1 = s[1][k], P2 = s[2][k];
+        return Px{make_float3(P0.x, P0.y, P0.z), make_float3(P0.w, P1.x, P1.y), make_float3(P1.z, P1.w, P2.x),
+                  make_float3(P2.y, P2.z, P2.w)};
+    };
+    struct Up {  // bands and upstream gradients
+        float k0, k1, k2, k3, k4, hA, hB;
+        float3 gA, gB;
+    };
+    auto upstream = [&](int k) {
+        const float4 K = s[3][k], G = s[4][k], HG = s[5][k];
+        return Up{K.x, K.y, K.z, K.w, G.x, HG.x, shB[k], make_float3(G.y, G.z, G.w), make_float3(HG.y, HG.z, HG.w)};
+    };
+    const Px Q = image(q0);
+    const Up U = upstream(q0);
+    const float3 zero = make_float3(0.f, 0.f, 0.f);
+    float3 dA = zero, dB = zero, da = zero, dn = zero;  // sum of coefficient * (c_q - c_r)
+    float3 eA = zero, eB = zero;                        // sum of w_rq g_r
+    // one pair (q, r) at the squared pixel distance r2: r's center term, and q's tap term where OWN
+    auto pair = [&](int k, float r2, auto own) {
+        constexpr bool OWN = decltype(own)::value;
+        const Px R = image(k);
+        const float3 xA = make_float3(Q.A.x - R.A.x, Q.A.y - R.A.y, Q.A.z - R.A.z);
+        const float3 xB = make_float3(Q.B.x - R.B.x, Q.B.y - R.B.y, Q.B.z - R.B.z);
+        const float3 xa = make_float3(Q.al.x - R.al.x, Q.al.y - R.al.y, Q.al.z - R.al.z);
+        const float3 xn = make_float3(Q.n.x - R.n.x, Q.n.y - R.n.y, Q.n.z - R.n.z);
+        const float DA = xA.x * xA.x + xA.y * xA.y + xA.z * xA.z, DB = xB.x * xB.x + xB.y * xB.y + xB.z * xB.z;
+        const float Da = xa.x * xa.x + xa.y * xa.y + xa.z * xa.z, Dn = xn.x * xn.x + xn.y * xn.y + xn.z * xn.z;
+        float cA = 0.f, cB = 0.f, ca = 0.f, cn = 0.f;
+        if constexpr (OWN)
         {
-            const int xs[3] = {qy, qy > 0 ? -qy : INT_MIN, qy <= H - 2 ? 2 * H - 2 - qy : INT_MIN};
-            for (int k = 0; k < 3; ++k)
-                if (xs[k] != INT_MIN && xs[k] - dy >= 0 && xs[k] - dy < H) pys[npy++] = xs[k] - dy;
+            const float sh = U.k2 * Da + (U.k3 * Dn + U.k4 * r2);
+            const float uA = fast_exp2(U.k0 * DA + sh) * (U.gA.x * R.A.x + U.gA.y * R.A.y + U.gA.z * R.A.z + U.hA);
+            const float uB = fast_exp2(U.k1 * DB + sh) * (U.gB.x * R.B.x + U.gB.y * R.B.y + U.gB.z * R.B.z + U.hB);
+            const float u = uA + uB;
+            cA = U.k0 * uA; cB = U.k1 * uB; ca = U.k2 * u; cn = U.k3 * u;
         }
-        for (int dx = -HALF; dx <= HALF; ++dx)
         {
-            const float pd = (float)(dx * dx + dy * dy) * inv_h2;
-            // own term: tap at q + d
-            {
-                const int k = q0 + dy * E + dx;
-                float3 iA, iB, ia, in;
-                unpack(k, iA, iB, ia, in);
-                const float eA = dist2(qA, iA), eB = dist2(qB, iB), ea = dist2(qa, ia), en = dist2(qn, in);
-                const float sh = -qb03.z * ea - qb03.w * en - qb4g.x * pd;
-                const float wA = __expf(-qb03.x * eA + sh), wB = __expf(-qb03.y * eB + sh);
-                const float uA = wA * (qgA.x * iA.x + qgA.y * iA.y + qgA.z * iA.z + qhA);
-                const float uB = wB * (qgB.x * iB.x + qgB.y * iB.y + qgB.z * iB.z + qhB);
-                const float tA = -2.f * qb03.x * uA, tB = -2.f * qb03.y * uB;
-                const float ta = -2.f * qb03.z * (uA + uB), tn = -2.f * qb03.w * (uA + uB);
-                dA.x += tA * (qA.x - iA.x); dA.y += tA * (qA.y - iA.y); dA.z += tA * (qA.z - iA.z);
-                dB.x += tB * (qB.x - iB.x); dB.y += tB * (qB.y - iB.y); dB.z += tB * (qB.z - iB.z);
-                da.x += ta * (qa.x - ia.x); da.y += ta * (qa.y - ia.y); da.z += ta * (qa.z - ia.z);
-                dn.x += tn * (qn.x - in.x); dn.y += tn * (qn.y - in.y); dn.z += tn * (qn.z - in.z);
-            }
-            // tap terms: centers p with mirror(p + d) = q
-            int pxs[3], npx = 0;
-            {
-                const int xs[3] = {qx, qx > 0 ? -qx : INT_MIN, qx <= W - 2 ? 2 * W - 2 - qx : INT_MIN};
-                for (int k = 0; k < 3; ++k)
-                    if (xs[k] != INT_MIN && xs[k] - dx >= 0 && xs[k] - dx < W) pxs[npx++] = xs[k] - dx;
-            }
-            for (int a = 0; a < npy; ++a)
-                for (int bq = 0; bq < npx; ++bq)
+            const Up V = upstream(k);
+            const float sh = V.k2 * Da + (V.k3 * Dn + V.k4 * r2);
+            const float wA = fast_exp2(V.k0 * DA + sh), wB = fast_exp2(V.k1 * DB + sh);
+            const float uA = wA * (V.gA.x * Q.A.x + V.gA.y * Q.A.y + V.gA.z * Q.A.z + V.hA);
+            const float uB = wB * (V.gB.x * Q.B.x + V.gB.y * Q.B.y + V.gB.z * Q.B.z + V.hB);
+            const float u = uA + uB;
+            cA += V.k0 * uA; cB += V.k1 * uB; ca += V.k2 * u; cn += V.k3 * u;
+            eA.x += wA * V.gA.x; eA.y += wA * V.gA.y; eA.z += wA * V.gA.z;
+            eB.x += wB * V.gB.x; eB.y += wB * V.gB.y; eB.z += wB * V.gB.z;
+        }
+        dA.x += cA * xA.x; dA.y += cA * xA.y; dA.z += cA * xA.z;
+        dB.x += cB * xB.x; dB.y += cB * xB.y; dB.z += cB * xB.z;
+        da.x += ca * xa.x; da.y += ca * xa.y; da.z += ca * xa.z;
+        dn.x += cn * xn.x; dn.y += cn * xn.y; dn.z += cn * xn.z;
+    };
+    const int dy1 = grp ? HALF : 0;
+#pragma unroll 1
+    for (int dy = grp ? 1 : -HALF; dy <= dy1; ++dy)
+    {
+        const int base = q0 + dy * E;
+        const float y2 = (float)(dy * dy);
+#pragma unroll
+        for (int dx = -HALF; dx <= HALF; ++dx) pair(base + dx, y2 + (float)(dx * dx), Yes{});
+    }
+    // a pixel at most HALF from the first or last row or column is reached through the reflection
+    if (live && (x0 <= HALF || y0 <= HALF || x0 + SF_T + HALF >= W || y0 + SF_T + HALF >= H))
+    {
+        // centers around the reflections of q (one or both axes reflected)
+        const int vy[3] = {qy, qy > 0 ? -qy : INT_MIN, qy <= H - 2 ? 2 * H - 2 - qy : INT_MIN};
+        const int vx[3] = {qx, qx > 0 ? -qx : INT_MIN, qx <= W - 2 ? 2 * W - 2 - qx : INT_MIN};
+        for (int a = 0; a < 9; ++a)
+        {
+            const int ay = a / 3, ax = a - 3 * ay;
+            if (a == 0 || vy[ay] == INT_MIN || vx[ax] == INT_MIN) continue;
+            const int py0 = max(0, vy[ay] - HALF), py1 = min(H - 1, vy[ay] + HALF);
+            const int px0 = max(0, vx[ax] - HALF), px1 = min(W - 1, vx[ax] + HALF);
+            for (int py = py0 + grp; py <= py1; py += 2)
+                for (int px = px0; px <= px1; ++px)
                 {
-                    const int k = (pys[a] - y0 + HALF) * E + (pxs[bq] - x0 + HALF);
-                    float3 pA, pB, pa, pn;
-                    unpack(k, pA, pB, pa, pn);
-                    const float4 b03 = s[3][k], b4g = s[4][k], hg = s[5][k];
-                    const float phB = s[6][k].x;
-                    const float3 gA = make_float3(b4g.y, b4g.z, b4g.w), gB = make_float3(hg.y, hg.z, hg.w);
-                    const float eA = dist2(pA, qA), eB = dist2(pB, qB), ea = dist2(pa, qa), en = dist2(pn, qn);
-                    const float sh = -b03.z * ea - b03.w * en - b4g.x * pd;
-                    const float wA = __expf(-b03.x * eA + sh), wB = __expf(-b03.y * eB + sh);
-                    const float uA = wA * (gA.x * qA.x + gA.y * qA.y + gA.z * qA.z + hg.x);
-                    const float uB = wB * (gB.x * qB.x + gB.y * qB.y + gB.z * qB.z + phB);
-                    const float tA = 2.f * b03.x * uA, tB = 2.f * b03.y * uB;
-                    const float ta = 2.f * b03.z * (uA + uB), tn = 2.f * b03.w * (uA + uB);
-                    dA.x += wA * gA.x + tA * (pA.x - qA.x);
-                    dA.y += wA * gA.y + tA * (pA.y - qA.y);
-                    dA.z += wA * gA.z + tA * (pA.z - qA.z);
-                    dB.x += wB * gB.x + tB * (pB.x - qB.x);
-                    dB.y += wB * gB.y + tB * (pB.y - qB.y);
-                    dB.z += wB * gB.z + tB * (pB.z - qB.z);
-                    da.x += ta * (pa.x - qa.x); da.y += ta * (pa.y - qa.y); da.z += ta * (pa.z - qa.z);
-                    dn.x += tn * (pn.x - qn.x); dn.y += tn * (pn.y - qn.y); dn.z += tn * (pn.z - qn.z);
+                    const int ey = py - vy[ay], ex = px - vx[ax];
+                    pair((py - y0 + HALF) * E + (px - x0 + HALF), (float)(ex * ex + ey * ey), No{});
                 }
         }
     }
+    // the second half of the rows joins through LDS (the tile is dead)
+    __syncthreads();
+    float *red = reinterpret_cast<float *>(&s[0][0]);  // [18][256]
+    static_assert(sizeof(s) >= 18 * 256 * sizeof(float), "reduction space");
+    if (grp)
+    {
+        const float v[18] = {dA.x, dA.y, dA.z, dB.x, dB.y, dB.z, da.x, da.y, da.z,
+                             dn.x, dn.y, dn.z, eA.x, eA.y, eA.z, eB.x, eB.y, eB.z};
+#pragma unroll
+        for (int k = 0; k < 18; ++k) red[k * 256 + t] = v[k];
+    }
+    __syncthreads();
+    if (grp || !live) return;
+    {
+        float3 *const v[6] = {&dA, &dB, &da, &dn, &eA, &eB};
+#pragma unroll
+        for (int k = 0; k < 6; ++k)
+        {
+            v[k]->x += red[(3 * k) * 256 + t];
+            v[k]->y += red[(3 * k + 1) * 256 + t];
+            v[k]->z += red[(3 * k + 2) * 256 + t];
+        }
+    }
+    // the coefficients hold k = -log2e b for the bands: -2 b = 2 ln2 k
+    constexpr float kScale = 2.f * 0.693147180559945309f;
     const size_t c = (size_t)qy * W + qx;
-    if (F.gia) st3(F.gia, c, dA);
-    if (F.gib) st3(F.gib, c, dB);
-    if (F.galb) st3(F.galb, c, da);
-    if (F.gnrm) st3(F.gnrm, c, dn);
+    if (F.gia) st3(F.gia, c, make_float3(eA.x + kScale * dA.x, eA.y + kScale * dA.y, eA.z + kScale * dA.z));
+    if (F.gib) st3(F.gib, c, make_float3(eB.x + kScale * dB.x, eB.y + kScale * dB.y, eB.z + kScale * dB.z));
+    if (F.galb) st3(F.galb, c, make_float3(kScale * da.x, kScale * da.y, kScale * da.z));
+    if (F.gnrm) st3(F.gnrm, c, make_float3(kScale * dn.x, kScale * dn.y, kScale * dn.z));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -534,13 +598,13 @@ hipError_t launch_sf_grad_inputs(int n, const SfFrame *fr, int win, hipStream_t 
     if (b.map.total == 0) return hipSuccess;
     switch (b.half)
     {
-    case 1: hipLaunchKernelGGL((sf_grad_inputs_tile<1>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 2: hipLaunchKernelGGL((sf_grad_inputs_tile<2>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 3: hipLaunchKernelGGL((sf_grad_inputs_tile<3>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 4: hipLaunchKernelGGL((sf_grad_inputs_tile<4>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 5: hipLaunchKernelGGL((sf_grad_inputs_tile<5>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 6: hipLaunchKernelGGL((sf_grad_inputs_tile<6>), dim3(b.map.total), dim3(256), 0, st, b); break;
-    case 7: hipLaunchKernelGGL((sf_grad_inputs_tile<7>), dim3(b.map.total), dim3(256), 0, st, b); break;
+    case 1: hipLaunchKernelGGL((sf_grad_inputs_tile<1>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 2: hipLaunchKernelGGL((sf_grad_inputs_tile<2>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 3: hipLaunchKernelGGL((sf_grad_inputs_tile<3>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 4: hipLaunchKernelGGL((sf_grad_inputs_tile<4>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 5: hipLaunchKernelGGL((sf_grad_inputs_tile<5>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 6: hipLaunchKernelGGL((sf_grad_inputs_tile<6>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 7: hipLaunchKernelGGL((sf_grad_inputs_tile<7>), dim3(b.map.total), dim3(512), 0, st, b); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -530,3 +530,19 @@ def test_reproject_validity_at_the_thresholds(ops, dev, H, W):
     assert np.array_equal(to_np(s), s_ref)
     for g, rr in zip(outs, o_ref):
         assert rel_l2(to_np(g), rr) <= 1e-6
+
+
+@pytest.mark.parametrize("B,H,W,win", [(1, 9, 70, 11), (1, 64, 7, 13), (2, 49, 50, 11), (1, 33, 48, 3),
+                                        (1, 53, 54, 11), (1, 9, 8, 15)])
+def test_spatial_filter_grad_inputs_edges(ops, dev, B, H, W, win):
+    """Images smaller than the window on one or both axes (every pixel reached through one or two
+    reflections), blocks without and with an image edge, the smallest and largest windows."""
+    args = sf_case(H, W, seed=5 * H + W, band_lo=0.1, band_hi=3.0, B=B)
+    cots = _cots(B, H, W, 12)
+    ref = O.spatial_filter_grad_inputs(*cots, *args, win_size=win)
+    got = ops.spatial_filter_grad_inputs(*[to_dev(c, dev) for c in cots], *[to_dev(a, dev) for a in args],
+                                         win_size=win)
+    for name, g, r in zip(("imga", "imgb", "albedo", "normal"), got, ref):
+        err = rel_l2(to_np(g), r)
+        _report(f"spatial_filter_grad_inputs {name} {B}x{H}x{W} win={win}", err)
+        assert err <= TOL, name
