@@ -135,7 +135,7 @@ int xdn_cross_regression_from_color(const float *color, const float *color2, con
 namespace {
 // Workspace of the cross-regression backward, per image (every buffer 256-B aligned).
 struct CrgLayout {
-    size_t var1, var2, beta, gq, u, gcen, evar, bytes;
+    size_t var1, var2, beta, fact, gq, u, gcen, evar, bytes;
     CrgLayout(int H, int W, int s)
     {
         const size_t N = px(H, W), C = (size_t)(H / s) * (W / s);
@@ -143,6 +143,7 @@ struct CrgLayout {
         var1 = o; o += al256(N * 4);
         var2 = o; o += al256(N * 4);
         beta = o; o += al256(C * 36 * 4);
+        fact = o; o += al256(C * 2 * 3 * 21 * 4);
         gq = o; o += al256(N * 2 * 16);
         u = o; o += al256(C * 36 * 4);
         gcen = o; o += al256(C * 24 * 4);
@@ -195,11 +196,12 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
             f.alb = albedo + b * N * 3;
             f.nrm = normal + b * N * 3;
             f.beta = reinterpret_cast<float *>(w + lay.beta);
+            f.fact = reinterpret_cast<float *>(w + lay.fact);
             f.H = H;
             f.W = W;
             xdn::CrgFrame &g = fr[i];
             g.y1 = f.y1; g.y2 = f.y2; g.alb = f.alb; g.nrm = f.nrm;
-            g.var1 = f.var1; g.var2 = f.var2; g.beta = f.beta;
+            g.var1 = f.var1; g.var2 = f.var2; g.beta = f.beta; g.fact = f.fact;
             g.gouta = grad_outa + b * N * 3;
             g.goutb = grad_outb + b * N * 3;
             g.gvara = grad_vara ? grad_vara + b * N : nullptr;

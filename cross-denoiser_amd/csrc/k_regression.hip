@@ -131,6 +131,7 @@ __global__ __launch_bounds__(256) void variance_kernel(VarBatch b)
 struct RegFrame {
     const float *y1, *y2, *var1, *var2, *alb, *nrm;
     float *beta;  // [Hs][Ws][2][18]
+    float *fact;  // [Hs][Ws][2][3][21] (FACT kernels)
     int H, W;
     int nfull;    // fast path with paired row tails: full 64-center blocks per center row, else 0
 };
@@ -170,7 +171,8 @@ constexpr int RG_ROW = RG_CX * RG_S + 2 * RG_H;
 // 21 tap rows the two center rows span), so a 1080p frame is 2,025 blocks instead of 2,160: two
 // rounds of the 1,024 resident at a time (four per CU) instead of three. Tile map per row pair p:
 // nfull blocks of row 2p, nfull of row 2p + 1, then the paired tail. Each lane sums its taps in the
-// same order either way.
+// same order either way. FACT: the centers' Cholesky factors are kept for the backward.
+template <bool FACT>
 __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
 {
     // [buffer][plane][pixel]; planes: (y1, var1), (y2, var2), (albedo, std1), (normal, std2)
@@ -267,6 +269,7 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
     if (!active) return;
     // Lane pair solves the three channels: split 0 -> channels 0 and 1, split 1 -> channel 2.
     float *out = F.beta + (((size_t)row_c * Ws + bx) * 2 + half) * 18;
+    float *fact = FACT ? F.fact + (((size_t)row_c * Ws + bx) * 2 + half) * (3 * kFact6) : nullptr;
     {
         Sys6 s0, s2;
         acc.system(0, s0);
@@ -277,8 +280,8 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
 #pragma unroll
         for (int k = 0; k < 6; ++k) s.x[k] = split ? s2.x[k] : s0.x[k];
         float be[6];
-        solve6(s, be);
         const int ch = split ? 2 : 0;
+        solve6(s, be, FACT ? fact + ch * kFact6 : nullptr);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + ch] = be[k];
     }
@@ -287,13 +290,14 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
         Sys6 s1;
         acc.system(1, s1);
         float be[6];
-        solve6(s1, be);
+        solve6(s1, be, FACT ? fact + kFact6 : nullptr);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + 1] = be[k];
     }
 }
 
 // Any window / sparsity: one lane per (center, half), direct loads.
+template <bool FACT>
 __global__ __launch_bounds__(256) void regression_generic(RegBatch b)
 {
     const int tile = xcd_tile(blockIdx.x, b.map.total);
@@ -333,7 +337,7 @@ __global__ __launch_bounds__(256) void regression_generic(RegBatch b)
         Sys6 s;
         acc.system(ch, s);
         float be[6];
-        solve6(s, be);
+        solve6(s, be, FACT ? F.fact + ((((size_t)by * Ws + bx) * 2 + half) * 3 + ch) * kFact6 : nullptr);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + ch] = be[k];
     }
@@ -555,6 +559,7 @@ hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, hipStream
         RegFrame &r = b.f[i];
         r.y1 = fr[i].y1; r.y2 = fr[i].y2; r.var1 = fr[i].var1; r.var2 = fr[i].var2;
         r.alb = fr[i].alb; r.nrm = fr[i].nrm; r.beta = fr[i].beta; r.H = fr[i].H; r.W = fr[i].W;
+        r.fact = fr[i].fact;
         const int Ws = r.W / s, Hs = r.H / s;
         // pair the rows' tail blocks where a tail holds at most half a block of centers
         const int rem = Ws % RG_CX;
@@ -574,10 +579,11 @@ hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, hipStream
     b.half_win = win / 2;
     b.sparsity = s;
     if (b.map.total == 0) return hipSuccess;
+    const bool fact = fr[0].fact != nullptr;  // all frames of a call or none
     if (fast)
-        hipLaunchKernelGGL(regression_rows, dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((fact ? regression_rows<true> : regression_rows<false>), dim3(b.map.total), dim3(256), 0, st, b);
     else
-        hipLaunchKernelGGL(regression_generic, dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((fact ? regression_generic<true> : regression_generic<false>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 

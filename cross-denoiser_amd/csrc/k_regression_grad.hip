@@ -13,16 +13,19 @@
 // Conventions at the kinks: max(0, .) passes the gradient where the value is > 0, the sumW guard
 // where sumW > 1e-7, and d sqrt(v)/dv is 0 where v == 0.
 //
-// Kernels (all batched over frames like the forward; one thread per pixel or per (center, half)):
-//   crg_recon_prep   per pixel: recompute the reconstruction sums, emit (g_acc, g_sumW)   [H][W][2]
-//   crg_center       per (center, half): gather g_beta over the pixels whose range holds the
-//                    center (recon adjoint, center side), rebuild M, solve u, then the
-//                    center side of the regression adjoint over the window             [Hs][Ws][2]
-//   crg_pixel        per pixel: recon adjoint (pixel side), regression adjoint (tap side,
-//                    all mirrored positions of the pixel), center-side terms of grid pixels,
-//                    variance adjoint (own term); writes grad albedo/normal and partial
-//                    grad imga/imgb
-//   crg_var_gather   per pixel: neighbour terms of the variance adjoint
+// Kernels (all batched over frames like the forward), in launch order; the crg_*_tile forms take the
+// windows that fit their LDS arrays (win 17 / sparsity 4 and smaller), the others any window with one
+// thread per pixel or per (center, half) and direct loads:
+//   crg_prep_tile, crg_recon_prep   per pixel: recompute the reconstruction sums, emit
+//                        (g_acc, g_sumW)                                                  [H][W][2]
+//   crg_center_tile, crg_center     per (center, half): gather g_beta over the pixels whose range holds
+//                        the center (recon adjoint, center side), solve u, then the center side of
+//                        the regression adjoint over the window                         [Hs][Ws][2]
+//   crg_pixel_tile, crg_pixel       per pixel: recon adjoint (pixel side), regression adjoint (tap
+//                        side, all mirrored positions of the pixel), center-side terms of grid
+//                        pixels, variance adjoint (own term); writes grad albedo/normal and partial
+//                        grad imga/imgb
+//   crg_var_gather       per pixel: neighbour terms of the variance adjoint
 #include "xdn_common.h"
 #include "xdn_kernels.h"
 #include "xdn_regression.h"
@@ -460,6 +463,488 @@ __global__ __launch_bounds__(256) void crg_pixel(CrgBatch b)
 }
 
 // ---------------------------------------------------------------------------------------------
+// Tiled forms of 1-3 for windows that fit LDS (win 17 / sparsity 4 and smaller)
+// ---------------------------------------------------------------------------------------------
+struct EdgeYes {
+    static constexpr bool value = true;
+};
+struct EdgeNo {
+    static constexpr bool value = false;
+};
+
+// Sum over the 16 lanes of a DPP row, the same bits in every lane (after each rotation the values
+// repeat with half the period, so both partners add the same two numbers).
+template <int R>
+__device__ __forceinline__ float row_ror_add(float v)
+{
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + R, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float v)
+{
+    return row_ror_add<1>(row_ror_add<2>(row_ror_add<4>(row_ror_add<8>(v))));
+}
+
+// Staged center records of a 16x16-pixel tile, in float4: beta A, beta B (18 floats each), with U: u A,
+// u B, then (y1, var1) (y2, var2) (albedo, std1) (normal, std2).
+template <bool U, int MAXC>
+struct CrgCenters {
+    static constexpr int REC = U ? 22 : 13, IMG = REC - 4;
+    int clo, rlo, ncx;
+    __device__ __forceinline__ void stage(const CrgFrame &F, float4 (*cs)[REC], int x0, int y0, int S, int HW)
+    {
+        const int H = F.H, W = F.W, Ws = W / S, Hs = H / S;
+        clo = max(0, (x0 - HW + S - 1) / S);
+        rlo = max(0, (y0 - HW + S - 1) / S);
+        if (x0 <= HW) clo = 0;
+        if (y0 <= HW) rlo = 0;
+        ncx = min(Ws - 1, (x0 + 15 + HW) / S) - clo + 1;
+        const int ncy = min(Hs - 1, (y0 + 15 + HW) / S) - rlo + 1;
+        for (int i = threadIdx.x; i < ncx * ncy * IMG; i += 256)
+        {
+            const int c = i / IMG, q = i - c * IMG, ry = c / ncx, rx = c - ry * ncx;
+            const size_t crec = ((size_t)(rlo + ry) * Ws + (clo + rx)) * 9;  // float4 of beta or u
+            const float4 *src = reinterpret_cast<const float4 *>(q < 9 ? F.beta : F.u);
+            cs[c][q] = src[crec + (q < 9 ? q : q - 9)];
+        }
+        for (int i = threadIdx.x; i < ncx * ncy; i += 256)
+        {
+            const int ry = i / ncx, rx = i - ry * ncx;
+            const size_t p = (size_t)((rlo + ry) * S) * W + (size_t)((clo + rx) * S);
+            const float3 a = ld3(F.y1, p), bb = ld3(F.y2, p), al = ld3(F.alb, p), nr = ld3(F.nrm, p);
+            const float v1 = F.var1[p], v2 = F.var2[p];
+            cs[i][IMG] = make_float4(a.x, a.y, a.z, v1);
+            cs[i][IMG + 1] = make_float4(bb.x, bb.y, bb.z, v2);
+            cs[i][IMG + 2] = make_float4(al.x, al.y, al.z, sqrtf(v1));
+            cs[i][IMG + 3] = make_float4(nr.x, nr.y, nr.z, sqrtf(v2));
+        }
+    }
+};
+// centers per tile axis
+static int crg_axis_centers(int S, int HW) { return (15 + 2 * HW) / S + 1; }
+
+// 1. (g_acc, g_sumW) of the reconstruction, both halves of a pixel per lane, its centers from LDS
+// (512x512, win 17: 58 -> 23 us against a lane's own loads of every center record).
+template <int MAXC>
+__global__ __launch_bounds__(256) void crg_prep_tile(CrgBatch b)
+{
+    typedef CrgCenters<false, MAXC> Rec;
+    __shared__ float4 cs[MAXC][Rec::REC];
+    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const CrgFrame &F = b.f[L.f];
+    const int S = b.sparsity, HW = b.half_win, H = F.H, W = F.W;
+    Rec rec;
+    rec.stage(F, cs, L.tx * 16, L.ty * 16, S, HW);
+    __syncthreads();
+    const int px = L.tx * 16 + (threadIdx.x & 15), py = L.ty * 16 + (threadIdx.x >> 4);
+    if (px >= W || py >= H) return;
+    const size_t p = (size_t)py * W + px;
+    const int sx = max(0, idivup(px - HW, S)), ex = min((W - 1) / S, (px + HW) / S);
+    const int sy = max(0, idivup(py - HW, S)), ey = min((H - 1) / S, (py + HW) / S);
+    const float3 ap = ld3(F.alb, p), np = ld3(F.nrm, p);
+    float3 fp[2] = {ld3(F.y1, p), ld3(F.y2, p)};
+    const float vp[2] = {F.var1[p], F.var2[p]};
+    const float sp[2] = {sqrtf(vp[0]), sqrtf(vp[1])};
+    float3 acc[2];
+    float sum[2] = {0.f, 0.f};
+    acc[0] = acc[1] = make_float3(0.f, 0.f, 0.f);
+    for (int iy = sy; iy <= ey; ++iy)
+        for (int ix = sx; ix <= ex; ++ix)
+        {
+            const float4 *c = cs[(iy - rec.rlo) * rec.ncx + (ix - rec.clo)];
+            const float4 A = c[Rec::IMG + 2], N = c[Rec::IMG + 3];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+            {
+                const float4 P = c[Rec::IMG + h];
+                float d[3][6], pred[3], inv;
+                const float w = recon_pair(fp[h], ap, np, vp[h], sp[h], make_float3(P.x, P.y, P.z),
+                                           make_float3(A.x, A.y, A.z), make_float3(N.x, N.y, N.z), P.w, h ? N.w : A.w,
+                                           reinterpret_cast<const float *>(c) + 18 * h, d, pred, inv);
+                acc[h].x += w * pred[0];
+                acc[h].y += w * pred[1];
+                acc[h].z += w * pred[2];
+                sum[h] += w;
+            }
+        }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        const float iv = 1.f / fmaxf(sum[h], 1e-7f);
+        const float3 go = ld3(h ? F.goutb : F.gouta, p);
+        float4 q;
+        q.x = acc[h].x * iv > 0.f ? go.x * iv : 0.f;
+        q.y = acc[h].y * iv > 0.f ? go.y * iv : 0.f;
+        q.z = acc[h].z * iv > 0.f ? go.z * iv : 0.f;
+        q.w = sum[h] > 1e-7f ? -(q.x * acc[h].x + q.y * acc[h].y + q.z * acc[h].z) * iv : 0.f;
+        F.gq[p * 2 + h] = q;
+    }
+}
+
+// 2. g_beta, u = M^-1 g_beta and the center-side gradients: a 4x4 block of centers per 512-lane
+// workgroup, 16 lanes per (center, half) that split the window's taps and add up with DPP rotations;
+// the pixels of the block's windows (image planes and the two g_acc planes, 29x29 px for win 17 /
+// sparsity 4: 81 KB, two blocks per CU) in LDS; the Cholesky factor from the forward instead of a
+// second accumulation of the normal equations. Every factor of a tap's adjoint that only depends on the
+// center is taken out of the sum, e.g. sum gd_2 = beta_2 sum w g_acc: 28 sums for the reconstruction and
+// 22 for the regression side instead of all of g_d. One lane per (center, half) had 512 waves for the
+// whole chip at 512x512 and direct loads for every tap: 496 -> 63 us (VALU-bound now).
+constexpr int CC_T = 4, CC_MAXPX = 29 * 29;
+__global__ __launch_bounds__(512, 4) void crg_center_tile(CrgBatch b)
+{
+    __shared__ float4 tl[6][CC_MAXPX];  // (y1, var1) (y2, var2) (albedo, std1) (normal, std2), g_acc A, B
+    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const CrgFrame &F = b.f[L.f];
+    const int S = b.sparsity, HW = b.half_win, H = F.H, W = F.W, Ws = W / S, Hs = H / S;
+    const int bx0 = L.tx * CC_T, by0 = L.ty * CC_T;
+    const int RW = (CC_T - 1) * S + 1 + 2 * HW, NP = RW * RW;
+    for (int i = threadIdx.x; i < NP; i += 512)
+    {
+        const int ly = i / RW, lx = i - ly * RW;
+        const int ux = bx0 * S - HW + lx, uy = by0 * S - HW + ly;
+        const size_t p = (size_t)mirror(min(uy, H - 1 + HW), H) * W + mirror(min(ux, W - 1 + HW), W);
+        const float3 a = ld3(F.y1, p), bb = ld3(F.y2, p), al = ld3(F.alb, p), nr = ld3(F.nrm, p);
+        const float v1 = F.var1[p], v2 = F.var2[p];
+        // a position outside the image is a regression tap (of the mirrored pixel) but no pixel of the
+        // reconstruction
+        float4 qa = make_float4(0.f, 0.f, 0.f, 0.f), qb = qa;
+        if (ux >= 0 && uy >= 0 && ux < W && uy < H) qa = F.gq[p * 2], qb = F.gq[p * 2 + 1];
+        tl[0][i] = make_float4(a.x, a.y, a.z, v1);
+        tl[1][i] = make_float4(bb.x, bb.y, bb.z, v2);
+        tl[2][i] = make_float4(al.x, al.y, al.z, sqrtf(v1));
+        tl[3][i] = make_float4(nr.x, nr.y, nr.z, sqrtf(v2));
+        tl[4][i] = qa;
+        tl[5][i] = qb;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 15, ch2 = threadIdx.x >> 4;
+    const int h = __builtin_amdgcn_readfirstlane(ch2 >> 4), ci = ch2 & 15;
+    const int bx = bx0 + (ci & 3), by = by0 + (ci >> 2);
+    const bool active = bx < Ws && by < Hs;  // the others run along (their sums are not stored)
+    const size_t crec = ((size_t)min(by, Hs - 1) * Ws + min(bx, Ws - 1)) * 2 + h;
+    const int corner = (ci >> 2) * S * RW + (ci & 3) * S, mid = corner + HW * RW + HW;
+    const float4 *own = tl[h], *oth = tl[1 - h], *alb = tl[2], *nrm = tl[3], *gq = tl[4 + h];
+    float3 fc, ac, nc;
+    float vc, sc;
+    {
+        const float4 P = own[mid], A = alb[mid], N = nrm[mid];
+        fc = make_float3(P.x, P.y, P.z); ac = make_float3(A.x, A.y, A.z); nc = make_float3(N.x, N.y, N.z);
+        vc = P.w;
+        sc = h ? N.w : A.w;
+    }
+    float bt[18];
+#pragma unroll
+    for (int k = 0; k < 18; ++k) bt[k] = F.beta[crec * 18 + k];
+    const float vce = vc + 1e-4f, sce = sc + 1e-2f;
+    // a pixel whose lower center bound rounds up past center 0 (idivup of a negative value)
+    const bool skx = bx == 0, sky = by == 0;
+    const bool edge = bx0 == 0 || by0 == 0;  // wave-uniform
+
+    const int W1 = 2 * HW + 1, n = W1 * W1;
+    const uint32_t magic = ((1u << 20) + W1 - 1) / W1;
+    struct Tap {
+        float3 df, da, dn;
+        float D, rS, E, inv, d1[3];
+    };
+    auto tap = [&](int i) {
+        const float4 P = own[i], A = alb[i], N = nrm[i];
+        Tap t;
+        t.df = make_float3(P.x - fc.x, P.y - fc.y, P.z - fc.z);
+        t.da = make_float3(A.x - ac.x, A.y - ac.y, A.z - ac.z);
+        t.dn = make_float3(N.x - nc.x, N.y - nc.y, N.z - nc.z);
+        t.D = t.df.x * t.df.x + t.df.y * t.df.y + t.df.z * t.df.z;
+        t.rS = fast_rcp(vce + P.w);
+        t.E = fast_exp2(-kLog2e * t.D * t.rS);
+        t.inv = fast_rcp(sce + (h ? N.w : A.w));
+        t.d1[0] = t.df.x * t.inv; t.d1[1] = t.df.y * t.inv; t.d1[2] = t.df.z * t.inv;
+        return t;
+    };
+    auto dot6 = [](const float *v, int c, const Tap &t) {  // v . d of channel c (v [6][3])
+        const float d2 = c == 0 ? t.da.x : (c == 1 ? t.da.y : t.da.z);
+        return v[c] + v[3 + c] * t.d1[c] + v[6 + c] * d2 + v[9 + c] * t.dn.x + v[12 + c] * t.dn.y + v[15 + c] * t.dn.z;
+    };
+
+    // (a) reconstruction adjoint over the pixels of the window
+    float gb[18], sD[3] = {0.f, 0.f, 0.f}, sT[3] = {0.f, 0.f, 0.f}, sG[3] = {0.f, 0.f, 0.f}, sV = 0.f;
+#pragma unroll
+    for (int k = 0; k < 18; ++k) gb[k] = 0.f;
+    for (int j = lane; j < n; j += 16)
+    {
+        const int row = (int)((uint32_t)j * magic >> 20), col = j - row * W1, i = corner + row * RW + col;
+        float4 q = gq[i];
+        if (edge)
+        {
+            // pixel coordinates row - HW + cy, col - HW + cx; center 0 is skipped by the pixels
+            // HW - S < p < HW, i.e. (center coordinate 0) window offsets 2 HW - S < row < 2 HW
+            if ((sky && row > 2 * HW - S && row < 2 * HW) || (skx && col > 2 * HW - S && col < 2 * HW))
+                q = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const Tap t = tap(i);
+        const float w = t.E + 1e-7f;
+        const float ga[3] = {q.x, q.y, q.z};
+        float gw = q.w;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            gw += ga[c] * dot6(bt, c, t);
+            const float wg = w * ga[c], m = wg * t.inv;
+            gb[c] += wg;
+            gb[3 + c] += wg * t.d1[c];
+            gb[6 + c] += wg * (c == 0 ? t.da.x : (c == 1 ? t.da.y : t.da.z));
+            gb[9 + c] += wg * t.dn.x;
+            gb[12 + c] += wg * t.dn.y;
+            gb[15 + c] += wg * t.dn.z;
+            sT[c] += m;
+            sG[c] += m * t.d1[c];
+        }
+        const float g1 = gw * t.E * t.rS;
+        sD[0] += g1 * t.df.x; sD[1] += g1 * t.df.y; sD[2] += g1 * t.df.z;
+        sV += g1 * t.D * t.rS;
+    }
+#pragma unroll
+    for (int k = 0; k < 18; ++k) gb[k] = row_sum(gb[k]);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) sD[c] = row_sum(sD[c]), sT[c] = row_sum(sT[c]), sG[c] = row_sum(sG[c]);
+    sV = row_sum(sV);
+    // the center is the Q side of the pair: minus the sums (dL/d df = -2 g1 df + gd_1 inv)
+    float gf[3], gal[3], gn[3] = {0.f, 0.f, 0.f}, gden = 0.f, gv = sV;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+        gf[c] = 2.f * sD[c] - bt[3 + c] * sT[c];
+        gal[c] = -bt[6 + c] * gb[c];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gn[k] -= bt[9 + 3 * k + c] * gb[c];
+        gden -= bt[3 + c] * sG[c];
+    }
+
+    // (b) u = M^-1 g_beta
+    float u[18];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+        float f[kFact6], x[6];
+#pragma unroll
+        for (int k = 0; k < kFact6; ++k) f[k] = F.fact[(crec * 3 + c) * kFact6 + k];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) x[k] = gb[k * 3 + c];
+        fact6_solve(f, x);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) u[k * 3 + c] = x[k];
+    }
+
+    // (c) regression adjoint, center side: with r = t - beta . d and s = u . d, gd_k = w (u_k r - beta_k s)
+    float sR[3] = {0.f, 0.f, 0.f}, sS[3] = {0.f, 0.f, 0.f}, sRi[3] = {0.f, 0.f, 0.f}, sSi[3] = {0.f, 0.f, 0.f};
+    float sRd[3] = {0.f, 0.f, 0.f}, sSd[3] = {0.f, 0.f, 0.f};
+    sD[0] = sD[1] = sD[2] = sV = 0.f;
+    for (int j = lane; j < n; j += 16)
+    {
+        const int row = (int)((uint32_t)j * magic >> 20), col = j - row * W1, i = corner + row * RW + col;
+        const float4 T = oth[i];
+        const Tap t = tap(i);
+        const float w = t.E + 1e-7f;
+        const float tv[3] = {T.x, T.y, T.z};
+        float gw = 0.f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            const float r = tv[c] - dot6(bt, c, t), s = dot6(u, c, t);
+            gw += s * r;
+            const float wr = w * r, ws = w * s, wri = wr * t.inv, wsi = ws * t.inv;
+            sR[c] += wr;
+            sS[c] += ws;
+            sRi[c] += wri;
+            sSi[c] += wsi;
+            sRd[c] += wri * t.d1[c];
+            sSd[c] += wsi * t.d1[c];
+        }
+        const float g1 = gw * t.E * t.rS;
+        sD[0] += g1 * t.df.x; sD[1] += g1 * t.df.y; sD[2] += g1 * t.df.z;
+        sV += g1 * t.D * t.rS;
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+        sR[c] = row_sum(sR[c]); sS[c] = row_sum(sS[c]); sRi[c] = row_sum(sRi[c]); sSi[c] = row_sum(sSi[c]);
+        sRd[c] = row_sum(sRd[c]); sSd[c] = row_sum(sSd[c]); sD[c] = row_sum(sD[c]);
+    }
+    gv += row_sum(sV);
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+        gf[c] += 2.f * sD[c] - (u[3 + c] * sRi[c] - bt[3 + c] * sSi[c]);
+        gal[c] -= u[6 + c] * sR[c] - bt[6 + c] * sS[c];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) gn[k] -= u[9 + 3 * k + c] * sR[c] - bt[9 + 3 * k + c] * sS[c];
+        gden -= u[3 + c] * sRd[c] - bt[3 + c] * sSd[c];
+    }
+    if (sc > 0.f) gv += 0.5f * gden / sc;
+    if (!active || lane != 0) return;
+    float *uo = F.u + crec * 18;
+#pragma unroll
+    for (int k = 0; k < 18; ++k) uo[k] = u[k];
+    float4 *go = reinterpret_cast<float4 *>(F.gcen + crec * 12);
+    go[0] = make_float4(gf[0], gf[1], gf[2], gal[0]);
+    go[1] = make_float4(gal[1], gal[2], gn[0], gn[1]);
+    go[2] = make_float4(gn[2], gv, 0.f, 0.f);
+}
+
+// 3. pixel-side and tap-side adjoints: the pairs of both loops are the same (pixel, center) pairs at the
+// same weight and delta, so one pass over the pixel's centers (records in LDS) serves both, with
+// alpha = w (g_acc - s) and rho = w r per channel, gd_k = beta_k alpha + u_k rho, r = t - pred. A tap
+// position reflected onto the pixel repeats the pair, so near an edge the regression terms are scaled
+// by how many of the pixel's positions lie in the center's window; the reconstruction leaves center
+// 0 out where its lower bound rounds up past it (EDGE tiles). 512x512, win 17: 202 -> 64 us.
+template <int MAXC>
+__global__ __launch_bounds__(256) void crg_pixel_tile(CrgBatch b)
+{
+    typedef CrgCenters<true, MAXC> Rec;
+    __shared__ float4 cs[MAXC][Rec::REC];
+    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const CrgFrame &F = b.f[L.f];
+    const int S = b.sparsity, HW = b.half_win, H = F.H, W = F.W, Ws = W / S, Hs = H / S;
+    const int x0 = L.tx * 16, y0 = L.ty * 16;
+    Rec rec;
+    rec.stage(F, cs, x0, y0, S, HW);
+    __syncthreads();
+    const int px = x0 + (threadIdx.x & 15), py = y0 + (threadIdx.x >> 4);
+    if (px >= W || py >= H) return;
+    const size_t p = (size_t)py * W + px;
+    const float3 ap = ld3(F.alb, p), np = ld3(F.nrm, p);
+    const float3 fp[2] = {ld3(F.y1, p), ld3(F.y2, p)};
+    const float vp[2] = {F.var1[p], F.var2[p]};
+    const float sp[2] = {sqrtf(vp[0]), sqrtf(vp[1])};
+    const float4 q[2] = {F.gq[p * 2], F.gq[p * 2 + 1]};
+    float gf[2][3], gt[2][3], gv[2] = {0.f, 0.f}, gden[2] = {0.f, 0.f};
+    float galb[3] = {0.f, 0.f, 0.f}, gnrm[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) gf[h][c] = gt[h][c] = 0.f;
+    // centers whose window holds the pixel
+    const int cy0 = py <= HW ? 0 : (py - HW + S - 1) / S, cy1 = min(Hs - 1, (py + HW) / S);
+    const int cx0 = px <= HW ? 0 : (px - HW + S - 1) / S, cx1 = min(Ws - 1, (px + HW) / S);
+    auto run = [&](auto edge) {
+        constexpr bool EDGE = decltype(edge)::value;
+        const int sx = EDGE ? max(0, idivup(px - HW, S)) : cx0, sy = EDGE ? max(0, idivup(py - HW, S)) : cy0;
+        for (int iy = cy0; iy <= cy1; ++iy)
+            for (int ix = cx0; ix <= cx1; ++ix)
+            {
+                const float4 *rc = cs[(iy - rec.rlo) * rec.ncx + (ix - rec.clo)];
+                const float4 A = rc[Rec::IMG + 2], N = rc[Rec::IMG + 3];
+                const float da[3] = {ap.x - A.x, ap.y - A.y, ap.z - A.z};
+                const float dn[3] = {np.x - N.x, np.y - N.y, np.z - N.z};
+                float mult = 1.f;
+                bool recon = true;
+                if constexpr (EDGE)
+                {
+                    const int cy = iy * S, cx = ix * S;
+                    const int my = 1 + (py >= 1 && py + cy <= HW) + (py <= H - 2 && 2 * (H - 1) - py - cy <= HW);
+                    const int mx = 1 + (px >= 1 && px + cx <= HW) + (px <= W - 2 && 2 * (W - 1) - px - cx <= HW);
+                    mult = (float)(my * mx);
+                    recon = iy >= sy && ix >= sx;
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                {
+                    const float *bt = reinterpret_cast<const float *>(rc) + 18 * h, *u = bt + 36;
+                    const float4 P = rc[Rec::IMG + h];
+                    const float3 tp = fp[1 - h];
+                    const float df[3] = {fp[h].x - P.x, fp[h].y - P.y, fp[h].z - P.z};
+                    const float D = df[0] * df[0] + df[1] * df[1] + df[2] * df[2];
+                    const float rS = fast_rcp((vp[h] + 1e-4f) + P.w);
+                    const float E = fast_exp2(-kLog2e * D * rS), w = E + 1e-7f;
+                    const float inv = fast_rcp((sp[h] + 1e-2f) + (h ? N.w : A.w));
+                    const float ga[3] = {recon ? q[h].x : 0.f, recon ? q[h].y : 0.f, recon ? q[h].z : 0.f};
+                    float gw = recon ? q[h].w : 0.f;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c)
+                    {
+                        const float d1 = df[c] * inv;
+                        const float pred = bt[c] + bt[3 + c] * d1 + bt[6 + c] * da[c] + bt[9 + c] * dn[0] +
+                                           bt[12 + c] * dn[1] + bt[15 + c] * dn[2];
+                        float s = u[c] + u[3 + c] * d1 + u[6 + c] * da[c] + u[9 + c] * dn[0] + u[12 + c] * dn[1] +
+                                  u[15 + c] * dn[2];
+                        float r = (c == 0 ? tp.x : (c == 1 ? tp.y : tp.z)) - pred;
+                        float wr = w * r;
+                        if constexpr (EDGE)
+                        {
+                            s *= mult;
+                            wr *= mult;
+                        }
+                        gw += ga[c] * pred + s * r;
+                        const float al = w * (ga[c] - s);
+                        const float g1 = (bt[3 + c] * al + u[3 + c] * wr) * inv;
+                        gf[h][c] += g1;
+                        gden[h] -= g1 * d1;
+                        gt[h][c] += w * s;
+                        galb[c] += bt[6 + c] * al + u[6 + c] * wr;
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) gnrm[k] += bt[9 + 3 * k + c] * al + u[9 + 3 * k + c] * wr;
+                    }
+                    const float g2 = gw * E * rS;
+#pragma unroll
+                    for (int c = 0; c < 3; ++c) gf[h][c] -= 2.f * g2 * df[c];
+                    gv[h] += g2 * D * rS;
+                }
+            }
+    };
+    if (x0 <= HW || y0 <= HW || x0 + 15 >= W - 1 - HW || y0 + 15 >= H - 1 - HW)
+        run(EdgeYes{});
+    else
+        run(EdgeNo{});
+
+    const bool grid = (px % S == 0) && (py % S == 0);
+    // 3x3 clamped neighbourhood (variance adjoint)
+    const int nx0 = max(0, px - 1), nx1 = min(W - 1, px + 1), ny0 = max(0, py - 1), ny1 = min(H - 1, py + 1);
+    const float in = 1.f / (float)((nx1 - nx0 + 1) * (ny1 - ny0 + 1) - 1);
+    float e[2][3];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+    {
+        float g = gv[h];
+        if (sp[h] > 0.f) g += 0.5f * gden[h] / sp[h];
+        // center-side terms when p is a regression center
+        if (grid)
+        {
+            const float4 *gc = reinterpret_cast<const float4 *>(F.gcen + (((size_t)(py / S) * Ws + px / S) * 2 + h) * 12);
+            const float4 g0 = gc[0], g1 = gc[1], g2 = gc[2];
+            gf[h][0] += g0.x; gf[h][1] += g0.y; gf[h][2] += g0.z;
+            galb[0] += g0.w; galb[1] += g1.x; galb[2] += g1.y;
+            gnrm[0] += g1.z; gnrm[1] += g1.w; gnrm[2] += g2.x;
+            g += g2.y;
+        }
+        // variance adjoint, own term: e = g_v * 2 (mean_neighbours - f_p)
+        const float *feat = h ? F.y2 : F.y1, *gvx = h ? F.gvarb : F.gvara;
+        if (gvx) g += gvx[p];
+        float m[3] = {0.f, 0.f, 0.f};
+        for (int yy = ny0; yy <= ny1; ++yy)
+            for (int xx = nx0; xx <= nx1; ++xx)
+            {
+                if (yy == py && xx == px) continue;
+                const float3 f = ld3(feat, (size_t)yy * W + xx);
+                m[0] += f.x; m[1] += f.y; m[2] += f.z;
+            }
+        const float fv[3] = {fp[h].x, fp[h].y, fp[h].z};
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            e[h][c] = 2.f * g * (m[c] * in - fv[c]);
+            gf[h][c] -= e[h][c];
+        }
+    }
+    // half A: features imga, target imgb; half B: features imgb, target imga
+    st3(F.gya, p, make_float3(gf[0][0] + gt[1][0], gf[0][1] + gt[1][1], gf[0][2] + gt[1][2]));
+    st3(F.gyb, p, make_float3(gf[1][0] + gt[0][0], gf[1][1] + gt[0][1], gf[1][2] + gt[0][2]));
+    st3(F.galb, p, make_float3(galb[0], galb[1], galb[2]));
+    st3(F.gnrm, p, make_float3(gnrm[0], gnrm[1], gnrm[2]));
+    float *eo = F.evar + p * 6;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) eo[3 * h + c] = e[h][c] * in;
+}
+
+// ---------------------------------------------------------------------------------------------
 // 4. per pixel: neighbour terms of the variance adjoint (the 3x3 relation is symmetric)
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void crg_var_gather(CrgBatch b)
@@ -504,11 +989,31 @@ hipError_t launch_cross_regression_grad(int n, const CrgFrame *fr, int win, int 
     b.sparsity = s;
     b.map = make_tilemap(n, tx, ty);
     if (b.map.total == 0) return hipSuccess;
-    hipLaunchKernelGGL(crg_recon_prep, dim3(b.map.total), dim3(256), 0, st, b);
+    // tiled kernels where a tile's center records (at most 64, or 200: 70 KB) and the pixels of a 4x4
+    // block of centers fit their LDS arrays: win 17 / sparsity 4 and smaller windows
+    const int HW = win / 2, axis = crg_axis_centers(s, HW), rw = (CC_T - 1) * s + 1 + 2 * HW;
+    const bool tiled = axis * axis <= 200 && rw * rw <= CC_MAXPX;
+    const bool few = axis * axis <= 64;
+    if (tiled)
+        for (int i = 0; i < n; ++i)
+        {
+            cx[i] = div_up_g(fr[i].W / s, CC_T);
+            cy[i] = div_up_g(fr[i].H / s, CC_T);
+        }
     CrgBatch bc = b;
     bc.map = make_tilemap(n, cx, cy);
-    if (bc.map.total > 0) hipLaunchKernelGGL(crg_center, dim3(bc.map.total), dim3(256), 0, st, bc);
-    hipLaunchKernelGGL(crg_pixel, dim3(b.map.total), dim3(256), 0, st, b);
+    if (tiled)
+    {
+        hipLaunchKernelGGL((few ? crg_prep_tile<64> : crg_prep_tile<200>), dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL(crg_center_tile, dim3(bc.map.total), dim3(512), 0, st, bc);
+        hipLaunchKernelGGL((few ? crg_pixel_tile<64> : crg_pixel_tile<200>), dim3(b.map.total), dim3(256), 0, st, b);
+    }
+    else
+    {
+        hipLaunchKernelGGL(crg_recon_prep, dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL(crg_center, dim3(bc.map.total), dim3(256), 0, st, bc);
+        hipLaunchKernelGGL(crg_pixel, dim3(b.map.total), dim3(256), 0, st, b);
+    }
     hipLaunchKernelGGL(crg_var_gather, dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
 }

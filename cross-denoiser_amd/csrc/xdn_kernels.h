@@ -20,6 +20,7 @@ struct CrFrame {
     float *beta;                  // [H/s][W/s][2][18]
     float *outa, *outb;           // [H/rs][W/rs][3]
     int H, W;
+    float *fact = nullptr;        // [H/s][W/s][2][3][21] Cholesky factors kept for the backward, or null
 };
 
 hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hipStream_t st);
@@ -31,6 +32,7 @@ hipError_t launch_recon(int n, const CrFrame *fr, int win, int s, int rs, hipStr
 struct CrgFrame {
     const float *y1, *y2, *alb, *nrm;
     const float *var1, *var2, *beta;     // [H][W], [H][W], [Hs][Ws][2][18]
+    const float *fact;                   // [Hs][Ws][2][3][21]
     const float *gouta, *goutb;          // [H][W][3]
     const float *gvara, *gvarb;          // [H][W] or null
     float4 *gq;                          // [H][W][2]

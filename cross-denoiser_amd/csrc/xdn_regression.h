@@ -13,9 +13,14 @@ struct Sys6 {
 
 __device__ __forceinline__ constexpr int up6(int r, int c) { return r * 6 - (r * (r - 1)) / 2 + (c - r); }
 
+// Lower triangle of a kept Cholesky factor (the diagonal holds reciprocals): (0,0) (1,0) (1,1) (2,0) ..
+__device__ __forceinline__ constexpr int lo6(int i, int j) { return i * (i + 1) / 2 + j; }
+constexpr int kFact6 = 21;
+
 // Ridge + Cholesky (cholesky_color :206-218 with the SQRT clamp :197-204) + forward/backward
-// substitution (:220-242) for one channel; all indices compile-time.
-__device__ __forceinline__ void solve6(const Sys6 &s, float beta[6])
+// substitution (:220-242) for one channel; all indices compile-time. `fact` (kFact6 floats, or null)
+// receives the factor for a later fact6_solve.
+__device__ __forceinline__ void solve6(const Sys6 &s, float beta[6], float *fact = nullptr)
 {
     float L[6][6];
 #pragma unroll
@@ -48,6 +53,32 @@ __device__ __forceinline__ void solve6(const Sys6 &s, float beta[6])
 #pragma unroll
         for (int k = 5; k > i; --k) acc += L[k][i] * beta[k];
         beta[i] = (w[i] - acc) / L[i][i];
+    }
+    if (fact)
+#pragma unroll
+        for (int i = 0; i < 6; ++i)
+#pragma unroll
+            for (int j = 0; j <= i; ++j) fact[lo6(i, j)] = i == j ? 1.f / L[i][i] : L[i][j];
+}
+
+// x -> M^-1 x for a kept factor.
+__device__ __forceinline__ void fact6_solve(const float *f, float x[6])
+{
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+    {
+        float acc = x[i];
+#pragma unroll
+        for (int k = 0; k < i; ++k) acc -= f[lo6(i, k)] * x[k];
+        x[i] = acc * f[lo6(i, i)];
+    }
+#pragma unroll
+    for (int i = 5; i >= 0; --i)
+    {
+        float acc = x[i];
+#pragma unroll
+        for (int k = 5; k > i; --k) acc -= f[lo6(k, i)] * x[k];
+        x[i] = acc * f[lo6(i, i)];
     }
 }
 

@@ -546,3 +546,19 @@ def test_spatial_filter_grad_inputs_edges(ops, dev, B, H, W, win):
         err = rel_l2(to_np(g), r)
         _report(f"spatial_filter_grad_inputs {name} {B}x{H}x{W} win={win}", err)
         assert err <= TOL, name
+
+
+@pytest.mark.parametrize("B,H,W,win,s", [(1, 20, 68, 17, 4), (2, 52, 12, 17, 4), (1, 36, 40, 27, 4), (1, 32, 24, 17, 2),
+                                         (1, 24, 20, 5, 4), (1, 17, 19, 3, 1)])
+def test_cross_regression_grad_windows(ops, dev, B, H, W, win, s):
+    """Images of a few center blocks (every pixel near an edge, partial blocks), windows whose center
+    records fit the small and the large LDS arrays, and windows too large for them."""
+    args = cr_grad_case(H, W, seed=3 * H + W, B=B)
+    cots = _cots(B, H, W, 17)
+    ref = O.cross_regression_grad(*args, *cots, win_size=win, sparsity=s)
+    got = ops.cross_regression_grad(*[to_dev(a, dev) for a in args], *[to_dev(c, dev) for c in cots],
+                                    win_size=win, sparsity=s)
+    for name, g, r in zip(("imga", "imgb", "albedo", "normal"), got, ref):
+        err = rel_l2(to_np(g), r)
+        _report(f"cross_regression_grad {name} {B}x{H}x{W} win={win} s={s}", err)
+        assert err <= CR_GRAD_TOL, name
