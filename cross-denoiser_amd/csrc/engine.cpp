@@ -195,7 +195,7 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             const int m = n - b0 < XDN_MAX_FRAMES / 2 ? n - b0 : XDN_MAX_FRAMES / 2;
             if (int e = hip_check(xdn::launch_variance(m, fr.data() + b0, 3, true, st), "variance")) return e;
         }
-        if (int e = hip_check(xdn::launch_regression(n, fr.data(), kRegWin, kSparsity, st), "regression")) return e;
+        if (int e = hip_check(xdn::launch_regression(n, fr.data(), kRegWin, kSparsity, true, st), "regression")) return e;
         if (int e = hip_check(xdn::launch_recon(n, fr.data(), kRegWin, kSparsity, 1, st), "recon")) return e;
     }
     // 2. reprojection of [out_log, ols1, ols2] of the previous frame (main.py:266, opacities one)

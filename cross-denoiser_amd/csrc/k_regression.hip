@@ -15,6 +15,8 @@
 //                      lanes that split the 17 tap columns 9/8 and are reduced with a lane swap.
 //                      61 FP32 accumulators per lane; 6x6 Cholesky per channel spread over the
 //                      lane pair. VALU-bound.
+//   regression_split   the same for launches of few blocks: the tap rows of 16 centers split over
+//                      four waves.
 //   recon_tile         fast path (win 17, sparsity 4, recon_scale 1): 16x16 pixels per
 //                      workgroup; the <= 8x8 centers the tile touches are staged in LDS (both
 //                      halves' coefficients and features), one pixel per lane, both halves.
@@ -296,6 +298,155 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
     }
 }
 
+// The same regression for launches that leave the chip idle: 16 centers of a center row per block, one
+// wave (16 centers x 2 halves x 2 tap splits) for each quarter of the tap rows, which stages its own rows
+// and loads the next one while it sums the current one. The four waves' sums meet in LDS, 21 accumulators
+// at a time, and 96 lanes solve one channel's system each. regression_rows has one wave per SIMD and 17
+// rows in a chain at 512x512 (256 blocks); the same taps are summed in another order here. 164 registers,
+// three waves per SIMD (at four waves it spills 160 B a lane and is slower at every size); three or
+// six waves of six or three rows, nine of two: slower from 360x480 on.
+constexpr int RS_CX = 16, RS_W = 4;  // centers, waves
+constexpr int RS_ROW = RS_CX * RG_S + 2 * RG_H;
+constexpr int RS_CHUNK = 21;                    // accumulators reduced at a time (3 x 21 >= 61)
+
+// The accumulators in a fixed order: the 10 shared ones, then per channel c01 .. c25 and x0 .. x5.
+constexpr int kAccShared = 10, kAccCh = 17, kAcc = kAccShared + 3 * kAccCh;
+__device__ __forceinline__ void acc_list(const RegAcc &a, float v[kAcc])
+{
+    const float sh[kAccShared] = {a.s00, a.s03, a.s04, a.s05, a.s33, a.s34, a.s35, a.s44, a.s45, a.s55};
+#pragma unroll
+    for (int k = 0; k < kAccShared; ++k) v[k] = sh[k];
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+    {
+        const float w[kAccCh] = {a.c01[c], a.c02[c], a.c11[c], a.c12[c], a.c22[c], a.c13[c], a.c14[c], a.c15[c], a.c23[c],
+                                 a.c24[c], a.c25[c], a.x0[c], a.x1[c], a.x2[c], a.x3[c], a.x4[c], a.x5[c]};
+#pragma unroll
+        for (int k = 0; k < kAccCh; ++k) v[kAccShared + c * kAccCh + k] = w[k];
+    }
+}
+
+__global__ __launch_bounds__(64 * RS_W, 3) void regression_split(RegBatch b)
+{
+    __shared__ float4 rows[RS_W][4][RS_ROW];       // one staged row per wave, planes as in regression_rows
+    __shared__ float sums[kAcc][2 * RS_CX];        // [accumulator][half * 16 + center]
+    static_assert(sizeof(rows) >= sizeof(float) * RS_W * RS_CHUNK * 2 * RS_CX, "reduction space");
+    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const RegFrame &F = b.f[L.f];
+    const int H = F.H, W = F.W, Ws = W / RG_S;
+    const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int by = L.ty, bx0 = L.tx * RS_CX;
+    const int split = lane & 1, ci = (lane >> 1) & (RS_CX - 1), half = lane >> 5;
+    const int cx = min(bx0 + ci, Ws - 1) * RG_S, cy = by * RG_S, px0 = bx0 * RG_S - RG_H;
+    const float *feat = half ? F.y2 : F.y1;
+    const size_t c = (size_t)cy * W + cx;
+    const float3 cw = ld3(feat, c), ca = ld3(F.alb, c), cn = ld3(F.nrm, c);
+    const float cvar = (half ? F.var2 : F.var1)[c];
+    const float cvar_e = cvar + 1e-4f;
+    const float cstd_e = sqrtf(cvar) + 1e-2f;
+    RegAcc acc;
+    acc.zero();
+    const int ncols = min(RS_ROW, W + 2 * RG_H - bx0 * RG_S);
+    constexpr int NS = (RS_ROW + 63) / 64;
+    float3 va[NS], vb[NS], val[NS], vn[NS];
+    float v1[NS], v2[NS];
+    auto fetch = [&](int r) {
+#pragma unroll
+        for (int u = 0; u < NS; ++u)
+        {
+            // columns past the last one needed repeat it: no branch around the loads
+            const int i = min(lane + 64 * u, ncols - 1);
+            const size_t p = (size_t)mirror(cy + r - RG_H, H) * W + mirror(px0 + i, W);
+            va[u] = ld3(F.y1, p); vb[u] = ld3(F.y2, p); val[u] = ld3(F.alb, p); vn[u] = ld3(F.nrm, p);
+            v1[u] = F.var1[p];
+            v2[u] = F.var2[p];
+        }
+    };
+    float4(*const row)[RS_ROW] = rows[wv];
+    auto commit = [&]() {
+#pragma unroll
+        for (int u = 0; u < NS; ++u)
+        {
+            const int i = lane + 64 * u;
+            if (i >= RS_ROW) continue;
+            row[0][i] = make_float4(va[u].x, va[u].y, va[u].z, v1[u]);
+            row[1][i] = make_float4(vb[u].x, vb[u].y, vb[u].z, v2[u]);
+            row[2][i] = make_float4(val[u].x, val[u].y, val[u].z, sqrtf(v1[u]));
+            row[3][i] = make_float4(vn[u].x, vn[u].y, vn[u].z, sqrtf(v2[u]));
+        }
+    };
+    const int col0 = ci * RG_S + (split ? RG_H + 1 : 0), ntap = split ? RG_H : RG_H + 1;
+    constexpr int NR = 2 * RG_H + 1;
+    const int r0 = NR * wv / RS_W, r1 = NR * (wv + 1) / RS_W;
+    fetch(r0);
+    for (int r = r0; r < r1; ++r)
+    {
+        commit();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the row is the wave's own
+        fetch(min(r + 1, r1 - 1));
+#pragma unroll
+        for (int k = 0; k < RG_H + 1; ++k)
+        {
+            if (k < ntap)
+            {
+                const int col = col0 + k;
+                const float4 P = row[half][col], T = row[1 - half][col], A = row[2][col], N = row[3][col];
+                const float3 dw = make_float3(P.x - cw.x, P.y - cw.y, P.z - cw.z);
+                const float w = reg_weight(dw, cvar_e, P.w);
+                const float inv = fast_rcp(cstd_e + (half ? N.w : A.w));
+                acc.add(w, inv, dw, make_float3(A.x - ca.x, A.y - ca.y, A.z - ca.z),
+                        make_float3(N.x - cn.x, N.y - cn.y, N.z - cn.z), make_float3(T.x, T.y, T.z));
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    // [wave][accumulator of the chunk][lane], over the staged rows
+    float *red = reinterpret_cast<float *>(&rows[0][0][0]);
+    float v[kAcc];
+    acc_list(acc, v);
+#pragma unroll
+    for (int k = 0; k < kAcc; ++k) v[k] = swap_add(v[k]);  // the two tap splits
+    constexpr int PAIRS = 2 * RS_CX;
+#pragma unroll
+    for (int k0 = 0; k0 < kAcc; k0 += RS_CHUNK)
+    {
+        __syncthreads();
+        if (!split)
+#pragma unroll
+            for (int k = 0; k < RS_CHUNK; ++k)
+                if (k0 + k < kAcc) red[(wv * RS_CHUNK + k) * PAIRS + (lane >> 1)] = v[k0 + k];
+        __syncthreads();
+        const int n = (kAcc - k0 < RS_CHUNK ? kAcc - k0 : RS_CHUNK) * PAIRS;
+        for (int e = t; e < n; e += 64 * RS_W)
+        {
+            float q[RS_W];
+#pragma unroll
+            for (int g = 0; g < RS_W; ++g) q[g] = red[g * RS_CHUNK * PAIRS + e];
+            (&sums[k0][0])[e] = (q[0] + q[1]) + (q[2] + q[3]);
+        }
+    }
+    __syncthreads();
+    // lane t < 96: channel t / 32 of (half, center) t % 32
+    const int pr = t & (PAIRS - 1), ch = t / PAIRS, sh = pr >> 4, sbx = bx0 + (pr & (RS_CX - 1));
+    if (ch >= 3 || sbx >= Ws) return;
+    Sys6 s;
+    {
+        auto g = [&](int k) { return sums[k][pr]; };
+        auto gc = [&](int k) { return sums[kAccShared + ch * kAccCh + k][pr]; };
+        const float a[21] = {g(0), gc(0), gc(1), g(1), g(2), g(3), gc(2), gc(3), gc(5), gc(6), gc(7),
+                             gc(4), gc(8), gc(9), gc(10), g(4), g(5), g(6), g(7), g(8), g(9)};
+#pragma unroll
+        for (int k = 0; k < 21; ++k) s.a[k] = a[k];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) s.x[k] = gc(11 + k);
+    }
+    const size_t rec = ((size_t)by * Ws + sbx) * 2 + sh;
+    float be[6];
+    solve6(s, be);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) F.beta[rec * 18 + k * 3 + ch] = be[k];
+}
+
 // Any window / sparsity: one lane per (center, half), direct loads.
 template <bool FACT>
 __global__ __launch_bounds__(256) void regression_generic(RegBatch b)
@@ -549,7 +700,15 @@ hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hip
     return hipGetLastError();
 }
 
-hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, hipStream_t st)
+// Up to this many blocks of regression_rows regression_split is the faster one. Whole operator, rows ->
+// split: 64 blocks (256x256) 62 -> 33 us, 256 (512x512) 70 -> 59, 540 (540x960) 118 -> 102, 900
+// (720x1280) 161 -> 175.
+constexpr int kRowsFewBlocks = 640;
+
+// batch_invariant: a frame's coefficients are the same bits whatever it is launched with, regression_rows
+// at any size: the training step, whose streams give the same results alone and batched, and the backward,
+// whose solves turn another summation order into up to 2e-5 of the normals' gradient.
+hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batch_invariant, hipStream_t st)
 {
     RegBatch b{};
     int tx[XDN_MAX_FRAMES], ty[XDN_MAX_FRAMES];
@@ -580,7 +739,17 @@ hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, hipStream
     b.sparsity = s;
     if (b.map.total == 0) return hipSuccess;
     const bool fact = fr[0].fact != nullptr;  // all frames of a call or none
-    if (fast)
+    if (fast && !batch_invariant && b.map.total <= kRowsFewBlocks)
+    {
+        for (int i = 0; i < n; ++i)
+        {
+            tx[i] = div_up(fr[i].W / s, RS_CX);
+            ty[i] = fr[i].H / s;
+        }
+        b.map = make_tilemap(n, tx, ty);
+        hipLaunchKernelGGL(regression_split, dim3(b.map.total), dim3(64 * RS_W), 0, st, b);
+    }
+    else if (fast)
         hipLaunchKernelGGL((fact ? regression_rows<true> : regression_rows<false>), dim3(b.map.total), dim3(256), 0, st, b);
     else
         hipLaunchKernelGGL((fact ? regression_generic<true> : regression_generic<false>), dim3(b.map.total), dim3(256), 0, st, b);

@@ -562,3 +562,17 @@ def test_cross_regression_grad_windows(ops, dev, B, H, W, win, s):
         err = rel_l2(to_np(g), r)
         _report(f"cross_regression_grad {name} {B}x{H}x{W} win={win} s={s}", err)
         assert err <= CR_GRAD_TOL, name
+
+
+@pytest.mark.parametrize("B,H,W", [(1, 12, 64), (1, 20, 68), (2, 36, 12), (1, 64, 260), (40, 64, 64)])
+def test_cross_regression_block_counts(ops, dev, B, H, W):
+    """The default window at sizes on both sides of the block count where the tap rows are split over
+    waves: whole and partial blocks of 16 and 64 centers, one and several center rows."""
+    ya, yb = log_images(H, W, seed=H + 2 * W, B=B)
+    args = [ya, yb, rand_img(H, W, seed=H, B=B), unit_normals(H, W, seed=W, B=B)]
+    ref = O.cross_regression(*args, 17, 4, 1)
+    got = ops.cross_regression(*[to_dev(a, dev) for a in args], win_size=17, sparsity=4)
+    for name, g, r in zip(("outa", "outb", "vara", "varb"), got, ref):
+        err = rel_l2(to_np(g), r)
+        _report(f"cross_regression {name} {B}x{H}x{W}", err)
+        assert err <= TOL, name
