@@ -305,6 +305,107 @@ __global__ __launch_bounds__(256) void sf_tile(SfBatch b)
     sf_tile_body<HALF, MODE>(b, nullptr);
 }
 
+// FWD and GRAD for launches that leave the chip idle: the window rows of a pixel are split over G threads
+// (groups of 256 threads of the block) whose sums meet in LDS, so a 16x16 tile runs 4 G waves instead of
+// a chain of 121 taps in four.
+template <int HALF, int MODE, int G>
+__global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
+{
+    static_assert(MODE == SF_FWD || MODE == SF_GRAD, "the training tile is not split");
+    constexpr int E = SF_T + 2 * HALF, NV = MODE == SF_FWD ? 8 : 5;
+    __shared__ float4 s[3][E * E];
+    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const SfFrame &F = b.f[L.f];
+    const int H = F.H, W = F.W;
+    const int x0 = L.tx * SF_T, y0 = L.ty * SF_T;
+    for (int i = threadIdx.x; i < E * E; i += 256 * G)
+    {
+        const int ly = i / E, lx = i - ly * E;
+        const int gy = mirror(min(y0 + ly - HALF, H - 1 + HALF), H), gx = mirror(min(x0 + lx - HALF, W - 1 + HALF), W);
+        const size_t p = (size_t)gy * W + gx;
+        const float3 a = ld3(F.ia, p), bb = ld3(F.ib, p), al = ld3(F.alb, p), n = ld3(F.nrm, p);
+        s[0][i] = make_float4(a.x, a.y, a.z, bb.x);
+        s[1][i] = make_float4(bb.y, bb.z, al.x, al.y);
+        s[2][i] = make_float4(al.z, n.x, n.y, n.z);
+    }
+    const int t = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int lx = t & (SF_T - 1), ly = t / SF_T;
+    const int cx = x0 + lx, cy = y0 + ly;
+    const bool live = cx < W && cy < H;
+    // lanes past the image run along on the last pixel (nothing of theirs is stored)
+    const size_t c = (size_t)min(cy, H - 1) * W + min(cx, W - 1);
+    SfCenter C;
+    sf_center_bands(C, F.band, c, HALF);
+    float3 gA = make_float3(0.f, 0.f, 0.f), gB = gA;
+    float hA = 0.f, hB = 0.f;
+    if constexpr (MODE == SF_GRAD)
+    {
+        gA = ld3(F.gaccA, c); gB = ld3(F.gaccB, c); hA = F.gwA[c]; hB = F.gwB[c];
+    }
+    __syncthreads();
+    const int q0 = (ly + HALF) * E + lx + HALF;
+    {
+        const float4 P0 = s[0][q0], P1 = s[1][q0], P2 = s[2][q0];
+        C.cA = make_float3(P0.x, P0.y, P0.z);
+        C.cB = make_float3(P0.w, P1.x, P1.y);
+        C.ca = make_float3(P1.z, P1.w, P2.x);
+        C.cn = make_float3(P2.y, P2.z, P2.w);
+    }
+    SfAcc acc;
+    sf_zero(acc);
+    constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
+    constexpr int R = 2 * HALF + 1;
+#pragma unroll 1
+    for (int dy = R * grp / G - HALF; dy < R * (grp + 1) / G - HALF; ++dy)
+    {
+        const float pdy = (float)(dy * dy) * inv_h2;
+        const float kdy = C.k4 * (float)(dy * dy);
+        const int base = q0 + dy * E;
+#pragma unroll
+        for (int dx = -HALF; dx <= HALF; ++dx)
+        {
+            const float4 P0 = s[0][base + dx], P1 = s[1][base + dx], P2 = s[2][base + dx];
+            sf_tap<MODE>(C, acc, make_float3(P0.x, P0.y, P0.z), make_float3(P0.w, P1.x, P1.y),
+                         make_float3(P1.z, P1.w, P2.x), make_float3(P2.y, P2.z, P2.w), pdy + (float)(dx * dx) * inv_h2,
+                         kdy + C.k4 * (float)(dx * dx), gA, hA, gB, hB);
+        }
+    }
+    float v[NV];
+    if constexpr (MODE == SF_FWD)
+    {
+        v[0] = acc.aA.x; v[1] = acc.aA.y; v[2] = acc.aA.z; v[3] = acc.aB.x;
+        v[4] = acc.aB.y; v[5] = acc.aB.z; v[6] = acc.sA; v[7] = acc.sB;
+    }
+    else
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] = acc.g[k];
+    __syncthreads();  // the tile is dead
+    float *red = reinterpret_cast<float *>(&s[0][0]);  // [G - 1][NV][256]
+    static_assert(sizeof(s) >= sizeof(float) * (G - 1) * NV * 256, "reduction space");
+    if (grp)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) red[((grp - 1) * NV + k) * 256 + t] = v[k];
+    __syncthreads();
+    if (grp || !live) return;
+#pragma unroll
+    for (int g = 1; g < G; ++g)
+#pragma unroll
+        for (int k = 0; k < NV; ++k) v[k] += red[((g - 1) * NV + k) * 256 + t];
+    if constexpr (MODE == SF_FWD)
+    {
+        st3(F.accA, c, make_float3(v[0], v[1], v[2]));
+        st3(F.accB, c, make_float3(v[3], v[4], v[5]));
+        F.wsA[c] = v[6];
+        F.wsB[c] = v[7];
+    }
+    else
+    {
+        float *o = F.gband + 5 * c;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) o[k] = -v[k];
+    }
+}
+
 // Five resident blocks per CU (32.5 KB of LDS each): 96 VGPRs instead of 106. The epilogue is kept
 // lean for it (see train_epilogue); one 8-byte value is still spilled there, none in the tap loop.
 template <int HALF>
@@ -570,12 +671,26 @@ static SfBatch sf_batch(int n, const SfFrame *fr, int win)
     return b;
 }
 
+// The splits by tiles of the launch, measured forward / band gradient in us a call: 256 tiles, one thread
+// 15.4 / 17.5, two 12.2 / 13.1, four 11.5 / 12.4; 480 tiles 20.0 / 21.4, 18.8 / 21.3, 20.9 / 22.5; from
+// 700 tiles on one thread is as fast as two, four are slower (1024 tiles: 32.8, 33.3, 40.0).
+template <int MODE>
+static void sf_launch(const SfBatch &b, hipStream_t st)
+{
+    if (b.map.total <= 256)
+        hipLaunchKernelGGL((sf_tile_split<5, MODE, 4>), dim3(b.map.total), dim3(1024), 0, st, b);
+    else if (b.map.total <= 512)
+        hipLaunchKernelGGL((sf_tile_split<5, MODE, 2>), dim3(b.map.total), dim3(512), 0, st, b);
+    else
+        hipLaunchKernelGGL((sf_tile<5, MODE>), dim3(b.map.total), dim3(256), 0, st, b);
+}
+
 hipError_t launch_sf_forward(int n, const SfFrame *fr, int win, hipStream_t st)
 {
     SfBatch b = sf_batch(n, fr, win);
     if (b.map.total == 0) return hipSuccess;
     if (b.half == 5)
-        hipLaunchKernelGGL((sf_tile<5, SF_FWD>), dim3(b.map.total), dim3(256), 0, st, b);
+        sf_launch<SF_FWD>(b, st);
     else
         hipLaunchKernelGGL((sf_generic<SF_FWD>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
@@ -586,7 +701,7 @@ hipError_t launch_sf_grad_band(int n, const SfFrame *fr, int win, hipStream_t st
     SfBatch b = sf_batch(n, fr, win);
     if (b.map.total == 0) return hipSuccess;
     if (b.half == 5)
-        hipLaunchKernelGGL((sf_tile<5, SF_GRAD>), dim3(b.map.total), dim3(256), 0, st, b);
+        sf_launch<SF_GRAD>(b, st);
     else
         hipLaunchKernelGGL((sf_generic<SF_GRAD>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
