@@ -95,8 +95,14 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+def raw_stream(index: int) -> int:
+    """hipStream_t of the current stream of GPU `index`. Every operator call asks for it; without the
+    torch.cuda.Stream object that takes 0.2 instead of 2.1 us."""
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return raw_stream(t.get_device())
 
 
 def version() -> str:

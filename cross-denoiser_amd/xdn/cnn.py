@@ -19,7 +19,7 @@ import math
 
 import torch
 
-from ._lib import check, lib, ptr
+from ._lib import check, lib, ptr, raw_stream
 
 CNN5_CHANNELS = (15, 32, 32, 32, 32, 6)
 
@@ -118,7 +118,7 @@ class _HipNet:
         self._inputs = None
 
     def _stream(self):
-        return torch.cuda.current_stream(self.device).cuda_stream
+        return raw_stream(self.params.get_device())
 
     def pack(self):
         check(self._fn("pack")(ptr(self.params), ptr(self.packed), self._stream()), f"{self.name} pack")

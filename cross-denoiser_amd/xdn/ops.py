@@ -37,6 +37,10 @@ __all__ = [
 
 
 def _img(t: torch.Tensor, name: str, channels: int | None = None) -> torch.Tensor:
+    if isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is torch.float32:
+        shape = t.shape
+        if len(shape) == 4 and (channels is None or shape[3] == channels):
+            return t.contiguous()
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.device.type != "cuda":
@@ -45,26 +49,25 @@ def _img(t: torch.Tensor, name: str, channels: int | None = None) -> torch.Tenso
         raise TypeError(f"{name} must be float32 (got {t.dtype})")
     if t.dim() != 4:
         raise ValueError(f"{name} must be NHWC rank 4 (got shape {tuple(t.shape)})")
-    if channels is not None and t.shape[3] != channels:
-        raise ValueError(f"{name} must have {channels} channels (got {t.shape[3]})")
-    return t.contiguous()
+    raise ValueError(f"{name} must have {channels} channels (got {t.shape[3]})")
 
 
 def _same_hw(ref: torch.Tensor, *ts) -> None:
+    bhw = ref.shape[:3]
     for name, t in ts:
-        if t.shape[:3] != ref.shape[:3]:
-            raise ValueError(f"{name} has shape {tuple(t.shape)}, expected [B,H,W] = {tuple(ref.shape[:3])}")
+        if t.shape[:3] != bhw:
+            raise ValueError(f"{name} has shape {tuple(t.shape)}, expected [B,H,W] = {tuple(bhw)}")
 
 
 # ---------------------------------------------------------------------------------------------
 def _cr_forward(imga, imgb, albedo, normal, win_size, sparsity, rs):
     B, H, W, C = imga.shape
-    outa = torch.empty((B, H // rs, W // rs, C), device=imga.device, dtype=torch.float32)
+    outa = imga.new_empty((B, H // rs, W // rs, C))
     outb = torch.empty_like(outa)
-    vara = torch.empty((B, H, W, 1), device=imga.device, dtype=torch.float32)
+    vara = imga.new_empty((B, H, W, 1))
     varb = torch.empty_like(vara)
     ws_bytes = lib.xdn_cross_regression_workspace_size(B, H, W, int(sparsity))
-    ws = torch.empty(max(ws_bytes, 4) // 4, device=imga.device, dtype=torch.float32)
+    ws = imga.new_empty(max(ws_bytes, 4) // 4)
     check(lib.xdn_cross_regression(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(outa), ptr(outb),
                                    ptr(vara), ptr(varb), ptr(ws), ws_bytes, B, H, W, int(win_size),
                                    int(sparsity), rs, stream_of(imga)), "cross_regression")
@@ -123,7 +126,7 @@ def cross_regression_grad(imga, imgb, albedo, normal, grad_outa, grad_outb, grad
     _same_hw(imga, ("imgb", imgb), ("albedo", albedo), ("normal", normal), ("grad_outa", ga), ("grad_outb", gb))
     outs = [torch.empty_like(imga) for _ in range(4)]
     ws_bytes = lib.xdn_cross_regression_grad_workspace_size(B, H, W, int(sparsity))
-    ws = torch.empty(max(ws_bytes, 4) // 4, device=imga.device, dtype=torch.float32)
+    ws = imga.new_empty(max(ws_bytes, 4) // 4)
     check(lib.xdn_cross_regression_grad(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(ga), ptr(gb), ptr(gva),
                                         ptr(gvb), *[ptr(o) for o in outs], ptr(ws), ws_bytes, B, H, W, int(win_size),
                                         int(sparsity), stream_of(imga)), "cross_regression_grad")
@@ -141,10 +144,10 @@ def cross_regression_from_color(color, color2, albedo, normal, win_size, sparsit
     B, H, W, _ = color.shape
     y1, y2 = torch.empty_like(color), torch.empty_like(color)
     outa, outb = torch.empty_like(color), torch.empty_like(color)
-    vara = torch.empty((B, H, W, 1), device=color.device, dtype=torch.float32)
+    vara = color.new_empty((B, H, W, 1))
     varb = torch.empty_like(vara)
     ws_bytes = lib.xdn_cross_regression_workspace_size(B, H, W, int(sparsity))
-    ws = torch.empty(max(ws_bytes, 4) // 4, device=color.device, dtype=torch.float32)
+    ws = color.new_empty(max(ws_bytes, 4) // 4)
     check(lib.xdn_cross_regression_from_color(ptr(color), ptr(color2), ptr(albedo), ptr(normal), ptr(y1), ptr(y2),
                                               ptr(outa), ptr(outb), ptr(vara), ptr(varb), ptr(ws), ws_bytes, B, H,
                                               W, int(win_size), int(sparsity), stream_of(color)),
@@ -156,7 +159,7 @@ def cross_regression_from_color(color, color2, albedo, normal, win_size, sparsit
 def _sf_forward(imga, imgb, albedo, normal, band, win_size):
     B, H, W, _ = imga.shape
     acca, accb = torch.empty_like(imga), torch.empty_like(imgb)
-    wa = torch.empty((B, H, W, 1), device=imga.device, dtype=torch.float32)
+    wa = imga.new_empty((B, H, W, 1))
     wb = torch.empty_like(wa)
     check(lib.xdn_spatial_filter(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(band), ptr(acca), ptr(accb),
                                  ptr(wa), ptr(wb), B, H, W, int(win_size), stream_of(imga)), "spatial_filter")
@@ -244,7 +247,7 @@ def temporal_screening(current1, current2, prev, prev1, prev2, reproj_success, w
     _same_hw(c1, ("current2", c2), ("prev", p), ("prev1", p1), ("prev2", p2), ("reproj_success", rs))
     B, H, W, _ = c1.shape
     o, o1, o2 = torch.empty_like(c1), torch.empty_like(c1), torch.empty_like(c1)
-    s = torch.empty((B, H, W, 1), device=c1.device, dtype=torch.float32)
+    s = c1.new_empty((B, H, W, 1))
     check(lib.xdn_temporal_screening(ptr(c1), ptr(c2), ptr(p), ptr(p1), ptr(p2), ptr(rs), ptr(o), ptr(o1), ptr(o2),
                                      ptr(s), B, H, W, int(win_curr), int(win_prev), stream_of(c1)),
           "temporal_screening")
@@ -263,7 +266,7 @@ def erode_temporal_screening(current1, current2, prev, prev1, prev2, success_mas
         raise ValueError("success_mask must be a [B,H,W,1] bool/uint8 tensor")
     B, H, W, _ = c1.shape
     o, o1, o2 = torch.empty_like(c1), torch.empty_like(c1), torch.empty_like(c1)
-    s = torch.empty((B, H, W, 1), device=c1.device, dtype=torch.float32)
+    s = c1.new_empty((B, H, W, 1))
     e = torch.empty_like(s)
     check(lib.xdn_erode_temporal_screening(ptr(c1), ptr(c2), ptr(p), ptr(p1), ptr(p2), ptr(m), ptr(e), ptr(o),
                                            ptr(o1), ptr(o2), ptr(s), B, H, W, int(win_curr), int(win_prev),

@@ -22,7 +22,7 @@ import ctypes
 import torch
 
 from . import cnn as cnn_mod
-from ._lib import check, lib, ptr
+from ._lib import check, lib, ptr, raw_stream, stream_of
 
 REGRESSION_WIDTH = 17   # scripts/main.py:71-74
 FILTER_WIDTH = 11
@@ -64,7 +64,7 @@ def filter_train(ols1, ols2, albedo, normal, param, success, success_prev, prev_
     ws_bytes = lib.xdn_filter_train_workspace_size(B, H, W)
     ws = torch.empty(max(ws_bytes, 4) // 4, device=dev, dtype=torch.float32)
     check(lib.xdn_filter_train(*[ptr(t) for t in ts], ptr(out_log), ptr(out), ptr(dparam), ptr(loss), ptr(avg),
-                               ptr(ws), ws_bytes, B, H, W, win_size, torch.cuda.current_stream(dev).cuda_stream),
+                               ptr(ws), ws_bytes, B, H, W, win_size, stream_of(ts[0])),
           "filter_train")
     return out_log, out, loss, avg, dparam
 
@@ -116,7 +116,7 @@ class Denoiser:
         check(lib.xdn_slot_init(ctypes.addressof(slot), self._stream()), "slot init")
 
     def _stream(self):
-        return torch.cuda.current_stream(self.device).cuda_stream
+        return raw_stream(self.params.get_device())
 
     def buffer(self, name: str, channels: int, dtype=torch.float32) -> torch.Tensor:
         """View of an intermediate of the last step inside the slot scratch (see SLOT_BUFFERS)."""
