@@ -72,12 +72,12 @@ struct Cnn5Layout {
 inline const Cnn5Layout kLay;
 
 // Workspace of cnn5 for B images of H x W: hidden activations, gradient ping-pong, and per layer
-// the weight-gradient partials of every block and the reduction stage (all five layers are reduced
-// together after the backward pass). The backward takes each ReLU derivative from the activation
+// the weight-gradient partials of every block (all five layers are reduced together after the backward
+// pass). The backward takes each ReLU derivative from the activation
 // itself (x > 0), so no mask is stored.
 struct Cnn5Ws {
     uint16_t *X[4], *dY[2];
-    float *part[5], *stage[5];
+    float *part[5];
     int nblk[5];     // weight-gradient blocks (partials) per image and layer
     int pstride[5];  // floats per partial (the first and last layers' partials are compact)
     size_t bytes;
@@ -96,8 +96,6 @@ struct Cnn5Ws {
             pstride[l] = l == 0 ? xdn::WG_PART_L1 : (l == 4 ? xdn::WG_PART_L5 : xdn::WG_PART);
             part[l] = reinterpret_cast<float *>(p + o);
             o += al256((size_t)B * nblk[l] * pstride[l] * 4);
-            stage[l] = reinterpret_cast<float *>(p + o);
-            o += al256((size_t)xdn::WG_SPLITS * pstride[l] * 4);
         }
         bytes = o;
     }
@@ -107,7 +105,7 @@ struct Cnn5Ws {
 // its flat gradient at grad + the layer's weight offset.
 inline xdn::RedJob cnn5_red_job(const Cnn5Ws &ws, int l, float *grad, int nblk_total)
 {
-    xdn::RedJob r{ws.part[l], ws.stage[l], grad + kLay.w_off[l], nblk_total, kCnn5[l].ci, kCnn5[l].co};
+    xdn::RedJob r{ws.part[l], grad + kLay.w_off[l], nblk_total, kCnn5[l].ci, kCnn5[l].co};
     if (l == 0 || l == 4)
     {
         r.compact = 1;
@@ -239,7 +237,7 @@ inline int unet_job_blocks(int job, int h, int w)
 struct UnetWs {
     char *buf[UNET_BUFS];
     size_t off[UNET_BUFS], frame_bytes[UNET_BUFS];
-    float *part[UNET_JOBS], *stage[UNET_JOBS];
+    float *part[UNET_JOBS];
     int nblk[UNET_JOBS];
     int h[3], w[3];
     size_t bytes;
@@ -262,8 +260,6 @@ struct UnetWs {
             nblk[j] = unet_job_blocks(j, h[lv], w[lv]);
             part[j] = reinterpret_cast<float *>(p + o);
             o += al256((size_t)B * nblk[j] * unet_job_pstride(j) * 4);
-            stage[j] = reinterpret_cast<float *>(p + o);
-            o += al256((size_t)xdn::WG_SPLITS * unet_job_pstride(j) * 4);
         }
         bytes = o;
     }
@@ -288,7 +284,7 @@ int unet_forward_frames(const UnetFrame *f, int n, hipStream_t st);
 // the backward pass up to the weight-gradient partials (reduced by the caller's jobs)
 int unet_backward_frames(const UnetFrame *f, int n, hipStream_t st);
 // reduction job of partial set `set` (nblk_total partials from part) into the flat gradient
-xdn::RedJob unet_red_job(int set, float *part, float *stage, float *grad, int nblk_total);
+xdn::RedJob unet_red_job(int set, float *part, float *grad, int nblk_total);
 // pack jobs of one parameter vector (3x3 fragments and FP32 copies of the 1x1 layers)
 void unet_pack_jobs(const float *params, void *packed, std::vector<xdn::UPackJob> &jobs);
 

@@ -241,13 +241,12 @@ int unet_backward_frames(const UnetFrame *F, int n, hipStream_t st)
     return wgrad(F, n, st, UW_0, 0, -1, -1, UB_DY0);                             // c1_1
 }
 
-xdn::RedJob unet_red_job(int set, float *part, float *stage, float *grad, int nblk_total)
+xdn::RedJob unet_red_job(int set, float *part, float *grad, int nblk_total)
 {
     const int l = kUnetJob[set].layer;
     const UnetLayer &L = kUnet[l];
     xdn::RedJob r;
     r.part = part;
-    r.stage = stage;
     r.grad = grad + kULay.w_off[l];
     r.nblk = nblk_total;
     r.ci = L.ci;
@@ -376,7 +375,7 @@ int xdn_unet_backward(const float *ols1, const float *ols2, const float *prev_ou
     if (int e = unet_backward_frames(F.data(), batch, S(stream))) return e;
     // the B images' partials of each set are contiguous: one job sums them into the one gradient
     std::vector<xdn::RedJob> jobs;
-    for (int j = 0; j < UNET_JOBS; ++j) jobs.push_back(unet_red_job(j, ws.part[j], ws.stage[j], grad, batch * ws.nblk[j]));
+    for (int j = 0; j < UNET_JOBS; ++j) jobs.push_back(unet_red_job(j, ws.part[j], grad, batch * ws.nblk[j]));
     return hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), S(stream)), "unet wgrad reduce");
 }
 

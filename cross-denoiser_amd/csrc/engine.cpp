@@ -6,8 +6,8 @@
 // as one: cross-regression (3), reprojection, erosion + screening, network forward (cnn5: layer 1,
 // then layers 2-5 in one row-streaming launch; the U-Net: 14 launches), fused filter + loss + backward, loss sums, network
 // backward (cnn5: 5 launches, the weight and data gradients of layers 2-5 fused; the
-// U-Net: 23 launches), one pair of
-// weight-gradient reductions, Adam, pack.
+// U-Net: 23 launches), one
+// weight-gradient reduction, Adam, pack.
 // Every slot owns its history, network, Adam moments and scratch; nothing is shared.
 #include <math.h>
 
@@ -297,14 +297,14 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
     // 6. network backward: layers 5..3 each in one fused launch (weight gradient and data gradient
     //    into the layer below), then layer 2's backward fused with layer 1's weight gradient (layer
     //    1's pre-activation gradient stays on chip); the per-block weight-gradient partials of every
-    //    (slot, layer) are reduced by one launch pair
+    //    (slot, layer) are reduced by one launch
     if (unet)
     {
         if (int e = unet_backward_frames(uf.data(), n, st)) return e;
         std::vector<xdn::RedJob> jobs;
         for (int i = 0; i < n; ++i)
             for (int j = 0; j < UNET_JOBS; ++j)
-                jobs.push_back(unet_red_job(j, uw[i].part[j], uw[i].stage[j], slots[i].grad, uw[i].nblk[j]));
+                jobs.push_back(unet_red_job(j, uw[i].part[j], slots[i].grad, uw[i].nblk[j]));
         if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st), "unet wgrad reduce")) return e;
     }
     else

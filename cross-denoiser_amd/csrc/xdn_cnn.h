@@ -8,7 +8,6 @@
 namespace xdn {
 
 constexpr int WG_PART = 9 * 1024 + 32;  // one block's partial: [9][32][32] weights + [32] bias
-constexpr int WG_SPLITS = 32;
 
 // Layer 1 forward: the five FP32 3-channel images -> bf16 32 channels, bias + ReLU.
 struct ConvFrame {
@@ -70,7 +69,6 @@ hipError_t launch_conv_l1(int n, const ConvFrame *fr, hipStream_t st);
 // [taps][ci][co] (or [co][ci] when transpose, taps 1) followed by [co] when bias.
 struct RedJob {
     const float *part;  // [nblk][pstride]
-    float *stage;       // [WG_SPLITS][pstride]
     float *grad;        // the layer's weights, then its bias
     int nblk, ci, co;
     int taps = 9, ci_off = 0, ci_cnt = -1, bias = 1, transpose = 0;
@@ -81,7 +79,7 @@ constexpr int compact_part(int taps, int cc, int co) { return taps * cc * co + c
 // the first layer's (15 -> 32) and the last layer's (32 -> 6) partials are compact
 constexpr int WG_PART_L1 = compact_part(9, 15, 32);
 constexpr int WG_PART_L5 = compact_part(9, 32, 6);
-constexpr int WG_MAX_JOBS = 48;  // per launch; longer job lists are split
+constexpr int WG_MAX_JOBS = 56;  // per launch; longer job lists are split
 hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st);
 hipError_t launch_pack(int n, const PackJob *jobs, hipStream_t st);
 // last: the network's last layer (dy = the FP32 6-channel gradient of the output, L5 fragments)
