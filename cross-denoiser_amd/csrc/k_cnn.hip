@@ -1152,13 +1152,13 @@ __global__ __launch_bounds__(512, 1) void conv3x3_bwd12(Bwd12Batch b)
 
 // Deterministic reduction of the per-block partials, batched over jobs (a job is one layer of one
 // frame): a block owns 32 entries of one job's flat gradient ([taps][ci][co] then [co], unpadded), eight
-// threads an entry. Thread g sums the partials g, g + 8, ... with 16 loads in flight, and the eight sums
-// meet in LDS in a fixed order. The grid holds each job's own blocks and nothing else. Bound by the
-// partials' bytes: 8.9 us for cnn5 at 717x1283 (35 MB), 16.1 us for the U-Net's 13 jobs at 1920x1080
-// (64 MB; sixteen threads an entry, or 64 entries a block: the same). Two launches with a staging buffer
-// and a grid of jobs x largest job x 32 splits took 8.5 + 9.6 and 15.6 + 9.6 us, and 18.7 + 10.2 + 10.2
-// for the 52 jobs of four 256x256 frames, now 9.9.
-constexpr int RED_E = 32, RED_G = 8;
+// threads an entry. The partials are summed in 32 contiguous splits, four to a thread, each in order with
+// its loads in flight eight at a time, and the splits' sums, in LDS, in order: one fixed order
+// whatever the launch. The grid holds each job's own blocks and nothing else. Bound by the partials'
+// bytes: 8.8 us for cnn5 at 717x1283 (35 MB), 16.7 us for the U-Net's 13 jobs at 1920x1080 (64 MB). Two
+// launches with a staging buffer and a grid of jobs x largest job x 32 splits took 8.5 + 9.6 and
+// 15.6 + 9.6 us, and 18.7 + 10.2 + 10.2 for the 52 jobs of four 256x256 frames, now 11.5.
+constexpr int RED_E = 32, RED_G = 8, RED_SPLITS = 32;
 struct RedBatch {
     int n;
     int begin[WG_MAX_JOBS + 1];  // first block of each job
@@ -1173,7 +1173,7 @@ __host__ __device__ inline int red_entries(const RedJob &J)
 
 __global__ __launch_bounds__(RED_E *RED_G) void wgrad_reduce(RedBatch b)
 {
-    __shared__ float red[RED_G][RED_E];
+    __shared__ float red[RED_SPLITS][RED_E];
     int lo = 0, hi = b.n - 1;  // the job whose blocks hold this one
     while (lo < hi)
     {
@@ -1203,38 +1203,31 @@ __global__ __launch_bounds__(RED_E *RED_G) void wgrad_reduce(RedBatch b)
     }
     // lanes past the last entry read entry 0's partials (their sum is not stored)
     const float *p = J.part + src;
-    const size_t step = (size_t)RED_G * J.pstride;
     const int nb = J.nblk;
-    constexpr int U = 16;
-    float s = 0.f;
-    int i = g;
-    p += (size_t)g * J.pstride;
-    for (; i + RED_G * (U - 1) < nb; i += RED_G * U, p += U * step)
+    constexpr int SPT = RED_SPLITS / RED_G, U = 8;  // splits a thread, loads in flight
+#pragma unroll
+    for (int k = 0; k < SPT; ++k)
     {
-        float v[U];
+        const int sp = g * SPT + k;
+        const int i0 = (int)((long)nb * sp / RED_SPLITS), i1 = (int)((long)nb * (sp + 1) / RED_SPLITS);
+        float s = 0.f;
+        for (int i = i0; i < i1; i += U)
+        {
+            float v[U];
 #pragma unroll
-        for (int k = 0; k < U; ++k) v[k] = p[k * step];
+            for (int j = 0; j < U; ++j) v[j] = i + j < i1 ? p[(size_t)(i + j) * J.pstride] : 0.f;
 #pragma unroll
-        for (int k = 0; k < U; ++k) s += v[k];
+            for (int j = 0; j < U; ++j)
+                if (i + j < i1) s += v[j];
+        }
+        red[sp][el] = s;
     }
-    {
-        float v[U];
-#pragma unroll
-        for (int k = 0; k < U; ++k) v[k] = i + RED_G * k < nb ? p[k * step] : 0.f;
-#pragma unroll
-        for (int k = 0; k < U; ++k) s += v[k];
-    }
-    red[g][el] = s;
     __syncthreads();
     if (g != 0 || e >= ne) return;
-    float r[RED_G];
+    float s = 0.f;
 #pragma unroll
-    for (int k = 0; k < RED_G; ++k) r[k] = red[k][el];
-#pragma unroll
-    for (int h = RED_G / 2; h > 0; h >>= 1)
-#pragma unroll
-        for (int k = 0; k < h; ++k) r[k] += r[k + h];
-    J.grad[dst] = r[0];
+    for (int k = 0; k < RED_SPLITS; ++k) s += red[k][el];
+    J.grad[dst] = s;
 }
 
 // ---------------------------------------------------------------------------------------------
