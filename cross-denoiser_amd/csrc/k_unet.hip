@@ -54,6 +54,26 @@ __device__ __forceinline__ uint32_t u_keep(uint32_t mw, uint32_t vw)
 }
 __device__ __forceinline__ float u_bf(const uint16_t *p, int i) { return __uint_as_float((uint32_t)p[i] << 16); }
 
+// Sum over the 64 lanes in every lane, pairing lanes 32, 16, 8, 4, 2 and 1 apart: lane swaps and DPP row
+// rotations (after each sum the values repeat with that period, so a rotation meets the same partner)
+// instead of six LDS permutes, with the sums of a __shfl_xor tree bit for bit (54 sums of head_bwd, 32 of
+// convT_bwd<32>: 1 us of a block each).
+template <int R>
+__device__ __forceinline__ float u_ror_add(float v)
+{
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + R, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float u_wave_sum(float v)
+{
+    const uint32_t a = __float_as_uint(v);
+    const auto s32 = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+    v = __uint_as_float((uint32_t)s32[0]) + __uint_as_float((uint32_t)s32[1]);
+    const uint32_t b = __float_as_uint(v);
+    const auto s16 = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    v = __uint_as_float((uint32_t)s16[0]) + __uint_as_float((uint32_t)s16[1]);
+    return u_ror_add<1>(u_ror_add<2>(u_ror_add<4>(u_ror_add<8>(v))));
+}
+
 static int udiv_up(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------------------------
@@ -841,7 +861,7 @@ hipError_t launch_pool_bwd(int C, int n, const PoolBwFrame *fr, hipStream_t st)
 // Transposed 1x1 stride-2 convolution
 // ---------------------------------------------------------------------------------------------
 struct CtBatch {
-    int n;
+    int n, gpw;  // gpw: 32-pixel groups per wave (forward)
     int blk_begin[XDN_MAX_FRAMES + 1];
     CtFrame f[XDN_MAX_FRAMES];
 };
@@ -858,11 +878,10 @@ __global__ __launch_bounds__(256) void convT1x1s2(CtBatch b)
 {
     constexpr int NI = C == 32 ? 16 : 8;  // accumulator rows holding output channels
     constexpr int NG = NI / 8;            // 16-B stores per output pixel and lane
-    constexpr int GPW = 4;                // 32-pixel groups per wave
     int f = 0;
     while (f + 1 < b.n && (int)blockIdx.x >= b.blk_begin[f + 1]) ++f;
     const CtFrame &F = b.f[f];
-    const int li = blockIdx.x - b.blk_begin[f];
+    const int li = blockIdx.x - b.blk_begin[f], GPW = b.gpw;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, px = lane & 31, h = lane >> 5;
     const int w = F.w_, np = F.h * w, W2 = 2 * w;
     // A operand of step s: W[co = px][ci = 2s + h]; the bias of the lane's outputs
@@ -1132,8 +1151,7 @@ __global__ __launch_bounds__(256) void convT_bwd(CtBatch b)
     }
     // bias sums: wave reduction in a fixed order, then the four waves
 #pragma unroll
-    for (int c = 0; c < C; ++c)
-        for (int off = 32; off > 0; off >>= 1) bacc[c] += __shfl_down(bacc[c], off);
+    for (int c = 0; c < C; ++c) bacc[c] = u_wave_sum(bacc[c]);
     // accumulators: C[row = ci][col = co]
 #pragma unroll
     for (int k = 0; k < (C == 32 ? 16 : 4); ++k)
@@ -1157,11 +1175,20 @@ static hipError_t convT_t(int n, const CtFrame *fr, hipStream_t st)
     CtBatch b{};
     b.n = n;
     int acc = 0;
+    if (!BWD)
+    {
+        // Pixel groups per wave (a wave loads the weights once): four where that leaves 192 blocks,
+        // fewer below. 254 blocks at four (C = 32, 1920x1080): 14.2 us, 15.4 at two, 18.8 at one; 128
+        // (C = 16, four 256x256 images): 8.2, 6.5, 6.6; 32 (C = 32): 12.0, 8.4, 6.6.
+        long np = 0;
+        for (int i = 0; i < n; ++i) np += (long)fr[i].h * fr[i].w_;
+        for (b.gpw = 4; b.gpw > 1 && np < (long)192 * b.gpw * 4 * 32; b.gpw >>= 1) {}
+    }
     for (int i = 0; i < n; ++i)
     {
         b.f[i] = fr[i];
         b.blk_begin[i] = acc;
-        acc += BWD ? fr[i].nblk : udiv_up(fr[i].h * fr[i].w_, 4 * 4 * 32);
+        acc += BWD ? fr[i].nblk : udiv_up(fr[i].h * fr[i].w_, b.gpw * 4 * 32);
     }
     b.blk_begin[n] = acc;
     if (acc == 0) return hipSuccess;
@@ -1214,41 +1241,55 @@ __global__ __launch_bounds__(256) void head_bwd(HeadBatch b)
     float g[54];
 #pragma unroll
     for (int e = 0; e < 54; ++e) g[e] = 0.f;
-    for (int p = li * 256 + tid; p < np; p += nblk * 256)
+    // The loads of four pixels are in flight together; each thread sums its pixels in order. At the
+    // HBM floor for 1920x1080 (116 MB, 27.7 -> 22.9 us); four 256x256 images: a chain of 16 pixels
+    // a thread in 64 blocks, 15.8 -> 10.7 us.
+    constexpr int U = 4;
+    const int step = nblk * 256;
+    for (int p0 = li * 256 + tid; p0 < np; p0 += U * step)
     {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(F.in + (size_t)p * 8);
-        const float in[8] = {u_lo(v.x), u_hi(v.x), u_lo(v.y), u_hi(v.y), u_lo(v.z), u_hi(v.z), u_lo(v.w), u_hi(v.w)};
-        float dp[6];
+        u32x4 v[U];
+        float d[U][6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) dp[k] = F.dparam[(size_t)p * 6 + k];
-        uint32_t o[4];
-#pragma unroll
-        for (int c = 0; c < 8; c += 2)
+        for (int u = 0; u < U; ++u)
         {
-            float s0 = 0.f, s1 = 0.f;
+            const int p = p0 + u * step < np ? p0 + u * step : p0;
+            v[u] = *reinterpret_cast<const u32x4 *>(F.in + (size_t)p * 8);
 #pragma unroll
-            for (int k = 0; k < 6; ++k)
-            {
-                s0 += w[c * 6 + k] * dp[k];
-                s1 += w[(c + 1) * 6 + k] * dp[k];
-            }
-            o[c / 2] = u_pack2(in[c] > 0.f ? s0 : 0.f, in[c + 1] > 0.f ? s1 : 0.f);
+            for (int k = 0; k < 6; ++k) d[u][k] = F.dparam[(size_t)p * 6 + k];
         }
-        *reinterpret_cast<u32x4 *>(F.din + (size_t)p * 8) = u32x4{o[0], o[1], o[2], o[3]};
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
+        for (int u = 0; u < U; ++u)
+        {
+            const int p = p0 + u * step;
+            if (p >= np) break;
+            const float in[8] = {u_lo(v[u].x), u_hi(v[u].x), u_lo(v[u].y), u_hi(v[u].y),
+                                 u_lo(v[u].z), u_hi(v[u].z), u_lo(v[u].w), u_hi(v[u].w)};
+            const float(&dp)[6] = d[u];
+            uint32_t o[4];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) g[c * 6 + k] += in[c] * dp[k];
+            for (int c = 0; c < 8; c += 2)
+            {
+                float s0 = 0.f, s1 = 0.f;
 #pragma unroll
-        for (int k = 0; k < 6; ++k) g[48 + k] += dp[k];
+                for (int k = 0; k < 6; ++k)
+                {
+                    s0 += w[c * 6 + k] * dp[k];
+                    s1 += w[(c + 1) * 6 + k] * dp[k];
+                }
+                o[c / 2] = u_pack2(in[c] > 0.f ? s0 : 0.f, in[c + 1] > 0.f ? s1 : 0.f);
+            }
+            *reinterpret_cast<u32x4 *>(F.din + (size_t)p * 8) = u32x4{o[0], o[1], o[2], o[3]};
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+#pragma unroll
+                for (int k = 0; k < 6; ++k) g[c * 6 + k] += in[c] * dp[k];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) g[48 + k] += dp[k];
+        }
     }
 #pragma unroll
-    for (int e = 0; e < 54; ++e)
-    {
-        float v = g[e];
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-        g[e] = v;
-    }
+    for (int e = 0; e < 54; ++e) g[e] = u_wave_sum(g[e]);
     if ((tid & 63) == 0)
 #pragma unroll
         for (int e = 0; e < 54; ++e) red[tid >> 6][e] = g[e];
