@@ -6,7 +6,7 @@
 //     every B fragment feeds up to three output rows. Forward
 //     (bias + ReLU -> bf16) and data gradient (flipped, transposed fragments; ReLU-masked, or
 //     plain for concat and pooled inputs). Channel counts are the stored ones (8, 16, 24, 32, 48).
-//   uwgrad<SRC, CA, CB, CO, MT>  weight gradient over 8x32-px strips, operands from pixel-major
+//   uwgrad<SRC, CA, CB, CO, MT, DEPTH>  weight gradient over 8x32-px strips, operands from pixel-major
 //     LDS tiles through ds_read_b64_tr_b16, one 32-channel input slice (MT) per instantiation,
 //     software-pipelined strip loop.
 //   maxpool2 / pool_bwd          2x2 max pool and its gradient (to the first maximum, plus the
@@ -115,8 +115,9 @@ __device__ __forceinline__ uint32_t u_cvt2(float a, float b)
 // the tile went back through LDS in 2-byte writes. Only the CI real channels are staged, in pixels of
 // an odd number of 16-B units (conflict-free b128 reads); the upper half of an odd last K chunk is
 // masked to zero as it is read. Bound by HBM at 8 output channels (1920x1080, before -> now: 8 -> 8
-// 28.3 -> 19.5 us for 66 MB, images -> 8 38.7 -> 34.0 us for 158 MB), by staging latency and MFMA issue
-// elsewhere (48 -> 16 at half resolution 37.7 -> 20.4 us); registers for four waves per SIMD with one K
+// 28.3 -> 19.5 us for 66 MB, images -> 8 38.7 -> 34.0 us for 158 MB, 24 -> 8 and the head 50 -> 46 us
+// with only the even pixels of the upsampled source read), by staging latency and MFMA issue elsewhere
+// (48 -> 16 at half resolution 37.7 -> 20.4 us); registers for four waves per SIMD with one K
 // chunk, three with two, two with three chunks or two channel tiles.
 template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
 __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 3 : 4)) void uconv3x3(UcBatch b)
@@ -141,6 +142,11 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
         const int gy = y0 + ly - 1, gx = x0 + lx - 1;
         return pix < NPX && gy >= 0 && gy < H && gx >= 0 && gx < W ? (uint32_t)(gy - yb) * (uint32_t)W + (uint32_t)gx : kUOob;
     };
+    // UPCAT: off the even image positions (odd tile-local ones: tiles start at even rows and columns) the
+    // first source is its layer's bias, staged from pixel (0, 1) while the other loads are in flight
+    u32x4 fill;
+    if constexpr (SRC == UC_SRC_UPCAT)
+        fill = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.a) + CA + 8 * (tid % (CA / 8)));
     // kernel fragments first: their loads are in flight together with the tile's
     u32x4 wf[9][KC][NT];
 #pragma unroll
@@ -152,10 +158,14 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
                 wf[t][kc][nt] = static_cast<const u32x4 *>(F.wfrag)[((t * KC + kc) * NT + nt) * 64 + lane];
     if constexpr (HEAD)
         if (tid < 54) hws[tid] = F.head_w[tid];
-    if constexpr (SRC == UC_SRC_BF16)
+    if constexpr (SRC != UC_SRC_IMAGES)
     {
         constexpr int QA = CA / 8, QB = CB / 8;
-        constexpr int NA = (NPX * QA + 255) / 256, NB = QB ? (NPX * QB + 255) / 256 : 0;
+        static_assert(256 % QA == 0, "a thread stages the same chunk of every pixel");
+        constexpr bool UP = SRC == UC_SRC_UPCAT;
+        constexpr int NPA = UP ? (LW / 2) * (LH / 2) : NPX;  // pixels loaded of the first source
+        auto apix = [](int e) { return UP ? (2 * (e / (LW / 2)) + 1) * LW + 2 * (e % (LW / 2)) + 1 : e; };
+        constexpr int NA = (NPA * QA + 255) / 256, NB = QB ? (NPX * QB + 255) / 256 : 0;
         const u_rsrc ra = u_buf(F.a, row0 * (CA * 2), npx * (CA * 2));
         u32x4 va[NA];
         u32x4 vb[NB ? NB : 1];
@@ -163,7 +173,7 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
         for (int u = 0; u < NA; ++u)
         {
             const int i = tid + 256 * u;
-            const uint32_t p = pixel(i / QA);
+            const uint32_t p = i < NPA * QA ? pixel(apix(i / QA)) : kUOob;
             va[u] = __builtin_amdgcn_raw_buffer_load_b128(ra, p == kUOob ? kUOob : p * (CA * 2) + (i % QA) * 16, 0, 0);
         }
         if constexpr (QB > 0)
@@ -177,11 +187,19 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
                 vb[u] = __builtin_amdgcn_raw_buffer_load_b128(rb, p == kUOob ? kUOob : p * (CB * 2) + (i % QB) * 16, 0, 0);
             }
         }
+        if constexpr (UP)
+#pragma unroll
+            for (int u = 0; u < (NPX * QA + 255) / 256; ++u)
+            {
+                const int i = tid + 256 * u, pix = i / QA;
+                if (i >= NPX * QA || (pix / LW & (pix % LW) & 1)) continue;
+                *reinterpret_cast<u32x4 *>(&lds[pix * PS + (i % QA) * 8]) = pixel(pix) != kUOob ? fill : u32x4{0u, 0u, 0u, 0u};
+            }
 #pragma unroll
         for (int u = 0; u < NA; ++u)
         {
             const int i = tid + 256 * u;
-            if (i < NPX * QA) *reinterpret_cast<u32x4 *>(&lds[(i / QA) * PS + (i % QA) * 8]) = va[u];
+            if (i < NPA * QA) *reinterpret_cast<u32x4 *>(&lds[apix(i / QA) * PS + (i % QA) * 8]) = va[u];
         }
         if constexpr (QB > 0)
 #pragma unroll
@@ -355,6 +373,10 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
 template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
 static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
 {
+    // bytes of one staged image row over all of a tile's 32-bit offsets, see kUOob
+    constexpr uint64_t row = (UT_H + 2) * (SRC == UC_SRC_IMAGES ? 12 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO);
+    for (int i = 0; i < n; ++i)
+        if (row * (uint64_t)fr[i].W >= kUOob) return hipErrorInvalidValue;  // wider than 4.9 million pixels
     UcBatch b{};
     int tx[XDN_MAX_FRAMES], ty[XDN_MAX_FRAMES];
     for (int i = 0; i < n; ++i)
@@ -382,7 +404,6 @@ hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st)
     case UC_F_16_32: return uconv_t<UC_SRC_BF16, 16, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_32_32: return uconv_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_48_16: return uconv_t<UC_SRC_BF16, 32, 16, 16, UC_EPI_RELU>(n, fr, st);
-    case UC_F_24_8: return uconv_t<UC_SRC_BF16, 16, 8, 8, UC_EPI_RELU>(n, fr, st);
     case UC_D_8_8: return uconv_t<UC_SRC_BF16, 8, 0, 8, UC_EPI_MASK>(n, fr, st);
     case UC_D_16_8: return uconv_t<UC_SRC_BF16, 16, 0, 8, UC_EPI_PLAIN>(n, fr, st);
     case UC_D_16_16: return uconv_t<UC_SRC_BF16, 16, 0, 16, UC_EPI_MASK>(n, fr, st);
@@ -390,13 +411,18 @@ hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st)
     case UC_D_32_32: return uconv_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_MASK>(n, fr, st);
     case UC_D_16_48: return uconv_t<UC_SRC_BF16, 16, 0, 48, UC_EPI_PLAIN>(n, fr, st);
     case UC_D_8_24: return uconv_t<UC_SRC_BF16, 8, 0, 24, UC_EPI_PLAIN>(n, fr, st);
-    case UC_F_24_8_HEAD: return uconv_t<UC_SRC_BF16, 16, 8, 8, UC_EPI_RELU, true>(n, fr, st);
+    case UC_F_24_8_HEAD: return uconv_t<UC_SRC_UPCAT, 16, 8, 8, UC_EPI_RELU, true>(n, fr, st);
     default: return hipErrorInvalidValue;
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// Weight gradient of a 3x3 layer: input slice [32 MT, 32 MT + 32) of concat[a, b] (or the images)
+// Weight gradient of a 3x3 layer: input slice [32 MT, 32 MT + 32) of concat[a, b] (or the images).
+// A block walks strips, at most two blocks a CU (their number fixes the partial sums), so what it spends
+// is the time between strips: staging without branches, strip-invariant offsets, DEPTH strips in flight,
+// only the even pixels of an upsampled source. HBM and the halo's L2 reads bound the images (1920x1080:
+// 41.4 us, 158 MB), LDS reads, barriers and latency the rest (24 channels 45 -> 33.6 us, 8 channels
+// 26.7 -> 20.3 us, 48 in two slices 18.8 + 11.8 -> 17.5 + 11.4 us).
 // ---------------------------------------------------------------------------------------------
 struct UwBatch {
     int n;
@@ -408,7 +434,7 @@ static_assert(sizeof(UwBatch) <= 4096, "kernel argument too large");
 constexpr int US_W = 32, US_H = 8;                // strip: 8 rows x 32 px
 constexpr int UX_C = US_W + 2, UX_R = US_H + 2;   // staged X: 10 rows x 34 px (1-px halo)
 
-template <int SRC, int CA, int CB, int CO, int MT>
+template <int SRC, int CA, int CB, int CO, int MT, int DEPTH>
 __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
 {
     // input-slice channels of this instantiation; staged channel counts (pixel strides) 16 or 32,
@@ -432,98 +458,183 @@ __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
     const int grp = (lane >> 4) & 1, s16 = lane & 15, jq = s16 >> 2, qq = s16 & 3;
     const int cbx = (XS > 16 ? 16 * grp : 0) + 4 * qq, cbd = (DS > 16 ? 16 * grp : 0) + 4 * qq;
 
-    constexpr int QX = XS / 8, QD = DS / 8;  // 16-byte chunks per staged pixel
-    constexpr int NX = SRC == UC_SRC_BF16 ? (UX_R * UX_C * QX + 255) / 256 : (UX_R * UX_C + 255) / 256;
-    constexpr int ND = US_H * US_W * QD / 256;
-    u32x4 rx[SRC == UC_SRC_BF16 ? NX : 1], rd[ND];
-    float fx[SRC == UC_SRC_BF16 ? 1 : NX][15];
-    auto fetch = [&](int s) {
-        const int y0 = (s / sx) * US_H, x0 = (s % sx) * US_W;
-#pragma unroll
-        for (int u = 0; u < NX; ++u)
-        {
-            if constexpr (SRC == UC_SRC_BF16)
-            {
-                const int i = tid + 256 * u, pix = i / QX, q = i % QX;
-                const int r = pix / UX_C, col = pix - r * UX_C;
-                const int gy = y0 - 1 + r, gx = x0 - 1 + col;
-                const int g = 32 * MT + 8 * q;  // first concat channel of this chunk
-                rx[u] = u32x4{0u, 0u, 0u, 0u};
-                if (i < UX_R * UX_C * QX && gy >= 0 && gy < H && gx >= 0 && gx < W)
-                {
-                    const size_t p = (size_t)gy * W + gx;
-                    if (g < CA)
-                        rx[u] = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.a) + p * CA + g);
-                    else if (g < CA + CB)
-                        rx[u] = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.b) + p * CB + (g - CA));
-                }
-            }
-            else
-            {
-                const int pix = tid + 256 * u;
-                const int r = pix / UX_C, col = pix - r * UX_C;
-                const int gy = y0 - 1 + r, gx = x0 - 1 + col;
-#pragma unroll
-                for (int j = 0; j < 15; ++j) fx[u][j] = 0.f;
-                if (pix < UX_R * UX_C && gy >= 0 && gy < H && gx >= 0 && gx < W)
-                {
-                    const size_t p = (size_t)gy * W + gx;
-#pragma unroll
-                    for (int im = 0; im < 5; ++im)
-                    {
-                        const float *sp = F.img[im] + 3 * p;
-                        fx[u][3 * im] = sp[0]; fx[u][3 * im + 1] = sp[1]; fx[u][3 * im + 2] = sp[2];
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < ND; ++u)
-        {
-            const int i = tid + 256 * u, pix = i / QD, q = i % QD;
-            const int r = pix / US_W, col = pix - r * US_W;
-            const int gy = y0 + r, gx = x0 + col;
-            rd[u] = u32x4{0u, 0u, 0u, 0u};
-            if (q < CO / 8 && gy < H && gx < W)
-                rd[u] = *reinterpret_cast<const u32x4 *>(F.dy + ((size_t)gy * W + gx) * CO + q * 8);
-        }
+    // Staging: 16-byte chunks of the sources' real channels (a slice lies in a, in b, or takes all of
+    // both), raw buffer loads as in uconv3x3 and no branch, so a strip's loads stay in flight
+    // through the two strips computed before it; the padding of the LDS pixels is cleared once.
+    constexpr int CAS = SRC == UC_SRC_IMAGES ? 0 : (CA - 32 * MT > 0 ? CS < CA ? CS : CA : 0);
+    constexpr int CBS = SRC == UC_SRC_IMAGES ? 0 : CS - CAS;
+    constexpr int AOFF = CAS ? 32 * MT : 0, BOFF = CAS ? 0 : 32 * MT - CA;
+    constexpr int QA = CAS / 8, QB = CBS / 8, QX = XS / 8, QD = DS / 8, QDR = CO / 8, NPX = UX_R * UX_C;
+    constexpr bool UP = SRC == UC_SRC_UPCAT && QA > 0;
+    constexpr int NPA = UP ? (UX_C / 2) * (UX_R / 2) : NPX;  // pixels loaded of a
+    auto apix = [](int e) { return UP ? (2 * (e / (UX_C / 2)) + 1) * UX_C + 2 * (e % (UX_C / 2)) + 1 : e; };
+    constexpr int NA = (NPA * QA + 255) / 256, NB = (NPX * QB + 255) / 256;
+    constexpr int NI = SRC == UC_SRC_IMAGES ? (NPX + 255) / 256 : 0;
+    static_assert(SRC == UC_SRC_IMAGES || ((QA == 0 || 256 % QA == 0) && CAS + CBS == CS), "slice of the concatenation");
+    struct Strip {
+        u32x4 a[NA ? NA : 1], b[NB ? NB : 1], d[QDR];
+        u32x3 im[NI ? NI : 1][5];
+        int ylo, yhi, xlo, xhi;  // UPCAT: staged rows and columns that lie in the image
     };
-    auto commit = [&]() {
+    u32x4 fill = {0u, 0u, 0u, 0u};
+    bool refill = true;  // UPCAT: the bias pixels of the staged tile have to be written (see uconv3x3)
+    if constexpr (UP)
+        fill = *reinterpret_cast<const u32x4 *>(static_cast<const uint16_t *>(F.a) + CA + AOFF + 8 * (tid % (QA ? QA : 1)));
+    // byte offsets from the strip's first staged pixel (row y0 - 1, column x0 - 1), the same for all
+    // strips; a strip at the image border replaces those outside by kUOob
+    auto offset = [&](int pix, int stride, int chunk) -> uint32_t {
+        const int r = pix / UX_C, col = pix - r * UX_C;
+        return ((uint32_t)r * (uint32_t)W + (uint32_t)col) * (uint32_t)stride + (uint32_t)chunk;
+    };
+    auto fetch = [&](Strip &R, int strip, bool on) {  // !on: no strip, every load out of range
+        // 32 -> 32: the offsets are computed anew for every strip (an identity DPP move keeps
+        // them in the loop); kept in registers they cost spills, 15.6 -> 20.4 us
+        const int ti = CO > 16 && CS > 16 ? __builtin_amdgcn_mov_dpp(tid, 0xE4, 0xf, 0xf, true) : tid;
+        const int s = on ? strip : 0, y0 = (s / sx) * US_H, x0 = (s % sx) * US_W;
+        // staged rows [ylo, yhi) and columns [xlo, xhi) lie in the image (readfirstlane: keeps the
+        // compiler from giving `on` a copy of the loads of its own, and a full wait where both meet)
+        const int ylo = y0 == 0, yhi = __builtin_amdgcn_readfirstlane(on ? min(UX_R, H - y0 + 1) : 0);
+        const int xlo = x0 == 0, xhi = min(UX_C, W - x0 + 1);
+        const bool inner = ylo == 0 && yhi == UX_R && xlo == 0 && xhi == UX_C;
+        const long base = ((long)y0 - 1) * W + x0 - 1;  // may lie before the image: only masked lanes do
+        const size_t span = (size_t)UX_R * W + UX_C;
+        auto outside = [&](int r, int col) { return r < ylo || r >= yhi || col < xlo || col >= xhi; };
+        uint32_t oa[NA ? NA : 1], ob[NB ? NB : 1], od[QDR], oi[NI ? NI : 1];
 #pragma unroll
-        for (int u = 0; u < NX; ++u)
+        for (int u = 0; u < NA; ++u)
         {
-            if constexpr (SRC == UC_SRC_BF16)
+            const int i = ti + 256 * u, e = i / (QA ? QA : 1);
+            oa[u] = e < NPA ? offset(apix(e), CA * 2, AOFF * 2 + (i % (QA ? QA : 1)) * 16) : kUOob;
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+        {
+            const int i = ti + 256 * u, pix = i / (QB ? QB : 1);
+            ob[u] = pix < NPX ? offset(pix, CB * 2, BOFF * 2 + (i % (QB ? QB : 1)) * 16) : kUOob;
+        }
+#pragma unroll
+        for (int u = 0; u < NI; ++u) oi[u] = ti + 256 * u < NPX ? offset(ti + 256 * u, 12, 0) : kUOob;
+#pragma unroll
+        for (int u = 0; u < QDR; ++u)
+        {
+            const int i = ti + 256 * u, pix = i / QDR;
+            od[u] = ((uint32_t)(pix / US_W + 1) * (uint32_t)W + (uint32_t)(pix % US_W + 1)) * (CO * 2) + (i % QDR) * 16;
+        }
+        R.ylo = ylo; R.yhi = yhi; R.xlo = xlo; R.xhi = xhi;
+        if (!inner)
+        {
+#pragma unroll
+            for (int u = 0; u < NA; ++u)
+            {
+                const int pix = apix((ti + 256 * u) / (QA ? QA : 1));
+                if (outside(pix / UX_C, pix % UX_C)) oa[u] = kUOob;
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+            {
+                const int pix = (ti + 256 * u) / (QB ? QB : 1);
+                if (outside(pix / UX_C, pix % UX_C)) ob[u] = kUOob;
+            }
+#pragma unroll
+            for (int u = 0; u < NI; ++u)
+                if (outside((ti + 256 * u) / UX_C, (ti + 256 * u) % UX_C)) oi[u] = kUOob;
+#pragma unroll
+            for (int u = 0; u < QDR; ++u)
+            {
+                const int pix = (ti + 256 * u) / QDR;
+                if (outside(pix / US_W + 1, pix % US_W + 1)) od[u] = kUOob;
+            }
+        }
+        if constexpr (QA > 0)
+        {
+            const u_rsrc r = u_buf(F.a, base * (CA * 2), span * (CA * 2));
+#pragma unroll
+            for (int u = 0; u < NA; ++u) R.a[u] = __builtin_amdgcn_raw_buffer_load_b128(r, oa[u], 0, 0);
+        }
+        if constexpr (QB > 0)
+        {
+            const u_rsrc r = u_buf(F.b, base * (CB * 2), span * (CB * 2));
+#pragma unroll
+            for (int u = 0; u < NB; ++u) R.b[u] = __builtin_amdgcn_raw_buffer_load_b128(r, ob[u], 0, 0);
+        }
+        if constexpr (SRC == UC_SRC_IMAGES)
+#pragma unroll
+            for (int im = 0; im < 5; ++im)
+            {
+                const u_rsrc r = u_buf(F.img[im], base * 12, span * 12);
+#pragma unroll
+                for (int u = 0; u < NI; ++u) R.im[u][im] = __builtin_amdgcn_raw_buffer_load_b96(r, oi[u], 0, 0);
+            }
+        const u_rsrc rd = u_buf(F.dy, base * (CO * 2), span * (CO * 2));
+#pragma unroll
+        for (int u = 0; u < QDR; ++u) R.d[u] = __builtin_amdgcn_raw_buffer_load_b128(rd, od[u], 0, 0);
+    };
+    auto commit = [&](Strip &R) {
+        if constexpr (UP)
+        {
+            // bias pixels stay from strip to strip but where a strip meets the image border
+            const bool border = R.ylo != 0 || R.yhi != UX_R || R.xlo != 0 || R.xhi != UX_C;
+            if (refill || border)
+                for (int i = tid; i < NPX * QA; i += 256)
+                {
+                    const int pix = i / QA, r = pix / UX_C, col = pix % UX_C;
+                    if (r & col & 1) continue;
+                    const bool in = r >= R.ylo && r < R.yhi && col >= R.xlo && col < R.xhi;
+                    *reinterpret_cast<u32x4 *>(&xs[pix * XS + (i % QA) * 8]) = in ? fill : u32x4{0u, 0u, 0u, 0u};
+                }
+            refill = border;
+        }
+        if constexpr (QA > 0)
+#pragma unroll
+            for (int u = 0; u < NA; ++u)
             {
                 const int i = tid + 256 * u;
-                if (i < UX_R * UX_C * QX) *reinterpret_cast<u32x4 *>(&xs[(i / QX) * XS + (i % QX) * 8]) = rx[u];
+                if (i < NPA * QA) *reinterpret_cast<u32x4 *>(&xs[apix(i / QA) * XS + (i % QA) * 8]) = R.a[u];
             }
-            else
+        if constexpr (QB > 0)
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+            {
+                const int i = tid + 256 * u;
+                if (i < NPX * QB) *reinterpret_cast<u32x4 *>(&xs[(i / QB) * XS + CAS + (i % QB) * 8]) = R.b[u];
+            }
+        if constexpr (SRC == UC_SRC_IMAGES)
+#pragma unroll
+            for (int u = 0; u < NI; ++u)
             {
                 const int pix = tid + 256 * u;
-                if (pix < UX_R * UX_C)
-                {
-                    u32x4 a, c, z = {0u, 0u, 0u, 0u};
-                    a.x = u_pack2(fx[u][0], fx[u][1]); a.y = u_pack2(fx[u][2], fx[u][3]);
-                    a.z = u_pack2(fx[u][4], fx[u][5]); a.w = u_pack2(fx[u][6], fx[u][7]);
-                    c.x = u_pack2(fx[u][8], fx[u][9]); c.y = u_pack2(fx[u][10], fx[u][11]);
-                    c.z = u_pack2(fx[u][12], fx[u][13]); c.w = u_pack2(fx[u][14], 0.f);
-                    *reinterpret_cast<u32x4 *>(&xs[pix * XS]) = a;
-                    *reinterpret_cast<u32x4 *>(&xs[pix * XS + 8]) = c;
-                    if constexpr (XS > 16)
-                    {
-                        *reinterpret_cast<u32x4 *>(&xs[pix * XS + 16]) = z;
-                        *reinterpret_cast<u32x4 *>(&xs[pix * XS + 24]) = z;
-                    }
-                }
-            }
-        }
+                if (pix >= NPX) continue;
+                float f[16];
 #pragma unroll
-        for (int u = 0; u < ND; ++u)
+                for (int im = 0; im < 5; ++im)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) f[3 * im + k] = __uint_as_float(R.im[u][im][k]);
+                f[15] = 0.f;
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    *reinterpret_cast<u32x4 *>(&xs[pix * XS + 8 * q]) =
+                        u32x4{u_cvt2(f[8 * q], f[8 * q + 1]), u_cvt2(f[8 * q + 2], f[8 * q + 3]),
+                              u_cvt2(f[8 * q + 4], f[8 * q + 5]), u_cvt2(f[8 * q + 6], f[8 * q + 7])};
+            }
+#pragma unroll
+        for (int u = 0; u < QDR; ++u)
         {
             const int i = tid + 256 * u;
-            *reinterpret_cast<u32x4 *>(&ds[(i / QD) * DS + (i % QD) * 8]) = rd[u];
+            *reinterpret_cast<u32x4 *>(&ds[(i / QDR) * DS + (i % QDR) * 8]) = R.d[u];
         }
     };
+    // padding chunks of the staged pixels
+    if constexpr (SRC != UC_SRC_IMAGES && QA + QB < QX)
+        for (int i = tid; i < NPX * (QX - QA - QB); i += 256)
+            *reinterpret_cast<u32x4 *>(&xs[i / (QX - QA - QB) * XS + 8 * (QA + QB + i % (QX - QA - QB))]) = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (QDR < QD)
+        for (int i = tid; i < US_H * US_W * (QD - QDR); i += 256)
+            *reinterpret_cast<u32x4 *>(&ds[i / (QD - QDR) * DS + 8 * (QDR + i % (QD - QDR))]) = u32x4{0u, 0u, 0u, 0u};
+
+    const StripWalk sw = xcd_strips(li, nblk, sx * sy);
+    Strip R[DEPTH];
+#pragma unroll
+    for (int k = 0; k < DEPTH; ++k) fetch(R[k], sw.first + k * sw.step, sw.first + k * sw.step < sw.end);
 
     // CO > 16: 32x32x16 MFMA, M = 32 input channels, N = 32 output channels, K = 16 px (8 px of row
     // 2wv + h per lane half). CO <= 16: 16x16x32 MFMA, M = 16 input channels (MTI tiles), N = 16
@@ -550,15 +661,7 @@ __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
             for (int k = 0; k < 16; ++k) acc[t][k] = 0.f;
     float db = 0.f;
     const int kg = lane >> 4;
-    const int nstrip = sx * sy;
-    const StripWalk sw = xcd_strips(li, nblk, nstrip);
-    if (sw.first < sw.end) fetch(sw.first);
-    for (int s = sw.first; s < sw.end; s += sw.step)
-    {
-        __syncthreads();
-        commit();
-        __syncthreads();
-        if (s + sw.step < sw.end) fetch(s + sw.step);
+    auto compute = [&]() {
         if constexpr (N16)
         {
             // lane group kg takes pixels 8kg .. 8kg+7 of the row; lane L of the group reads the
@@ -586,7 +689,7 @@ __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
                                 __builtin_bit_cast(bf16x8, B), acc16[dy * 3 + sh][m], 0, 0, 0);
                         }
             }
-            continue;
+            return;
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c)
@@ -605,7 +708,20 @@ __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
                     acc[dy * 3 + sh] = u_mfma(u32x4{a0.x, a0.y, a1.x, a1.y}, B, acc[dy * 3 + sh]);
                 }
         }
-    }
+    };
+    for (int s = sw.first; s < sw.end; s += DEPTH * sw.step)
+#pragma unroll
+        for (int k = 0; k < DEPTH; ++k)
+        {
+            const int c = s + k * sw.step;
+            if (c >= sw.end) break;  // uniform across the block
+            __syncthreads();
+            commit(R[k]);
+            __syncthreads();
+            // unconditional at two strips in flight: the next commit then waits for its own strip alone
+            if (DEPTH > 1 || c + sw.step < sw.end) fetch(R[k], c + DEPTH * sw.step, c + DEPTH * sw.step < sw.end);
+            compute();
+        }
     // compact partial [9][CS][CO] + [CO] of this input slice
     float *out = F.part + (size_t)li * compact_part(9, CS, CO);
     float *red = reinterpret_cast<float *>(lds);  // [4 waves][1024]
@@ -658,21 +774,32 @@ int ublocks(int H, int W)
     return strips < 1 ? 1 : (strips < 512 ? strips : 512);
 }
 
+// Two strips in flight where a block walks more than two (1920x1080, 16 strips: 24 channels 33.6 us, 38.5
+// with one; 8 channels 20.3, 26.7), one below (256x256, one strip: 13.8 us, 15.3 with two; the images 10.6,
+// 13.8) and where 32 outputs leave no registers for two.
 template <int SRC, int CA, int CB, int CO, int MT>
 static hipError_t uwgrad_t(int n, const UwFrame *fr, hipStream_t st)
 {
+    constexpr int pix = SRC == UC_SRC_IMAGES ? 16 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO;
+    for (int i = 0; i < n; ++i)  // a strip's 32-bit offsets
+        if ((uint64_t)pix * (UX_R * (uint64_t)fr[i].W + UX_C) >= kUOob) return hipErrorInvalidValue;
     UwBatch b{};
     b.n = n;
     int acc = 0;
+    bool deep = false;
     for (int i = 0; i < n; ++i)
     {
         b.f[i] = fr[i];
         b.blk_begin[i] = acc;
         acc += fr[i].nblk;
+        deep |= udiv_up(fr[i].W, US_W) * udiv_up(fr[i].H, US_H) > 2 * fr[i].nblk;
     }
     b.blk_begin[n] = acc;
     if (acc == 0) return hipSuccess;
-    hipLaunchKernelGGL((uwgrad<SRC, CA, CB, CO, MT>), dim3(acc), dim3(256), 0, st, b);
+    if (CO <= 16 && deep)
+        hipLaunchKernelGGL((uwgrad<SRC, CA, CB, CO, MT, CO <= 16 ? 2 : 1>), dim3(acc), dim3(256), 0, st, b);
+    else
+        hipLaunchKernelGGL((uwgrad<SRC, CA, CB, CO, MT, 1>), dim3(acc), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 
@@ -688,9 +815,9 @@ hipError_t launch_uwgrad(int kind, int n, const UwFrame *fr, hipStream_t st)
     case UW_16_16: return uwgrad_t<UC_SRC_BF16, 16, 0, 16, 0>(n, fr, st);
     case UW_16_32: return uwgrad_t<UC_SRC_BF16, 16, 0, 32, 0>(n, fr, st);
     case UW_32_32: return uwgrad_t<UC_SRC_BF16, 32, 0, 32, 0>(n, fr, st);
-    case UW_48_16_M0: return uwgrad_t<UC_SRC_BF16, 32, 16, 16, 0>(n, fr, st);
+    case UW_48_16_M0: return uwgrad_t<UC_SRC_UPCAT, 32, 16, 16, 0>(n, fr, st);
     case UW_48_16_M1: return uwgrad_t<UC_SRC_BF16, 32, 16, 16, 1>(n, fr, st);
-    case UW_24_8: return uwgrad_t<UC_SRC_BF16, 16, 8, 8, 0>(n, fr, st);
+    case UW_24_8: return uwgrad_t<UC_SRC_UPCAT, 16, 8, 8, 0>(n, fr, st);
     default: return hipErrorInvalidValue;
     }
 }

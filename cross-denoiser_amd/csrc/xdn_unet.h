@@ -26,7 +26,9 @@
 
 namespace xdn {
 
-enum { UC_SRC_BF16 = 0, UC_SRC_IMAGES = 1 };
+// UC_SRC_UPCAT: the first source is a transposed 1x1 stride-2 layer's output. Off the even positions it
+// holds that layer's bias, so only the even ones are read; the rest take the pixel (0, 1).
+enum { UC_SRC_BF16 = 0, UC_SRC_IMAGES = 1, UC_SRC_UPCAT = 2 };
 enum { UC_EPI_RELU = 0, UC_EPI_MASK = 1, UC_EPI_PLAIN = 2 };
 
 // 3x3 'same' convolution over concat[a (CA ch), b (CB ch)] (or the five images), forward or data
@@ -52,7 +54,6 @@ enum {
     UC_F_16_32,   // 16 -> 32 ReLU
     UC_F_32_32,   // 32 -> 32 ReLU
     UC_F_48_16,   // concat 32+16 -> 16 ReLU
-    UC_F_24_8,    // concat 16+8 -> 8 ReLU
     UC_D_8_8,     // dgrad dY 8 -> dX 8, masked
     UC_D_16_8,    // dgrad dY 16 -> dX 8, unmasked (pool input)
     UC_D_16_16,   // dgrad dY 16 -> dX 16, masked
@@ -60,7 +61,7 @@ enum {
     UC_D_32_32,   // dgrad dY 32 -> dX 32, masked
     UC_D_16_48,   // dgrad dY 16 -> dX 48, unmasked (concat input)
     UC_D_8_24,    // dgrad dY 8 -> dX 24, unmasked (concat input)
-    UC_F_24_8_HEAD,  // UC_F_24_8 with the 1x1 head 8 -> 6 (FP32) applied to its bf16 output
+    UC_F_24_8_HEAD,  // concat 16 (upsampled) + 8 -> 8 ReLU, then the 1x1 head 8 -> 6 (FP32) on the bf16 output
     UC_KINDS
 };
 
@@ -81,9 +82,9 @@ enum {
     UW_16_16,     // 16 x 16
     UW_16_32,     // 16 x 32
     UW_32_32,     // 32 x 32
-    UW_48_16_M0,  // concat 32+16 x 16, input channels 0-31
+    UW_48_16_M0,  // concat 32 (upsampled) + 16 x 16, input channels 0-31
     UW_48_16_M1,  // concat 32+16 x 16, input channels 32-47
-    UW_24_8,      // concat 16+8 x 8
+    UW_24_8,      // concat 16 (upsampled) + 8 x 8
     UW_KINDS
 };
 hipError_t launch_uwgrad(int kind, int n, const UwFrame *fr, hipStream_t st);

@@ -296,6 +296,15 @@ def test_unet_forward_backward(dev, B, H, W):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("H,W", [(256, 1024), (268, 1028)])
+def test_unet_weight_gradient_strips_per_block(dev, H, W):
+    """Full-resolution weight gradients of two strips a block at most (1024 strips over 512 blocks:
+    one strip in flight) and of two or three (1122 strips: two in flight, ragged right and bottom
+    edges), with the bars of test_unet_forward_backward."""
+    test_unet_forward_backward(dev, 1, H, W)
+
+
+@pytest.mark.gpu
 def test_unet_adam_step_and_repack(dev):
     """A Keras Adam step on the U-Net parameters, then the packed fragments follow the update."""
     from xdn import cnn
