@@ -281,18 +281,19 @@ int xdn_spatial_filter_grad(const float *grad_acca, const float *grad_accb, cons
         "spatial_filter_grad");
 }
 
-int xdn_spatial_filter_grad_inputs(const float *grad_acca, const float *grad_accb, const float *grad_wgtsuma,
-                                   const float *grad_wgtsumb, const float *imga, const float *imgb,
-                                   const float *img_albedo, const float *img_normal, const float *band,
-                                   float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
-                                   int batch, int height, int width, int win_size, void *stream)
+// The image gradients, and the band gradient with them where grad_band is given.
+static int sf_input_grads(const float *grad_acca, const float *grad_accb, const float *grad_wgtsuma,
+                          const float *grad_wgtsumb, const float *imga, const float *imgb,
+                          const float *img_albedo, const float *img_normal, const float *band,
+                          float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal, float *grad_band,
+                          int batch, int height, int width, int win_size, void *stream, const char *name)
 {
     if (int e = sf_common_check(batch, height, width, win_size)) return e;
     if (win_size / 2 > 7) return fail(XDN_EINVAL, "input gradients support win_size <= 15");
     if (batch == 0) return XDN_OK;  // empty batch: nothing to read or write
     if (!grad_acca || !grad_accb || !grad_wgtsuma || !grad_wgtsumb || !imga || !imgb || !img_albedo || !img_normal ||
         !band)
-        return fail(XDN_EINVAL, "spatial_filter_grad_inputs: null tensor");
+        return fail(XDN_EINVAL, "%s: null tensor", name);
     const size_t N = px(height, width);
     auto off = [](float *p, size_t o) { return p ? p + o : nullptr; };
     return sf_run(
@@ -304,9 +305,33 @@ int xdn_spatial_filter_grad_inputs(const float *grad_acca, const float *grad_acc
             f.gwA = grad_wgtsuma + b * N; f.gwB = grad_wgtsumb + b * N;
             f.gia = off(grad_imga, b * N * 3); f.gib = off(grad_imgb, b * N * 3);
             f.galb = off(grad_albedo, b * N * 3); f.gnrm = off(grad_normal, b * N * 3);
+            f.gband = off(grad_band, b * N * 5);
         },
         [&](int n, const xdn::SfFrame *fr) { return xdn::launch_sf_grad_inputs(n, fr, win_size, S(stream)); },
-        "spatial_filter_grad_inputs");
+        name);
+}
+
+int xdn_spatial_filter_backward(const float *grad_acca, const float *grad_accb, const float *grad_wgtsuma,
+                                const float *grad_wgtsumb, const float *imga, const float *imgb,
+                                const float *img_albedo, const float *img_normal, const float *band,
+                                float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
+                                float *grad_band, int batch, int height, int width, int win_size, void *stream)
+{
+    if (batch > 0 && !grad_band) return fail(XDN_EINVAL, "spatial_filter_backward: null tensor");
+    return sf_input_grads(grad_acca, grad_accb, grad_wgtsuma, grad_wgtsumb, imga, imgb, img_albedo, img_normal, band,
+                          grad_imga, grad_imgb, grad_albedo, grad_normal, grad_band, batch, height, width, win_size,
+                          stream, "spatial_filter_backward");
+}
+
+int xdn_spatial_filter_grad_inputs(const float *grad_acca, const float *grad_accb, const float *grad_wgtsuma,
+                                   const float *grad_wgtsumb, const float *imga, const float *imgb,
+                                   const float *img_albedo, const float *img_normal, const float *band,
+                                   float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
+                                   int batch, int height, int width, int win_size, void *stream)
+{
+    return sf_input_grads(grad_acca, grad_accb, grad_wgtsuma, grad_wgtsumb, imga, imgb, img_albedo, img_normal, band,
+                          grad_imga, grad_imgb, grad_albedo, grad_normal, nullptr, batch, height, width, win_size,
+                          stream, "spatial_filter_grad_inputs");
 }
 
 int xdn_reproject(const float *mvec, int n_list, const float *const *inputs, const int *dims, const float *linear_z,

@@ -13,7 +13,7 @@
 //                    accumulation, loss and the whole pointwise backward (aggregation ->
 //                    weights -> band transform) in the epilogue; writes the output image and
 //                    d loss / d network output                                  VALU-bound
-//   sf_grad_inputs   gradient w.r.t. the four images, gather form (no atomics): every pixel
+//   sf_grad_inputs   gradient w.r.t. the four images (and the bands with BAND), gather form (no atomics): every pixel
 //                    collects its own-center term and the terms of all centers whose (mirrored)
 //                    window contains it, both from one pass over its window; two threads a pixel
 //   sf_generic       any window size, direct loads (forward / grad)
@@ -47,37 +47,44 @@ struct SfCenter {
 struct SfAcc {
     float3 aA, aB;
     float sA, sB;
-    // GRAD: band-gradient accumulators; TRAIN: moments sum w*d_k*(c,1)
-    float g[5];
-    float4 MA[4], MB[4];
+    float4 MA[4], MB[4];  // TRAIN: moments sum w*d_k*(c,1)
 };
+
+// One tap of the band gradient: g[k] += u * distance, with r2 the squared pixel distance. The roundings are
+// spelled out so that every kernel that computes the band gradient gives the same bits.
+__device__ __forceinline__ float2 sf_grad_tap(float (&g)[5], const float4 k, float k4, float DA, float DB, float Da,
+                                              float Dn, float r2, float3 gA, float hA, float3 iA, float3 gB, float hB,
+                                              float3 iB)
+{
+#pragma clang fp contract(off)
+    const float sh = fmaf(k.z, Da, fmaf(k.w, Dn, k4 * r2));
+    const float uA = fast_exp2(fmaf(k.x, DA, sh)) * fmaf(gA.z, iA.z, fmaf(gA.y, iA.y, fmaf(gA.x, iA.x, hA)));
+    const float uB = fast_exp2(fmaf(k.y, DB, sh)) * fmaf(gB.z, iB.z, fmaf(gB.y, iB.y, fmaf(gB.x, iB.x, hB)));
+    const float u = uA + uB;
+    g[0] = fmaf(uA, DA, g[0]);
+    g[1] = fmaf(uB, DB, g[1]);
+    g[2] = fmaf(u, Da, g[2]);
+    g[3] = fmaf(u, Dn, g[3]);
+    g[4] = fmaf(u, r2, g[4]);
+    return make_float2(uA, uB);
+}
+
+// |v|^2 in the roundings of dist2.
+__device__ __forceinline__ float norm2(float3 v) { return fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y)); }
+__device__ __forceinline__ float3 sub3(float3 a, float3 b) { return make_float3(a.x - b.x, a.y - b.y, a.z - b.z); }
 
 template <int MODE>
 __device__ __forceinline__ void sf_tap(const SfCenter &C, SfAcc &acc, float3 iA, float3 iB, float3 ia, float3 in,
-                                       float pd, float kpd, float3 gA, float hA, float3 gB, float hB)
+                                       float pd, float kpd)
 {
     const float dA = dist2(C.cA, iA), dB = dist2(C.cB, iB), dal = dist2(C.ca, ia), dn = dist2(C.cn, in);
     const float sh = C.k2 * dal + (C.k3 * dn + kpd);
     const float wA = fast_exp2(C.k0 * dA + sh);
     const float wB = fast_exp2(C.k1 * dB + sh);
-    if (MODE == SF_FWD || MODE == SF_TRAIN)
-    {
-        acc.aA.x += wA * iA.x; acc.aA.y += wA * iA.y; acc.aA.z += wA * iA.z;
-        acc.aB.x += wB * iB.x; acc.aB.y += wB * iB.y; acc.aB.z += wB * iB.z;
-        acc.sA += wA;
-        acc.sB += wB;
-    }
-    if (MODE == SF_GRAD)
-    {
-        const float uA = wA * (gA.x * iA.x + gA.y * iA.y + gA.z * iA.z + hA);
-        const float uB = wB * (gB.x * iB.x + gB.y * iB.y + gB.z * iB.z + hB);
-        const float uS = uA + uB;
-        acc.g[0] += uA * dA;
-        acc.g[1] += uB * dB;
-        acc.g[2] += uS * dal;
-        acc.g[3] += uS * dn;
-        acc.g[4] += uS * pd;
-    }
+    acc.aA.x += wA * iA.x; acc.aA.y += wA * iA.y; acc.aA.z += wA * iA.z;
+    acc.aB.x += wB * iB.x; acc.aB.y += wB * iB.y; acc.aB.z += wB * iB.z;
+    acc.sA += wA;
+    acc.sB += wB;
     if (MODE == SF_TRAIN)
     {
         const float mA[4] = {wA * dA, wA * dal, wA * dn, wA * pd};
@@ -97,8 +104,6 @@ __device__ __forceinline__ void sf_zero(SfAcc &a)
 {
     a.aA = a.aB = make_float3(0.f, 0.f, 0.f);
     a.sA = a.sB = 0.f;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) a.g[k] = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; ++k) a.MA[k] = a.MB[k] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
@@ -243,12 +248,6 @@ __device__ __forceinline__ void sf_tile_body(const Batch &b, float *red)
         }
         else
             sf_center_bands(C, F.band, c, HALF);
-        float3 gA = make_float3(0.f, 0.f, 0.f), gB = gA;
-        float hA = 0.f, hB = 0.f;
-        if constexpr (MODE == SF_GRAD)
-        {
-            gA = ld3(F.gaccA, c); gB = ld3(F.gaccB, c); hA = F.gwA[c]; hB = F.gwB[c];
-        }
         SfAcc acc;
         sf_zero(acc);
         constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
@@ -265,7 +264,7 @@ __device__ __forceinline__ void sf_tile_body(const Batch &b, float *red)
                 const float pd = pdy + (float)(dx * dx) * inv_h2;
                 const float kpd = kdy + C.k4 * (float)(dx * dx);
                 sf_tap<MODE>(C, acc, make_float3(P0.x, P0.y, P0.z), make_float3(P0.w, P1.x, P1.y),
-                             make_float3(P1.z, P1.w, P2.x), make_float3(P2.y, P2.z, P2.w), pd, kpd, gA, hA, gB, hB);
+                             make_float3(P1.z, P1.w, P2.x), make_float3(P2.y, P2.z, P2.w), pd, kpd);
             }
         }
         if constexpr (MODE == SF_FWD)
@@ -274,12 +273,6 @@ __device__ __forceinline__ void sf_tile_body(const Batch &b, float *red)
             st3(F.accB, c, acc.aB);
             F.wsA[c] = acc.sA;
             F.wsB[c] = acc.sB;
-        }
-        else if constexpr (MODE == SF_GRAD)
-        {
-            float *o = F.gband + 5 * (size_t)c;
-#pragma unroll
-            for (int k = 0; k < 5; ++k) o[k] = -acc.g[k];
         }
         else
         {
@@ -299,15 +292,15 @@ __device__ __forceinline__ void sf_tile_body(const Batch &b, float *red)
     }
 }
 
-template <int HALF, int MODE>
+template <int HALF>
 __global__ __launch_bounds__(256) void sf_tile(SfBatch b)
 {
-    sf_tile_body<HALF, MODE>(b, nullptr);
+    sf_tile_body<HALF, SF_FWD>(b, nullptr);
 }
 
-// FWD and GRAD for launches that leave the chip idle: the window rows of a pixel are split over G threads
-// (groups of 256 threads of the block) whose sums meet in LDS, so a 16x16 tile runs 4 G waves instead of
-// a chain of 121 taps in four.
+// The window rows of a pixel are split over G threads (groups of 256 threads of the block) whose sums meet in
+// LDS: FWD and GRAD for launches that leave the chip idle, where a 16x16 tile then runs 4 G waves instead of a
+// chain of 121 taps in four, and GRAD at every size.
 template <int HALF, int MODE, int G>
 __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
 {
@@ -353,21 +346,25 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
     }
     SfAcc acc;
     sf_zero(acc);
+    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
     constexpr int R = 2 * HALF + 1;
 #pragma unroll 1
     for (int dy = R * grp / G - HALF; dy < R * (grp + 1) / G - HALF; ++dy)
     {
-        const float pdy = (float)(dy * dy) * inv_h2;
-        const float kdy = C.k4 * (float)(dy * dy);
+        const float y2 = (float)(dy * dy), kdy = C.k4 * y2;
         const int base = q0 + dy * E;
 #pragma unroll
         for (int dx = -HALF; dx <= HALF; ++dx)
         {
             const float4 P0 = s[0][base + dx], P1 = s[1][base + dx], P2 = s[2][base + dx];
-            sf_tap<MODE>(C, acc, make_float3(P0.x, P0.y, P0.z), make_float3(P0.w, P1.x, P1.y),
-                         make_float3(P1.z, P1.w, P2.x), make_float3(P2.y, P2.z, P2.w), pdy + (float)(dx * dx) * inv_h2,
-                         kdy + C.k4 * (float)(dx * dx), gA, hA, gB, hB);
+            const float3 iA = make_float3(P0.x, P0.y, P0.z), iB = make_float3(P0.w, P1.x, P1.y);
+            const float3 ia = make_float3(P1.z, P1.w, P2.x), in = make_float3(P2.y, P2.z, P2.w);
+            if constexpr (MODE == SF_FWD)
+                sf_tap<MODE>(C, acc, iA, iB, ia, in, 0.f, kdy + C.k4 * (float)(dx * dx));
+            else
+                sf_grad_tap(g, make_float4(C.k0, C.k1, C.k2, C.k3), C.k4, norm2(sub3(C.cA, iA)), norm2(sub3(C.cB, iB)),
+                            norm2(sub3(C.ca, ia)), norm2(sub3(C.cn, in)), y2 + (float)(dx * dx), gA, hA, iA, gB, hB, iB);
         }
     }
     float v[NV];
@@ -378,7 +375,7 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
     }
     else
 #pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] = acc.g[k];
+        for (int k = 0; k < NV; ++k) v[k] = g[k];
     __syncthreads();  // the tile is dead
     float *red = reinterpret_cast<float *>(&s[0][0]);  // [G - 1][NV][256]
     static_assert(sizeof(s) >= sizeof(float) * (G - 1) * NV * 256, "reduction space");
@@ -402,7 +399,7 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
     {
         float *o = F.gband + 5 * c;
 #pragma unroll
-        for (int k = 0; k < NV; ++k) o[k] = -v[k];
+        for (int k = 0; k < NV; ++k) o[k] = (k == 4 ? -inv_h2 : -1.f) * v[k];
     }
 }
 
@@ -437,14 +434,18 @@ __global__ __launch_bounds__(256) void sf_generic(SfBatch b)
     }
     SfAcc acc;
     sf_zero(acc);
-    const float inv_h2 = 1.f / (float)(HALF * HALF);
+    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     for (int dy = -HALF; dy <= HALF; ++dy)
         for (int dx = -HALF; dx <= HALF; ++dx)
         {
             const size_t i = (size_t)mirror(cy + dy, H) * W + mirror(cx + dx, W);
             const float r2 = (float)(dx * dx + dy * dy);
-            sf_tap<MODE>(C, acc, ld3(F.ia, i), ld3(F.ib, i), ld3(F.alb, i), ld3(F.nrm, i), r2 * inv_h2,
-                         C.k4 * r2, gA, hA, gB, hB);
+            const float3 iA = ld3(F.ia, i), iB = ld3(F.ib, i), ia = ld3(F.alb, i), in = ld3(F.nrm, i);
+            if (MODE == SF_FWD)
+                sf_tap<MODE>(C, acc, iA, iB, ia, in, 0.f, C.k4 * r2);
+            else
+                sf_grad_tap(g, make_float4(C.k0, C.k1, C.k2, C.k3), C.k4, norm2(sub3(C.cA, iA)), norm2(sub3(C.cB, iB)),
+                            norm2(sub3(C.ca, ia)), norm2(sub3(C.cn, in)), r2, gA, hA, iA, gB, hB, iB);
         }
     if (MODE == SF_FWD)
     {
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(256) void sf_generic(SfBatch b)
     {
         float *o = F.gband + 5 * c;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) o[k] = -acc.g[k];
+        for (int k = 0; k < 5; ++k) o[k] = k == 4 ? -g[k] / (float)(HALF * HALF) : -g[k];
     }
 }
 
@@ -478,9 +479,12 @@ __global__ __launch_bounds__(256) void sf_generic(SfBatch b)
 // axis, they are taps of the centers p around q' too, at the distances of (p, q) and the pixel
 // distance of p - q'; those pairs are a second loop that only blocks at an edge run.
 // LDS: the tile plus halo of every per-pixel quantity (25 floats), 26x26 pixels for win 11: 67.6 KB, two
-// blocks per CU, so a pixel's window rows are split over two threads (rows dy <= 0 and dy > 0, joined
+// blocks per CU, so a pixel's window rows are split over two threads (rows dy < 0 and dy >= 0, joined
 // through LDS) for four waves per SIMD instead of two. VALU-bound: 512x512, win 11: 247 -> 102 us
 // (128 us with one thread per pixel).
+// BAND: the band gradient too. Its terms are the own terms' u against the pair's distances, which are at
+// hand here: five FMAs a pair instead of a second launch that recomputes distances and weights (forward and
+// both gradients at 512x512 163 -> 145 us, at 1920x1080 1044 -> 770 us).
 // ---------------------------------------------------------------------------------------------
 struct Yes {
     static constexpr bool value = true;
@@ -489,7 +493,7 @@ struct No {
     static constexpr bool value = false;
 };
 
-template <int HALF>
+template <int HALF, bool BAND>
 __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
 {
     constexpr int E = SF_T + 2 * HALF;
@@ -557,24 +561,20 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
     const float3 zero = make_float3(0.f, 0.f, 0.f);
     float3 dA = zero, dB = zero, da = zero, dn = zero;  // sum of coefficient * (c_q - c_r)
     float3 eA = zero, eB = zero;                        // sum of w_rq g_r
+    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};             // BAND: sum of u_qr * distance
     // one pair (q, r) at the squared pixel distance r2: r's center term, and q's tap term where OWN
     auto pair = [&](int k, float r2, auto own) {
         constexpr bool OWN = decltype(own)::value;
         const Px R = image(k);
-        const float3 xA = make_float3(Q.A.x - R.A.x, Q.A.y - R.A.y, Q.A.z - R.A.z);
-        const float3 xB = make_float3(Q.B.x - R.B.x, Q.B.y - R.B.y, Q.B.z - R.B.z);
-        const float3 xa = make_float3(Q.al.x - R.al.x, Q.al.y - R.al.y, Q.al.z - R.al.z);
-        const float3 xn = make_float3(Q.n.x - R.n.x, Q.n.y - R.n.y, Q.n.z - R.n.z);
-        const float DA = xA.x * xA.x + xA.y * xA.y + xA.z * xA.z, DB = xB.x * xB.x + xB.y * xB.y + xB.z * xB.z;
-        const float Da = xa.x * xa.x + xa.y * xa.y + xa.z * xa.z, Dn = xn.x * xn.x + xn.y * xn.y + xn.z * xn.z;
+        const float3 xA = sub3(Q.A, R.A), xB = sub3(Q.B, R.B), xa = sub3(Q.al, R.al), xn = sub3(Q.n, R.n);
+        const float DA = norm2(xA), DB = norm2(xB), Da = norm2(xa), Dn = norm2(xn);
         float cA = 0.f, cB = 0.f, ca = 0.f, cn = 0.f;
         if constexpr (OWN)
         {
-            const float sh = U.k2 * Da + (U.k3 * Dn + U.k4 * r2);
-            const float uA = fast_exp2(U.k0 * DA + sh) * (U.gA.x * R.A.x + U.gA.y * R.A.y + U.gA.z * R.A.z + U.hA);
-            const float uB = fast_exp2(U.k1 * DB + sh) * (U.gB.x * R.B.x + U.gB.y * R.B.y + U.gB.z * R.B.z + U.hB);
-            const float u = uA + uB;
-            cA = U.k0 * uA; cB = U.k1 * uB; ca = U.k2 * u; cn = U.k3 * u;
+            const float2 u2 = sf_grad_tap(g, make_float4(U.k0, U.k1, U.k2, U.k3), U.k4, DA, DB, Da, Dn, r2, U.gA, U.hA,
+                                          R.A, U.gB, U.hB, R.B);
+            const float u = u2.x + u2.y;
+            cA = U.k0 * u2.x; cB = U.k1 * u2.y; ca = U.k2 * u; cn = U.k3 * u;
         }
         {
             const Up V = upstream(k);
@@ -592,9 +592,9 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
         da.x += ca * xa.x; da.y += ca * xa.y; da.z += ca * xa.z;
         dn.x += cn * xn.x; dn.y += cn * xn.y; dn.z += cn * xn.z;
     };
-    const int dy1 = grp ? HALF : 0;
+    const int dy1 = grp ? HALF : -1;  // the split of sf_tile_split<GRAD>, for the same sums
 #pragma unroll 1
-    for (int dy = grp ? 1 : -HALF; dy <= dy1; ++dy)
+    for (int dy = grp ? 0 : -HALF; dy <= dy1; ++dy)
     {
         const int base = q0 + dy * E;
         const float y2 = (float)(dy * dy);
@@ -623,14 +623,18 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
     }
     // the second half of the rows joins through LDS (the tile is dead)
     __syncthreads();
-    float *red = reinterpret_cast<float *>(&s[0][0]);  // [18][256]
-    static_assert(sizeof(s) >= 18 * 256 * sizeof(float), "reduction space");
+    constexpr int NV = BAND ? 23 : 18;
+    float *red = reinterpret_cast<float *>(&s[0][0]);  // [NV][256]
+    static_assert(sizeof(s) >= NV * 256 * sizeof(float), "reduction space");
     if (grp)
     {
         const float v[18] = {dA.x, dA.y, dA.z, dB.x, dB.y, dB.z, da.x, da.y, da.z,
                              dn.x, dn.y, dn.z, eA.x, eA.y, eA.z, eB.x, eB.y, eB.z};
 #pragma unroll
         for (int k = 0; k < 18; ++k) red[k * 256 + t] = v[k];
+        if constexpr (BAND)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) red[(18 + k) * 256 + t] = g[k];
     }
     __syncthreads();
     if (grp || !live) return;
@@ -651,6 +655,12 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
     if (F.gib) st3(F.gib, c, make_float3(eB.x + kScale * dB.x, eB.y + kScale * dB.y, eB.z + kScale * dB.z));
     if (F.galb) st3(F.galb, c, make_float3(kScale * da.x, kScale * da.y, kScale * da.z));
     if (F.gnrm) st3(F.gnrm, c, make_float3(kScale * dn.x, kScale * dn.y, kScale * dn.z));
+    if constexpr (BAND)
+    {
+        float *o = F.gband + 5 * c;
+#pragma unroll
+        for (int k = 0; k < 5; ++k) o[k] = (k == 4 ? -inv_h2 : -1.f) * (g[k] + red[(18 + k) * 256 + t]);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -679,10 +689,10 @@ static void sf_launch(const SfBatch &b, hipStream_t st)
 {
     if (b.map.total <= 256)
         hipLaunchKernelGGL((sf_tile_split<5, MODE, 4>), dim3(b.map.total), dim3(1024), 0, st, b);
-    else if (b.map.total <= 512)
+    else if (MODE == SF_GRAD || b.map.total <= 512)
         hipLaunchKernelGGL((sf_tile_split<5, MODE, 2>), dim3(b.map.total), dim3(512), 0, st, b);
     else
-        hipLaunchKernelGGL((sf_tile<5, MODE>), dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((sf_tile<5>), dim3(b.map.total), dim3(256), 0, st, b);
 }
 
 hipError_t launch_sf_forward(int n, const SfFrame *fr, int win, hipStream_t st)
@@ -707,19 +717,34 @@ hipError_t launch_sf_grad_band(int n, const SfFrame *fr, int win, hipStream_t st
     return hipGetLastError();
 }
 
+// One launch computes both gradients where the band gradient takes the sums of two threads a pixel anyway;
+// up to 256 tiles it takes four, and a second launch costs less than a chain twice as long.
+static bool sf_grad_fused(const SfBatch &b) { return b.f[0].gband && b.half == 5 && b.map.total > 256; }
+
+template <int HALF>
+static void sf_grad_inputs_launch(const SfBatch &b, hipStream_t st)
+{
+    if (HALF == 5 && sf_grad_fused(b))
+        hipLaunchKernelGGL((sf_grad_inputs_tile<5, true>), dim3(b.map.total), dim3(512), 0, st, b);
+    else
+        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, false>), dim3(b.map.total), dim3(512), 0, st, b);
+}
+
 hipError_t launch_sf_grad_inputs(int n, const SfFrame *fr, int win, hipStream_t st)
 {
     SfBatch b = sf_batch(n, fr, win);
     if (b.map.total == 0) return hipSuccess;
+    if (b.f[0].gband && !sf_grad_fused(b))
+        if (hipError_t e = launch_sf_grad_band(n, fr, win, st)) return e;
     switch (b.half)
     {
-    case 1: hipLaunchKernelGGL((sf_grad_inputs_tile<1>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 2: hipLaunchKernelGGL((sf_grad_inputs_tile<2>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 3: hipLaunchKernelGGL((sf_grad_inputs_tile<3>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 4: hipLaunchKernelGGL((sf_grad_inputs_tile<4>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 5: hipLaunchKernelGGL((sf_grad_inputs_tile<5>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 6: hipLaunchKernelGGL((sf_grad_inputs_tile<6>), dim3(b.map.total), dim3(512), 0, st, b); break;
-    case 7: hipLaunchKernelGGL((sf_grad_inputs_tile<7>), dim3(b.map.total), dim3(512), 0, st, b); break;
+    case 1: sf_grad_inputs_launch<1>(b, st); break;
+    case 2: sf_grad_inputs_launch<2>(b, st); break;
+    case 3: sf_grad_inputs_launch<3>(b, st); break;
+    case 4: sf_grad_inputs_launch<4>(b, st); break;
+    case 5: sf_grad_inputs_launch<5>(b, st); break;
+    case 6: sf_grad_inputs_launch<6>(b, st); break;
+    case 7: sf_grad_inputs_launch<7>(b, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

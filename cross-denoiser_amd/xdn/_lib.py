@@ -39,6 +39,7 @@ PROTOTYPES = {
     "xdn_spatial_filter": (_I, [_P] * 9 + [_I] * 4 + [_P]),
     "xdn_spatial_filter_grad": (_I, [_P] * 10 + [_I] * 4 + [_P]),
     "xdn_spatial_filter_grad_inputs": (_I, [_P] * 13 + [_I] * 4 + [_P]),
+    "xdn_spatial_filter_backward": (_I, [_P] * 14 + [_I] * 4 + [_P]),
     "xdn_reproject": (_I, [_P, _I, _PP, _IP] + [_P] * 8 + [_PP] + [_I] * 3 + [_P]),
     "xdn_temporal_screening": (_I, [_P] * 10 + [_I] * 5 + [_P]),
     "xdn_erode_temporal_screening": (_I, [_P] * 11 + [_I] * 5 + [_P]),

@@ -192,6 +192,17 @@ class _SpatialFilterFn(torch.autograd.Function):
 
         g_acca, g_accb, g_wa, g_wb = z(g_acca, 3), z(g_accb, 3), z(g_wa, 1), z(g_wb, 1)
         need = ctx.needs_input_grad
+        if need[4] and any(need[:4]) and ctx.win_size <= 15:  # both gradients in one pass over the windows
+            imga, imgb, albedo, normal, band = _sf_check(imga, imgb, albedo, normal, band)
+            g_acca, g_accb = _img(g_acca, "grad_acca", 3), _img(g_accb, "grad_accb", 3)
+            g_wa, g_wb = _img(g_wa, "grad_wgtsuma", 1), _img(g_wb, "grad_wgtsumb", 1)
+            out = [torch.empty_like(t) if w else None
+                   for t, w in zip((imga, imgb, albedo, normal, band), need)]
+            check(lib.xdn_spatial_filter_backward(ptr(g_acca), ptr(g_accb), ptr(g_wa), ptr(g_wb), ptr(imga),
+                                                  ptr(imgb), ptr(albedo), ptr(normal), ptr(band),
+                                                  *[ptr(o) for o in out], B, H, W, int(ctx.win_size),
+                                                  stream_of(imga)), "spatial_filter_backward")
+            return (*out, None)
         g_band = None
         if need[4]:
             g_band = spatial_filter_grad(g_acca, g_accb, g_wa, g_wb, imga, imgb, albedo, normal, band,

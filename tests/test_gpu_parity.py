@@ -548,6 +548,28 @@ def test_spatial_filter_grad_inputs_edges(ops, dev, B, H, W, win):
         assert err <= TOL, name
 
 
+@pytest.mark.parametrize("B,H,W,win", [(1, 9, 70, 11), (2, 177, 181, 11), (1, 257, 256, 11), (1, 33, 48, 3),
+                                        (1, 9, 8, 15), (1, 20, 24, 17)])
+def test_spatial_filter_backward_all_inputs(ops, dev, B, H, W, win):
+    """Band and image gradients of one backward pass, in one launch (more than 256 tiles) or two: the bits
+    of the two separate ops; windows past 15x15 are refused as by the image gradients."""
+    args = [to_dev(a, dev) for a in sf_case(H, W, seed=5 * H + W, band_lo=0.1, band_hi=3.0, B=B)]
+    cots = [to_dev(c, dev) for c in _cots(B, H, W, 12)]
+    leaves = [a.clone().requires_grad_(True) for a in args]
+    outs = ops.spatial_filter(*leaves, win_size=win)
+    if win > 15:
+        with pytest.raises(ValueError):
+            torch.autograd.grad(outs, leaves, cots)
+        return
+    got = torch.autograd.grad(outs, leaves, cots)
+    ref = list(ops.spatial_filter_grad_inputs(*cots, *args, win_size=win))
+    ref.append(ops.spatial_filter_grad(*cots, *args, win_size=win))
+    for name, g, r in zip(("imga", "imgb", "albedo", "normal", "band"), got, ref):
+        assert torch.equal(g, r), name
+    err = rel_l2(to_np(got[4]), O.spatial_filter_grad(*map(to_np, cots), *map(to_np, args), win_size=win))
+    assert err <= TOL
+
+
 @pytest.mark.parametrize("B,H,W,win,s", [(1, 20, 68, 17, 4), (2, 52, 12, 17, 4), (1, 36, 40, 27, 4), (1, 32, 24, 17, 2),
                                          (1, 24, 20, 5, 4), (1, 17, 19, 3, 1)])
 def test_cross_regression_grad_windows(ops, dev, B, H, W, win, s):
