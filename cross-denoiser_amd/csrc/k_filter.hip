@@ -16,7 +16,7 @@
 //   sf_grad_inputs   gradient w.r.t. the four images (and the bands with BAND), gather form (no atomics): every pixel
 //                    collects its own-center term and the terms of all centers whose (mirrored)
 //                    window contains it, both from one pass over its window; two threads a pixel
-//   sf_generic       any window size, direct loads (forward / grad)
+//   sf_generic       windows past 15x15, direct loads (forward / grad)
 #include "xdn_common.h"
 #include "xdn_kernels.h"
 
@@ -306,7 +306,8 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
 {
     static_assert(MODE == SF_FWD || MODE == SF_GRAD, "the training tile is not split");
     constexpr int E = SF_T + 2 * HALF, NV = MODE == SF_FWD ? 8 : 5;
-    __shared__ float4 s[3][E * E];
+    constexpr int RED = (G - 1) * NV * 256;  // floats of the reduction, which reuses the tile
+    __shared__ float4 s[3][E * E > RED / 12 ? E * E : (RED + 11) / 12];
     const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
     const SfFrame &F = b.f[L.f];
     const int H = F.H, W = F.W;
@@ -378,7 +379,7 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
         for (int k = 0; k < NV; ++k) v[k] = g[k];
     __syncthreads();  // the tile is dead
     float *red = reinterpret_cast<float *>(&s[0][0]);  // [G - 1][NV][256]
-    static_assert(sizeof(s) >= sizeof(float) * (G - 1) * NV * 256, "reduction space");
+    static_assert(sizeof(s) >= sizeof(float) * RED, "reduction space");
     if (grp)
 #pragma unroll
         for (int k = 0; k < NV; ++k) red[((grp - 1) * NV + k) * 256 + t] = v[k];
@@ -684,48 +685,56 @@ static SfBatch sf_batch(int n, const SfFrame *fr, int win)
 // The splits by tiles of the launch, measured forward / band gradient in us a call: 256 tiles, one thread
 // 15.4 / 17.5, two 12.2 / 13.1, four 11.5 / 12.4; 480 tiles 20.0 / 21.4, 18.8 / 21.3, 20.9 / 22.5; from
 // 700 tiles on one thread is as fast as two, four are slower (1024 tiles: 32.8, 33.3, 40.0).
-template <int MODE>
+template <int HALF, int MODE>
 static void sf_launch(const SfBatch &b, hipStream_t st)
 {
     if (b.map.total <= 256)
-        hipLaunchKernelGGL((sf_tile_split<5, MODE, 4>), dim3(b.map.total), dim3(1024), 0, st, b);
+        hipLaunchKernelGGL((sf_tile_split<HALF, MODE, 4>), dim3(b.map.total), dim3(1024), 0, st, b);
     else if (MODE == SF_GRAD || b.map.total <= 512)
-        hipLaunchKernelGGL((sf_tile_split<5, MODE, 2>), dim3(b.map.total), dim3(512), 0, st, b);
+        hipLaunchKernelGGL((sf_tile_split<HALF, MODE, 2>), dim3(b.map.total), dim3(512), 0, st, b);
     else
-        hipLaunchKernelGGL((sf_tile<5>), dim3(b.map.total), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((sf_tile<HALF>), dim3(b.map.total), dim3(256), 0, st, b);
+}
+
+// Windows up to 15x15 have tiled kernels; larger ones take direct loads (win 7, 512x512: forward 43 -> 19,
+// band gradient 43 -> 19 us; 1920x1080: 294 -> 122, 271 -> 141).
+template <int MODE>
+static hipError_t sf_dispatch(const SfBatch &b, hipStream_t st)
+{
+    if (b.map.total == 0) return hipSuccess;
+    switch (b.half)
+    {
+    case 1: sf_launch<1, MODE>(b, st); break;
+    case 2: sf_launch<2, MODE>(b, st); break;
+    case 3: sf_launch<3, MODE>(b, st); break;
+    case 4: sf_launch<4, MODE>(b, st); break;
+    case 5: sf_launch<5, MODE>(b, st); break;
+    case 6: sf_launch<6, MODE>(b, st); break;
+    case 7: sf_launch<7, MODE>(b, st); break;
+    default: hipLaunchKernelGGL((sf_generic<MODE>), dim3(b.map.total), dim3(256), 0, st, b);
+    }
+    return hipGetLastError();
 }
 
 hipError_t launch_sf_forward(int n, const SfFrame *fr, int win, hipStream_t st)
 {
-    SfBatch b = sf_batch(n, fr, win);
-    if (b.map.total == 0) return hipSuccess;
-    if (b.half == 5)
-        sf_launch<SF_FWD>(b, st);
-    else
-        hipLaunchKernelGGL((sf_generic<SF_FWD>), dim3(b.map.total), dim3(256), 0, st, b);
-    return hipGetLastError();
+    return sf_dispatch<SF_FWD>(sf_batch(n, fr, win), st);
 }
 
 hipError_t launch_sf_grad_band(int n, const SfFrame *fr, int win, hipStream_t st)
 {
-    SfBatch b = sf_batch(n, fr, win);
-    if (b.map.total == 0) return hipSuccess;
-    if (b.half == 5)
-        sf_launch<SF_GRAD>(b, st);
-    else
-        hipLaunchKernelGGL((sf_generic<SF_GRAD>), dim3(b.map.total), dim3(256), 0, st, b);
-    return hipGetLastError();
+    return sf_dispatch<SF_GRAD>(sf_batch(n, fr, win), st);
 }
 
 // One launch computes both gradients where the band gradient takes the sums of two threads a pixel anyway;
 // up to 256 tiles it takes four, and a second launch costs less than a chain twice as long.
-static bool sf_grad_fused(const SfBatch &b) { return b.f[0].gband && b.half == 5 && b.map.total > 256; }
+static bool sf_grad_fused(const SfBatch &b) { return b.f[0].gband && b.map.total > 256; }
 
 template <int HALF>
 static void sf_grad_inputs_launch(const SfBatch &b, hipStream_t st)
 {
-    if (HALF == 5 && sf_grad_fused(b))
-        hipLaunchKernelGGL((sf_grad_inputs_tile<5, true>), dim3(b.map.total), dim3(512), 0, st, b);
+    if (sf_grad_fused(b))
+        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, true>), dim3(b.map.total), dim3(512), 0, st, b);
     else
         hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, false>), dim3(b.map.total), dim3(512), 0, st, b);
 }

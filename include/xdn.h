@@ -110,8 +110,7 @@ int xdn_spatial_filter_grad_inputs(const float *grad_acca, const float *grad_acc
                                    float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
                                    int batch, int height, int width, int win_size, void *stream);
 
-/* Both gradients of SpatialFilter, in one pass over the windows of an 11x11 filter on more than 256 16x16
- * tiles: the image gradients (each may be NULL) and grad_band [B,H,W,5], the bits of
+/* Both gradients of SpatialFilter, in one pass over the windows on more than 256 16x16 tiles: the image gradients (each may be NULL) and grad_band [B,H,W,5], the bits of
  * xdn_spatial_filter_grad. win_size <= 15. */
 int xdn_spatial_filter_backward(const float *grad_acca, const float *grad_accb, const float *grad_wgtsuma,
                                 const float *grad_wgtsumb, const float *imga, const float *imgb,

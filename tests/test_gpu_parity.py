@@ -548,8 +548,23 @@ def test_spatial_filter_grad_inputs_edges(ops, dev, B, H, W, win):
         assert err <= TOL, name
 
 
+@pytest.mark.parametrize("H,W,win", [(2, 5, 3), (5, 3, 5), (37, 41, 7), (270, 260, 7), (370, 370, 3), (21, 39, 9),
+                                      (30, 17, 13), (8, 50, 15), (261, 257, 15), (20, 23, 17)])
+def test_spatial_filter_windows(ops, dev, H, W, win):
+    """Every window with a tiled kernel and one without, images down to the smallest, on launches of each
+    split of the window rows."""
+    args = sf_case(H, W, seed=7 * H + W, band_lo=0.1, band_hi=3.0)
+    cots = _cots(1, H, W, 13)
+    dargs = [to_dev(a, dev) for a in args]
+    for name, g, r in zip(("acca", "accb", "wa", "wb"), ops.spatial_filter(*dargs, win_size=win),
+                          O.spatial_filter(*args, win_size=win)):
+        assert rel_l2(to_np(g), r) <= TOL, name
+    got = ops.spatial_filter_grad(*[to_dev(c, dev) for c in cots], *dargs, win_size=win)
+    assert rel_l2(to_np(got), O.spatial_filter_grad(*cots, *args, win_size=win)) <= TOL
+
+
 @pytest.mark.parametrize("B,H,W,win", [(1, 9, 70, 11), (2, 177, 181, 11), (1, 257, 256, 11), (1, 33, 48, 3),
-                                        (1, 9, 8, 15), (1, 20, 24, 17)])
+                                        (1, 260, 261, 7), (2, 181, 179, 3), (1, 9, 8, 15), (1, 20, 24, 17)])
 def test_spatial_filter_backward_all_inputs(ops, dev, B, H, W, win):
     """Band and image gradients of one backward pass, in one launch (more than 256 tiles) or two: the bits
     of the two separate ops; windows past 15x15 are refused as by the image gradients."""
