@@ -64,10 +64,31 @@ size_t xdn_cross_regression_workspace_size(int batch, int height, int width, int
     return (size_t)batch * (size_t)(height / sparsity) * (size_t)(width / sparsity) * 36 * sizeof(float);
 }
 
+namespace {
+// What the backward needs of the forward, per image (256-B aligned): coefficients and Cholesky factors.
+struct CrState {
+    size_t beta, fact, bytes;
+    CrState(int H, int W, int s)
+    {
+        const size_t C = (size_t)(H / s) * (W / s);
+        beta = 0;
+        fact = al256(C * 36 * 4);
+        bytes = fact + al256(C * 2 * 3 * 21 * 4);
+    }
+};
+}  // namespace
+
+size_t xdn_cross_regression_state_size(int batch, int height, int width, int sparsity)
+{
+    if (batch <= 0 || height <= 0 || width <= 0 || sparsity <= 0) return 0;
+    return (size_t)batch * CrState(height, width, sparsity).bytes;
+}
+
+// keep: ws is the state of a later backward instead of the coefficients alone.
 static int cross_regression_impl(const float *color, const float *color2, const float *imga, const float *imgb,
                                  const float *albedo, const float *normal, float *y1, float *y2, float *outa,
                                  float *outb, float *vara, float *varb, void *ws, size_t ws_bytes, int B, int H,
-                                 int W, int win, int s, int rs, void *stream)
+                                 int W, int win, int s, int rs, bool keep, void *stream)
 {
     if (int e = check_shape(B, H, W)) return e;
     if (win < 1 || s < 1 || rs < 1) return fail(XDN_EINVAL, "win_size, sparsity and recon_scale must be >= 1");
@@ -78,10 +99,11 @@ static int cross_regression_impl(const float *color, const float *color2, const 
     if (B == 0) return XDN_OK;  // empty batch: nothing to read or write
     if ((!color && (!imga || !imgb)) || !albedo || !normal || !outa || !outb || !vara || !varb)
         return fail(XDN_EINVAL, "cross_regression: null tensor");
-    if (!ws || ws_bytes < xdn_cross_regression_workspace_size(B, H, W, s))
-        return fail(XDN_EINVAL, "workspace too small: %zu < %zu", ws_bytes, xdn_cross_regression_workspace_size(B, H, W, s));
+    const size_t need = keep ? xdn_cross_regression_state_size(B, H, W, s) : xdn_cross_regression_workspace_size(B, H, W, s);
+    if (!ws || ws_bytes < need) return fail(XDN_EINVAL, "workspace too small: %zu < %zu", ws_bytes, need);
     const bool fused = color != nullptr;
-    const size_t N = px(H, W), Nr = px(H / rs, W / rs), Nb = (size_t)(H / s) * (W / s) * 36;
+    const CrState state(H, W, s);
+    const size_t N = px(H, W), Nr = px(H / rs, W / rs), Nb = keep ? state.bytes : (size_t)(H / s) * (W / s) * 36 * 4;
     for (int b0 = 0; b0 < B; b0 += XDN_MAX_FRAMES / 2)
     {
         const int n = B - b0 < XDN_MAX_FRAMES / 2 ? B - b0 : XDN_MAX_FRAMES / 2;
@@ -98,14 +120,16 @@ static int cross_regression_impl(const float *color, const float *color2, const 
             f.var2 = varb + b * N;
             f.alb = albedo + b * N * 3;
             f.nrm = normal + b * N * 3;
-            f.beta = static_cast<float *>(ws) + b * Nb;
+            char *w = static_cast<char *>(ws) + b * Nb;
+            f.beta = reinterpret_cast<float *>(w);
+            f.fact = keep ? reinterpret_cast<float *>(w + state.fact) : nullptr;
             f.outa = outa + b * Nr * 3;
             f.outb = outb + b * Nr * 3;
             f.H = H;
             f.W = W;
         }
         if (int e = hip_check(xdn::launch_variance(n, fr.data(), 3, fused, S(stream)), "variance")) return e;
-        if (int e = hip_check(xdn::launch_regression(n, fr.data(), win, s, false, S(stream)), "regression")) return e;
+        if (int e = hip_check(xdn::launch_regression(n, fr.data(), win, s, keep, S(stream)), "regression")) return e;
         if (int e = hip_check(xdn::launch_recon(n, fr.data(), win, s, rs, S(stream)), "recon")) return e;
     }
     return XDN_OK;
@@ -117,7 +141,17 @@ int xdn_cross_regression(const float *imga, const float *imgb, const float *albe
 {
     return cross_regression_impl(nullptr, nullptr, imga, imgb, albedo, normal, nullptr, nullptr, outa, outb, out_vara,
                                  out_varb, workspace, workspace_bytes, batch, height, width, win_size, sparsity,
-                                 recon_scale, stream);
+                                 recon_scale, false, stream);
+}
+
+int xdn_cross_regression_keep(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                              float *outa, float *outb, float *out_vara, float *out_varb, void *state,
+                              size_t state_bytes, int batch, int height, int width, int win_size, int sparsity,
+                              void *stream)
+{
+    return cross_regression_impl(nullptr, nullptr, imga, imgb, albedo, normal, nullptr, nullptr, outa, outb, out_vara,
+                                 out_varb, state, state_bytes, batch, height, width, win_size, sparsity, 1, true,
+                                 stream);
 }
 
 int xdn_cross_regression_from_color(const float *color, const float *color2, const float *albedo, const float *normal,
@@ -129,21 +163,20 @@ int xdn_cross_regression_from_color(const float *color, const float *color2, con
         return fail(XDN_EINVAL, "color, color2, y1 and y2 are required");
     return cross_regression_impl(color, color2, nullptr, nullptr, albedo, normal, y1, y2, outa, outb, out_vara,
                                  out_varb, workspace, workspace_bytes, batch, height, width, win_size, sparsity, 1,
-                                 stream);
+                                 false, stream);
 }
 
 namespace {
 // Workspace of the cross-regression backward, per image (every buffer 256-B aligned).
 struct CrgLayout {
-    size_t var1, var2, beta, fact, gq, u, gcen, evar, bytes;
-    CrgLayout(int H, int W, int s)
+    size_t var1, var2, state, gq, u, gcen, evar, bytes;
+    CrgLayout(int H, int W, int s, bool kept)
     {
         const size_t N = px(H, W), C = (size_t)(H / s) * (W / s);
         size_t o = 0;
         var1 = o; o += al256(N * 4);
         var2 = o; o += al256(N * 4);
-        beta = o; o += al256(C * 36 * 4);
-        fact = o; o += al256(C * 2 * 3 * 21 * 4);
+        state = o; o += kept ? 0 : CrState(H, W, s).bytes;
         gq = o; o += al256(N * 2 * 16);
         u = o; o += al256(C * 36 * 4);
         gcen = o; o += al256(C * 24 * 4);
@@ -156,14 +189,21 @@ struct CrgLayout {
 size_t xdn_cross_regression_grad_workspace_size(int batch, int height, int width, int sparsity)
 {
     if (batch <= 0 || height <= 0 || width <= 0 || sparsity <= 0) return 0;
-    return (size_t)batch * CrgLayout(height, width, sparsity).bytes;
+    return (size_t)batch * CrgLayout(height, width, sparsity, false).bytes;
 }
 
-int xdn_cross_regression_grad(const float *imga, const float *imgb, const float *albedo, const float *normal,
-                              const float *grad_outa, const float *grad_outb, const float *grad_vara,
-                              const float *grad_varb, float *grad_imga, float *grad_imgb, float *grad_albedo,
-                              float *grad_normal, void *workspace, size_t workspace_bytes, int B, int H, int W,
-                              int win, int s, void *stream)
+size_t xdn_cross_regression_grad_kept_workspace_size(int batch, int height, int width, int sparsity)
+{
+    if (batch <= 0 || height <= 0 || width <= 0 || sparsity <= 0) return 0;
+    return (size_t)batch * CrgLayout(height, width, sparsity, true).bytes;
+}
+
+// state: what xdn_cross_regression_keep left, or null: computed here, in the workspace.
+static int cross_regression_grad_impl(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                                      const void *state, const float *grad_outa, const float *grad_outb,
+                                      const float *grad_vara, const float *grad_varb, float *grad_imga,
+                                      float *grad_imgb, float *grad_albedo, float *grad_normal, void *workspace,
+                                      size_t workspace_bytes, int B, int H, int W, int win, int s, void *stream)
 {
     if (int e = check_shape(B, H, W)) return e;
     if (win < 1 || s < 1) return fail(XDN_EINVAL, "win_size and sparsity must be >= 1");
@@ -173,10 +213,11 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
     if (!imga || !imgb || !albedo || !normal || !grad_outa || !grad_outb || !grad_imga || !grad_imgb ||
         !grad_albedo || !grad_normal)
         return fail(XDN_EINVAL, "cross_regression_grad: null tensor");
-    const size_t need = xdn_cross_regression_grad_workspace_size(B, H, W, s);
+    const CrgLayout lay(H, W, s, state != nullptr);
+    const CrState kept(H, W, s);
+    const size_t need = (size_t)B * lay.bytes;
     if (!workspace || workspace_bytes < need)
         return fail(XDN_EINVAL, "workspace too small: %zu < %zu", workspace_bytes, need);
-    const CrgLayout lay(H, W, s);
     const size_t N = px(H, W);
     for (int b0 = 0; b0 < B; b0 += XDN_MAX_FRAMES / 2)
     {
@@ -195,8 +236,9 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
             f.var2 = reinterpret_cast<float *>(w + lay.var2);
             f.alb = albedo + b * N * 3;
             f.nrm = normal + b * N * 3;
-            f.beta = reinterpret_cast<float *>(w + lay.beta);
-            f.fact = reinterpret_cast<float *>(w + lay.fact);
+            char *st = state ? const_cast<char *>(static_cast<const char *>(state)) + b * kept.bytes : w + lay.state;
+            f.beta = reinterpret_cast<float *>(st + kept.beta);
+            f.fact = reinterpret_cast<float *>(st + kept.fact);
             f.H = H;
             f.W = W;
             xdn::CrgFrame &g = fr[i];
@@ -218,12 +260,39 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
             g.W = W;
         }
         if (int e = hip_check(xdn::launch_variance(n, fw.data(), 3, false, S(stream)), "variance")) return e;
-        if (int e = hip_check(xdn::launch_regression(n, fw.data(), win, s, true, S(stream)), "regression")) return e;
+        if (!state)
+            if (int e = hip_check(xdn::launch_regression(n, fw.data(), win, s, true, S(stream)), "regression")) return e;
         if (int e = hip_check(xdn::launch_cross_regression_grad(n, fr.data(), win, s, S(stream)),
                               "cross_regression_grad"))
             return e;
     }
     return XDN_OK;
+}
+
+int xdn_cross_regression_grad(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                              const float *grad_outa, const float *grad_outb, const float *grad_vara,
+                              const float *grad_varb, float *grad_imga, float *grad_imgb, float *grad_albedo,
+                              float *grad_normal, void *workspace, size_t workspace_bytes, int B, int H, int W,
+                              int win, int s, void *stream)
+{
+    return cross_regression_grad_impl(imga, imgb, albedo, normal, nullptr, grad_outa, grad_outb, grad_vara, grad_varb,
+                                      grad_imga, grad_imgb, grad_albedo, grad_normal, workspace, workspace_bytes, B, H,
+                                      W, win, s, stream);
+}
+
+int xdn_cross_regression_grad_kept(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                                   const void *state, size_t state_bytes, const float *grad_outa,
+                                   const float *grad_outb, const float *grad_vara, const float *grad_varb,
+                                   float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
+                                   void *workspace, size_t workspace_bytes, int B, int H, int W, int win, int s,
+                                   void *stream)
+{
+    const size_t need = xdn_cross_regression_state_size(B, H, W, s);
+    if (B > 0 && (!state || state_bytes < need))
+        return fail(XDN_EINVAL, "cross_regression_grad_kept: state too small: %zu < %zu", state_bytes, need);
+    return cross_regression_grad_impl(imga, imgb, albedo, normal, state, grad_outa, grad_outb, grad_vara, grad_varb,
+                                      grad_imga, grad_imgb, grad_albedo, grad_normal, workspace, workspace_bytes, B, H,
+                                      W, win, s, stream);
 }
 
 static int sf_common_check(int B, int H, int W, int win)

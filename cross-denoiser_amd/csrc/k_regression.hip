@@ -716,7 +716,8 @@ hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hip
 constexpr int kRowsFewBlocks = 640;
 
 // batch_invariant: a frame's coefficients are the same bits whatever it is launched with, regression_rows
-// at any size: the training step, whose streams give the same results alone and batched, and the backward,
+// at any size: the training step, whose streams give the same results alone and batched, and the backward (or the
+// forward that keeps its factors for one),
 // whose solves turn another summation order into up to 2e-5 of the normals' gradient.
 hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batch_invariant, hipStream_t st)
 {

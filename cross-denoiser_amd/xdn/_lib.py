@@ -36,6 +36,10 @@ PROTOTYPES = {
     "xdn_cross_regression_from_color": (_I, [_P] * 10 + [_P, _Z] + [_I] * 5 + [_P]),
     "xdn_cross_regression_grad_workspace_size": (_Z, [_I, _I, _I, _I]),
     "xdn_cross_regression_grad": (_I, [_P] * 12 + [_P, _Z] + [_I] * 5 + [_P]),
+    "xdn_cross_regression_state_size": (_Z, [_I, _I, _I, _I]),
+    "xdn_cross_regression_keep": (_I, [_P] * 8 + [_P, _Z] + [_I] * 5 + [_P]),
+    "xdn_cross_regression_grad_kept_workspace_size": (_Z, [_I, _I, _I, _I]),
+    "xdn_cross_regression_grad_kept": (_I, [_P] * 5 + [_Z] + [_P] * 8 + [_P, _Z] + [_I] * 5 + [_P]),
     "xdn_spatial_filter": (_I, [_P] * 9 + [_I] * 4 + [_P]),
     "xdn_spatial_filter_grad": (_I, [_P] * 10 + [_I] * 4 + [_P]),
     "xdn_spatial_filter_grad_inputs": (_I, [_P] * 13 + [_I] * 4 + [_P]),

@@ -60,37 +60,44 @@ def _same_hw(ref: torch.Tensor, *ts) -> None:
 
 
 # ---------------------------------------------------------------------------------------------
-def _cr_forward(imga, imgb, albedo, normal, win_size, sparsity, rs):
+def _cr_forward(imga, imgb, albedo, normal, win_size, sparsity, rs, keep=False):
+    """The op's four outputs and, with `keep`, the state that its backward takes (else None)."""
     B, H, W, C = imga.shape
     outa = imga.new_empty((B, H // rs, W // rs, C))
     outb = torch.empty_like(outa)
     vara = imga.new_empty((B, H, W, 1))
     varb = torch.empty_like(vara)
+    if keep:
+        n = lib.xdn_cross_regression_state_size(B, H, W, sparsity)
+        state = imga.new_empty(max(n, 4) // 4)
+        check(lib.xdn_cross_regression_keep(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(outa), ptr(outb),
+                                            ptr(vara), ptr(varb), ptr(state), n, B, H, W, win_size, sparsity,
+                                            stream_of(imga)), "cross_regression")
+        return (outa, outb, vara, varb), state
     ws_bytes = lib.xdn_cross_regression_workspace_size(B, H, W, int(sparsity))
     ws = imga.new_empty(max(ws_bytes, 4) // 4)
     check(lib.xdn_cross_regression(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(outa), ptr(outb),
                                    ptr(vara), ptr(varb), ptr(ws), ws_bytes, B, H, W, int(win_size),
                                    int(sparsity), rs, stream_of(imga)), "cross_regression")
-    return outa, outb, vara, varb
+    return (outa, outb, vara, varb), None
 
 
 class _CrossRegressionFn(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, imga, imgb, albedo, normal, win_size, sparsity, rs):
-        outs = _cr_forward(imga, imgb, albedo, normal, win_size, sparsity, rs)
-        ctx.save_for_backward(imga, imgb, albedo, normal)
+    def forward(ctx, imga, imgb, albedo, normal, win_size, sparsity, rs, keep):
+        outs, state = _cr_forward(imga, imgb, albedo, normal, win_size, sparsity, rs, keep)
+        ctx.save_for_backward(imga, imgb, albedo, normal, state)
         ctx.args = (win_size, sparsity, rs)
         return outs
 
     @staticmethod
     def backward(ctx, g_outa, g_outb, g_vara, g_varb):
-        imga, imgb, albedo, normal = ctx.saved_tensors
+        imga, imgb, albedo, normal, state = ctx.saved_tensors
         win_size, sparsity, rs = ctx.args
         if rs != 1:
             raise NotImplementedError("cross_regression backward supports recon_scale 1 only")
-        g = cross_regression_grad(imga, imgb, albedo, normal, g_outa, g_outb, g_vara, g_varb, win_size=win_size,
-                                  sparsity=sparsity)
-        return g[0], g[1], g[2], g[3], None, None, None
+        g = _cr_grad(imga, imgb, albedo, normal, g_outa, g_outb, g_vara, g_varb, win_size, sparsity, state)
+        return g[0], g[1], g[2], g[3], None, None, None, None
 
 
 def cross_regression(imga, imgb, albedo, normal, win_size, sparsity, recon_scale=1, name=None):
@@ -105,13 +112,20 @@ def cross_regression(imga, imgb, albedo, normal, win_size, sparsity, recon_scale
         raise ValueError("recon_scale must be less than or equal to sparsity")
     if H % recon_scale or W % recon_scale:
         raise ValueError("Image height and width must be divisible by recon_scale")
-    return _CrossRegressionFn.apply(imga, imgb, albedo, normal, int(win_size), int(sparsity), int(recon_scale))
+    keep = (recon_scale == 1 and torch.is_grad_enabled()
+            and any(t.requires_grad for t in (imga, imgb, albedo, normal)))
+    return _CrossRegressionFn.apply(imga, imgb, albedo, normal, int(win_size), int(sparsity), int(recon_scale), keep)
 
 
 def cross_regression_grad(imga, imgb, albedo, normal, grad_outa, grad_outb, grad_vara=None, grad_varb=None, *,
                           win_size, sparsity):
     """(d imga, d imgb, d albedo, d normal) of cross_regression (recon_scale 1), window weights
     recomputed. ``grad_vara``/``grad_varb`` may be None (zero)."""
+    return _cr_grad(imga, imgb, albedo, normal, grad_outa, grad_outb, grad_vara, grad_varb, win_size, sparsity, None)
+
+
+def _cr_grad(imga, imgb, albedo, normal, grad_outa, grad_outb, grad_vara, grad_varb, win_size, sparsity, state):
+    """The gradients, from the forward's kept `state` where there is one."""
     imga, imgb = _img(imga, "imga", 3), _img(imgb, "imgb", 3)
     albedo, normal = _img(albedo, "albedo", 3), _img(normal, "normal", 3)
     B, H, W, _ = imga.shape
@@ -125,11 +139,22 @@ def cross_regression_grad(imga, imgb, albedo, normal, grad_outa, grad_outb, grad
     gva, gvb = g(grad_vara, "grad_vara", 1), g(grad_varb, "grad_varb", 1)
     _same_hw(imga, ("imgb", imgb), ("albedo", albedo), ("normal", normal), ("grad_outa", ga), ("grad_outb", gb))
     outs = [torch.empty_like(imga) for _ in range(4)]
-    ws_bytes = lib.xdn_cross_regression_grad_workspace_size(B, H, W, int(sparsity))
+    win_size, sparsity = int(win_size), int(sparsity)
+    cots, stream = [ptr(t) for t in (ga, gb, gva, gvb)], stream_of(imga)
+    if state is None:
+        ws_bytes = lib.xdn_cross_regression_grad_workspace_size(B, H, W, sparsity)
+        ws = imga.new_empty(max(ws_bytes, 4) // 4)
+        check(lib.xdn_cross_regression_grad(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), *cots,
+                                            *[ptr(o) for o in outs], ptr(ws), ws_bytes, B, H, W, win_size, sparsity,
+                                            stream), "cross_regression_grad")
+        return tuple(outs)
+    if state.device != imga.device or state.dtype != torch.float32 or not state.is_contiguous():
+        raise ValueError("cross_regression: the saved state is no longer a contiguous float32 tensor of its device")
+    ws_bytes = lib.xdn_cross_regression_grad_kept_workspace_size(B, H, W, sparsity)
     ws = imga.new_empty(max(ws_bytes, 4) // 4)
-    check(lib.xdn_cross_regression_grad(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(ga), ptr(gb), ptr(gva),
-                                        ptr(gvb), *[ptr(o) for o in outs], ptr(ws), ws_bytes, B, H, W, int(win_size),
-                                        int(sparsity), stream_of(imga)), "cross_regression_grad")
+    check(lib.xdn_cross_regression_grad_kept(ptr(imga), ptr(imgb), ptr(albedo), ptr(normal), ptr(state),
+                                             4 * state.numel(), *cots, *[ptr(o) for o in outs], ptr(ws), ws_bytes,
+                                             B, H, W, win_size, sparsity, stream), "cross_regression_grad")
     return tuple(outs)
 
 

@@ -82,6 +82,23 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
                               float *grad_normal, void *workspace, size_t workspace_bytes, int batch, int height,
                               int width, int win_size, int sparsity, void *stream);
 
+/* The op for a caller that will differentiate it (recon_scale 1): `state`, caller-owned,
+ * xdn_cross_regression_state_size() bytes, receives the regression coefficients and Cholesky factors, and
+ * xdn_cross_regression_grad_kept on the same images gives the gradients of xdn_cross_regression_grad, bit
+ * for bit, without running the regression again. The state is only read there. */
+size_t xdn_cross_regression_state_size(int batch, int height, int width, int sparsity);
+int xdn_cross_regression_keep(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                              float *outa, float *outb, float *out_vara, float *out_varb, void *state,
+                              size_t state_bytes, int batch, int height, int width, int win_size, int sparsity,
+                              void *stream);
+size_t xdn_cross_regression_grad_kept_workspace_size(int batch, int height, int width, int sparsity);
+int xdn_cross_regression_grad_kept(const float *imga, const float *imgb, const float *albedo, const float *normal,
+                                   const void *state, size_t state_bytes, const float *grad_outa,
+                                   const float *grad_outb, const float *grad_vara, const float *grad_varb,
+                                   float *grad_imga, float *grad_imgb, float *grad_albedo, float *grad_normal,
+                                   void *workspace, size_t workspace_bytes, int batch, int height, int width,
+                                   int win_size, int sparsity, void *stream);
+
 /* ---------------------------------------------------------------------------------------------
  * SpatialFilter op: replaces REGISTER_OP("SpatialFilter") / SpatialFilterOp::Compute
  * (ops/regression.cc:59-86, 235-282) and SpatialFilterFunc (ops/regression.cu.cc:502-517).

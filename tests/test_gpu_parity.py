@@ -585,6 +585,25 @@ def test_spatial_filter_backward_all_inputs(ops, dev, B, H, W, win):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("B,H,W,win,s", [(1, 32, 40, 17, 4), (9, 24, 28, 17, 4), (1, 36, 40, 27, 4), (2, 26, 24, 13, 2)])
+def test_cross_regression_autograd_kept_state(ops, dev, B, H, W, win, s):
+    """The backward from the forward's kept factors: the bits of cross_regression_grad, twice in a row,
+    with more images than one launch takes and for windows without tiled kernels."""
+    args = [to_dev(a, dev) for a in cr_grad_case(H, W, seed=H + W, B=B)]
+    cots = [to_dev(c, dev) for c in _cots(B, H, W, 17)]
+    leaves = [a.clone().requires_grad_(True) for a in args]
+    outs = ops.cross_regression(*leaves, win_size=win, sparsity=s)
+    ref = ops.cross_regression_grad(*args, *cots, win_size=win, sparsity=s)
+    for _ in range(2):
+        got = torch.autograd.grad(outs, leaves, cots, retain_graph=True)
+        for name, g, r in zip(("imga", "imgb", "albedo", "normal"), got, ref):
+            assert torch.equal(g, r), name
+    with torch.no_grad():
+        plain = ops.cross_regression(*leaves, win_size=win, sparsity=s)
+    for o, r in zip(outs, plain):
+        assert rel_l2(to_np(o.detach()), to_np(r)) <= TOL
+
+
 @pytest.mark.parametrize("B,H,W,win,s", [(1, 20, 68, 17, 4), (2, 52, 12, 17, 4), (1, 36, 40, 27, 4), (1, 32, 24, 17, 2),
                                          (1, 24, 20, 5, 4), (1, 17, 19, 3, 1)])
 def test_cross_regression_grad_windows(ops, dev, B, H, W, win, s):
