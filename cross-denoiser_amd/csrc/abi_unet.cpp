@@ -16,35 +16,40 @@ namespace {
 
 using Frames = const UnetFrame *;
 
-// 3x3 convolution of layer l over every image: forward from concat[a, b] (the images when a < 0)
-// into buffer out, or (dgrad) data gradient from buffer a into out, masked by buffer mask's ReLU
-// (unmasked when mask < 0).
-int conv(Frames F, int n, hipStream_t st, int kind, int l, int a, int b, int out, int mask, bool dgrad,
-         const char *what)
+// 3x3 convolution of layer l over image U: forward from concat[a, b] (the images when a < 0) into buffer
+// out, or (dgrad) data gradient from buffer a into out, masked by buffer mask's ReLU (unmasked when
+// mask < 0).
+xdn::UcFrame conv_frame(const UnetFrame &U, int l, int a, int b, int out, int mask, bool dgrad)
 {
     const int lv = kUnet[l].level;
+    xdn::UcFrame f;
+    memset(&f, 0, sizeof(f));
+    if (a >= 0)
+        f.a = U.buf[a];
+    else
+        for (int k = 0; k < 5; ++k) f.img[k] = U.img[k];
+    f.b = b >= 0 ? U.buf[b] : nullptr;
+    f.out = U.buf[out];
+    f.mask = mask >= 0 ? reinterpret_cast<const uint16_t *>(U.buf[mask]) : nullptr;
+    f.wfrag = U.pk + (dgrad ? kULay.dg_off[l] : kULay.fwd_off[l]);
+    f.bias = reinterpret_cast<const float *>(U.pk + kULay.bias_off[l]);
+    f.H = U.h[lv];
+    f.W = U.w[lv];
+    return f;
+}
+
+// forward of 3x3 layer l over every image
+int conv(Frames F, int n, hipStream_t st, int kind, int l, int a, int b, int out, const char *what)
+{
     std::vector<xdn::UcFrame> fr(n);
     for (int i = 0; i < n; ++i)
     {
-        const UnetFrame &U = F[i];
-        xdn::UcFrame &f = fr[i];
-        memset(&f, 0, sizeof(f));
-        if (a >= 0)
-            f.a = U.buf[a];
-        else
-            for (int k = 0; k < 5; ++k) f.img[k] = U.img[k];
-        f.b = b >= 0 ? U.buf[b] : nullptr;
-        f.out = U.buf[out];
-        f.mask = mask >= 0 ? reinterpret_cast<const uint16_t *>(U.buf[mask]) : nullptr;
-        f.wfrag = U.pk + (dgrad ? kULay.dg_off[l] : kULay.fwd_off[l]);
-        f.bias = reinterpret_cast<const float *>(U.pk + kULay.bias_off[l]);
+        fr[i] = conv_frame(F[i], l, a, b, out, -1, false);
         if (kind == xdn::UC_F_24_8_HEAD)
         {
-            f.head_w = reinterpret_cast<const float *>(U.pk + kULay.master_off[11]);
-            f.head_out = U.param;
+            fr[i].head_w = reinterpret_cast<const float *>(F[i].pk + kULay.master_off[11]);
+            fr[i].head_out = F[i].param;
         }
-        f.H = U.h[lv];
-        f.W = U.w[lv];
     }
     return hip_check(xdn::launch_uconv(kind, n, fr.data(), st), what);
 }
@@ -81,27 +86,44 @@ int convT(Frames F, int n, hipStream_t st, int l, int in, int out)
 }
 
 // weight gradient of partial set j over concat[a, b] (or the images) and dY buffer dy
-int wgrad(Frames F, int n, hipStream_t st, int kind, int j, int a, int b, int dy)
+xdn::UwFrame wgrad_frame(const UnetFrame &U, int j, int a, int b, int dy)
 {
     const int lv = kUnetJob[j].level;
-    std::vector<xdn::UwFrame> fr(n);
+    xdn::UwFrame f;
+    memset(&f, 0, sizeof(f));
+    if (a >= 0)
+        f.a = U.buf[a];
+    else
+        for (int k = 0; k < 5; ++k) f.img[k] = U.img[k];
+    f.b = b >= 0 ? U.buf[b] : nullptr;
+    f.dy = reinterpret_cast<const uint16_t *>(U.buf[dy]);
+    f.part = U.part[j];
+    f.nblk = U.nblk[j];
+    f.H = U.h[lv];
+    f.W = U.w[lv];
+    return f;
+}
+
+// both gradients of 3x3 layer l over concat[a, b]: weights from dY buffer dy into partial set j (channels 32
+// and up into the next one), data into buffer out, masked by buffer mask's ReLU (unmasked when mask < 0)
+int backward(Frames F, int n, hipStream_t st, int kind, int l, int j, int a, int b, int dy, int out, int mask)
+{
+    std::vector<xdn::UwFrame> wf(n);
+    std::vector<xdn::UcFrame> cf(n);
     for (int i = 0; i < n; ++i)
     {
-        const UnetFrame &U = F[i];
-        xdn::UwFrame &f = fr[i];
-        memset(&f, 0, sizeof(f));
-        if (a >= 0)
-            f.a = U.buf[a];
-        else
-            for (int k = 0; k < 5; ++k) f.img[k] = U.img[k];
-        f.b = b >= 0 ? U.buf[b] : nullptr;
-        f.dy = reinterpret_cast<const uint16_t *>(U.buf[dy]);
-        f.part = U.part[j];
-        f.nblk = U.nblk[j];
-        f.H = U.h[lv];
-        f.W = U.w[lv];
+        wf[i] = wgrad_frame(F[i], j, a, b, dy);
+        if (kind == xdn::UBW_48_16) wf[i].part_m1 = F[i].part[j + 1];
+        cf[i] = conv_frame(F[i], l, dy, -1, out, mask, true);
     }
-    return hip_check(xdn::launch_uwgrad(kind, n, fr.data(), st), "unet wgrad");
+    return hip_check(xdn::launch_ubackward(kind, n, wf.data(), cf.data(), st), "unet layer backward");
+}
+
+int wgrad_images(Frames F, int n, hipStream_t st, int j, int dy)
+{
+    std::vector<xdn::UwFrame> fr(n);
+    for (int i = 0; i < n; ++i) fr[i] = wgrad_frame(F[i], j, -1, -1, dy);
+    return hip_check(xdn::launch_uwgrad_images(n, fr.data(), st), "unet wgrad");
 }
 
 // transposed layer l backward (partial set j): input buffer in, gradient of its output in buffer
@@ -194,20 +216,20 @@ int unet_forward_frames(const UnetFrame *F, int n, hipStream_t st)
 {
     using namespace xdn;
     int e = 0;
-    if ((e = conv(F, n, st, UC_F_0, 0, -1, -1, UB_A0, -1, false, "unet c1_1"))) return e;
-    if ((e = conv(F, n, st, UC_F_8_8, 1, UB_A0, -1, UB_A1, -1, false, "unet c1_2"))) return e;
+    if ((e = conv(F, n, st, UC_F_0, 0, -1, -1, UB_A0, "unet c1_1"))) return e;
+    if ((e = conv(F, n, st, UC_F_8_8, 1, UB_A0, -1, UB_A1, "unet c1_2"))) return e;
     if ((e = pool(F, n, st, 8, UB_A1, UB_P1))) return e;
-    if ((e = conv(F, n, st, UC_F_8_16, 2, UB_P1, -1, UB_A2, -1, false, "unet c2_1"))) return e;
-    if ((e = conv(F, n, st, UC_F_16_16, 3, UB_A2, -1, UB_A3, -1, false, "unet c2_2"))) return e;
+    if ((e = conv(F, n, st, UC_F_8_16, 2, UB_P1, -1, UB_A2, "unet c2_1"))) return e;
+    if ((e = conv(F, n, st, UC_F_16_16, 3, UB_A2, -1, UB_A3, "unet c2_2"))) return e;
     if ((e = pool(F, n, st, 16, UB_A3, UB_P2))) return e;
-    if ((e = conv(F, n, st, UC_F_16_32, 4, UB_P2, -1, UB_A4, -1, false, "unet c3_1"))) return e;
-    if ((e = conv(F, n, st, UC_F_32_32, 5, UB_A4, -1, UB_A5, -1, false, "unet c3_2"))) return e;
+    if ((e = conv(F, n, st, UC_F_16_32, 4, UB_P2, -1, UB_A4, "unet c3_1"))) return e;
+    if ((e = conv(F, n, st, UC_F_32_32, 5, UB_A4, -1, UB_A5, "unet c3_2"))) return e;
     if ((e = convT(F, n, st, 6, UB_A5, UB_A6))) return e;                                       // c3_3
-    if ((e = conv(F, n, st, UC_F_48_16, 7, UB_A6, UB_A3, UB_A7, -1, false, "unet c4_1"))) return e;  // [c3_3, c2_2]
-    if ((e = conv(F, n, st, UC_F_16_16, 8, UB_A7, -1, UB_A8, -1, false, "unet c4_2"))) return e;
+    if ((e = conv(F, n, st, UC_F_48_16, 7, UB_A6, UB_A3, UB_A7, "unet c4_1"))) return e;  // [c3_3, c2_2]
+    if ((e = conv(F, n, st, UC_F_16_16, 8, UB_A7, -1, UB_A8, "unet c4_2"))) return e;
     if ((e = convT(F, n, st, 9, UB_A8, UB_A9))) return e;                                       // c4_3
     // c5_1 over [c4_3, c1_2], with the 1x1 head applied in its epilogue
-    return conv(F, n, st, UC_F_24_8_HEAD, 10, UB_A9, UB_A1, UB_A10, -1, false, "unet c5_1 + head");
+    return conv(F, n, st, UC_F_24_8_HEAD, 10, UB_A9, UB_A1, UB_A10, "unet c5_1 + head");
 }
 
 int unet_backward_frames(const UnetFrame *F, int n, hipStream_t st)
@@ -215,30 +237,21 @@ int unet_backward_frames(const UnetFrame *F, int n, hipStream_t st)
     using namespace xdn;
     int e = 0;
     if ((e = head_bwd(F, n, st))) return e;                                      // dY10, set 12
-    if ((e = wgrad(F, n, st, UW_24_8, 11, UB_A9, UB_A1, UB_DY10))) return e;     // c5_1
-    if ((e = conv(F, n, st, UC_D_8_24, 10, UB_DY10, -1, UB_DC5, -1, true, "unet c5_1 dgrad"))) return e;
+    if ((e = backward(F, n, st, UBW_24_8, 10, 11, UB_A9, UB_A1, UB_DY10, UB_DC5, -1))) return e;    // c5_1
     if ((e = convT_bwd(F, n, st, 9, 10, UB_A8, UB_DC5, UB_DY8))) return e;       // c4_3 <- dC5[:, 0:16]
-    if ((e = wgrad(F, n, st, UW_16_16, 9, UB_A7, -1, UB_DY8))) return e;         // c4_2
-    if ((e = conv(F, n, st, UC_D_16_16, 8, UB_DY8, -1, UB_DY7, UB_A7, true, "unet c4_2 dgrad"))) return e;
-    if ((e = wgrad(F, n, st, UW_48_16_M0, 7, UB_A6, UB_A3, UB_DY7))) return e;   // c4_1, inputs 0-31
-    if ((e = wgrad(F, n, st, UW_48_16_M1, 8, UB_A6, UB_A3, UB_DY7))) return e;   // c4_1, inputs 32-47
-    if ((e = conv(F, n, st, UC_D_16_48, 7, UB_DY7, -1, UB_DC4, -1, true, "unet c4_1 dgrad"))) return e;
+    if ((e = backward(F, n, st, UBW_16_16, 8, 9, UB_A7, -1, UB_DY8, UB_DY7, UB_A7))) return e;      // c4_2
+    if ((e = backward(F, n, st, UBW_48_16, 7, 7, UB_A6, UB_A3, UB_DY7, UB_DC4, -1))) return e;      // c4_1
     if ((e = convT_bwd(F, n, st, 6, 6, UB_A5, UB_DC4, UB_DY5))) return e;        // c3_3 <- dC4[:, 0:32]
-    if ((e = wgrad(F, n, st, UW_32_32, 5, UB_A4, -1, UB_DY5))) return e;         // c3_2
-    if ((e = conv(F, n, st, UC_D_32_32, 5, UB_DY5, -1, UB_DY4, UB_A4, true, "unet c3_2 dgrad"))) return e;
-    if ((e = wgrad(F, n, st, UW_16_32, 4, UB_P2, -1, UB_DY4))) return e;         // c3_1
-    if ((e = conv(F, n, st, UC_D_32_16, 4, UB_DY4, -1, UB_DP2, -1, true, "unet c3_1 dgrad"))) return e;
+    if ((e = backward(F, n, st, UBW_32_32, 5, 5, UB_A4, -1, UB_DY5, UB_DY4, UB_A4))) return e;      // c3_2
+    if ((e = backward(F, n, st, UBW_16_32, 4, 4, UB_P2, -1, UB_DY4, UB_DP2, -1))) return e;         // c3_1
     // c2_2's output feeds the second pool and the skip into c4_1 (dC4[:, 32:48])
     if ((e = pool_bwd(F, n, st, 16, UB_DP2, UB_A3, UB_DC4, 32, UB_DY3))) return e;
-    if ((e = wgrad(F, n, st, UW_16_16, 3, UB_A2, -1, UB_DY3))) return e;         // c2_2
-    if ((e = conv(F, n, st, UC_D_16_16, 3, UB_DY3, -1, UB_DY2, UB_A2, true, "unet c2_2 dgrad"))) return e;
-    if ((e = wgrad(F, n, st, UW_8_16, 2, UB_P1, -1, UB_DY2))) return e;          // c2_1
-    if ((e = conv(F, n, st, UC_D_16_8, 2, UB_DY2, -1, UB_DP1, -1, true, "unet c2_1 dgrad"))) return e;
+    if ((e = backward(F, n, st, UBW_16_16, 3, 3, UB_A2, -1, UB_DY3, UB_DY2, UB_A2))) return e;      // c2_2
+    if ((e = backward(F, n, st, UBW_8_16, 2, 2, UB_P1, -1, UB_DY2, UB_DP1, -1))) return e;          // c2_1
     // c1_2's output feeds the first pool and the skip into c5_1 (dC5[:, 16:24])
     if ((e = pool_bwd(F, n, st, 8, UB_DP1, UB_A1, UB_DC5, 16, UB_DY1))) return e;
-    if ((e = wgrad(F, n, st, UW_8_8, 1, UB_A0, -1, UB_DY1))) return e;           // c1_2
-    if ((e = conv(F, n, st, UC_D_8_8, 1, UB_DY1, -1, UB_DY0, UB_A0, true, "unet c1_2 dgrad"))) return e;
-    return wgrad(F, n, st, UW_0, 0, -1, -1, UB_DY0);                             // c1_1
+    if ((e = backward(F, n, st, UBW_8_8, 1, 1, UB_A0, -1, UB_DY1, UB_DY0, UB_A0))) return e;        // c1_2
+    return wgrad_images(F, n, st, 0, UB_DY0);                                    // c1_1
 }
 
 xdn::RedJob unet_red_job(int set, float *part, float *grad, int nblk_total)

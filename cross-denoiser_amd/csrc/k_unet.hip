@@ -6,9 +6,11 @@
 //     every B fragment feeds up to three output rows. Forward
 //     (bias + ReLU -> bf16) and data gradient (flipped, transposed fragments; ReLU-masked, or
 //     plain for concat and pooled inputs). Channel counts are the stored ones (8, 16, 24, 32, 48).
-//   uwgrad<SRC, CA, CB, CO, MT, DEPTH>  weight gradient over 8x32-px strips, operands from pixel-major
+//   uwgrad_block<SRC, CA, CB, CO, MT, DEPTH>  weight gradient over 8x32-px strips, operands from pixel-major
 //     LDS tiles through ds_read_b64_tr_b16, one 32-channel input slice (MT) per instantiation,
 //     software-pipelined strip loop.
+//   ubackward                    weight and data gradient of a layer in one launch (uwgrad_images: the
+//                                first layer's weight gradient alone).
 //   maxpool2 / pool_bwd          2x2 max pool and its gradient (to the first maximum, plus the
 //     skip-connection gradient, ReLU-masked).
 //   convT1x1s2 / convT_bwd       transposed 1x1 stride-2 convolution and its gradients.
@@ -119,18 +121,23 @@ __device__ __forceinline__ uint32_t u_cvt2(float a, float b)
 // with only the even pixels of the upsampled source read), by staging latency and MFMA issue elsewhere
 // (48 -> 16 at half resolution 37.7 -> 20.4 us); registers for four waves per SIMD with one K
 // chunk, three with two, two with three chunks or two channel tiles.
-template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
-__global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 3 : 4)) void uconv3x3(UcBatch b)
+constexpr int uconv_lds(int src, int ci, bool head)  // 16-bit elements
+{
+    const int q = (src == UC_SRC_IMAGES ? 16 : ci) / 8;
+    return (UT_W + 2) * (UT_H + 2) * 8 * (q | 1) + (head ? 2 * 54 : 0);
+}
+
+template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD>
+__device__ __forceinline__ void uconv_block(const UcBatch &b, int bid, uint16_t *lds)
 {
     static_assert(!HEAD || (CO == 8 && EPI == UC_EPI_RELU), "the head follows the 8-channel ReLU layer");
     constexpr int CI = SRC == UC_SRC_IMAGES ? 16 : CA + CB;
     constexpr int KC = (CI + 15) / 16, QL = CI / 8, PS = 8 * (QL | 1);
     constexpr int NT = (CO + 31) / 32, NG = CO / 8;
     constexpr int LW = UT_W + 2, LH = UT_H + 2, NPX = LW * LH;
-    __shared__ __attribute__((aligned(16))) uint16_t lds[NPX * PS];
-    __shared__ float hws[HEAD ? 54 : 1];  // head weights [8][6] and bias [6], read behind the MFMAs
+    float *hws = reinterpret_cast<float *>(lds + NPX * PS);  // head weights [8][6], bias [6], read behind the MFMAs
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, px = lane & 31, h = lane >> 5;
-    const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
+    const TileLoc L = locate(b.map, xcd_tile(bid, b.map.total));
     const UcFrame &F = b.f[L.f];
     const int H = F.H, W = F.W;
     const int x0 = L.tx * UT_W, y0 = L.ty * UT_H;
@@ -371,13 +378,20 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
 }
 
 template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
-static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
+__global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 3 : 4)) void uconv3x3(UcBatch b)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t lds[uconv_lds(SRC, CA + CB, HEAD)];
+    uconv_block<SRC, CA, CB, CO, EPI, HEAD>(b, blockIdx.x, lds);
+}
+
+// False: a row is too wide for the 32-bit offsets.
+template <int SRC, int CA, int CB, int CO>
+static bool uconv_batch(UcBatch &b, int n, const UcFrame *fr)
 {
     // bytes of one staged image row over all of a tile's 32-bit offsets, see kUOob
     constexpr uint64_t row = (UT_H + 2) * (SRC == UC_SRC_IMAGES ? 12 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO);
     for (int i = 0; i < n; ++i)
-        if (row * (uint64_t)fr[i].W >= kUOob) return hipErrorInvalidValue;  // wider than 4.9 million pixels
-    UcBatch b{};
+        if (row * (uint64_t)fr[i].W >= kUOob) return false;  // wider than 4.9 million pixels
     int tx[XDN_MAX_FRAMES], ty[XDN_MAX_FRAMES];
     for (int i = 0; i < n; ++i)
     {
@@ -386,6 +400,14 @@ static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
         ty[i] = udiv_up(fr[i].H, UT_H);
     }
     b.map = make_tilemap(n, tx, ty);
+    return true;
+}
+
+template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
+static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
+{
+    UcBatch b{};
+    if (!uconv_batch<SRC, CA, CB, CO>(b, n, fr)) return hipErrorInvalidValue;
     if (b.map.total == 0) return hipSuccess;
     hipLaunchKernelGGL((uconv3x3<SRC, CA, CB, CO, EPI, HEAD>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
@@ -404,13 +426,6 @@ hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st)
     case UC_F_16_32: return uconv_t<UC_SRC_BF16, 16, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_32_32: return uconv_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_48_16: return uconv_t<UC_SRC_BF16, 32, 16, 16, UC_EPI_RELU>(n, fr, st);
-    case UC_D_8_8: return uconv_t<UC_SRC_BF16, 8, 0, 8, UC_EPI_MASK>(n, fr, st);
-    case UC_D_16_8: return uconv_t<UC_SRC_BF16, 16, 0, 8, UC_EPI_PLAIN>(n, fr, st);
-    case UC_D_16_16: return uconv_t<UC_SRC_BF16, 16, 0, 16, UC_EPI_MASK>(n, fr, st);
-    case UC_D_32_16: return uconv_t<UC_SRC_BF16, 32, 0, 16, UC_EPI_PLAIN>(n, fr, st);
-    case UC_D_32_32: return uconv_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_MASK>(n, fr, st);
-    case UC_D_16_48: return uconv_t<UC_SRC_BF16, 16, 0, 48, UC_EPI_PLAIN>(n, fr, st);
-    case UC_D_8_24: return uconv_t<UC_SRC_BF16, 8, 0, 24, UC_EPI_PLAIN>(n, fr, st);
     case UC_F_24_8_HEAD: return uconv_t<UC_SRC_UPCAT, 16, 8, 8, UC_EPI_RELU, true>(n, fr, st);
     default: return hipErrorInvalidValue;
     }
@@ -421,8 +436,8 @@ hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st)
 // A block walks strips, at most two blocks a CU (their number fixes the partial sums), so what it spends
 // is the time between strips: staging without branches, strip-invariant offsets, DEPTH strips in flight,
 // only the even pixels of an upsampled source. HBM and the halo's L2 reads bound the images (1920x1080:
-// 41.4 us, 158 MB), LDS reads, barriers and latency the rest (24 channels 45 -> 33.6 us, 8 channels
-// 26.7 -> 20.3 us, 48 in two slices 18.8 + 11.8 -> 17.5 + 11.4 us).
+// 41.4 us, 158 MB), LDS reads, barriers and latency the rest (in launches of their own with two strips in
+// flight, 24 channels 45 -> 33.6 us, 8 channels 26.7 -> 20.3 us, 48 in two slices 18.8 + 11.8 -> 17.5 + 11.4 us).
 // ---------------------------------------------------------------------------------------------
 struct UwBatch {
     int n;
@@ -434,23 +449,29 @@ static_assert(sizeof(UwBatch) <= 4096, "kernel argument too large");
 constexpr int US_W = 32, US_H = 8;                // strip: 8 rows x 32 px
 constexpr int UX_C = US_W + 2, UX_R = US_H + 2;   // staged X: 10 rows x 34 px (1-px halo)
 
+constexpr int uw_slice(int src, int ci, int mt) { return src == UC_SRC_IMAGES ? 15 : (ci - 32 * mt < 32 ? ci - 32 * mt : 32); }
+constexpr int uwgrad_tile(int src, int ci, int co, int mt)  // 16-bit elements, at least 4 x 1024 floats
+{
+    const int n = UX_R * UX_C * (uw_slice(src, ci, mt) <= 16 ? 16 : 32) + US_H * US_W * (co <= 16 ? 16 : 32);
+    return n > 8192 ? n : 8192;
+}
+constexpr int uwgrad_lds(int src, int ci, int co, int mt) { return uwgrad_tile(src, ci, co, mt) + 2 * 4 * 32; }
+
 template <int SRC, int CA, int CB, int CO, int MT, int DEPTH>
-__global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
+__device__ __forceinline__ void uwgrad_block(const UwBatch &b, int bid, uint16_t *lds)
 {
     // input-slice channels of this instantiation; staged channel counts (pixel strides) 16 or 32,
     // zero-padded: with 16 the lane groups 0 and 1 read the same channels, so the accumulator rows
     // (or columns) 16-31 repeat 0-15 and are not written out
-    constexpr int CS = SRC == UC_SRC_IMAGES ? 15 : ((CA + CB - 32 * MT) < 32 ? (CA + CB - 32 * MT) : 32);
+    constexpr int CS = uw_slice(SRC, CA + CB, MT);
     constexpr int XS = CS <= 16 ? 16 : 32, DS = CO <= 16 ? 16 : 32;
-    constexpr int X_ELEMS = UX_R * UX_C * XS, D_ELEMS = US_H * US_W * DS;
-    constexpr int LDS_ELEMS = (X_ELEMS + D_ELEMS) > 8192 ? (X_ELEMS + D_ELEMS) : 8192;  // >= 4 x 1024 floats
-    __shared__ __attribute__((aligned(16))) uint16_t lds[LDS_ELEMS];
-    __shared__ float dbs[4][32];
+    constexpr int X_ELEMS = UX_R * UX_C * XS;
+    float(*dbs)[32] = reinterpret_cast<float(*)[32]>(lds + uwgrad_tile(SRC, CA + CB, CO, MT));
     uint16_t *xs = lds, *ds = lds + X_ELEMS;
     int f = 0;
-    while (f + 1 < b.n && (int)blockIdx.x >= b.blk_begin[f + 1]) ++f;
+    while (f + 1 < b.n && bid >= b.blk_begin[f + 1]) ++f;
     const UwFrame &F = b.f[f];
-    const int li = blockIdx.x - b.blk_begin[f], nblk = b.blk_begin[f + 1] - b.blk_begin[f];
+    const int li = bid - b.blk_begin[f], nblk = b.blk_begin[f + 1] - b.blk_begin[f];
     const int H = F.H, W = F.W;
     const int sx = (W + US_W - 1) / US_W, sy = (H + US_H - 1) / US_H;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, h = lane >> 5, ch = lane & 31;
@@ -723,9 +744,8 @@ __global__ __launch_bounds__(256, 2) void uwgrad(UwBatch b)
             compute();
         }
     // compact partial [9][CS][CO] + [CO] of this input slice
-    float *out = F.part + (size_t)li * compact_part(9, CS, CO);
+    float *out = (MT ? F.part_m1 : F.part) + (size_t)li * compact_part(9, CS, CO);
     float *red = reinterpret_cast<float *>(lds);  // [4 waves][1024]
-    static_assert(sizeof(lds) >= 4 * 1024 * sizeof(float), "reduction buffer");
 #pragma unroll
     for (int t = 0; t < 9; ++t)
     {
@@ -774,50 +794,124 @@ int ublocks(int H, int W)
     return strips < 1 ? 1 : (strips < 512 ? strips : 512);
 }
 
-// Two strips in flight where a block walks more than two (1920x1080, 16 strips: 24 channels 33.6 us, 38.5
-// with one; 8 channels 20.3, 26.7), one below (256x256, one strip: 13.8 us, 15.3 with two; the images 10.6,
-// 13.8) and where 32 outputs leave no registers for two.
-template <int SRC, int CA, int CB, int CO, int MT>
-static hipError_t uwgrad_t(int n, const UwFrame *fr, hipStream_t st)
+template <int DEPTH>
+__global__ __launch_bounds__(256, 2) void uwgrad_images(UwBatch b)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t lds[uwgrad_lds(UC_SRC_IMAGES, 0, 8, 0)];
+    uwgrad_block<UC_SRC_IMAGES, 0, 0, 8, 0, DEPTH>(b, blockIdx.x, lds);
+}
+
+// False: a row is too wide for the 32-bit offsets.
+template <int SRC, int CA, int CB, int CO>
+static bool uwgrad_batch(UwBatch &b, int n, const UwFrame *fr, int &blocks)
 {
     constexpr int pix = SRC == UC_SRC_IMAGES ? 16 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO;
     for (int i = 0; i < n; ++i)  // a strip's 32-bit offsets
-        if ((uint64_t)pix * (UX_R * (uint64_t)fr[i].W + UX_C) >= kUOob) return hipErrorInvalidValue;
-    UwBatch b{};
+        if ((uint64_t)pix * (UX_R * (uint64_t)fr[i].W + UX_C) >= kUOob) return false;
     b.n = n;
-    int acc = 0;
-    bool deep = false;
+    blocks = 0;
     for (int i = 0; i < n; ++i)
     {
         b.f[i] = fr[i];
-        b.blk_begin[i] = acc;
-        acc += fr[i].nblk;
-        deep |= udiv_up(fr[i].W, US_W) * udiv_up(fr[i].H, US_H) > 2 * fr[i].nblk;
+        b.blk_begin[i] = blocks;
+        blocks += fr[i].nblk;
     }
-    b.blk_begin[n] = acc;
-    if (acc == 0) return hipSuccess;
-    if (CO <= 16 && deep)
-        hipLaunchKernelGGL((uwgrad<SRC, CA, CB, CO, MT, CO <= 16 ? 2 : 1>), dim3(acc), dim3(256), 0, st, b);
+    b.blk_begin[n] = blocks;
+    return true;
+}
+
+// The first layer's weight gradient. Two strips in flight where a block walks more than two, one below
+// (256x256, one strip: 10.6 us, 13.8 with two).
+hipError_t launch_uwgrad_images(int n, const UwFrame *fr, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    if (n > XDN_MAX_FRAMES) return hipErrorInvalidValue;
+    UwBatch b{};
+    int blocks;
+    if (!uwgrad_batch<UC_SRC_IMAGES, 0, 0, 8>(b, n, fr, blocks)) return hipErrorInvalidValue;
+    if (blocks == 0) return hipSuccess;
+    bool deep = false;
+    for (int i = 0; i < n; ++i) deep |= udiv_up(fr[i].W, US_W) * udiv_up(fr[i].H, US_H) > 2 * fr[i].nblk;
+    if (deep)
+        hipLaunchKernelGGL((uwgrad_images<2>), dim3(blocks), dim3(256), 0, st, b);
     else
-        hipLaunchKernelGGL((uwgrad<SRC, CA, CB, CO, MT, 1>), dim3(acc), dim3(256), 0, st, b);
+        hipLaunchKernelGGL((uwgrad_images<1>), dim3(blocks), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 
-hipError_t launch_uwgrad(int kind, int n, const UwFrame *fr, hipStream_t st)
+// ---------------------------------------------------------------------------------------------
+// A layer's weight gradient and data gradient in one launch. Both wait for dY alone; as two launches they
+// were two latencies in a row on small images (four 256x256 streams: 32 tiles and 64 strips at quarter
+// resolution) and two nearly empty last waves on large ones. The first blocks take the weight gradient (both
+// slices of the 48-channel layer), at most two a CU and the longest to run, the others the data gradient's
+// tiles, which fill in behind them; each part starts at a multiple of eight blocks, so that its XCD order
+// holds. The block bodies are those of separate kernels: the same bits. U-Net backward, two launches -> one:
+// 256x256 153 -> 108 us, four of them 187 -> 147, 512x512 172 -> 132, 1280x720 281 -> 235, 1920x1080
+// 442 -> 391, 3840x2160 1393 -> 1311. One strip in flight (two: 397 at 1920x1080); three waves per SIMD
+// where two are given: 409; data gradient first: 422; both parts interleaved: 433.
+// ---------------------------------------------------------------------------------------------
+struct UbBatch {
+    UwBatch w;
+    UcBatch c;
+    int w_blocks;
+};
+static_assert(sizeof(UbBatch) <= 4096, "kernel argument too large");
+
+__host__ __device__ constexpr int up8(int n) { return (n + 7) & ~7; }
+
+template <int SRC, int CA, int CB, int CO, int EPI, int WAVES>
+__global__ __launch_bounds__(256, WAVES) void ubackward(UbBatch b)
+{
+    constexpr int CI = CA + CB;
+    constexpr bool two = CI > 32;  // input slices
+    constexpr int LW = uwgrad_lds(SRC, CI, CO, 0), LC = uconv_lds(UC_SRC_BF16, CO, false);
+    __shared__ __attribute__((aligned(16))) uint16_t lds[LW > LC ? LW : LC];
+    int bid = blockIdx.x;
+    const int wb = up8(b.w_blocks);
+    if (bid < wb)
+    {
+        if (bid < b.w_blocks) uwgrad_block<SRC, CA, CB, CO, 0, 1>(b.w, bid, lds);
+        return;
+    }
+    bid -= wb;
+    if constexpr (two)
+    {
+        if (bid < wb)
+        {
+            if (bid < b.w_blocks) uwgrad_block<UC_SRC_BF16, CA, CB, CO, 1, 1>(b.w, bid, lds);
+            return;
+        }
+        bid -= wb;
+    }
+    uconv_block<UC_SRC_BF16, CO, 0, CI, EPI, false>(b.c, bid, lds);
+}
+
+template <int SRC, int CA, int CB, int CO, int EPI, int WAVES>
+static hipError_t ubackward_t(int n, const UwFrame *wfr, const UcFrame *cfr, hipStream_t st)
+{
+    constexpr int CI = CA + CB;
+    UbBatch b{};
+    if (!uwgrad_batch<SRC, CA, CB, CO>(b.w, n, wfr, b.w_blocks)) return hipErrorInvalidValue;
+    if (!uconv_batch<UC_SRC_BF16, CO, 0, CI>(b.c, n, cfr)) return hipErrorInvalidValue;
+    if (b.c.map.total == 0) return hipSuccess;
+    const int blocks = up8(b.w_blocks) * (CI > 32 ? 2 : 1) + b.c.map.total;
+    hipLaunchKernelGGL((ubackward<SRC, CA, CB, CO, EPI, WAVES>), dim3(blocks), dim3(256), 0, st, b);
+    return hipGetLastError();
+}
+
+hipError_t launch_ubackward(int kind, int n, const UwFrame *wfr, const UcFrame *cfr, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
     if (n > XDN_MAX_FRAMES) return hipErrorInvalidValue;
     switch (kind)
     {
-    case UW_0: return uwgrad_t<UC_SRC_IMAGES, 0, 0, 8, 0>(n, fr, st);
-    case UW_8_8: return uwgrad_t<UC_SRC_BF16, 8, 0, 8, 0>(n, fr, st);
-    case UW_8_16: return uwgrad_t<UC_SRC_BF16, 8, 0, 16, 0>(n, fr, st);
-    case UW_16_16: return uwgrad_t<UC_SRC_BF16, 16, 0, 16, 0>(n, fr, st);
-    case UW_16_32: return uwgrad_t<UC_SRC_BF16, 16, 0, 32, 0>(n, fr, st);
-    case UW_32_32: return uwgrad_t<UC_SRC_BF16, 32, 0, 32, 0>(n, fr, st);
-    case UW_48_16_M0: return uwgrad_t<UC_SRC_UPCAT, 32, 16, 16, 0>(n, fr, st);
-    case UW_48_16_M1: return uwgrad_t<UC_SRC_BF16, 32, 16, 16, 1>(n, fr, st);
-    case UW_24_8: return uwgrad_t<UC_SRC_UPCAT, 16, 8, 8, 0>(n, fr, st);
+    case UBW_8_8: return ubackward_t<UC_SRC_BF16, 8, 0, 8, UC_EPI_MASK, 4>(n, wfr, cfr, st);
+    case UBW_8_16: return ubackward_t<UC_SRC_BF16, 8, 0, 16, UC_EPI_PLAIN, 4>(n, wfr, cfr, st);
+    case UBW_16_16: return ubackward_t<UC_SRC_BF16, 16, 0, 16, UC_EPI_MASK, 4>(n, wfr, cfr, st);
+    case UBW_16_32: return ubackward_t<UC_SRC_BF16, 16, 0, 32, UC_EPI_PLAIN, 2>(n, wfr, cfr, st);
+    case UBW_32_32: return ubackward_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_MASK, 2>(n, wfr, cfr, st);
+    case UBW_48_16: return ubackward_t<UC_SRC_UPCAT, 32, 16, 16, UC_EPI_PLAIN, 2>(n, wfr, cfr, st);
+    case UBW_24_8: return ubackward_t<UC_SRC_UPCAT, 16, 8, 8, UC_EPI_PLAIN, 2>(n, wfr, cfr, st);
     default: return hipErrorInvalidValue;
     }
 }

@@ -54,13 +54,6 @@ enum {
     UC_F_16_32,   // 16 -> 32 ReLU
     UC_F_32_32,   // 32 -> 32 ReLU
     UC_F_48_16,   // concat 32+16 -> 16 ReLU
-    UC_D_8_8,     // dgrad dY 8 -> dX 8, masked
-    UC_D_16_8,    // dgrad dY 16 -> dX 8, unmasked (pool input)
-    UC_D_16_16,   // dgrad dY 16 -> dX 16, masked
-    UC_D_32_16,   // dgrad dY 32 -> dX 16, unmasked (pool input)
-    UC_D_32_32,   // dgrad dY 32 -> dX 32, masked
-    UC_D_16_48,   // dgrad dY 16 -> dX 48, unmasked (concat input)
-    UC_D_8_24,    // dgrad dY 8 -> dX 24, unmasked (concat input)
     UC_F_24_8_HEAD,  // concat 16 (upsampled) + 8 -> 8 ReLU, then the 1x1 head 8 -> 6 (FP32) on the bf16 output
     UC_KINDS
 };
@@ -73,21 +66,23 @@ struct UwFrame {
     const float *img[5];
     const uint16_t *dy;         // bf16 [H][W][CO]
     float *part;                // [nblk][compact_part(9, cs, CO)]
+    float *part_m1;             // the same of input channels 32 and up
     int H, W, nblk;
 };
+hipError_t launch_uwgrad_images(int n, const UwFrame *fr, hipStream_t st);  // images (15) x dY 8
+
+// The gradients of a 3x3 layer below the first: weights (wfr: input and dY) and data (cfr: dY into the input's
+// gradient), in one launch on small images.
+hipError_t launch_ubackward(int kind, int n, const UwFrame *wfr, const UcFrame *cfr, hipStream_t st);
 enum {
-    UW_0 = 0,     // images (15) x dY 8
-    UW_8_8,       // 8 x 8
-    UW_8_16,      // 8 x 16
-    UW_16_16,     // 16 x 16
-    UW_16_32,     // 16 x 32
-    UW_32_32,     // 32 x 32
-    UW_48_16_M0,  // concat 32 (upsampled) + 16 x 16, input channels 0-31
-    UW_48_16_M1,  // concat 32+16 x 16, input channels 32-47
-    UW_24_8,      // concat 16 (upsampled) + 8 x 8
-    UW_KINDS
+    UBW_8_8 = 0,  // layer 8 -> 8, data gradient masked
+    UBW_8_16,     // 8 -> 16, unmasked (pool input)
+    UBW_16_16,    // 16 -> 16, masked
+    UBW_16_32,    // 16 -> 32, unmasked (pool input)
+    UBW_32_32,    // 32 -> 32, masked
+    UBW_48_16,    // concat 32 (upsampled) + 16 -> 16, unmasked
+    UBW_24_8,     // concat 16 (upsampled) + 8 -> 8, unmasked
 };
-hipError_t launch_uwgrad(int kind, int n, const UwFrame *fr, hipStream_t st);
 
 // 2x2 max pool (valid), bf16 [H][W][C] -> [H/2][W/2][C].
 struct PoolFrame {
