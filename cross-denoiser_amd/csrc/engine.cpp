@@ -178,10 +178,11 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
         else
             cw.emplace_back(sc[i].cnn_ws, 1, s.height, s.width);
     }
+    const bool regress = stages & XDN_STAGE_REGRESS, reproject = stages & XDN_STAGE_REPROJECT;
+    std::vector<xdn::CrFrame> fr(n);
     // 1. cross-regression with the log1p prologue (variance launches hold 2 frames per slot)
-    if (stages & XDN_STAGE_REGRESS)
+    if (regress)
     {
-        std::vector<xdn::CrFrame> fr(n);
         for (int i = 0; i < n; ++i)
         {
             const xdn_slot &s = slots[i];
@@ -196,17 +197,19 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             if (int e = hip_check(xdn::launch_variance(m, fr.data() + b0, 3, true, st), "variance")) return e;
         }
         if (int e = hip_check(xdn::launch_regression(n, fr.data(), kRegWin, kSparsity, true, st), "regression")) return e;
-        if (int e = hip_check(xdn::launch_recon(n, fr.data(), kRegWin, kSparsity, 1, st), "recon")) return e;
+        if (!reproject)
+            if (int e = hip_check(xdn::launch_recon(n, fr.data(), kRegWin, kSparsity, 1, st), "recon")) return e;
     }
-    // 2. reprojection of [out_log, ols1, ols2] of the previous frame (main.py:266, opacities one)
-    if (stages & XDN_STAGE_REPROJECT)
+    // 2. reprojection of [out_log, ols1, ols2] of the previous frame (main.py:266, opacities one), in one
+    //    launch with the reconstruction where both are asked for
+    if (reproject)
     {
-        std::vector<xdn::RpFrame> fr(n);
+        std::vector<xdn::RpFrame> rp(n);
         const int dims[3] = {3, 3, 3};
         for (int i = 0; i < n; ++i)
         {
             const xdn_slot &s = slots[i];
-            xdn::RpFrame &f = fr[i];
+            xdn::RpFrame &f = rp[i];
             memset(&f, 0, sizeof(f));
             f.mvec = s.mvec; f.linZ = s.linear_z; f.prevLinZ = s.prev_linear_z; f.nrm = s.normal;
             f.prevNrm = s.prev_normal; f.pnFw = s.pn_fwidth; f.opac = sc[i].ones; f.prevOpac = sc[i].ones;
@@ -215,7 +218,9 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             f.out[0] = sc[i].rp[0]; f.out[1] = sc[i].rp[1]; f.out[2] = sc[i].rp[2];
             f.H = s.height; f.W = s.width;
         }
-        if (int e = hip_check(xdn::launch_reproject(n, fr.data(), 3, dims, true, st), "reproject")) return e;
+        const hipError_t e = regress ? xdn::launch_recon_reproject(n, fr.data(), kRegWin, kSparsity, rp.data(), st)
+                                     : xdn::launch_reproject(n, rp.data(), 3, dims, true, st);
+        if (int rc = hip_check(e, regress ? "recon + reproject" : "reproject")) return rc;
     }
     if (!(stages & XDN_STAGE_FINISH)) return XDN_OK;
     // 3. 3x3 erosion + temporal screening (win_curr 7, win_prev 1, main.py:270-280)

@@ -87,6 +87,10 @@ struct RpFrame {
 hipError_t launch_reproject(int n, const RpFrame *fr, int n_list, const int *dims, bool unit_opacity,
                             hipStream_t st);
 
+// launch_recon (win 17, sparsity 4, recon_scale 1) and launch_reproject (three 3-channel buffers, unit
+// opacities) of the same frames in one launch; neither reads what the other writes.
+hipError_t launch_recon_reproject(int n, const CrFrame *fr, int win, int s, const RpFrame *rp, hipStream_t st);
+
 // Temporal screening (optionally with the 3x3 erosion of a u8 success mask fused in).
 struct TsFrame {
     const float *c1, *c2, *prev, *prev1, *prev2;
