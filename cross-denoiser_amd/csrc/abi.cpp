@@ -555,7 +555,7 @@ int xdn_filter_train(const float *ols1, const float *ols2, const float *albedo, 
             sc[i] = (float)(1.0 / (3.0 * (double)N));
             outp[i] = avg_loss + b;
         }
-        if (int e = hip_check(xdn::launch_filter_train(n, fr.data(), win_size, S(stream)), "filter_train")) return e;
+        if (int e = hip_check(xdn::launch_filter_train(n, fr.data(), win_size, false, S(stream)), "filter_train")) return e;
         if (avg_loss)
             if (int e = hip_check(xdn::launch_sums(n, pp.data(), cnt.data(), sc.data(), outp.data(), S(stream)), "loss sum"))
                 return e;

@@ -294,7 +294,7 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
                 tick.alpha[tick.n] = sc[i].adam_alpha;
                 ++tick.n;
             }
-        if (int e = hip_check(xdn::launch_filter_train(n, fr.data(), kFilterWin, st), "filter_train")) return e;
+        if (int e = hip_check(xdn::launch_filter_train(n, fr.data(), kFilterWin, true, st), "filter_train")) return e;
         if (int e = hip_check(xdn::launch_sums(n, parts.data(), cnt.data(), scale.data(), outp.data(), st, &tick),
                               "loss"))
             return e;

@@ -118,6 +118,17 @@ __device__ __forceinline__ void sf_center_bands(SfCenter &C, const float *band, 
     C.k4 = -kLog2e * b[4] / (float)(half * half);
 }
 
+// The same from the network's raw output (band transform of scripts/main.py:110-113).
+__device__ __forceinline__ void sf_center_param(SfCenter &C, const float *param, uint32_t c, int half)
+{
+    const float *pr = param + 6 * (size_t)c;
+    float bnd[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) bnd[k] = 1.f / (pr[k] * pr[k] + 1e-4f);
+    C.k0 = -kLog2e * bnd[0]; C.k1 = -kLog2e * bnd[1]; C.k2 = -kLog2e * bnd[2];
+    C.k3 = -kLog2e * bnd[3]; C.k4 = -kLog2e * bnd[4] / (float)(half * half);
+}
+
 // Epilogue of the fused training kernel for one pixel; returns the pixel's loss sum.
 // Follows aggregation_loss (scripts/main.py:214-248), its analytic gradient, the band-gradient
 // contraction (regression.cu.cc:58-80) and the band/alpha transform (main.py:111-113).
@@ -239,12 +250,7 @@ __device__ __forceinline__ void sf_tile_body(const Batch &b, float *red)
         }
         if constexpr (MODE == SF_TRAIN)
         {
-            const float *pr = F.param + 6 * (size_t)c;
-            float bnd[5];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) bnd[k] = 1.f / (pr[k] * pr[k] + 1e-4f);
-            C.k0 = -kLog2e * bnd[0]; C.k1 = -kLog2e * bnd[1]; C.k2 = -kLog2e * bnd[2];
-            C.k3 = -kLog2e * bnd[3]; C.k4 = -kLog2e * bnd[4] / (float)(HALF * HALF);
+            sf_center_param(C, F.param, c, HALF);
         }
         else
             sf_center_bands(C, F.band, c, HALF);
@@ -411,6 +417,94 @@ __global__ __launch_bounds__(256, 5) void sf_train_tile(TrBatch b)
 {
     __shared__ float red[4];
     sf_tile_body<HALF, SF_TRAIN>(b, red);
+}
+
+// The training tile for launches that leave the chip idle: the window rows of a pixel are split over two
+// threads as in sf_tile_split, their 40 sums joined in LDS twenty at a time, over the tile.
+template <int HALF>
+__global__ __launch_bounds__(512) void sf_train_split(TrBatch b)
+{
+    constexpr int G = 2, E = SF_T + 2 * HALF, NV = 40, CH = 20, R = 2 * HALF + 1;
+    __shared__ float4 s[3][E * E];
+    __shared__ float red[4];
+    static_assert(sizeof(s) >= sizeof(float) * CH * 256, "reduction space");
+    const int tile = xcd_tile(blockIdx.x, b.map.total);
+    const TileLoc L = locate(b.map, tile);
+    const TrainFrame &F = b.f[L.f];
+    const int H = F.H, W = F.W;
+    const int x0 = L.tx * SF_T, y0 = L.ty * SF_T;
+    for (int i = threadIdx.x; i < E * E; i += 256 * G)
+    {
+        const int ly = i / E, lx = i - ly * E;
+        const int gy = mirror(min(y0 + ly - HALF, H - 1 + HALF), H), gx = mirror(min(x0 + lx - HALF, W - 1 + HALF), W);
+        const size_t p = (size_t)gy * W + gx;
+        const float3 a = ld3(F.ols1, p), bb = ld3(F.ols2, p), al = ld3(F.alb, p), n = ld3(F.nrm, p);
+        s[0][i] = make_float4(a.x, a.y, a.z, bb.x);
+        s[1][i] = make_float4(bb.y, bb.z, al.x, al.y);
+        s[2][i] = make_float4(al.z, n.x, n.y, n.z);
+    }
+    const int t = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const int lx = t & (SF_T - 1), ly = t / SF_T;
+    const int cx = x0 + lx, cy = y0 + ly;
+    const bool live = cx < W && cy < H;
+    // lanes past the image run along on the last pixel (nothing of theirs is stored)
+    const uint32_t c = (uint32_t)min(cy, H - 1) * (uint32_t)W + (uint32_t)min(cx, W - 1);
+    SfCenter C;
+    sf_center_param(C, F.param, c, HALF);
+    __syncthreads();
+    const int q0 = (ly + HALF) * E + lx + HALF;
+    {
+        const float4 P0 = s[0][q0], P1 = s[1][q0], P2 = s[2][q0];
+        C.cA = make_float3(P0.x, P0.y, P0.z);
+        C.cB = make_float3(P0.w, P1.x, P1.y);
+        C.ca = make_float3(P1.z, P1.w, P2.x);
+        C.cn = make_float3(P2.y, P2.z, P2.w);
+    }
+    SfAcc acc;
+    sf_zero(acc);
+    constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
+#pragma unroll 1
+    for (int dy = R * grp / G - HALF; dy < R * (grp + 1) / G - HALF; ++dy)
+    {
+        const float y2 = (float)(dy * dy), kdy = C.k4 * y2, pdy = y2 * inv_h2;
+        const int base = q0 + dy * E;
+#pragma unroll
+        for (int dx = -HALF; dx <= HALF; ++dx)
+        {
+            const float4 P0 = s[0][base + dx], P1 = s[1][base + dx], P2 = s[2][base + dx];
+            sf_tap<SF_TRAIN>(C, acc, make_float3(P0.x, P0.y, P0.z), make_float3(P0.w, P1.x, P1.y),
+                             make_float3(P1.z, P1.w, P2.x), make_float3(P2.y, P2.z, P2.w),
+                             pdy + (float)(dx * dx) * inv_h2, kdy + C.k4 * (float)(dx * dx));
+        }
+    }
+    float *const v[NV] = {&acc.aA.x, &acc.aA.y, &acc.aA.z, &acc.aB.x, &acc.aB.y, &acc.aB.z, &acc.sA, &acc.sB,
+                          &acc.MA[0].x, &acc.MA[0].y, &acc.MA[0].z, &acc.MA[0].w, &acc.MA[1].x, &acc.MA[1].y,
+                          &acc.MA[1].z, &acc.MA[1].w, &acc.MA[2].x, &acc.MA[2].y, &acc.MA[2].z, &acc.MA[2].w,
+                          &acc.MA[3].x, &acc.MA[3].y, &acc.MA[3].z, &acc.MA[3].w, &acc.MB[0].x, &acc.MB[0].y,
+                          &acc.MB[0].z, &acc.MB[0].w, &acc.MB[1].x, &acc.MB[1].y, &acc.MB[1].z, &acc.MB[1].w,
+                          &acc.MB[2].x, &acc.MB[2].y, &acc.MB[2].z, &acc.MB[2].w, &acc.MB[3].x, &acc.MB[3].y,
+                          &acc.MB[3].z, &acc.MB[3].w};
+    float *part = reinterpret_cast<float *>(&s[0][0]);  // [CH][256]
+#pragma unroll
+    for (int k0 = 0; k0 < NV; k0 += CH)
+    {
+        __syncthreads();  // the tile, or the first half of the sums, is read
+        if (grp)
+#pragma unroll
+            for (int k = 0; k < CH; ++k) part[k * 256 + t] = *v[k0 + k];
+        __syncthreads();
+        if (!grp)
+#pragma unroll
+            for (int k = 0; k < CH; ++k) *v[k0 + k] += part[k * 256 + t];
+    }
+    float lsum = 0.f;
+    if (!grp && live) lsum = train_epilogue(F, c, acc, 1.f / (3.f * (float)H * (float)W), C.cA, C.cB);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_down(lsum, off);
+    const bool lane0 = __lane_id() == 0;
+    if (!grp && lane0) red[wave] = lsum;
+    __syncthreads();
+    if (wave == 0 && lane0) F.loss_part[tile - b.map.begin[L.f]] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // Any window size: direct loads with the mirror boundary.
@@ -761,7 +855,8 @@ hipError_t launch_sf_grad_inputs(int n, const SfFrame *fr, int win, hipStream_t 
 
 int filter_train_tiles(int H, int W) { return div_up(W, SF_T) * div_up(H, SF_T); }
 
-hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, hipStream_t st)
+// batch_invariant: a frame's results are the same bits whatever it is launched with.
+hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool batch_invariant, hipStream_t st)
 {
     if (win / 2 != 5) return hipErrorInvalidValue;
     TrBatch b{};
@@ -774,7 +869,12 @@ hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, hipStream_t
     }
     b.map = make_tilemap(n, tx, ty);
     if (b.map.total == 0) return hipSuccess;
-    hipLaunchKernelGGL((sf_train_tile<5>), dim3(b.map.total), dim3(256), 0, st, b);
+    // operator call, one thread -> two: 64 tiles 28.4 -> 23.9 us (the host's launch rate), 256 30.8 -> 25.6; no
+    // gain from 420 tiles on (39.4, 39.2; 1024: 66.1, 67.1), and four threads are no faster at any size
+    if (!batch_invariant && b.map.total <= 256)
+        hipLaunchKernelGGL((sf_train_split<5>), dim3(b.map.total), dim3(512), 0, st, b);
+    else
+        hipLaunchKernelGGL((sf_train_tile<5>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 

@@ -401,6 +401,16 @@ def test_filter_train(dev, B, H, W):
         assert err <= TOL, name
 
 
+@pytest.mark.parametrize("B,H,W", [(1, 256, 250), (1, 257, 250), (3, 16, 7), (1, 6, 6)])
+def test_filter_train_tiles(dev, B, H, W):
+    """256 tiles (two threads a pixel), 272 (one), one tile per image, the smallest image."""
+    from xdn import pipeline
+    case = train_case(H, W, seed=3 * H + W, B=B)
+    got = pipeline.filter_train(*[to_dev(a, dev) for a in case], want_loss=True)
+    for name, g, r in zip(("out_log", "out", "loss", "avg_loss", "dparam"), got, train_oracle(*case)):
+        assert rel_l2(to_np(g), r) <= TOL, name
+
+
 def test_adam_keras(dev):
     from xdn._lib import check, lib, ptr
     r = np.random.default_rng(0)
