@@ -38,13 +38,14 @@ xdn::UcFrame conv_frame(const UnetFrame &U, int l, int a, int b, int out, int ma
     return f;
 }
 
-// forward of 3x3 layer l over every image
-int conv(Frames F, int n, hipStream_t st, int kind, int l, int a, int b, int out, const char *what)
+// forward of 3x3 layer l over every image (its 2x2 max pool into buffer pooled, if any)
+int conv(Frames F, int n, hipStream_t st, int kind, int l, int a, int b, int out, const char *what, int pooled = -1)
 {
     std::vector<xdn::UcFrame> fr(n);
     for (int i = 0; i < n; ++i)
     {
         fr[i] = conv_frame(F[i], l, a, b, out, -1, false);
+        if (pooled >= 0) fr[i].pooled = F[i].buf[pooled];
         if (kind == xdn::UC_F_24_8_HEAD)
         {
             fr[i].head_w = reinterpret_cast<const float *>(F[i].pk + kULay.master_off[11]);
@@ -52,16 +53,6 @@ int conv(Frames F, int n, hipStream_t st, int kind, int l, int a, int b, int out
         }
     }
     return hip_check(xdn::launch_uconv(kind, n, fr.data(), st), what);
-}
-
-int pool(Frames F, int n, hipStream_t st, int C, int in, int out)
-{
-    const int lv = kUnetBuf[in].level;
-    std::vector<xdn::PoolFrame> fr(n);
-    for (int i = 0; i < n; ++i)
-        fr[i] = xdn::PoolFrame{reinterpret_cast<const uint16_t *>(F[i].buf[in]),
-                               reinterpret_cast<uint16_t *>(F[i].buf[out]), F[i].h[lv], F[i].w[lv]};
-    return hip_check(xdn::launch_maxpool(C, n, fr.data(), st), "unet max pool");
 }
 
 const float *master(const UnetFrame &U, int l) { return reinterpret_cast<const float *>(U.pk + kULay.master_off[l]); }
@@ -217,11 +208,9 @@ int unet_forward_frames(const UnetFrame *F, int n, hipStream_t st)
     using namespace xdn;
     int e = 0;
     if ((e = conv(F, n, st, UC_F_0, 0, -1, -1, UB_A0, "unet c1_1"))) return e;
-    if ((e = conv(F, n, st, UC_F_8_8, 1, UB_A0, -1, UB_A1, "unet c1_2"))) return e;
-    if ((e = pool(F, n, st, 8, UB_A1, UB_P1))) return e;
+    if ((e = conv(F, n, st, UC_F_8_8_POOL, 1, UB_A0, -1, UB_A1, "unet c1_2 + pool", UB_P1))) return e;
     if ((e = conv(F, n, st, UC_F_8_16, 2, UB_P1, -1, UB_A2, "unet c2_1"))) return e;
-    if ((e = conv(F, n, st, UC_F_16_16, 3, UB_A2, -1, UB_A3, "unet c2_2"))) return e;
-    if ((e = pool(F, n, st, 16, UB_A3, UB_P2))) return e;
+    if ((e = conv(F, n, st, UC_F_16_16_POOL, 3, UB_A2, -1, UB_A3, "unet c2_2 + pool", UB_P2))) return e;
     if ((e = conv(F, n, st, UC_F_16_32, 4, UB_P2, -1, UB_A4, "unet c3_1"))) return e;
     if ((e = conv(F, n, st, UC_F_32_32, 5, UB_A4, -1, UB_A5, "unet c3_2"))) return e;
     if ((e = convT(F, n, st, 6, UB_A5, UB_A6))) return e;                                       // c3_3

@@ -11,8 +11,9 @@
 //     software-pipelined strip loop.
 //   ubackward                    weight and data gradient of a layer in one launch (uwgrad_images: the
 //                                first layer's weight gradient alone).
-//   maxpool2 / pool_bwd          2x2 max pool and its gradient (to the first maximum, plus the
-//     skip-connection gradient, ReLU-masked).
+//   pool_bwd                     gradient of the 2x2 max pool (to the first maximum, plus the
+//     skip-connection gradient, ReLU-masked); the pool itself is in the epilogue of the layer before it,
+//     uconv3x3<..., POOL>.
 //   convT1x1s2 / convT_bwd       transposed 1x1 stride-2 convolution and its gradients.
 //   head_bwd                     gradients of the 1x1 8->6 output convolution (its forward runs in
 //                                the epilogue of the last 3x3 layer, uconv3x3<..., HEAD>).
@@ -127,10 +128,11 @@ constexpr int uconv_lds(int src, int ci, bool head)  // 16-bit elements
     return (UT_W + 2) * (UT_H + 2) * 8 * (q | 1) + (head ? 2 * 54 : 0);
 }
 
-template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD>
+template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD, bool POOL = false>
 __device__ __forceinline__ void uconv_block(const UcBatch &b, int bid, uint16_t *lds)
 {
     static_assert(!HEAD || (CO == 8 && EPI == UC_EPI_RELU), "the head follows the 8-channel ReLU layer");
+    static_assert(!POOL || (CO <= 16 && EPI == UC_EPI_RELU), "the pool takes nonnegative activations");
     constexpr int CI = SRC == UC_SRC_IMAGES ? 16 : CA + CB;
     constexpr int KC = (CI + 15) / 16, QL = CI / 8, PS = 8 * (QL | 1);
     constexpr int NT = (CO + 31) / 32, NG = CO / 8;
@@ -291,6 +293,7 @@ __device__ __forceinline__ void uconv_block(const UcBatch &b, int bid, uint16_t 
                 }
             }
 
+    uint32_t above[POOL ? 2 * NG : 1];  // POOL: the packed channels of the row above
     // head: output channels 3h .. 3h + 2 of the lane's pixel
     float hw[HEAD ? 24 : 1], hb[3] = {0.f, 0.f, 0.f};
     if constexpr (HEAD)
@@ -323,6 +326,48 @@ __device__ __forceinline__ void uconv_block(const UcBatch &b, int bid, uint16_t 
             }
             d[2 * j] = u_cvt2(v[0], v[1]);
             d[2 * j + 1] = u_cvt2(v[2], v[3]);
+        }
+        if constexpr (POOL)
+        {
+            // 2x2 maximum of the stored activations: row pairs in a lane, column pairs in adjacent lanes.
+            // Nonnegative bf16 values order as int16. A launch of its own read them all again:
+            // the step of four 256x256 streams 414 -> 407 us, the network at 1920x1080 630 -> 621.
+            typedef __attribute__((ext_vector_type(2))) short s16x2;
+            auto max2 = [](uint32_t x, uint32_t y) {
+                return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, x), __builtin_bit_cast(s16x2, y)));
+            };
+            uint32_t m[2 * NG];
+#pragma unroll
+            for (int k = 0; k < 2 * NG; ++k)
+            {
+                if (!(orow & 1))
+                {
+                    above[k] = d[k];
+                    continue;
+                }
+                const uint32_t v = max2(above[k], d[k]);
+                m[k] = max2(v, (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true));
+            }
+            if (orow & 1)
+            {
+                const u_rsrc rp = u_buf(F.pooled, orow0 / 4 * (CO * 2), onpx / 4 * (CO * 2));
+                const uint32_t p2 = (uint32_t)((4 * wv + orow) >> 1) * (uint32_t)(W / 2) + (uint32_t)((x0 + px) >> 1);
+                const bool st = in && !(px & 1);
+                if constexpr (NG == 1)
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{m[0], m[1]}, rp, st ? p2 * 16 + 8 * h : kUOob, 0, 0);
+                else
+                {
+                    u32x4 v;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                    {
+                        const auto sw = __builtin_amdgcn_permlane32_swap(m[e], m[2 + e], false, false);
+                        v[e] = (uint32_t)sw[0];
+                        v[2 + e] = (uint32_t)sw[1];
+                    }
+                    __builtin_amdgcn_raw_buffer_store_b128(v, rp, st ? p2 * 32 + 16 * h : kUOob, 0, 0);
+                }
+            }
         }
         // two groups of 8 channels: each half-wave gathers one whole group of its pixels
 #pragma unroll
@@ -379,11 +424,11 @@ __device__ __forceinline__ void uconv_block(const UcBatch &b, int bid, uint16_t 
     }
 }
 
-template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
+template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD, bool POOL>
 __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 3 : 4)) void uconv3x3(UcBatch b)
 {
     __shared__ __attribute__((aligned(16))) uint16_t lds[uconv_lds(SRC, CA + CB, HEAD)];
-    uconv_block<SRC, CA, CB, CO, EPI, HEAD>(b, blockIdx.x, lds);
+    uconv_block<SRC, CA, CB, CO, EPI, HEAD, POOL>(b, blockIdx.x, lds);
 }
 
 // False: a row is too wide for the 32-bit offsets.
@@ -405,13 +450,16 @@ static bool uconv_batch(UcBatch &b, int n, const UcFrame *fr)
     return true;
 }
 
-template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false>
+template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false, bool POOL = false>
 static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
 {
     UcBatch b{};
     if (!uconv_batch<SRC, CA, CB, CO>(b, n, fr)) return hipErrorInvalidValue;
     if (b.map.total == 0) return hipSuccess;
-    hipLaunchKernelGGL((uconv3x3<SRC, CA, CB, CO, EPI, HEAD>), dim3(b.map.total), dim3(256), 0, st, b);
+    if (POOL)
+        for (int i = 0; i < n; ++i)
+            if (fr[i].H % 2 || fr[i].W % 2) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((uconv3x3<SRC, CA, CB, CO, EPI, HEAD, POOL>), dim3(b.map.total), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 
@@ -422,9 +470,10 @@ hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st)
     switch (kind)
     {
     case UC_F_0: return uconv_t<UC_SRC_IMAGES, 0, 0, 8, UC_EPI_RELU>(n, fr, st);
-    case UC_F_8_8: return uconv_t<UC_SRC_BF16, 8, 0, 8, UC_EPI_RELU>(n, fr, st);
+    case UC_F_8_8_POOL: return uconv_t<UC_SRC_BF16, 8, 0, 8, UC_EPI_RELU, false, true>(n, fr, st);
     case UC_F_8_16: return uconv_t<UC_SRC_BF16, 8, 0, 16, UC_EPI_RELU>(n, fr, st);
     case UC_F_16_16: return uconv_t<UC_SRC_BF16, 16, 0, 16, UC_EPI_RELU>(n, fr, st);
+    case UC_F_16_16_POOL: return uconv_t<UC_SRC_BF16, 16, 0, 16, UC_EPI_RELU, false, true>(n, fr, st);
     case UC_F_16_32: return uconv_t<UC_SRC_BF16, 16, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_32_32: return uconv_t<UC_SRC_BF16, 32, 0, 32, UC_EPI_RELU>(n, fr, st);
     case UC_F_48_16: return uconv_t<UC_SRC_BF16, 32, 16, 16, UC_EPI_RELU>(n, fr, st);
@@ -919,13 +968,8 @@ hipError_t launch_ubackward(int kind, int n, const UwFrame *wfr, const UcFrame *
 }
 
 // ---------------------------------------------------------------------------------------------
-// Max pool and its gradient
+// Gradient of the max pool (its forward is in uconv3x3<..., POOL>)
 // ---------------------------------------------------------------------------------------------
-struct PoolBatch {
-    int n, total;
-    int begin[XDN_MAX_FRAMES + 1];  // first item of each frame
-    PoolFrame f[XDN_MAX_FRAMES];
-};
 struct PoolBwBatch {
     int n, total;
     int begin[XDN_MAX_FRAMES + 1];
@@ -937,38 +981,6 @@ __device__ __forceinline__ int item_frame(const int *begin, int n, int i)
     int f = 0;
     while (f + 1 < n && i >= begin[f + 1]) ++f;
     return f;
-}
-
-// one item = one pooled pixel x one 8-channel chunk
-template <int C>
-__global__ __launch_bounds__(256) void maxpool2(PoolBatch b)
-{
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= b.total) return;
-    const int f = item_frame(b.begin, b.n, i);
-    const PoolFrame &F = b.f[f];
-    const int W2 = F.W / 2;
-    const int li = i - b.begin[f], q = li % (C / 8), p2 = li / (C / 8);
-    const int y = p2 / W2, x = p2 - y * W2;
-    u32x4 v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-        v[k] = *reinterpret_cast<const u32x4 *>(F.in + ((size_t)(2 * y + (k >> 1)) * F.W + 2 * x + (k & 1)) * C + q * 8);
-    uint32_t o[4];
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-    {
-        float lo = -__builtin_inff(), hi = -__builtin_inff();
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-        {
-            const uint32_t word = w == 0 ? v[k].x : (w == 1 ? v[k].y : (w == 2 ? v[k].z : v[k].w));
-            lo = fmaxf(lo, u_lo(word));
-            hi = fmaxf(hi, u_hi(word));
-        }
-        o[w] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
-    }
-    *reinterpret_cast<u32x4 *>(F.out + (size_t)p2 * C + q * 8) = u32x4{o[0], o[1], o[2], o[3]};
 }
 
 // one item = one 2x2 window x one 8-channel chunk: vector loads of the window's four activations,
@@ -1024,33 +1036,6 @@ __global__ __launch_bounds__(256) void pool_bwd(PoolBwBatch b)
         *reinterpret_cast<u32x4 *>(F.dy + pix[k] * C + q * 8) =
             u32x4{u_pack2(r[k][0], r[k][1]), u_pack2(r[k][2], r[k][3]), u_pack2(r[k][4], r[k][5]),
                   u_pack2(r[k][6], r[k][7])};
-}
-
-template <int C>
-static hipError_t maxpool_t(int n, const PoolFrame *fr, hipStream_t st)
-{
-    PoolBatch b{};
-    b.n = n;
-    int acc = 0;
-    for (int i = 0; i < n; ++i)
-    {
-        b.f[i] = fr[i];
-        b.begin[i] = acc;
-        acc += (fr[i].H / 2) * (fr[i].W / 2) * (C / 8);
-    }
-    b.begin[n] = b.total = acc;
-    if (acc == 0) return hipSuccess;
-    hipLaunchKernelGGL(maxpool2<C>, dim3(udiv_up(acc, 256)), dim3(256), 0, st, b);
-    return hipGetLastError();
-}
-
-hipError_t launch_maxpool(int C, int n, const PoolFrame *fr, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    if (n > XDN_MAX_FRAMES) return hipErrorInvalidValue;
-    if (C == 8) return maxpool_t<8>(n, fr, st);
-    if (C == 16) return maxpool_t<16>(n, fr, st);
-    return hipErrorInvalidValue;
 }
 
 template <int C>

@@ -42,15 +42,17 @@ struct UcFrame {
     const float *bias;          // [NT * 32] (RELU)
     const float *head_w;        // UC_F_24_8_HEAD: the 1x1 head, FP32 [8][6] then [6]
     float *head_out;            // UC_F_24_8_HEAD: its output, FP32 [H][W][6]
+    void *pooled;               // *_POOL: the 2x2 maximum of out, bf16 [H/2][W/2][CO] (H, W even)
     int H, W;
 };
 // kind = index into the instantiated (SRC, CA, CB, CO, EPI) table of k_unet.hip
 hipError_t launch_uconv(int kind, int n, const UcFrame *fr, hipStream_t st);
 enum {
     UC_F_0 = 0,   // images -> 8, ReLU
-    UC_F_8_8,     // 8 -> 8 ReLU
+    UC_F_8_8_POOL,  // 8 -> 8 ReLU and its 2x2 max pool
     UC_F_8_16,    // 8 -> 16 ReLU
     UC_F_16_16,   // 16 -> 16 ReLU
+    UC_F_16_16_POOL,  // the same and its 2x2 max pool
     UC_F_16_32,   // 16 -> 32 ReLU
     UC_F_32_32,   // 32 -> 32 ReLU
     UC_F_48_16,   // concat 32+16 -> 16 ReLU
@@ -83,14 +85,6 @@ enum {
     UBW_48_16,    // concat 32 (upsampled) + 16 -> 16, unmasked
     UBW_24_8,     // concat 16 (upsampled) + 8 -> 8, unmasked
 };
-
-// 2x2 max pool (valid), bf16 [H][W][C] -> [H/2][W/2][C].
-struct PoolFrame {
-    const uint16_t *in;
-    uint16_t *out;
-    int H, W;  // of the input
-};
-hipError_t launch_maxpool(int C, int n, const PoolFrame *fr, hipStream_t st);
 
 // Gradient into a pooled activation act [H][W][C]: the pooled gradient (bf16 [H/2][W/2][C]) goes to
 // the first maximum of each 2x2 window (row-major), the skip gradient (bf16 [H][W][sstride], channels
