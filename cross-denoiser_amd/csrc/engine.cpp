@@ -264,12 +264,12 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
         if (int e = hip_check(xdn::launch_fwd_stream(n, sf.data(), st), "cnn forward")) return e;
     }
     // 5. fused spatial filter + temporal accumulation + loss + backward to the network output
+    std::vector<const float *> parts(n);
+    std::vector<int> cnt(n);
+    std::vector<float> scale(n);
+    std::vector<float *> outp(n);
     {
         std::vector<xdn::TrainFrame> fr(n);
-        std::vector<const float *> parts(n);
-        std::vector<int> cnt(n);
-        std::vector<float> scale(n);
-        std::vector<float *> outp(n);
         for (int i = 0; i < n; ++i)
         {
             const xdn_slot &s = slots[i];
@@ -284,25 +284,22 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             scale[i] = (float)(1.0 / (3.0 * (double)px(s.height, s.width)));
             outp[i] = s.avg_loss;
         }
-        // the loss-sum launch also advances the device Adam step counters used by step 7
-        xdn::AdamTick tick{};
-        tick.lr = lr; tick.b1 = kAdamB1; tick.b2 = kAdamB2;
-        for (int i = 0; i < n; ++i)
-            if (slots[i].adam_t)
-            {
-                tick.counter[tick.n] = slots[i].adam_t;
-                tick.alpha[tick.n] = sc[i].adam_alpha;
-                ++tick.n;
-            }
         if (int e = hip_check(xdn::launch_filter_train(n, fr.data(), kFilterWin, true, st), "filter_train")) return e;
-        if (int e = hip_check(xdn::launch_sums(n, parts.data(), cnt.data(), scale.data(), outp.data(), st, &tick),
-                              "loss"))
-            return e;
     }
     // 6. network backward: layers 5..3 each in one fused launch (weight gradient and data gradient
     //    into the layer below), then layer 2's backward fused with layer 1's weight gradient (layer
     //    1's pre-activation gradient stays on chip); the per-block weight-gradient partials of every
-    //    (slot, layer) are reduced by one launch
+    //    (slot, layer) are reduced by one launch, which also advances the device Adam step counters
+    //    used by step 7
+    xdn::AdamTick tick{};
+    tick.lr = lr; tick.b1 = kAdamB1; tick.b2 = kAdamB2;
+    for (int i = 0; i < n; ++i)
+        if (slots[i].adam_t)
+        {
+            tick.counter[tick.n] = slots[i].adam_t;
+            tick.alpha[tick.n] = sc[i].adam_alpha;
+            ++tick.n;
+        }
     if (unet)
     {
         if (int e = unet_backward_frames(uf.data(), n, st)) return e;
@@ -310,7 +307,7 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
         for (int i = 0; i < n; ++i)
             for (int j = 0; j < UNET_JOBS; ++j)
                 jobs.push_back(unet_red_job(j, uw[i].part[j], slots[i].grad, uw[i].nblk[j]));
-        if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st), "unet wgrad reduce")) return e;
+        if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st, &tick), "unet wgrad reduce")) return e;
     }
     else
     {
@@ -343,9 +340,9 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             jobs.push_back(cnn5_red_job(cw[i], 0, s.grad, cw[i].nblk[0]));
         }
         if (int e = hip_check(xdn::launch_bwd12(n, f12.data(), st), "cnn backward")) return e;
-        if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st), "cnn wgrad reduce")) return e;
+        if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st, &tick), "cnn wgrad reduce")) return e;
     }
-    // 7. Keras Adam on every slot's parameters and the bf16 fragments: the cnn5 update writes each
+    // 7. Keras Adam on every slot's parameters, with the loss sums of step 5, and the bf16 fragments: the cnn5 update writes each
     //    weight's fragment slots itself; the U-Net's fragments are rebuilt by one packing launch
     {
         std::vector<xdn::AdamJob> jobs(n);
@@ -367,7 +364,8 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             jobs[i].packed = unet ? nullptr : s.packed;
             if (unet) unet_pack_jobs(s.params, s.packed, upj);
         }
-        if (int e = hip_check(xdn::launch_adam(n, jobs.data(), b1, b2, eps, st, unet ? nullptr : lay), "adam"))
+        const xdn::LossSums sums{n, parts.data(), cnt.data(), scale.data(), outp.data()};
+        if (int e = hip_check(xdn::launch_adam(n, jobs.data(), b1, b2, eps, st, unet ? nullptr : lay, &sums), "adam"))
             return e;
         if (unet)
             if (int e = hip_check(xdn::launch_upack((int)upj.size(), upj.data(), st), "unet pack")) return e;

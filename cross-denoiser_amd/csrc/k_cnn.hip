@@ -27,6 +27,7 @@
 //                     gradient (flipped/transposed) convolutions.
 #include "xdn_common.h"
 #include "xdn_cnn.h"
+#include "xdn_misc.h"
 
 namespace xdn {
 
@@ -1163,6 +1164,7 @@ struct RedBatch {
     int n;
     int begin[WG_MAX_JOBS + 1];  // first block of each job
     RedJob j[WG_MAX_JOBS];
+    AdamTick tick;  // the last block's, where tick.n > 0
 };
 static_assert(sizeof(RedBatch) <= 4096, "kernel argument too large");
 
@@ -1174,6 +1176,19 @@ __host__ __device__ inline int red_entries(const RedJob &J)
 __global__ __launch_bounds__(RED_E *RED_G) void wgrad_reduce(RedBatch b)
 {
     __shared__ float red[RED_SPLITS][RED_E];
+    if ((int)blockIdx.x == b.begin[b.n])
+    {
+        // one thread per counter: the double-precision step size is computed beside the sums
+        if ((int)threadIdx.x < b.tick.n)
+        {
+            const int i = threadIdx.x;
+            const int t = *b.tick.counter[i] + 1;
+            *b.tick.counter[i] = t;
+            *b.tick.alpha[i] = (float)((double)b.tick.lr * sqrt(1.0 - pow((double)b.tick.b2, (double)t)) /
+                                       (1.0 - pow((double)b.tick.b1, (double)t)));
+        }
+        return;
+    }
     int lo = 0, hi = b.n - 1;  // the job whose blocks hold this one
     while (lo < hi)
     {
@@ -1392,8 +1407,9 @@ hipError_t launch_fwd_stream(int n, const FwdStreamFrame *fr, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st)
+hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st, const AdamTick *tick)
 {
+    if (tick && (tick->n < 0 || tick->n > XDN_MAX_FRAMES)) return hipErrorInvalidValue;
     for (int j0 = 0; j0 < n; j0 += WG_MAX_JOBS)
     {
         RedBatch b{};
@@ -1406,6 +1422,8 @@ hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st)
             blocks += div_up(red_entries(b.j[i]), RED_E);
         }
         b.begin[b.n] = blocks;
+        if (tick && j0 == 0) b.tick = *tick;
+        if (b.tick.n > 0) ++blocks;
         if (blocks == 0) continue;
         hipLaunchKernelGGL(wgrad_reduce, dim3(blocks), dim3(RED_E * RED_G), 0, st, b);
         if (hipError_t e = hipGetLastError()) return e;

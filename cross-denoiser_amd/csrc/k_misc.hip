@@ -6,15 +6,66 @@
 
 namespace xdn {
 
+// out[f] = scale[f] * sum(parts[f][0 .. count[f])) in a fixed order (one workgroup per frame).
+struct BlockSums {
+    int n;
+    const float *parts[XDN_MAX_FRAMES];
+    int count[XDN_MAX_FRAMES];
+    float scale[XDN_MAX_FRAMES];
+    float *out[XDN_MAX_FRAMES];
+};
+
+__device__ __forceinline__ void block_sum(const BlockSums &b, int f, float *red)
+{
+    // eight loads in flight per thread; the sum keeps the order i, i + 256, ...
+    float s = 0.f;
+    const int cnt = b.count[f];
+    const float *pp = b.parts[f];
+    for (int i0 = threadIdx.x; i0 < cnt; i0 += 8 * 256)
+    {
+        float v[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] = i0 + 256 * k < cnt ? pp[i0 + 256 * k] : 0.f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (i0 + 256 * k < cnt) s += v[k];
+    }
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1)
+    {
+        if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *b.out[f] = red[0] * b.scale[f];
+}
+
+static bool set_sums(BlockSums &b, int n, const float *const *parts, const int *count, const float *scale, float *const *out)
+{
+    if (n < 0 || n > XDN_MAX_FRAMES) return false;
+    b.n = n;
+    for (int i = 0; i < n; ++i)
+    {
+        b.parts[i] = parts[i];
+        b.count[i] = count[i];
+        b.scale[i] = scale[i];
+        b.out[i] = out[i];
+    }
+    return true;
+}
+
 // Keras Adam (tf.keras.optimizers.Adam as used by scripts/main.py:81,303):
 //   m += (g - m)(1 - b1); v += (g^2 - v)(1 - b2); p -= alpha m / (sqrt(v) + eps),
 //   alpha = lr sqrt(1 - b2^t) / (1 - b1^t) (computed in double on the host, or on the device from a
-//   step counter by the loss-sum launch that precedes the update).
+//   step counter by the weight-gradient reduction that precedes the update). The training step's loss sums
+//   ride along, the first blocks (a launch of their own before the network's backward: 96x96 step 198.3 -> 195.2
+//   us, four 256x256 U-Net streams 379 -> 375).
 struct AdamBatch {
     int n;
     AdamJob j[XDN_MAX_FRAMES];
     AdamPackLayer lay[ADAM_PACK_LAYERS];
     float b1, b2, eps;
+    BlockSums sums;
 };
 static_assert(sizeof(AdamBatch) <= 4096, "kernel argument too large");
 
@@ -50,7 +101,13 @@ __device__ __forceinline__ void pack_param(const AdamBatch &b, char *pk, int i, 
 
 __global__ __launch_bounds__(256) void adam_kernel(AdamBatch b)
 {
-    const AdamJob &J = b.j[blockIdx.y];
+    if ((int)blockIdx.y < b.sums.n)
+    {
+        __shared__ float red[256];
+        if (blockIdx.x == 0) block_sum(b.sums, blockIdx.y, red);
+        return;
+    }
+    const AdamJob &J = b.j[blockIdx.y - b.sums.n];
     const float alpha = J.alpha_dev ? *J.alpha_dev : J.alpha;
     char *pk = static_cast<char *>(J.packed);
     for (int i = blockIdx.x * 256 + threadIdx.x; i < J.count; i += gridDim.x * 256)
@@ -68,10 +125,11 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamBatch b)
 }
 
 hipError_t launch_adam(int n, const AdamJob *jobs, float b1, float b2, float eps, hipStream_t st,
-                       const AdamPackLayer *layers)
+                       const AdamPackLayer *layers, const LossSums *sums)
 {
     AdamBatch b{};
     b.n = n;
+    if (sums && !set_sums(b.sums, sums->n, sums->parts, sums->count, sums->scale, sums->out)) return hipErrorInvalidValue;
     for (int i = 0; i < n; ++i)
         if (jobs[i].packed && !layers) return hipErrorInvalidValue;
     if (layers)
@@ -85,83 +143,25 @@ hipError_t launch_adam(int n, const AdamJob *jobs, float b1, float b2, float eps
     b.b1 = b1;
     b.b2 = b2;
     b.eps = eps;
-    if (n == 0 || maxc == 0) return hipSuccess;
-    const int gx = (maxc + 255) / 256 < 256 ? (maxc + 255) / 256 : 256;
-    hipLaunchKernelGGL(adam_kernel, dim3(gx, n), dim3(256), 0, st, b);
+    if (n == 0 || (maxc == 0 && b.sums.n == 0)) return hipSuccess;
+    const int gx = maxc < 1 ? 1 : ((maxc + 255) / 256 < 256 ? (maxc + 255) / 256 : 256);
+    hipLaunchKernelGGL(adam_kernel, dim3(gx, b.sums.n + n), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 
-// out[f] = scale[f] * sum(parts[f][0 .. count[f])) in a fixed order (one workgroup per frame).
-// Optionally also the Adam step counters' advance (one extra block, one thread per counter, so its
-// double-precision step size runs beside the sums).
-struct SumBatch {
-    int n;
-    const float *parts[XDN_MAX_FRAMES];
-    int count[XDN_MAX_FRAMES];
-    float scale[XDN_MAX_FRAMES];
-    float *out[XDN_MAX_FRAMES];
-    AdamTick tick;
-};
-static_assert(sizeof(SumBatch) <= 4096, "kernel argument too large");
-
-__global__ __launch_bounds__(256) void sum_kernel(SumBatch b)
+__global__ __launch_bounds__(256) void sum_kernel(BlockSums b)
 {
     __shared__ float red[256];
-    const int f = blockIdx.x;
-    if (f == b.n)
-    {
-        if (threadIdx.x < b.tick.n)
-        {
-            const int i = threadIdx.x;
-            const int t = *b.tick.counter[i] + 1;
-            *b.tick.counter[i] = t;
-            *b.tick.alpha[i] = (float)((double)b.tick.lr * sqrt(1.0 - pow((double)b.tick.b2, (double)t)) /
-                                       (1.0 - pow((double)b.tick.b1, (double)t)));
-        }
-        return;
-    }
-    // eight loads in flight per thread; the sum keeps the order i, i + 256, ...
-    float s = 0.f;
-    const int cnt = b.count[f];
-    const float *pp = b.parts[f];
-    for (int i0 = threadIdx.x; i0 < cnt; i0 += 8 * 256)
-    {
-        float v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = i0 + 256 * k < cnt ? pp[i0 + 256 * k] : 0.f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            if (i0 + 256 * k < cnt) s += v[k];
-    }
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 128; off > 0; off >>= 1)
-    {
-        if (threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *b.out[f] = red[0] * b.scale[f];
+    block_sum(b, blockIdx.x, red);
 }
 
 hipError_t launch_sums(int n, const float *const *parts, const int *count, const float *scale, float *const *out,
-                       hipStream_t st, const AdamTick *tick)
+                       hipStream_t st)
 {
-    SumBatch b{};
-    b.n = n;
-    if (tick)
-    {
-        if (tick->n < 0 || tick->n > XDN_MAX_FRAMES || tick->n > n) return hipErrorInvalidValue;
-        b.tick = *tick;
-    }
-    for (int i = 0; i < n; ++i)
-    {
-        b.parts[i] = parts[i];
-        b.count[i] = count[i];
-        b.scale[i] = scale[i];
-        b.out[i] = out[i];
-    }
+    BlockSums b{};
+    if (!set_sums(b, n, parts, count, scale, out)) return hipErrorInvalidValue;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(sum_kernel, dim3(n + (b.tick.n > 0 ? 1 : 0)), dim3(256), 0, st, b);
+    hipLaunchKernelGGL(sum_kernel, dim3(n), dim3(256), 0, st, b);
     return hipGetLastError();
 }
 

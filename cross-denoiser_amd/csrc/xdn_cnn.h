@@ -80,7 +80,9 @@ constexpr int compact_part(int taps, int cc, int co) { return taps * cc * co + c
 constexpr int WG_PART_L1 = compact_part(9, 15, 32);
 constexpr int WG_PART_L5 = compact_part(9, 32, 6);
 constexpr int WG_MAX_JOBS = 56;  // per launch; longer job lists are split
-hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st);
+// tick: Adam step counters that the same launch advances (the update follows it on the stream)
+struct AdamTick;
+hipError_t launch_wgrad_reduce(int n, const RedJob *jobs, hipStream_t st, const AdamTick *tick = nullptr);
 hipError_t launch_pack(int n, const PackJob *jobs, hipStream_t st);
 // last: the network's last layer (dy = the FP32 6-channel gradient of the output, L5 fragments)
 hipError_t launch_bwd(int n, const BwdFrame *fr, bool last, hipStream_t st);

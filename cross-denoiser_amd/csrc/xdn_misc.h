@@ -25,8 +25,16 @@ struct AdamPackLayer {
 };
 constexpr int ADAM_PACK_LAYERS = 5;
 
+// sums: loss sums taken by the same launch (see launch_sums)
+struct LossSums {
+    int n;
+    const float *const *parts;
+    const int *count;
+    const float *scale;
+    float *const *out;
+};
 hipError_t launch_adam(int n, const AdamJob *jobs, float b1, float b2, float eps, hipStream_t st,
-                       const AdamPackLayer *layers = nullptr);
+                       const AdamPackLayer *layers = nullptr, const LossSums *sums = nullptr);
 // Device Adam step counters: per entry t = ++(*counter[i]); alpha[i] = lr * sqrt(1 - b2^t) / (1 - b1^t)
 // (double, rounded once).
 struct AdamTick {
@@ -35,10 +43,9 @@ struct AdamTick {
     float *alpha[XDN_MAX_FRAMES];
     float lr, b1, b2;
 };
-// out[f] = scale[f] * sum(parts[f][0 .. count[f])); with `tick` the same launch also advances those
-// Adam step counters (the training step's loss sum precedes its Adam update on the stream).
+// out[f] = scale[f] * sum(parts[f][0 .. count[f]))
 hipError_t launch_sums(int n, const float *const *parts, const int *count, const float *scale, float *const *out,
-                       hipStream_t st, const AdamTick *tick = nullptr);
+                       hipStream_t st);
 
 // Frame report (displayed frame and RelL2 partial sums) of one image; see frame_error_kernel.
 struct ErrFrame {
