@@ -285,7 +285,5 @@ int unet_forward_frames(const UnetFrame *f, int n, hipStream_t st);
 int unet_backward_frames(const UnetFrame *f, int n, hipStream_t st);
 // reduction job of partial set `set` (nblk_total partials from part) into the flat gradient
 xdn::RedJob unet_red_job(int set, float *part, float *grad, int nblk_total);
-// pack jobs of one parameter vector (3x3 fragments and FP32 copies of the 1x1 layers)
-void unet_pack_jobs(const float *params, void *packed, std::vector<xdn::UPackJob> &jobs);
 
 }  // namespace xdn_abi

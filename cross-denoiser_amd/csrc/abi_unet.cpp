@@ -262,7 +262,8 @@ xdn::RedJob unet_red_job(int set, float *part, float *grad, int nblk_total)
     return r;
 }
 
-void unet_pack_jobs(const float *params, void *packed, std::vector<xdn::UPackJob> &jobs)
+// pack jobs of one parameter vector (3x3 fragments and FP32 copies of the 1x1 layers)
+static void unet_pack_jobs(const float *params, void *packed, std::vector<xdn::UPackJob> &jobs)
 {
     char *pk = static_cast<char *>(packed);
     for (int l = 0; l < UNET_LAYERS; ++l)

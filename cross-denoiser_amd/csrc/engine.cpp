@@ -342,16 +342,23 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
         if (int e = hip_check(xdn::launch_bwd12(n, f12.data(), st), "cnn backward")) return e;
         if (int e = hip_check(xdn::launch_wgrad_reduce((int)jobs.size(), jobs.data(), st, &tick), "cnn wgrad reduce")) return e;
     }
-    // 7. Keras Adam on every slot's parameters, with the loss sums of step 5, and the bf16 fragments: the cnn5 update writes each
-    //    weight's fragment slots itself; the U-Net's fragments are rebuilt by one packing launch
+    // 7. Keras Adam on every slot's parameters, with the loss sums of step 5; the update writes each weight's
+    //    fragment slots itself
     {
         std::vector<xdn::AdamJob> jobs(n);
-        std::vector<xdn::UPackJob> upj;
         xdn::AdamPackLayer lay[xdn::ADAM_PACK_LAYERS];
-        for (int l = 0; l < 5; ++l)
-            lay[l] = xdn::AdamPackLayer{(int)kLay.w_off[l], (int)kLay.b_off[l], kCnn5[l].ci, kCnn5[l].co,
-                                        (int)kLay.fwd_off[l], l > 0 ? (int)kLay.dg_off[l] : -1,
-                                        (int)kLay.bias_off[l]};
+        const int n_lay = unet ? UNET_LAYERS : 5;
+        static_assert(UNET_LAYERS <= xdn::ADAM_PACK_LAYERS, "layers of the fragment layout");
+        for (int l = 0; l < n_lay; ++l)
+            if (unet)
+                lay[l] = xdn::AdamPackLayer{(int)kULay.w_off[l], (int)kULay.b_off[l], kUnet[l].ci, kUnet[l].co,
+                                            (int)kULay.fwd_off[l], l > 0 ? (int)kULay.dg_off[l] : -1,
+                                            (int)kULay.bias_off[l],
+                                            kUnet[l].type == UL_CONV ? -1 : (int)kULay.master_off[l]};
+            else
+                lay[l] = xdn::AdamPackLayer{(int)kLay.w_off[l], (int)kLay.b_off[l], kCnn5[l].ci, kCnn5[l].co,
+                                            (int)kLay.fwd_off[l], l > 0 ? (int)kLay.dg_off[l] : -1,
+                                            (int)kLay.bias_off[l], -1};
         const float b1 = kAdamB1, b2 = kAdamB2, eps = 1e-7f;
         for (int i = 0; i < n; ++i)
         {
@@ -361,14 +368,10 @@ int xdn_denoise_stages(const xdn_slot *slots, int n_slots, float lr, int stages,
             jobs[i].count = (int)(unet ? kULay.count : kLay.count);
             jobs[i].alpha = (float)((double)lr * sqrt(1.0 - pow((double)b2, t)) / (1.0 - pow((double)b1, t)));
             jobs[i].alpha_dev = s.adam_t ? sc[i].adam_alpha : nullptr;
-            jobs[i].packed = unet ? nullptr : s.packed;
-            if (unet) unet_pack_jobs(s.params, s.packed, upj);
+            jobs[i].packed = s.packed;
         }
         const xdn::LossSums sums{n, parts.data(), cnt.data(), scale.data(), outp.data()};
-        if (int e = hip_check(xdn::launch_adam(n, jobs.data(), b1, b2, eps, st, unet ? nullptr : lay, &sums), "adam"))
-            return e;
-        if (unet)
-            if (int e = hip_check(xdn::launch_upack((int)upj.size(), upj.data(), st), "unet pack")) return e;
+        if (int e = hip_check(xdn::launch_adam(n, jobs.data(), b1, b2, eps, st, lay, n_lay, &sums), "adam")) return e;
     }
     return XDN_OK;
 }

@@ -4,6 +4,8 @@
 #include "xdn_common.h"
 #include "xdn_misc.h"
 
+#include <limits.h>
+
 namespace xdn {
 
 // out[f] = scale[f] * sum(parts[f][0 .. count[f])) in a fixed order (one workgroup per frame).
@@ -81,6 +83,11 @@ __device__ __forceinline__ void pack_param(const AdamBatch &b, char *pk, int i, 
     for (int k = 1; k < ADAM_PACK_LAYERS; ++k)
         if (i >= b.lay[k].w_off) l = k;
     const AdamPackLayer &g = b.lay[l];
+    if (g.copy_off >= 0)
+    {
+        reinterpret_cast<float *>(pk + g.copy_off)[i - g.w_off] = x;
+        return;
+    }
     if (i >= g.b_off)
     {
         reinterpret_cast<float *>(pk + g.bias_off)[i - g.b_off] = x;
@@ -94,8 +101,8 @@ __device__ __forceinline__ void pack_param(const AdamBatch &b, char *pk, int i, 
     }
     if (g.dg_off >= 0)
     {
-        const int kcd = (g.co + 15) >> 4, kc = co >> 4, h = (co >> 3) & 1, jj = co & 7;
-        reinterpret_cast<uint16_t *>(pk + g.dg_off)[(((8 - t) * kcd + kc) * 64 + 32 * h + ci) * 8 + jj] = v;
+        const int kcd = (g.co + 15) >> 4, ntd = (g.ci + 31) >> 5, kc = co >> 4, h = (co >> 3) & 1, jj = co & 7;
+        reinterpret_cast<uint16_t *>(pk + g.dg_off)[((((8 - t) * kcd + kc) * ntd + (ci >> 5)) * 64 + 32 * h + (ci & 31)) * 8 + jj] = v;
     }
 }
 
@@ -125,15 +132,18 @@ __global__ __launch_bounds__(256) void adam_kernel(AdamBatch b)
 }
 
 hipError_t launch_adam(int n, const AdamJob *jobs, float b1, float b2, float eps, hipStream_t st,
-                       const AdamPackLayer *layers, const LossSums *sums)
+                       const AdamPackLayer *layers, int n_layers, const LossSums *sums)
 {
     AdamBatch b{};
     b.n = n;
     if (sums && !set_sums(b.sums, sums->n, sums->parts, sums->count, sums->scale, sums->out)) return hipErrorInvalidValue;
     for (int i = 0; i < n; ++i)
-        if (jobs[i].packed && !layers) return hipErrorInvalidValue;
-    if (layers)
-        for (int l = 0; l < ADAM_PACK_LAYERS; ++l) b.lay[l] = layers[l];
+        if (jobs[i].packed && (!layers || n_layers < 1 || n_layers > ADAM_PACK_LAYERS)) return hipErrorInvalidValue;
+    for (int l = 0; l < ADAM_PACK_LAYERS; ++l)
+        if (l < n_layers)
+            b.lay[l] = layers[l];
+        else
+            b.lay[l].w_off = INT_MAX;
     int maxc = 0;
     for (int i = 0; i < n; ++i)
     {

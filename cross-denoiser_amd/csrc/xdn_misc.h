@@ -17,13 +17,14 @@ struct AdamJob {
 // Fragment layout of a network whose flat parameters are, per layer, a [9][ci][co] kernel then a
 // [co] bias: per layer a forward B-fragment block frag[t][kc][lane][8] (element 8h + j of lane
 // 32h + n holds W[t][16 kc + 8h + j][n]), a data-gradient block (W[8 - t][n][16 kc + 8h + j], none
-// when dg_off < 0) and an FP32 bias block; offsets in bytes from the packed base. Entries outside
-// ci x co are not written (they stay as the full packing left them: zero).
+// when dg_off < 0; more than 32 input channels make blocks [t][kc][ci / 32]) and an FP32 bias block;
+// offsets in bytes from the packed base. Entries outside ci x co are not written (they stay as the full
+// packing left them: zero). A layer with copy_off >= 0 is kept as an FP32 copy of its kernel and bias instead.
 struct AdamPackLayer {
     int w_off, b_off, ci, co;
-    int fwd_off, dg_off, bias_off;
+    int fwd_off, dg_off, bias_off, copy_off;
 };
-constexpr int ADAM_PACK_LAYERS = 5;
+constexpr int ADAM_PACK_LAYERS = 12;  // at most
 
 // sums: loss sums taken by the same launch (see launch_sums)
 struct LossSums {
@@ -34,7 +35,7 @@ struct LossSums {
     float *const *out;
 };
 hipError_t launch_adam(int n, const AdamJob *jobs, float b1, float b2, float eps, hipStream_t st,
-                       const AdamPackLayer *layers = nullptr, const LossSums *sums = nullptr);
+                       const AdamPackLayer *layers = nullptr, int n_layers = 0, const LossSums *sums = nullptr);
 // Device Adam step counters: per entry t = ++(*counter[i]); alpha[i] = lr * sqrt(1 - b2^t) / (1 - b1^t)
 // (double, rounded once).
 struct AdamTick {
