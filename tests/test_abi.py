@@ -188,3 +188,31 @@ def test_single_op_null_buffers_are_rejected_without_gpu():
     assert rejected(lib.xdn_cnn5_pack(None, None, None))
     # nothing to update: no buffers needed
     assert lib.xdn_adam(None, None, None, None, 0, 1, 1e-3, 0.9, 0.999, 1e-7, None) in (0, -1)
+
+
+def test_kept_state_and_combined_backward_without_gpu():
+    """The entry points that keep or combine gradients: empty batches are no-ops, missing buffers, a state
+    too small and windows past 15x15 are refused before anything is launched."""
+    from xdn._lib import lib
+    N, H, W = None, 32, 48
+
+    def rejected(rc, text):
+        return rc == -1 and text in lib.xdn_last_error().decode()
+
+    assert lib.xdn_spatial_filter_backward(*([N] * 14 + [0, H, W, 11, N])) == 0
+    assert lib.xdn_cross_regression_keep(*([N] * 8 + [N, 0, 0, H, W, 17, 4, N])) == 0
+    assert lib.xdn_cross_regression_grad_kept(*([N] * 5 + [0] + [N] * 8 + [N, 0, 0, H, W, 17, 4, N])) == 0
+    assert rejected(lib.xdn_spatial_filter_backward(*([N] * 14 + [1, H, W, 11, N])), "null")
+    p = 1 << 20  # never dereferenced
+    assert rejected(lib.xdn_spatial_filter_backward(*([N] * 13 + [p, 1, H, W, 17, N])), "win_size <= 15")
+    assert rejected(lib.xdn_cross_regression_keep(*([N] * 8 + [p, 1 << 30, 1, H, W, 17, 4, N])), "null")
+    size = lib.xdn_cross_regression_state_size(1, H, W, 4)
+    assert size >= (H // 4) * (W // 4) * 2 * (18 + 63) * 4
+    assert rejected(lib.xdn_cross_regression_keep(*([p] * 8 + [p, size - 1, 1, H, W, 17, 4, N])), "too small")
+    assert rejected(lib.xdn_cross_regression_grad_kept(*([p] * 5 + [size - 1] + [p] * 8 + [p, 1 << 30, 1, H, W, 17, 4, N])),
+                    "too small")
+    full, kept = (f(1, H, W, 4) for f in (lib.xdn_cross_regression_grad_workspace_size,
+                                         lib.xdn_cross_regression_grad_kept_workspace_size))
+    assert full == kept + size
+    assert rejected(lib.xdn_cross_regression_grad_kept(*([p] * 5 + [size] + [p] * 8 + [p, kept - 1, 1, H, W, 17, 4, N])),
+                    "too small")
