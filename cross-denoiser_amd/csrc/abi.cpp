@@ -65,15 +65,18 @@ size_t xdn_cross_regression_workspace_size(int batch, int height, int width, int
 }
 
 namespace {
-// What the backward needs of the forward, per image (256-B aligned): coefficients and Cholesky factors.
+// What the backward needs of the forward, per image (256-B aligned): coefficients, Cholesky factors and
+// variances (a copy: the outputs are the caller's to overwrite).
 struct CrState {
-    size_t beta, fact, bytes;
+    size_t beta, fact, var1, var2, bytes;
     CrState(int H, int W, int s)
     {
         const size_t C = (size_t)(H / s) * (W / s);
         beta = 0;
         fact = al256(C * 36 * 4);
-        bytes = fact + al256(C * 2 * 3 * 21 * 4);
+        var1 = fact + al256(C * 2 * 3 * 21 * 4);
+        var2 = var1 + al256(px(H, W) * 4);
+        bytes = var2 + al256(px(H, W) * 4);
     }
 };
 }  // namespace
@@ -123,6 +126,8 @@ static int cross_regression_impl(const float *color, const float *color2, const 
             char *w = static_cast<char *>(ws) + b * Nb;
             f.beta = reinterpret_cast<float *>(w);
             f.fact = keep ? reinterpret_cast<float *>(w + state.fact) : nullptr;
+            f.var1_kept = keep ? reinterpret_cast<float *>(w + state.var1) : nullptr;
+            f.var2_kept = keep ? reinterpret_cast<float *>(w + state.var2) : nullptr;
             f.outa = outa + b * Nr * 3;
             f.outb = outb + b * Nr * 3;
             f.H = H;
@@ -169,13 +174,11 @@ int xdn_cross_regression_from_color(const float *color, const float *color2, con
 namespace {
 // Workspace of the cross-regression backward, per image (every buffer 256-B aligned).
 struct CrgLayout {
-    size_t var1, var2, state, gq, u, gcen, evar, bytes;
+    size_t state, gq, u, gcen, evar, bytes;
     CrgLayout(int H, int W, int s, bool kept)
     {
         const size_t N = px(H, W), C = (size_t)(H / s) * (W / s);
         size_t o = 0;
-        var1 = o; o += al256(N * 4);
-        var2 = o; o += al256(N * 4);
         state = o; o += kept ? 0 : CrState(H, W, s).bytes;
         gq = o; o += al256(N * 2 * 16);
         u = o; o += al256(C * 36 * 4);
@@ -232,11 +235,11 @@ static int cross_regression_grad_impl(const float *imga, const float *imgb, cons
             f = xdn::CrFrame{};
             f.y1 = const_cast<float *>(imga + b * N * 3);
             f.y2 = const_cast<float *>(imgb + b * N * 3);
-            f.var1 = reinterpret_cast<float *>(w + lay.var1);
-            f.var2 = reinterpret_cast<float *>(w + lay.var2);
             f.alb = albedo + b * N * 3;
             f.nrm = normal + b * N * 3;
             char *st = state ? const_cast<char *>(static_cast<const char *>(state)) + b * kept.bytes : w + lay.state;
+            f.var1 = reinterpret_cast<float *>(st + kept.var1);
+            f.var2 = reinterpret_cast<float *>(st + kept.var2);
             f.beta = reinterpret_cast<float *>(st + kept.beta);
             f.fact = reinterpret_cast<float *>(st + kept.fact);
             f.H = H;
@@ -259,9 +262,11 @@ static int cross_regression_grad_impl(const float *imga, const float *imgb, cons
             g.H = H;
             g.W = W;
         }
-        if (int e = hip_check(xdn::launch_variance(n, fw.data(), 3, false, S(stream)), "variance")) return e;
         if (!state)
+        {
+            if (int e = hip_check(xdn::launch_variance(n, fw.data(), 3, false, S(stream)), "variance")) return e;
             if (int e = hip_check(xdn::launch_regression(n, fw.data(), win, s, true, S(stream)), "regression")) return e;
+        }
         if (int e = hip_check(xdn::launch_cross_regression_grad(n, fr.data(), win, s, S(stream)),
                               "cross_regression_grad"))
             return e;

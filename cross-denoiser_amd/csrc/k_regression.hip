@@ -36,6 +36,7 @@ struct VarFrame {
     const float *in;   // y (already log) or raw colour when log_in is set
     float *y_out;      // log1p(colour) when log_in is set, else unused
     float *var;        // [H][W]
+    float *kept;       // a second copy for a later backward, or null
     int H, W;
 };
 struct VarBatch {
@@ -126,6 +127,7 @@ __global__ __launch_bounds__(256) void variance_kernel(VarBatch b)
             var += d * d;
         }
         F.var[(size_t)cy * W + cx] = var;
+        if (F.kept) F.kept[(size_t)cy * W + cx] = var;
     }
 }
 
@@ -727,6 +729,7 @@ hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hip
             v.in = log_in ? (h ? fr[i].color2 : fr[i].color) : (h ? fr[i].y2 : fr[i].y1);
             v.y_out = h ? fr[i].y2 : fr[i].y1;
             v.var = h ? fr[i].var2 : fr[i].var1;
+            v.kept = h ? fr[i].var2_kept : fr[i].var1_kept;
             v.H = fr[i].H;
             v.W = fr[i].W;
             tx[m] = div_up(v.W, VT_X);

@@ -21,6 +21,7 @@ struct CrFrame {
     float *outa, *outb;           // [H/rs][W/rs][3]
     int H, W;
     float *fact = nullptr;        // [H/s][W/s][2][3][21] Cholesky factors kept for the backward, or null
+    float *var1_kept = nullptr, *var2_kept = nullptr;  // second copies of var1, var2 for it, or null
 };
 
 hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hipStream_t st);

@@ -83,9 +83,9 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
                               int width, int win_size, int sparsity, void *stream);
 
 /* The op for a caller that will differentiate it (recon_scale 1): `state`, caller-owned,
- * xdn_cross_regression_state_size() bytes, receives the regression coefficients and Cholesky factors, and
- * xdn_cross_regression_grad_kept on the same images gives the gradients of xdn_cross_regression_grad, bit
- * for bit, without running the regression again. The state is only read there. */
+ * xdn_cross_regression_state_size() bytes, receives the regression coefficients, Cholesky factors and
+ * variances, and xdn_cross_regression_grad_kept on the same images gives the gradients of
+ * xdn_cross_regression_grad, bit for bit, without running the variance and the regression again. The state is only read there. */
 size_t xdn_cross_regression_state_size(int batch, int height, int width, int sparsity);
 int xdn_cross_regression_keep(const float *imga, const float *imgb, const float *albedo, const float *normal,
                               float *outa, float *outb, float *out_vara, float *out_varb, void *state,
