@@ -216,3 +216,24 @@ def test_kept_state_and_combined_backward_without_gpu():
     assert full == kept + size
     assert rejected(lib.xdn_cross_regression_grad_kept(*([p] * 5 + [size] + [p] * 8 + [p, kept - 1, 1, H, W, 17, 4, N])),
                     "too small")
+
+
+def test_cpu_tensors_are_refused_before_any_launch(monkeypatch):
+    """The entry points without tensor checks of their own: a CPU tensor is a ValueError and no library
+    call is made. torch's raw stream getter accepts a CPU tensor's device index, -1, where there is a GPU."""
+    import torch
+
+    from xdn import cnn, pipeline
+    from xdn._lib import lib
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 0)
+    launched = []
+    for name in ("xdn_filter_train", "xdn_cnn5_pack", "xdn_unet_pack", "xdn_slot_init"):
+        monkeypatch.setattr(lib, name, lambda *a, name=name: launched.append(name) or 0)
+    img, one = torch.zeros(1, 16, 16, 3), torch.ones(1, 16, 16, 1)
+    calls = [lambda: pipeline.filter_train(img, img, img, img, torch.zeros(1, 16, 16, 6), one, one, img, one, img, img)]
+    calls += [lambda n=n: cnn.make(n, "cpu", shape=(1, 16, 16)) for n in ("cnn5", "unet")]
+    calls += [lambda n=n: pipeline.Denoiser(16, 16, device="cpu", network=n) for n in ("cnn5", "unet")]
+    for call in calls:
+        with pytest.raises(ValueError, match="GPU"):
+            call()
+    assert not launched
