@@ -613,13 +613,15 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
         sf_center_bands(C, F.band, p, HALF);
         float3 gA = ld3(F.gaccA, p), gB = ld3(F.gaccB, p);
         float hA = F.gwA[p], hB = F.gwB[p];
-        // a window position outside the image is a tap (of the mirrored pixel's values) but no center:
-        // its weights are exp2(-inf) = 0 and its upstream gradients zero
+        // a window position outside the image is a tap (of the mirrored pixel's values) but no center: its
+        // weights are exp2(-inf) = 0, also at an infinite distance (-1 inf, where 0 inf would be NaN), and its
+        // upstream gradients zero
         const int ux = x0 + lx - HALF, uy = y0 + ly - HALF;
         if (ux < 0 || uy < 0 || ux >= W || uy >= H)
         {
-            C.k0 = C.k1 = C.k2 = C.k3 = hA = hB = 0.f;
+            C.k0 = C.k1 = C.k2 = C.k3 = -1.f;
             C.k4 = -__builtin_inff();
+            hA = hB = 0.f;
             gA = gB = make_float3(0.f, 0.f, 0.f);
         }
         s[0][i] = make_float4(a.x, a.y, a.z, bb.x);

@@ -642,3 +642,28 @@ def test_cross_regression_block_counts(ops, dev, B, H, W):
         err = rel_l2(to_np(g), r)
         _report(f"cross_regression {name} {B}x{H}x{W}", err)
         assert err <= TOL, name
+
+
+@pytest.mark.parametrize("H,W,win", [(40, 37, 11), (9, 8, 15), (20, 33, 3), (272, 256, 11)])
+def test_spatial_filter_grads_with_infinite_guides(ops, dev, H, W, win):
+    """An infinite albedo and a normal whose square overflows, in the corner and beside each edge: their pixels
+    have weight 0 in every other pixel's window, as they have at a large finite albedo, so every other pixel's
+    gradients of the two colors and the normal are the same bits, and finite."""
+    args = sf_case(H, W, seed=H * W, band_lo=0.1, band_hi=3.0)
+    cots = [to_dev(c, dev) for c in _cots(1, H, W, 19)]
+    far, inf = [a.copy() for a in args], [a.copy() for a in args]
+    rest = np.ones((1, H, W), bool)
+    for y, x in ((0, 0), (1, W // 2), (H // 2, 1), (H - 2, W // 2), (H // 2, W - 2)):
+        rest[0, y, x] = False
+        far[2][0, y, x], inf[2][0, y, x] = 1e15, np.inf
+        far[3][0, y, x, 1] = inf[3][0, y, x, 1] = 1e30
+    grads = []
+    for a in (far, inf):
+        leaves = [to_dev(v, dev).requires_grad_(True) for v in a]
+        grads.append(torch.autograd.grad(ops.spatial_filter(*leaves, win_size=win), leaves, cots))
+    ref = O.spatial_filter_grad_inputs(*map(to_np, cots), *far, win_size=win)
+    for k, name in ((0, "imga"), (1, "imgb"), (3, "normal")):
+        got, at_inf = (to_np(g[k])[rest] for g in grads)
+        assert np.isfinite(got).all(), name
+        assert np.array_equal(got, at_inf), name
+        assert rel_l2(got, ref[k][rest]) <= TOL, name
