@@ -321,12 +321,13 @@ int xdn_unet_pack(const float *params, void *packed, void *stream)
     return hip_check(xdn::launch_upack((int)jobs.size(), jobs.data(), S(stream)), "unet pack");
 }
 
-static int unet_check(int B, int H, int W, size_t ws_bytes)
+static int unet_check(int B, int H, int W, int max_w, size_t ws_bytes)
 {
     if (B < 0 || H <= 0 || W <= 0) return fail(XDN_EINVAL, "unet: invalid shape [%d, %d, %d]", B, H, W);
     if (B > XDN_MAX_FRAMES) return fail(XDN_EINVAL, "unet: batch must be <= %d", XDN_MAX_FRAMES);
     // two 2x2 poolings and two 2x upsamplings must give back the full size for the concatenations
     if (H % 4 || W % 4) return fail(XDN_EINVAL, "unet: height and width must be multiples of 4 (got %d x %d)", H, W);
+    if (W > max_w) return fail(XDN_EINVAL, "unet: frames at most %d pixels wide (got %d)", max_w, W);
     if (ws_bytes < xdn_unet_workspace_size(B, H, W)) return fail(XDN_EINVAL, "unet: workspace too small");
     return XDN_OK;
 }
@@ -350,7 +351,7 @@ int xdn_unet_forward(const float *ols1, const float *ols2, const float *prev_out
                      const float *normal, const void *packed, float *param, void *workspace, size_t workspace_bytes,
                      int batch, int height, int width, void *stream)
 {
-    if (int e = unet_check(batch, height, width, workspace_bytes)) return e;
+    if (int e = unet_check(batch, height, width, xdn::UNET_MAX_W_FORWARD, workspace_bytes)) return e;
     if (batch == 0) return XDN_OK;  // empty batch: nothing to read or write
     if (!ols1 || !ols2 || !prev_out || !albedo || !normal || !packed || !param || !workspace)
         return fail(XDN_EINVAL, "unet forward: null buffer");
@@ -364,7 +365,7 @@ int xdn_unet_backward(const float *ols1, const float *ols2, const float *prev_ou
                       const float *normal, const float *dparam, const void *packed, float *grad, void *workspace,
                       size_t workspace_bytes, int batch, int height, int width, void *stream)
 {
-    if (int e = unet_check(batch, height, width, workspace_bytes)) return e;
+    if (int e = unet_check(batch, height, width, xdn::UNET_MAX_W_BACKWARD, workspace_bytes)) return e;
     if (batch == 0)  // empty batch: the gradient is a sum over no images
     {
         if (!grad) return fail(XDN_EINVAL, "unet backward: null buffer");

@@ -77,6 +77,8 @@ int check_slot(const xdn_slot &s)
         return fail(XDN_EINVAL, "slots hold frames of fewer than 2^32 pixels (got %d x %d)", s.height, s.width);
     if (s.network == XDN_NET_CNN5 && (size_t)s.height * s.width >= kCnn5MaxPx)
         return fail(XDN_EINVAL, "cnn5 slots hold frames of fewer than 2^25 pixels (got %d x %d)", s.height, s.width);
+    if (s.network == XDN_NET_UNET && s.width > xdn::UNET_MAX_W_BACKWARD)
+        return fail(XDN_EINVAL, "U-Net slots hold frames at most %d pixels wide (got %d)", xdn::UNET_MAX_W_BACKWARD, s.width);
     return XDN_OK;
 }
 

@@ -96,7 +96,6 @@ constexpr int UT_W = 32, UT_H = 16;
 typedef __amdgpu_buffer_rsrc_t u_rsrc;
 typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
 typedef __attribute__((ext_vector_type(3))) unsigned int u32x3;
-constexpr uint32_t kUOob = 0xFFFFFFF0u;
 __device__ __forceinline__ u_rsrc u_buf(const void *p, size_t off, size_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(p) + off), (short)0, (int)(uint32_t)bytes,
@@ -431,14 +430,21 @@ __global__ __launch_bounds__(256, CO > 32 || CA + CB > 32 ? 2 : (CA + CB > 16 ? 
     uconv_block<SRC, CA, CB, CO, EPI, HEAD, POOL>(b, blockIdx.x, lds);
 }
 
-// False: a row is too wide for the 32-bit offsets.
-template <int SRC, int CA, int CB, int CO>
+// Bytes of the widest pixel that a tile stages or stores (a source, the output or mask, the FP32 head).
+constexpr int widest_pixel(int src, int ca, int cb, int co, bool head)
+{
+    const int in = src == UC_SRC_IMAGES ? 12 : 2 * (ca > cb ? ca : cb), out = head ? 24 : 2 * co;
+    return in > out ? in : out;
+}
+
+// False: a row is too wide for this instantiation's 32-bit offsets (at its own level of the network; the entry
+// points refuse such frames before they launch anything, see UNET_MAX_W_FORWARD).
+template <int SRC, int CA, int CB, int CO, bool HEAD>
 static bool uconv_batch(UcBatch &b, int n, const UcFrame *fr)
 {
-    // bytes of one staged image row over all of a tile's 32-bit offsets, see kUOob
-    constexpr uint64_t row = (UT_H + 2) * (SRC == UC_SRC_IMAGES ? 12 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO);
+    constexpr uint64_t row = (UT_H + 2) * widest_pixel(SRC, CA, CB, CO, HEAD);
     for (int i = 0; i < n; ++i)
-        if (row * (uint64_t)fr[i].W >= kUOob) return false;  // wider than 4.9 million pixels
+        if (row * (uint64_t)fr[i].W >= kUOob) return false;
     int tx[XDN_MAX_FRAMES], ty[XDN_MAX_FRAMES];
     for (int i = 0; i < n; ++i)
     {
@@ -454,7 +460,7 @@ template <int SRC, int CA, int CB, int CO, int EPI, bool HEAD = false, bool POOL
 static hipError_t uconv_t(int n, const UcFrame *fr, hipStream_t st)
 {
     UcBatch b{};
-    if (!uconv_batch<SRC, CA, CB, CO>(b, n, fr)) return hipErrorInvalidValue;
+    if (!uconv_batch<SRC, CA, CB, CO, HEAD>(b, n, fr)) return hipErrorInvalidValue;
     if (b.map.total == 0) return hipSuccess;
     if (POOL)
         for (int i = 0; i < n; ++i)
@@ -856,7 +862,7 @@ __global__ __launch_bounds__(256, 2) void uwgrad_images(UwBatch b)
 template <int SRC, int CA, int CB, int CO>
 static bool uwgrad_batch(UwBatch &b, int n, const UwFrame *fr, int &blocks)
 {
-    constexpr int pix = SRC == UC_SRC_IMAGES ? 16 : 2 * (CA > CB ? CA : CB) > 2 * CO ? 2 * (CA > CB ? CA : CB) : 2 * CO;
+    constexpr int pix = widest_pixel(SRC, CA, CB, CO, false);
     for (int i = 0; i < n; ++i)  // a strip's 32-bit offsets
         if ((uint64_t)pix * (UX_R * (uint64_t)fr[i].W + UX_C) >= kUOob) return false;
     b.n = n;
@@ -943,7 +949,7 @@ static hipError_t ubackward_t(int n, const UwFrame *wfr, const UcFrame *cfr, hip
     constexpr int CI = CA + CB;
     UbBatch b{};
     if (!uwgrad_batch<SRC, CA, CB, CO>(b.w, n, wfr, b.w_blocks)) return hipErrorInvalidValue;
-    if (!uconv_batch<UC_SRC_BF16, CO, 0, CI>(b.c, n, cfr)) return hipErrorInvalidValue;
+    if (!uconv_batch<UC_SRC_BF16, CO, 0, CI, false>(b.c, n, cfr)) return hipErrorInvalidValue;
     if (b.c.map.total == 0) return hipSuccess;
     const int blocks = up8(b.w_blocks) * (CI > 32 ? 2 : 1) + b.c.map.total;
     hipLaunchKernelGGL((ubackward<SRC, CA, CB, CO, EPI, WAVES>), dim3(blocks), dim3(256), 0, st, b);

@@ -31,6 +31,13 @@ namespace xdn {
 enum { UC_SRC_BF16 = 0, UC_SRC_IMAGES = 1, UC_SRC_UPCAT = 2 };
 enum { UC_EPI_RELU = 0, UC_EPI_MASK = 1, UC_EPI_PLAIN = 2 };
 
+// The 3x3 kernels address a tile with 32-bit offsets from its first row, below kUOob. Widest frames at full
+// resolution, by the bytes a pixel column takes in the 18 rows of a tile: 16 channels to c5_1 (and 32 to c4_1 at
+// half the width), the 24 of c5_1's data gradient (48 of c4_1's). Checked before a call launches anything.
+constexpr uint32_t kUOob = 0xFFFFFFF0u;
+constexpr int UNET_MAX_W_FORWARD = (int)((kUOob - 1) / (18 * 32));   // 7,456,540
+constexpr int UNET_MAX_W_BACKWARD = (int)((kUOob - 1) / (18 * 48));  // 4,971,026
+
 // 3x3 'same' convolution over concat[a (CA ch), b (CB ch)] (or the five images), forward or data
 // gradient (the data gradient is the same kernel on dY with the flipped, transposed fragments).
 struct UcFrame {

@@ -19,7 +19,9 @@
  *     to grad.
  *   - Frame size: the cnn5 entry points and cnn5 slots take frames of fewer than 2^25 pixels (the
  *     network kernels address their 64 B/px activations with 32-bit offsets; 7680x4320 fits), the
- *     spatial-filter entry points and every slot fewer than 2^32; larger ones are XDN_EINVAL.
+ *     spatial-filter entry points and every slot fewer than 2^32; the U-Net takes frames at most
+ *     7,456,540 pixels wide forward and 4,971,026 backward and in a slot (32-bit offsets within a
+ *     tile's rows); larger ones are XDN_EINVAL.
  */
 #ifndef XDN_H
 #define XDN_H

@@ -190,6 +190,28 @@ def test_single_op_null_buffers_are_rejected_without_gpu():
     assert lib.xdn_adam(None, None, None, None, 0, 1, 1e-3, 0.9, 0.999, 1e-7, None) in (0, -1)
 
 
+def test_unet_rows_past_32_bit_offsets_are_rejected_without_gpu():
+    """The U-Net's kernels address the rows of a tile with 32-bit offsets: wider frames are refused before
+    anything is launched, in the network's calls and in a slot; at the limit the next failure is the
+    missing buffers."""
+    from xdn import pipeline
+    from xdn._lib import lib
+    N, big = None, 1 << 62
+
+    def fails(rc, text):
+        return rc == -1 and text in lib.xdn_last_error().decode()
+
+    assert fails(lib.xdn_unet_forward(*([N] * 7 + [N, big, 1, 4, 7456544, N])), "at most 7456540 pixels wide")
+    assert fails(lib.xdn_unet_forward(*([N] * 7 + [N, big, 1, 4, 7456540, N])), "null")
+    assert fails(lib.xdn_unet_backward(*([N] * 8 + [N, big, 1, 4, 4971028, N])), "at most 4971026 pixels wide")
+    assert fails(lib.xdn_unet_backward(*([N] * 8 + [N, big, 1, 4, 4971024, N])), "null")
+    s = pipeline.XdnSlot()
+    s.network, s.height, s.width = pipeline.NETWORKS["unet"], 12, 4971028
+    assert fails(lib.xdn_denoise_step(ctypes.addressof(s), 1, 1e-3, None), "at most 4971026 pixels wide")
+    s.width = 4971024
+    assert fails(lib.xdn_denoise_step(ctypes.addressof(s), 1, 1e-3, None), "null")
+
+
 def test_kept_state_and_combined_backward_without_gpu():
     """The entry points that keep or combine gradients: empty batches are no-ops, missing buffers, a state
     too small and windows past 15x15 are refused before anything is launched."""
