@@ -73,6 +73,22 @@ __device__ __forceinline__ float2 sf_grad_tap(float (&g)[5], const float4 k, flo
 __device__ __forceinline__ float norm2(float3 v) { return fmaf(v.z, v.z, fmaf(v.x, v.x, v.y * v.y)); }
 __device__ __forceinline__ float3 sub3(float3 a, float3 b) { return make_float3(a.x - b.x, a.y - b.y, a.z - b.z); }
 
+// One tap of sf_tap<SF_FWD> at the squared pixel distances y2 and x2, with the roundings spelled out: an image's sums
+// are the same bits in every kernel that takes its window rows in the same groups. (sf_tile leaves them to the
+// compiler: the images it serves are served by no other kernel.)
+__device__ __forceinline__ void sf_fwd_tap(const SfCenter &C, SfAcc &acc, float3 iA, float3 iB, float3 ia, float3 in,
+                                           float y2, float x2)
+{
+#pragma clang fp contract(off)
+    const float sh = fmaf(C.k2, norm2(sub3(C.ca, ia)), fmaf(C.k3, norm2(sub3(C.cn, in)), fmaf(C.k4, y2, C.k4 * x2)));
+    const float wA = fast_exp2(fmaf(C.k0, norm2(sub3(C.cA, iA)), sh));
+    const float wB = fast_exp2(fmaf(C.k1, norm2(sub3(C.cB, iB)), sh));
+    acc.aA.x = fmaf(wA, iA.x, acc.aA.x); acc.aA.y = fmaf(wA, iA.y, acc.aA.y); acc.aA.z = fmaf(wA, iA.z, acc.aA.z);
+    acc.aB.x = fmaf(wB, iB.x, acc.aB.x); acc.aB.y = fmaf(wB, iB.y, acc.aB.y); acc.aB.z = fmaf(wB, iB.z, acc.aB.z);
+    acc.sA += wA;
+    acc.sB += wB;
+}
+
 template <int MODE>
 __device__ __forceinline__ void sf_tap(const SfCenter &C, SfAcc &acc, float3 iA, float3 iB, float3 ia, float3 in,
                                        float pd, float kpd)
@@ -305,15 +321,24 @@ __global__ __launch_bounds__(256, 5) void sf_tile(SfBatch b)
     sf_tile_body<HALF, SF_FWD>(b, nullptr);
 }
 
-// The window rows of a pixel are split over G threads (groups of 256 threads of the block) whose sums meet in
-// LDS: FWD and GRAD for launches that leave the chip idle, where a 16x16 tile then runs 4 G waves instead of a
-// chain of 121 taps in four, and GRAD at every size.
-template <int HALF, int MODE, int G>
-__global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
+// First of the window rows of group p of P, from the middle row.
+template <int HALF, int P>
+__device__ __forceinline__ int sf_row0(int p)
+{
+    return (2 * HALF + 1) * p / P - HALF;
+}
+
+// The window rows of a pixel are summed in P groups, each from zero and the groups' sums added in order, by G
+// threads (groups of 256 threads of the block, each taking P / G row groups, whose sums meet in LDS): G = 4 or 2
+// for launches that leave the chip idle, where a 16x16 tile then runs 4 G waves instead of a chain of 121 taps in
+// four, and GRAD at every size. P is the image's, so that its bits do not depend on what it is launched with.
+template <int HALF, int MODE, int G, int P>
+__global__ __launch_bounds__(256 * G, G == 1 ? 5 : 1) void sf_tile_split(SfBatch b)
 {
     static_assert(MODE == SF_FWD || MODE == SF_GRAD, "the training tile is not split");
-    constexpr int E = SF_T + 2 * HALF, NV = MODE == SF_FWD ? 8 : 5;
-    constexpr int RED = (G - 1) * NV * 256;  // floats of the reduction, which reuses the tile
+    static_assert(P % G == 0, "whole row groups a thread");
+    constexpr int E = SF_T + 2 * HALF, NV = MODE == SF_FWD ? 8 : 5, Q = P / G;
+    constexpr int RED = (P - Q) * NV * 256;  // floats of the reduction, which reuses the tile
     __shared__ float4 s[3][E * E > RED / 12 ? E * E : (RED + 11) / 12];
     const TileLoc L = locate(b.map, xcd_tile(blockIdx.x, b.map.total));
     const SfFrame &F = b.f[L.f];
@@ -352,50 +377,66 @@ __global__ __launch_bounds__(256 * G) void sf_tile_split(SfBatch b)
         C.ca = make_float3(P1.z, P1.w, P2.x);
         C.cn = make_float3(P2.y, P2.z, P2.w);
     }
-    SfAcc acc;
-    sf_zero(acc);
-    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
     constexpr float inv_h2 = 1.f / (float)(HALF * HALF);
-    constexpr int R = 2 * HALF + 1;
+    float sum[Q][NV];  // of the thread's row groups
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+    {
+        SfAcc acc;
+        sf_zero(acc);
+        float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        const int dy1 = sf_row0<HALF, P>(Q * grp + q + 1);
 #pragma unroll 1
-    for (int dy = R * grp / G - HALF; dy < R * (grp + 1) / G - HALF; ++dy)
-    {
-        const float y2 = (float)(dy * dy), kdy = C.k4 * y2;
-        const int base = q0 + dy * E;
-#pragma unroll
-        for (int dx = -HALF; dx <= HALF; ++dx)
+        for (int dy = sf_row0<HALF, P>(Q * grp + q); dy < dy1; ++dy)
         {
-            const float4 P0 = s[0][base + dx], P1 = s[1][base + dx], P2 = s[2][base + dx];
-            const float3 iA = make_float3(P0.x, P0.y, P0.z), iB = make_float3(P0.w, P1.x, P1.y);
-            const float3 ia = make_float3(P1.z, P1.w, P2.x), in = make_float3(P2.y, P2.z, P2.w);
-            if constexpr (MODE == SF_FWD)
-                sf_tap<MODE>(C, acc, iA, iB, ia, in, 0.f, kdy + C.k4 * (float)(dx * dx));
-            else
-                sf_grad_tap(g, make_float4(C.k0, C.k1, C.k2, C.k3), C.k4, norm2(sub3(C.cA, iA)), norm2(sub3(C.cB, iB)),
-                            norm2(sub3(C.ca, ia)), norm2(sub3(C.cn, in)), y2 + (float)(dx * dx), gA, hA, iA, gB, hB, iB);
+            const float y2 = (float)(dy * dy);
+            const int base = q0 + dy * E;
+#pragma unroll
+            for (int dx = -HALF; dx <= HALF; ++dx)
+            {
+                const float4 P0 = s[0][base + dx], P1 = s[1][base + dx], P2 = s[2][base + dx];
+                const float3 iA = make_float3(P0.x, P0.y, P0.z), iB = make_float3(P0.w, P1.x, P1.y);
+                const float3 ia = make_float3(P1.z, P1.w, P2.x), in = make_float3(P2.y, P2.z, P2.w);
+                if constexpr (MODE == SF_FWD)
+                    sf_fwd_tap(C, acc, iA, iB, ia, in, y2, (float)(dx * dx));
+                else
+                    sf_grad_tap(g, make_float4(C.k0, C.k1, C.k2, C.k3), C.k4, norm2(sub3(C.cA, iA)),
+                                norm2(sub3(C.cB, iB)), norm2(sub3(C.ca, ia)), norm2(sub3(C.cn, in)),
+                                y2 + (float)(dx * dx), gA, hA, iA, gB, hB, iB);
+            }
         }
+        if constexpr (MODE == SF_FWD)
+        {
+            const float a[8] = {acc.aA.x, acc.aA.y, acc.aA.z, acc.aB.x, acc.aB.y, acc.aB.z, acc.sA, acc.sB};
+#pragma unroll
+            for (int k = 0; k < NV; ++k) sum[q][k] = a[k];
+        }
+        else
+#pragma unroll
+            for (int k = 0; k < NV; ++k) sum[q][k] = g[k];
+        if (G == 1 && q > 0)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) sum[0][k] += sum[q][k];
     }
-    float v[NV];
-    if constexpr (MODE == SF_FWD)
+    float(&v)[NV] = sum[0];
+    if constexpr (G > 1)
     {
-        v[0] = acc.aA.x; v[1] = acc.aA.y; v[2] = acc.aA.z; v[3] = acc.aB.x;
-        v[4] = acc.aB.y; v[5] = acc.aB.z; v[6] = acc.sA; v[7] = acc.sB;
+        __syncthreads();  // the tile is dead
+        float *red = reinterpret_cast<float *>(&s[0][0]);  // [P - Q][NV][256]
+        static_assert(sizeof(s) >= sizeof(float) * RED, "reduction space");
+        if (grp)
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+#pragma unroll
+                for (int k = 0; k < NV; ++k) red[((Q * (grp - 1) + q) * NV + k) * 256 + t] = sum[q][k];
+        __syncthreads();
+        if (grp) return;
+#pragma unroll
+        for (int p = 1; p < P; ++p)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) v[k] += p < Q ? sum[p][k] : red[((p - Q) * NV + k) * 256 + t];
     }
-    else
-#pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] = g[k];
-    __syncthreads();  // the tile is dead
-    float *red = reinterpret_cast<float *>(&s[0][0]);  // [G - 1][NV][256]
-    static_assert(sizeof(s) >= sizeof(float) * RED, "reduction space");
-    if (grp)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) red[((grp - 1) * NV + k) * 256 + t] = v[k];
-    __syncthreads();
-    if (grp || !live) return;
-#pragma unroll
-    for (int g = 1; g < G; ++g)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) v[k] += red[((g - 1) * NV + k) * 256 + t];
+    if (!live) return;
     if constexpr (MODE == SF_FWD)
     {
         st3(F.accA, c, make_float3(v[0], v[1], v[2]));
@@ -589,7 +630,7 @@ struct No {
     static constexpr bool value = false;
 };
 
-template <int HALF, bool BAND>
+template <int HALF, bool BAND, int P>
 __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
 {
     constexpr int E = SF_T + 2 * HALF;
@@ -690,10 +731,16 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
         da.x += ca * xa.x; da.y += ca * xa.y; da.z += ca * xa.z;
         dn.x += cn * xn.x; dn.y += cn * xn.y; dn.z += cn * xn.z;
     };
-    const int dy1 = grp ? HALF : -1;  // the split of sf_tile_split<GRAD>, for the same sums
+    // the row groups of sf_tile_split<GRAD>, for the same sums
+    const int dy0 = grp ? 0 : -HALF, dy1 = grp ? HALF : -1, mid = sf_row0<HALF, 4>(2 * grp + 1);
+    static_assert(P == 2 || P == 4, "row groups of the band gradient");
+    float g0[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // BAND, P = 4: the first of the thread's two row groups
 #pragma unroll 1
-    for (int dy = grp ? 0 : -HALF; dy <= dy1; ++dy)
+    for (int dy = dy0; dy <= dy1; ++dy)
     {
+        if (BAND && P == 4 && dy == mid)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) g0[k] = g[k], g[k] = 0.f;
         const int base = q0 + dy * E;
         const float y2 = (float)(dy * dy);
 #pragma unroll
@@ -721,7 +768,7 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
     }
     // the second half of the rows joins through LDS (the tile is dead)
     __syncthreads();
-    constexpr int NV = BAND ? 23 : 18;
+    constexpr int NV = !BAND ? 18 : (P == 4 ? 28 : 23);
     float *red = reinterpret_cast<float *>(&s[0][0]);  // [NV][256]
     static_assert(sizeof(s) >= NV * 256 * sizeof(float), "reduction space");
     if (grp)
@@ -732,7 +779,11 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
         for (int k = 0; k < 18; ++k) red[k * 256 + t] = v[k];
         if constexpr (BAND)
 #pragma unroll
-            for (int k = 0; k < 5; ++k) red[(18 + k) * 256 + t] = g[k];
+            for (int k = 0; k < 5; ++k)
+            {
+                if (P == 4) red[(23 + k) * 256 + t] = g0[k];
+                red[(18 + k) * 256 + t] = g[k];
+            }
     }
     __syncthreads();
     if (grp || !live) return;
@@ -757,7 +808,12 @@ __global__ __launch_bounds__(512) void sf_grad_inputs_tile(SfBatch b)
     {
         float *o = F.gband + 5 * c;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) o[k] = (k == 4 ? -inv_h2 : -1.f) * (g[k] + red[(18 + k) * 256 + t]);
+        for (int k = 0; k < 5; ++k)
+        {
+            float v = g[k];
+            if (P == 4) v = (g0[k] + v) + red[(23 + k) * 256 + t];
+            o[k] = (k == 4 ? -inv_h2 : -1.f) * (v + red[(18 + k) * 256 + t]);
+        }
     }
 }
 
@@ -779,16 +835,33 @@ static SfBatch sf_batch(int n, const SfFrame *fr, int win)
     return b;
 }
 
-// The splits by tiles of the launch, measured forward / band gradient in us a call: 256 tiles, one thread
+template <int HALF, int MODE, int G, int P>
+static void sf_launch_split(const SfBatch &b, hipStream_t st)
+{
+    hipLaunchKernelGGL((sf_tile_split<HALF, MODE, G, P>), dim3(b.map.total), dim3(256 * G), 0, st, b);
+}
+
+// Tiles of one image (a launch's images have one size).
+static int sf_own_tiles(const SfBatch &b) { return div_up(b.f[0].W, SF_T) * div_up(b.f[0].H, SF_T); }
+
+// Threads a pixel by the tiles of the launch, row groups by those of one image alone (an image's bits do not
+// depend on its batch). Measured at win 11, forward / band gradient in us a call: 256 tiles, one thread
 // 15.4 / 17.5, two 12.2 / 13.1, four 11.5 / 12.4; 480 tiles 20.0 / 21.4, 18.8 / 21.3, 20.9 / 22.5; from
-// 700 tiles on one thread is as fast as two, four are slower (1024 tiles: 32.8, 33.3, 40.0).
+// 700 tiles on one thread is as fast as two, four are slower (1024 tiles: 32.8, 33.3, 40.0). One thread with its
+// rows in four groups instead of one: four images of 256 tiles 33.0 -> 34.0, sixteen 115 -> 118; the other windows
+// to 15 alike (win 3 24.6, win 7 54.0 -> 55.7, win 15 206 -> 211 for the sixteen).
 template <int HALF, int MODE>
 static void sf_launch(const SfBatch &b, hipStream_t st)
 {
-    if (b.map.total <= 256)
-        hipLaunchKernelGGL((sf_tile_split<HALF, MODE, 4>), dim3(b.map.total), dim3(1024), 0, st, b);
-    else if (MODE == SF_GRAD || b.map.total <= 512)
-        hipLaunchKernelGGL((sf_tile_split<HALF, MODE, 2>), dim3(b.map.total), dim3(512), 0, st, b);
+    const int own = sf_own_tiles(b), total = b.map.total;
+    if (total <= 256)
+        sf_launch_split<HALF, MODE, 4, 4>(b, st);
+    else if (MODE == SF_GRAD || total <= 512)
+        own <= 256 ? sf_launch_split<HALF, MODE, 2, 4>(b, st) : sf_launch_split<HALF, MODE, 2, 2>(b, st);
+    else if (own <= 256)
+        sf_launch_split<HALF, SF_FWD, 1, 4>(b, st);
+    else if (own <= 512)
+        sf_launch_split<HALF, SF_FWD, 1, 2>(b, st);
     else
         hipLaunchKernelGGL((sf_tile<HALF>), dim3(b.map.total), dim3(256), 0, st, b);
 }
@@ -830,10 +903,12 @@ static bool sf_grad_fused(const SfBatch &b) { return b.f[0].gband && b.map.total
 template <int HALF>
 static void sf_grad_inputs_launch(const SfBatch &b, hipStream_t st)
 {
-    if (sf_grad_fused(b))
-        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, true>), dim3(b.map.total), dim3(512), 0, st, b);
+    if (!sf_grad_fused(b))
+        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, false, 2>), dim3(b.map.total), dim3(512), 0, st, b);
+    else if (sf_own_tiles(b) <= 256)
+        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, true, 4>), dim3(b.map.total), dim3(512), 0, st, b);
     else
-        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, false>), dim3(b.map.total), dim3(512), 0, st, b);
+        hipLaunchKernelGGL((sf_grad_inputs_tile<HALF, true, 2>), dim3(b.map.total), dim3(512), 0, st, b);
 }
 
 hipError_t launch_sf_grad_inputs(int n, const SfFrame *fr, int win, hipStream_t st)

@@ -667,3 +667,25 @@ def test_spatial_filter_grads_with_infinite_guides(ops, dev, H, W, win):
         assert np.isfinite(got).all(), name
         assert np.array_equal(got, at_inf), name
         assert rel_l2(got, ref[k][rest]) <= TOL, name
+
+
+@pytest.mark.parametrize("B,H,W,win", [(5, 120, 140, 11), (17, 120, 140, 11), (2, 290, 280, 11), (5, 130, 125, 7),
+                                        (9, 130, 125, 3), (2, 270, 260, 3), (9, 130, 125, 15), (2, 30, 40, 17)])
+def test_spatial_filter_batch_bits(ops, dev, B, H, W, win):
+    """An image's results are the same bits alone and in a batch: launches of up to 256, 512 and more tiles of
+    images of up to 256 and 512, and a batch of more images than one launch takes."""
+    args = [to_dev(a, dev) for a in sf_case(H, W, seed=H + 3 * W, band_lo=0.1, band_hi=3.0, B=B)]
+    cots = [to_dev(c, dev) for c in _cots(B, H, W, 21)]
+
+    def results(a, c):
+        out = list(ops.spatial_filter(*a, win_size=win)) + [ops.spatial_filter_grad(*c, *a, win_size=win)]
+        if win <= 15:
+            leaves = [v.clone().requires_grad_(True) for v in a]
+            out += torch.autograd.grad(ops.spatial_filter(*leaves, win_size=win), leaves, c)
+        return out
+
+    batch = results(args, cots)
+    for b in (0, B - 1):
+        alone = results([a[b:b + 1] for a in args], [c[b:b + 1] for c in cots])
+        for k, (g, r) in enumerate(zip(batch, alone)):
+            assert torch.equal(g[b:b + 1], r), (b, k)
