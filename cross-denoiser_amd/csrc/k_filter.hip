@@ -933,8 +933,9 @@ hipError_t launch_sf_grad_inputs(int n, const SfFrame *fr, int win, hipStream_t 
 
 int filter_train_tiles(int H, int W) { return div_up(W, SF_T) * div_up(H, SF_T); }
 
-// batch_invariant: a frame's results are the same bits whatever it is launched with.
-hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool batch_invariant, hipStream_t st)
+// A frame's results are the same bits whatever it is launched with: with `step` those of one thread a pixel at any
+// size, else its own tiles decide. (A launch's frames have one size without `step`.)
+hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool step, hipStream_t st)
 {
     if (win / 2 != 5) return hipErrorInvalidValue;
     TrBatch b{};
@@ -948,8 +949,9 @@ hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool batch_
     b.map = make_tilemap(n, tx, ty);
     if (b.map.total == 0) return hipSuccess;
     // operator call, one thread -> two: 64 tiles 28.4 -> 23.9 us (the host's launch rate), 256 30.8 -> 25.6; no
-    // gain from 420 tiles on (39.4, 39.2; 1024: 66.1, 67.1), and four threads are no faster at any size
-    if (!batch_invariant && b.map.total <= 256)
+    // gain from 420 tiles on (39.4, 39.2; 1024: 66.1, 67.1; sixteen images of 256: 243, 244-249), and four threads
+    // are no faster at any size
+    if (!step && tx[0] * ty[0] <= 256)
         hipLaunchKernelGGL((sf_train_split<5>), dim3(b.map.total), dim3(512), 0, st, b);
     else
         hipLaunchKernelGGL((sf_train_tile<5>), dim3(b.map.total), dim3(256), 0, st, b);

@@ -73,7 +73,7 @@ struct TrainFrame {
     float *loss_part;                   // one partial sum per tile
     int H, W;
 };
-hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool batch_invariant, hipStream_t st);
+hipError_t launch_filter_train(int n, const TrainFrame *fr, int win, bool step, hipStream_t st);
 int filter_train_tiles(int H, int W);
 
 // Reprojection.

@@ -5,7 +5,8 @@
  * Conventions
  *   - Every image is a contiguous NHWC float32 device buffer [B, H, W, C] (C stated per argument),
  *     the layout of the reference ops (scripts/ops.py). B images are processed independently; the
- *     spatial-filter entry points give an image the same bits alone and in any batch.
+ *     spatial-filter entry points and xdn_filter_train give an image the same bits alone and in any
+ *     batch.
  *   - `stream` is a hipStream_t (NULL = default stream). All work is enqueued on it; no entry
  *     point synchronizes, allocates device memory or keeps device state between calls (the one
  *     exception, xdn_filter_train_noalloc, uses a fixed array of the library instead of a

@@ -689,3 +689,16 @@ def test_spatial_filter_batch_bits(ops, dev, B, H, W, win):
         alone = results([a[b:b + 1] for a in args], [c[b:b + 1] for c in cots])
         for k, (g, r) in enumerate(zip(batch, alone)):
             assert torch.equal(g[b:b + 1], r), (b, k)
+
+
+@pytest.mark.parametrize("B,H,W", [(5, 120, 140), (17, 64, 72), (2, 256, 256), (2, 272, 256)])
+def test_filter_train_batch_bits(dev, B, H, W):
+    """An image's results are the same bits alone and in a batch: images of up to 256 tiles in launches of
+    more, a batch of more images than one launch takes, images of 272 tiles."""
+    from xdn import pipeline
+    case = [to_dev(a, dev) for a in train_case(H, W, seed=H + 3 * W, B=B)]
+    batch = pipeline.filter_train(*case, want_loss=True)
+    for b in (0, B - 1):
+        alone = pipeline.filter_train(*[a[b:b + 1] for a in case], want_loss=True)
+        for name, g, r in zip(("out_log", "out", "loss", "avg_loss", "dparam"), batch, alone):
+            assert torch.equal(g[b:b + 1], r), (b, name)
