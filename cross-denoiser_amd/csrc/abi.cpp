@@ -134,7 +134,7 @@ static int cross_regression_impl(const float *color, const float *color2, const 
             f.W = W;
         }
         if (int e = hip_check(xdn::launch_variance(n, fr.data(), 3, fused, S(stream)), "variance")) return e;
-        if (int e = hip_check(xdn::launch_regression(n, fr.data(), win, s, keep, S(stream)), "regression")) return e;
+        if (int e = hip_check(xdn::launch_regression(n, fr.data(), win, s, false, S(stream)), "regression")) return e;
         if (int e = hip_check(xdn::launch_recon(n, fr.data(), win, s, rs, S(stream)), "recon")) return e;
     }
     return XDN_OK;
@@ -265,7 +265,7 @@ static int cross_regression_grad_impl(const float *imga, const float *imgb, cons
         if (!state)
         {
             if (int e = hip_check(xdn::launch_variance(n, fw.data(), 3, false, S(stream)), "variance")) return e;
-            if (int e = hip_check(xdn::launch_regression(n, fw.data(), win, s, true, S(stream)), "regression")) return e;
+            if (int e = hip_check(xdn::launch_regression(n, fw.data(), win, s, false, S(stream)), "regression")) return e;
         }
         if (int e = hip_check(xdn::launch_cross_regression_grad(n, fr.data(), win, s, S(stream)),
                               "cross_regression_grad"))

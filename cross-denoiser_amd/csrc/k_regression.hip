@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
 // The same regression for launches that leave the chip idle: 16 centers of a center row per block, one
 // wave (16 centers x 2 halves x 2 tap splits) for each quarter of the tap rows, which stages its own rows
 // and loads the next one while it sums the current one. The four waves' sums meet in LDS, 21 accumulators
-// at a time, and 96 lanes solve one channel's system each. regression_rows has one wave per SIMD and 17
+// at a time, and 96 lanes solve one channel's system each. FACT as in regression_rows. regression_rows has one wave per SIMD and 17
 // rows in a chain at 512x512 (256 blocks); the same taps are summed in another order here. 164 registers,
 // three waves per SIMD (at four waves it spills 160 B a lane and is slower at every size); three or
 // six waves of six or three rows, nine of two: slower from 360x480 on.
@@ -330,6 +330,7 @@ __device__ __forceinline__ void acc_list(const RegAcc &a, float v[kAcc])
     }
 }
 
+template <bool FACT>
 __global__ __launch_bounds__(64 * RS_W, 3) void regression_split(RegBatch b)
 {
     __shared__ float4 rows[RS_W][4][RS_ROW];       // one staged row per wave, planes as in regression_rows
@@ -446,7 +447,7 @@ __global__ __launch_bounds__(64 * RS_W, 3) void regression_split(RegBatch b)
     }
     const size_t rec = ((size_t)by * Ws + sbx) * 2 + sh;
     float be[6];
-    solve6(s, be);
+    solve6(s, be, FACT ? F.fact + (rec * 3 + ch) * kFact6 : nullptr);
 #pragma unroll
     for (int k = 0; k < 6; ++k) F.beta[rec * 18 + k * 3 + ch] = be[k];
 }
@@ -745,14 +746,17 @@ hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hip
 
 // Up to this many blocks of regression_rows regression_split is the faster one. Whole operator, rows ->
 // split: 64 blocks (256x256) 62 -> 33 us, 256 (512x512) 70 -> 59, 540 (540x960) 118 -> 102, 900
-// (720x1280) 161 -> 175.
+// (720x1280) 161 -> 175. It is a frame's own blocks that count, so that its bits do not depend on its batch; in
+// larger launches of such frames: 3 x 540x960 256 -> 252, 8 x 384x384 209 -> 200, 4 x 512x512 169 -> 179,
+// 8 x 512x512 315 -> 338.
 constexpr int kRowsFewBlocks = 640;
 
-// batch_invariant: a frame's coefficients are the same bits whatever it is launched with, regression_rows
-// at any size: the training step, whose streams give the same results alone and batched, and the backward (or the
-// forward that keeps its factors for one),
-// whose solves turn another summation order into up to 2e-5 of the normals' gradient.
-hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batch_invariant, hipStream_t st)
+// A frame's coefficients are the same bits whatever it is launched with: regression_rows at any size with `step`
+// (the training step, where another order in one layer would move the next frame's bf16 activations), else what its
+// own size asks for, whether the factors are kept for a backward or not. (A launch's frames have one size without
+// `step`.) Against 64 bits the split's shorter sums are the more accurate: 512x512, rows -> split, outputs 2.1e-7 ->
+// 1.6e-7, gradients of the colors 3.3e-7 -> 1.9e-7, of the normals 1.3e-5 -> 5.7e-6 relative L2.
+hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool step, hipStream_t st)
 {
     RegBatch b{};
     int tx[XDN_MAX_FRAMES], ty[XDN_MAX_FRAMES];
@@ -783,7 +787,7 @@ hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batc
     b.sparsity = s;
     if (b.map.total == 0) return hipSuccess;
     const bool fact = fr[0].fact != nullptr;  // all frames of a call or none
-    if (fast && !batch_invariant && b.map.total <= kRowsFewBlocks)
+    if (fast && !step && tx[0] * ty[0] <= kRowsFewBlocks)
     {
         for (int i = 0; i < n; ++i)
         {
@@ -791,7 +795,7 @@ hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batc
             ty[i] = fr[i].H / s;
         }
         b.map = make_tilemap(n, tx, ty);
-        hipLaunchKernelGGL(regression_split, dim3(b.map.total), dim3(64 * RS_W), 0, st, b);
+        hipLaunchKernelGGL((fact ? regression_split<true> : regression_split<false>), dim3(b.map.total), dim3(64 * RS_W), 0, st, b);
     }
     else if (fast)
         hipLaunchKernelGGL((fact ? regression_rows<true> : regression_rows<false>), dim3(b.map.total), dim3(256), 0, st, b);

@@ -25,7 +25,7 @@ struct CrFrame {
 };
 
 hipError_t launch_variance(int n, const CrFrame *fr, int which, bool log_in, hipStream_t st);
-hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool batch_invariant, hipStream_t st);
+hipError_t launch_regression(int n, const CrFrame *fr, int win, int s, bool step, hipStream_t st);
 hipError_t launch_recon(int n, const CrFrame *fr, int win, int s, int rs, hipStream_t st);
 
 // Backward of cross_regression with respect to its inputs (recon_scale 1). var1/var2/beta hold

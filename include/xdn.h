@@ -4,9 +4,8 @@
  *
  * Conventions
  *   - Every image is a contiguous NHWC float32 device buffer [B, H, W, C] (C stated per argument),
- *     the layout of the reference ops (scripts/ops.py). B images are processed independently; the
- *     spatial-filter entry points and xdn_filter_train give an image the same bits alone and in any
- *     batch.
+ *     the layout of the reference ops (scripts/ops.py). B images are processed independently; an
+ *     operator gives an image the same bits alone and in any batch.
  *   - `stream` is a hipStream_t (NULL = default stream). All work is enqueued on it; no entry
  *     point synchronizes, allocates device memory or keeps device state between calls (the one
  *     exception, xdn_filter_train_noalloc, uses a fixed array of the library instead of a
@@ -89,7 +88,8 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
 /* The op for a caller that will differentiate it (recon_scale 1): `state`, caller-owned,
  * xdn_cross_regression_state_size() bytes, receives the regression coefficients, Cholesky factors and
  * variances, and xdn_cross_regression_grad_kept on the same images gives the gradients of
- * xdn_cross_regression_grad, bit for bit, without running the variance and the regression again. The state is only read there. */
+ * xdn_cross_regression_grad, bit for bit, without running the variance and the regression again. The outputs
+ * are those of xdn_cross_regression, bit for bit. The state is only read by the backward. */
 size_t xdn_cross_regression_state_size(int batch, int height, int width, int sparsity);
 int xdn_cross_regression_keep(const float *imga, const float *imgb, const float *albedo, const float *normal,
                               float *outa, float *outb, float *out_vara, float *out_varb, void *state,
@@ -329,7 +329,9 @@ size_t xdn_slot_scratch_bytes(int height, int width);
 int xdn_slot_scratch_offsets(int height, int width, size_t *offsets);
 /* Fills the slot's constant scratch and packs its network; call once when the slot is admitted. */
 int xdn_slot_init(const xdn_slot *slot, void *stream);
-/* One frame for each of n_slots (<= 16) slots, enqueued on `stream`. */
+/* One frame for each of n_slots (<= 16) slots, enqueued on `stream`. A stream's results are the same bits alone
+ * and in any batch; its regression and filter sums keep one order at every frame size, where the operators
+ * above take another on small images, so the two may differ in the last bits there. */
 int xdn_denoise_step(const xdn_slot *slots, int n_slots, float learning_rate, void *stream);
 
 /* The same step in parts, so that consecutive frames of a stream can overlap on two HIP streams.

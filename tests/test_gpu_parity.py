@@ -702,3 +702,25 @@ def test_filter_train_batch_bits(dev, B, H, W):
         alone = pipeline.filter_train(*[a[b:b + 1] for a in case], want_loss=True)
         for name, g, r in zip(("out_log", "out", "loss", "avg_loss", "dparam"), batch, alone):
             assert torch.equal(g[b:b + 1], r), (b, name)
+
+
+@pytest.mark.parametrize("B,H,W,win,s", [(5, 260, 516, 17, 4), (9, 128, 256, 17, 4), (2, 720, 1280, 17, 4), (3, 40, 36, 9, 4)])
+def test_cross_regression_batch_bits(ops, dev, B, H, W, win, s):
+    """An image's outputs and gradients are the same bits alone and in a batch, and its outputs the same with and
+    without a gradient asked for: images whose tap rows are split in launches of more blocks than one alone
+    may have, a batch of more images than one launch takes, images past the split, another window."""
+    args = [to_dev(a, dev) for a in cr_grad_case(H, W, seed=H + W, B=B)]
+    cots = [to_dev(c, dev) for c in _cots(B, H, W, 23)]
+
+    def results(a, c):
+        leaves = [v.clone().requires_grad_(True) for v in a]
+        outs = ops.cross_regression(*leaves, win_size=win, sparsity=s)
+        for o, p in zip(outs, ops.cross_regression(*a, win_size=win, sparsity=s)):
+            assert torch.equal(o.detach(), p)
+        return [o.detach() for o in outs] + list(torch.autograd.grad(outs, leaves, c))
+
+    batch = results(args, cots)
+    for b in (0, B - 1):
+        alone = results([a[b:b + 1].contiguous() for a in args], [c[b:b + 1].contiguous() for c in cots])
+        for k, (g, r) in enumerate(zip(batch, alone)):
+            assert torch.equal(g[b:b + 1], r), (b, k)
