@@ -266,33 +266,21 @@ __global__ __launch_bounds__(256) void crg_center(CrgBatch b)
         }
     }
 
-    // (b) normal equations of the center (as the forward) and u = M^-1 g_beta per channel
-    RegAcc acc;
-    acc.zero();
-    const float cvar_e = vc + 1e-4f, cstd_e = sc + 1e-2f;
-    for (int iy = cy - HW; iy <= cy + HW; ++iy)
-        for (int ix = cx - HW; ix <= cx + HW; ++ix)
-        {
-            const size_t i = (size_t)mirror(iy, H) * W + mirror(ix, W);
-            const float3 iw = ld3(feat, i), ia = ld3(F.alb, i), in = ld3(F.nrm, i), it = ld3(tgt, i);
-            const float ivar = var[i];
-            const float3 dw = sub3(iw, fc);
-            const float w = reg_weight(dw, cvar_e, ivar);
-            const float inv = fast_rcp(cstd_e + sqrtf(ivar));
-            acc.add(w, inv, dw, sub3(ia, ac), sub3(in, nc), it);
-        }
+    // (b) u = M^-1 g_beta per channel, from the Cholesky factors of the forward (running the normal equations
+    // again was a third pass over the window: 256x256, forward + backward, win 27 / sparsity 4 1626 -> 1406 us,
+    // win 17 / sparsity 1 2453 -> 2327)
     float u[18];
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch)
     {
-        Sys6 s;
-        acc.system(ch, s);
+        float f[kFact6], x[6];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) s.x[k] = gb[k * 3 + ch];
-        float uc[6];
-        solve6(s, uc);
+        for (int k = 0; k < kFact6; ++k) f[k] = F.fact[(crec * 3 + ch) * kFact6 + k];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) u[k * 3 + ch] = uc[k];
+        for (int k = 0; k < 6; ++k) x[k] = gb[k * 3 + ch];
+        fact6_solve(f, x);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) u[k * 3 + ch] = x[k];
     }
 
     // (c) regression adjoint, center side
