@@ -295,6 +295,9 @@ int xdn_cross_regression_grad_kept(const float *imga, const float *imgb, const f
     const size_t need = xdn_cross_regression_state_size(B, H, W, s);
     if (B > 0 && (!state || state_bytes < need))
         return fail(XDN_EINVAL, "cross_regression_grad_kept: state too small: %zu < %zu", state_bytes, need);
+    if (B > 0 && state_bytes != need)
+        return fail(XDN_EINVAL, "cross_regression_grad_kept: the state is of another shape or sparsity: %zu bytes, expected %zu",
+                    state_bytes, need);
     return cross_regression_grad_impl(imga, imgb, albedo, normal, state, grad_outa, grad_outb, grad_vara, grad_varb,
                                       grad_imga, grad_imgb, grad_albedo, grad_normal, workspace, workspace_bytes, B, H,
                                       W, win, s, stream);

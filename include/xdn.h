@@ -89,7 +89,10 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
  * xdn_cross_regression_state_size() bytes, receives the regression coefficients, Cholesky factors and
  * variances, and xdn_cross_regression_grad_kept on the same images gives the gradients of
  * xdn_cross_regression_grad, bit for bit, without running the variance and the regression again. The outputs
- * are those of xdn_cross_regression, bit for bit. The state is only read by the backward. */
+ * are those of xdn_cross_regression, bit for bit. The state is only read by the backward, which takes the
+ * batch, height, width, win_size and sparsity of the call that left it: state_bytes has to be their state size
+ * exactly, so another shape or sparsity is XDN_EINVAL; another win_size cannot be told from it and gives wrong
+ * gradients. */
 size_t xdn_cross_regression_state_size(int batch, int height, int width, int sparsity);
 int xdn_cross_regression_keep(const float *imga, const float *imgb, const float *albedo, const float *normal,
                               float *outa, float *outb, float *out_vara, float *out_varb, void *state,

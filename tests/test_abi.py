@@ -240,6 +240,21 @@ def test_kept_state_and_combined_backward_without_gpu():
                     "too small")
 
 
+def test_kept_state_of_another_shape_or_sparsity_is_rejected_without_gpu():
+    """The backward reads the state in the layout of its own arguments, so a state of another size is refused,
+    not only one that is too small: a finer sparsity's, a larger batch's, a larger image's."""
+    from xdn._lib import lib
+    p, H, W = 1 << 20, 32, 48  # p is never dereferenced
+
+    def call(state_bytes, s=4):
+        return lib.xdn_cross_regression_grad_kept(*([p] * 5 + [state_bytes] + [p] * 8 + [p, 0, 1, H, W, 17, s, None]))
+
+    size = lib.xdn_cross_regression_state_size
+    for wrong in (size(1, H, W, 2), size(2, H, W, 4), size(1, H, 2 * W, 4), size(1, H, W, 4) + 256):
+        assert call(wrong) == -1 and "another shape or sparsity" in lib.xdn_last_error().decode()
+    assert call(size(1, H, W, 4)) == -1 and "workspace too small" in lib.xdn_last_error().decode()
+
+
 def test_cpu_tensors_are_refused_before_any_launch(monkeypatch):
     """The entry points without tensor checks of their own: a CPU tensor is a ValueError and no library
     call is made. torch's raw stream getter accepts a CPU tensor's device index, -1, where there is a GPU."""
