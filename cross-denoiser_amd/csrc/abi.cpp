@@ -74,7 +74,7 @@ struct CrState {
         const size_t C = (size_t)(H / s) * (W / s);
         beta = 0;
         fact = al256(C * 36 * 4);
-        var1 = fact + al256(C * 2 * 3 * 21 * 4);
+        var1 = fact + al256(xdn::fact_floats(C) * 4);
         var2 = var1 + al256(px(H, W) * 4);
         bytes = var2 + al256(px(H, W) * 4);
     }
@@ -125,7 +125,7 @@ static int cross_regression_impl(const float *color, const float *color2, const 
             f.nrm = normal + b * N * 3;
             char *w = static_cast<char *>(ws) + b * Nb;
             f.beta = reinterpret_cast<float *>(w);
-            f.fact = keep ? reinterpret_cast<float *>(w + state.fact) : nullptr;
+            f.fact = keep ? reinterpret_cast<float4 *>(w + state.fact) : nullptr;
             f.var1_kept = keep ? reinterpret_cast<float *>(w + state.var1) : nullptr;
             f.var2_kept = keep ? reinterpret_cast<float *>(w + state.var2) : nullptr;
             f.outa = outa + b * Nr * 3;
@@ -241,7 +241,7 @@ static int cross_regression_grad_impl(const float *imga, const float *imgb, cons
             f.var1 = reinterpret_cast<float *>(st + kept.var1);
             f.var2 = reinterpret_cast<float *>(st + kept.var2);
             f.beta = reinterpret_cast<float *>(st + kept.beta);
-            f.fact = reinterpret_cast<float *>(st + kept.fact);
+            f.fact = reinterpret_cast<float4 *>(st + kept.fact);
             f.H = H;
             f.W = W;
             xdn::CrgFrame &g = fr[i];

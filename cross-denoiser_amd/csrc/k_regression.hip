@@ -137,7 +137,7 @@ __global__ __launch_bounds__(256) void variance_kernel(VarBatch b)
 struct RegFrame {
     const float *y1, *y2, *var1, *var2, *alb, *nrm;
     float *beta;  // [Hs][Ws][2][18]
-    float *fact;  // [Hs][Ws][2][3][21] (FACT kernels)
+    float4 *fact; // Cholesky factors, see fact_at (FACT kernels)
     int H, W;
     int nfull;    // fast path with paired row tails: full 64-center blocks per center row, else 0
 };
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
     if (!active) return;
     // Lane pair solves the three channels: split 0 -> channels 0 and 1, split 1 -> channel 2.
     float *out = F.beta + (((size_t)row_c * Ws + bx) * 2 + half) * 18;
-    float *fact = FACT ? F.fact + (((size_t)row_c * Ws + bx) * 2 + half) * (3 * kFact6) : nullptr;
+    const size_t centers = (size_t)Hs * Ws, center = (size_t)row_c * Ws + bx;
     {
         Sys6 s0, s2;
         acc.system(0, s0);
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
         for (int k = 0; k < 6; ++k) s.x[k] = split ? s2.x[k] : s0.x[k];
         float be[6];
         const int ch = split ? 2 : 0;
-        solve6(s, be, FACT ? fact + ch * kFact6 : nullptr);
+        solve6(s, be, FACT ? F.fact + fact_at(centers, center, half, ch) : nullptr, centers);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + ch] = be[k];
     }
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void regression_rows(RegBatch b)
         Sys6 s1;
         acc.system(1, s1);
         float be[6];
-        solve6(s1, be, FACT ? fact + kFact6 : nullptr);
+        solve6(s1, be, FACT ? F.fact + fact_at(centers, center, half, 1) : nullptr, centers);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + 1] = be[k];
     }
@@ -445,9 +445,9 @@ __global__ __launch_bounds__(64 * RS_W, 3) void regression_split(RegBatch b)
 #pragma unroll
         for (int k = 0; k < 6; ++k) s.x[k] = gc(11 + k);
     }
-    const size_t rec = ((size_t)by * Ws + sbx) * 2 + sh;
+    const size_t centers = (size_t)(H / RG_S) * Ws, center = (size_t)by * Ws + sbx, rec = center * 2 + sh;
     float be[6];
-    solve6(s, be, FACT ? F.fact + (rec * 3 + ch) * kFact6 : nullptr);
+    solve6(s, be, FACT ? F.fact + fact_at(centers, center, sh, ch) : nullptr, centers);
 #pragma unroll
     for (int k = 0; k < 6; ++k) F.beta[rec * 18 + k * 3 + ch] = be[k];
 }
@@ -486,14 +486,15 @@ __global__ __launch_bounds__(256) void regression_generic(RegBatch b)
             acc.add(w, inv, dw, make_float3(ia.x - ca.x, ia.y - ca.y, ia.z - ca.z),
                     make_float3(in.x - cn.x, in.y - cn.y, in.z - cn.z), it);
         }
-    float *out = F.beta + (((size_t)by * Ws + bx) * 2 + half) * 18;
+    const size_t centers = (size_t)Hs * Ws, center = (size_t)by * Ws + bx;
+    float *out = F.beta + (center * 2 + half) * 18;
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch)
     {
         Sys6 s;
         acc.system(ch, s);
         float be[6];
-        solve6(s, be, FACT ? F.fact + ((((size_t)by * Ws + bx) * 2 + half) * 3 + ch) * kFact6 : nullptr);
+        solve6(s, be, FACT ? F.fact + fact_at(centers, center, half, ch) : nullptr, centers);
 #pragma unroll
         for (int k = 0; k < 6; ++k) out[k * 3 + ch] = be[k];
     }

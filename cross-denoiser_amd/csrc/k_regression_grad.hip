@@ -273,12 +273,10 @@ __global__ __launch_bounds__(256) void crg_center(CrgBatch b)
 #pragma unroll
     for (int ch = 0; ch < 3; ++ch)
     {
-        float f[kFact6], x[6];
-#pragma unroll
-        for (int k = 0; k < kFact6; ++k) f[k] = F.fact[(crec * 3 + ch) * kFact6 + k];
+        float x[6];
 #pragma unroll
         for (int k = 0; k < 6; ++k) x[k] = gb[k * 3 + ch];
-        fact6_solve(f, x);
+        fact6_solve(F.fact + fact_at((size_t)Hs * Ws, crec >> 1, h, ch), (size_t)Hs * Ws, x);
 #pragma unroll
         for (int k = 0; k < 6; ++k) u[k * 3 + ch] = x[k];
     }
@@ -710,12 +708,10 @@ __global__ __launch_bounds__(512, 4) void crg_center_tile(CrgBatch b)
 #pragma unroll
     for (int c = 0; c < 3; ++c)
     {
-        float f[kFact6], x[6];
-#pragma unroll
-        for (int k = 0; k < kFact6; ++k) f[k] = F.fact[(crec * 3 + c) * kFact6 + k];
+        float x[6];
 #pragma unroll
         for (int k = 0; k < 6; ++k) x[k] = gb[k * 3 + c];
-        fact6_solve(f, x);
+        fact6_solve(F.fact + fact_at((size_t)Hs * Ws, crec >> 1, h, c), (size_t)Hs * Ws, x);
 #pragma unroll
         for (int k = 0; k < 6; ++k) u[k * 3 + c] = x[k];
     }

@@ -11,6 +11,10 @@
 
 namespace xdn {
 
+// A kept Cholesky factor of a 6x6 system: six float4 (21 floats and padding), see fact_at.
+constexpr int kFact4 = 6;
+constexpr size_t fact_floats(size_t centers) { return centers * (2 * 3 * kFact4 * 4); }
+
 // Cross-regression family (variance, regression, recon). Unused pointers may be null.
 struct CrFrame {
     const float *color, *color2;  // raw colour (only for the fused log1p prologue)
@@ -20,7 +24,7 @@ struct CrFrame {
     float *beta;                  // [H/s][W/s][2][18]
     float *outa, *outb;           // [H/rs][W/rs][3]
     int H, W;
-    float *fact = nullptr;        // [H/s][W/s][2][3][21] Cholesky factors kept for the backward, or null
+    float4 *fact = nullptr;       // Cholesky factors kept for the backward (see fact_at), or null
     float *var1_kept = nullptr, *var2_kept = nullptr;  // second copies of var1, var2 for it, or null
 };
 
@@ -33,7 +37,7 @@ hipError_t launch_recon(int n, const CrFrame *fr, int win, int s, int rs, hipStr
 struct CrgFrame {
     const float *y1, *y2, *alb, *nrm;
     const float *var1, *var2, *beta;     // [H][W], [H][W], [Hs][Ws][2][18]
-    const float *fact;                   // [Hs][Ws][2][3][21]
+    const float4 *fact;                  // Cholesky factors (see fact_at)
     const float *gouta, *goutb;          // [H][W][3]
     const float *gvara, *gvarb;          // [H][W] or null
     float4 *gq;                          // [H][W][2]

@@ -86,7 +86,7 @@ int xdn_cross_regression_grad(const float *imga, const float *imgb, const float 
                               int width, int win_size, int sparsity, void *stream);
 
 /* The op for a caller that will differentiate it (recon_scale 1): `state`, caller-owned,
- * xdn_cross_regression_state_size() bytes, receives the regression coefficients, Cholesky factors and
+ * xdn_cross_regression_state_size() bytes (720 a center and 8 a pixel), receives the regression coefficients, Cholesky factors and
  * variances, and xdn_cross_regression_grad_kept on the same images gives the gradients of
  * xdn_cross_regression_grad, bit for bit, without running the variance and the regression again. The outputs
  * are those of xdn_cross_regression, bit for bit. The state is only read by the backward, which takes the

@@ -729,7 +729,7 @@ def test_cross_regression_batch_bits(ops, dev, B, H, W, win, s):
 @pytest.mark.parametrize("H,W,win,s", [(36, 40, 27, 4), (20, 24, 17, 1), (32, 40, 17, 4), (24, 26, 13, 2)])
 def test_cross_regression_backward_solves_with_the_kept_factors(ops, dev, H, W, win, s):
     """At windows with tiled kernels and without, the backward reads the Cholesky factors that the forward kept
-    (laid out after the coefficients) instead of running the normal equations again: without them it
+    (laid out between the coefficients and the two variances) instead of running the normal equations again: without them it
     has nothing to solve with."""
     centers = (H // s) * (W // s)
     al64 = lambda n: (n + 63) // 64 * 64  # buffers of whole 256 bytes, in floats
@@ -737,7 +737,7 @@ def test_cross_regression_backward_solves_with_the_kept_factors(ops, dev, H, W, 
     def lose_the_factors(t):
         if t.dim() == 1:  # the kept state
             t = t.clone()
-            t[al64(36 * centers):al64(36 * centers) + 126 * centers] = float("nan")
+            t[al64(36 * centers):-2 * al64(H * W)] = float("nan")
         return t
 
     leaves = [to_dev(a, dev).requires_grad_(True) for a in cr_grad_case(H, W, seed=H + W)]
