@@ -57,10 +57,16 @@ __device__ __forceinline__ bool reproj_valid(int W, int H, int px, int py, float
 // A pixel whose bilinear taps all fail takes the mean of its valid 3x3 neighbours. With a tenth of the
 // pixels disoccluded nearly every wave holds a few such pixels, and walking the nine neighbours in
 // place ran nine dependent round trips for a handful of live lanes. The block queues them in LDS
-// instead and gives every (pixel, neighbour) pair a lane: RP_PAIRS / 9 pixels per round, all their
+// instead and gives every (pixel, neighbour) pair a lane: RP_ROUND pixels per round, all their
 // validity inputs in flight together, then all their values; the values are summed in neighbour order
 // from LDS, so the sums are those of the walk. HBM-bound gather: 3840x2160, three 3-channel buffers,
-// 10% disoccluded: 363 -> 340 us (153 B/px, 3.7 TB/s).
+// 10% disoccluded: 363 -> 340 us (153 B/px, 3.7 TB/s). Where most of a block's pixels are queued (a scene cut, a
+// disoccluded region) the rounds cost more than they hide: a lane then takes a queued pixel and walks its neighbours.
+// 1920x1080, rounds alone -> with the walk, nothing valid: three 3-channel buffers 106 -> 55 us (every pixel walking in
+// place: 53), one buffer 163 -> 58, four 4-channel ones 184 -> 111. The more floats a neighbour holds the longer the
+// rounds stay the faster ones (pixels invalid at random, rounds and walk as fast: one buffer at about 85 queued of 256,
+// three 3-channel ones at 115, four 4-channel ones at 140).
+__device__ __forceinline__ int rp_walk_above(int floats) { return 80 + 4 * floats; }
 constexpr int RP_ROUND = 28;               // queued pixels per round (28 x 9 = 252 of 256 lanes)
 struct RpQueued {
     int ipx, ipy, c;                       // c: pixel of the block (thread index)
@@ -215,6 +221,55 @@ __device__ __forceinline__ void reproject_block(const RpBatch &b, int bid, RpSha
     }
     __syncthreads();
     const int nq = queued;
+    int floats = FNL * FD;
+    if (FNL == 0)
+        for (int l = 0; l < nl; ++l) floats += b.dims[l];
+    if (nq > rp_walk_above(floats))
+    {
+        if ((int)threadIdx.x >= nq) return;
+        const RpQueued Q = queue[threadIdx.x];
+        const float3 n = make_float3(Q.nx, Q.ny, Q.nz);
+        float acc[ML][MD];
+#pragma unroll
+        for (int l = 0; l < ML; ++l)
+#pragma unroll
+            for (int k = 0; k < MD; ++k) acc[l][k] = 0.f;
+        int nvalid = 0;
+#pragma unroll 1
+        for (int j = 0; j < 9; ++j)
+        {
+            const int qx = Q.ipx + j % 3 - 1, qy = Q.ipy + j / 3 - 1;
+            if (qx >= W || qx < 0 || qy >= H || qy < 0) continue;
+            const size_t qi = (size_t)qy * W + qx;
+            if (!UNIT_OPAC && F.prevOpac[qi] == 0.f) continue;
+            if (!reproj_valid(W, H, Q.ipx, Q.ipy, Q.Z, F.prevLinZ[3 * qi], Q.fwZ, n, ld3(F.prevNrm, qi), Q.fwN)) continue;
+#pragma unroll
+            for (int l = 0; l < ML; ++l)
+            {
+                if (l >= nl) break;
+                const int d = FNL > 0 ? FD : b.dims[l];
+                const float *src = F.in[l] + qi * d;
+#pragma unroll
+                for (int k = 0; k < MD; ++k)
+                    if (k < d) acc[l][k] += src[k];
+            }
+            ++nvalid;
+        }
+        const float inv = nvalid > 0 ? 1.f / (float)nvalid : 0.f;
+        const size_t c = (size_t)(by0 + Q.c / RP_TX) * W + bx0 + (Q.c & (RP_TX - 1));
+#pragma unroll
+        for (int l = 0; l < ML; ++l)
+        {
+            if (l >= nl) break;
+            const int d = FNL > 0 ? FD : b.dims[l];
+            float *dst = F.out[l] + c * d;
+#pragma unroll
+            for (int k = 0; k < MD; ++k)
+                if (k < d) dst[k] = nvalid > 0 ? acc[l][k] * inv : 0.f;
+        }
+        F.success[c] = nvalid > 0 ? 1 : 0;
+        return;
+    }
     const int q = threadIdx.x / 9, nb = threadIdx.x - 9 * q;  // this lane's pixel of the round and neighbour
     for (int q0 = 0; q0 < nq; q0 += RP_ROUND)
     {

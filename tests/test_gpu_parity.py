@@ -745,3 +745,27 @@ def test_cross_regression_backward_solves_with_the_kept_factors(ops, dev, H, W, 
         outs = ops.cross_regression(*leaves, win_size=win, sparsity=s)
     for g in torch.autograd.grad(outs, leaves, [to_dev(c, dev) for c in _cots(1, H, W, 25)]):
         assert torch.isnan(g).any()
+
+
+@pytest.mark.parametrize("dims", [(3, 3, 3), (4, 1)])
+@pytest.mark.parametrize("invalid", [0.6, 0.75, 0.9, 1.0])
+def test_reproject_mostly_disoccluded(ops, dev, invalid, dims):
+    """Blocks with few, about half and all of their pixels in the 3x3 fallback, ragged at the right and bottom:
+    the mask bit for bit, the values to 1e-6, with transparent pixels now and in the history."""
+    H, W = 21, 150
+    r = np.random.default_rng(int(100 * invalid))
+    sh = (1, H, W)
+    lz, plz = np.ones(sh + (3,), np.float32), np.ones(sh + (3,), np.float32)
+    lz[..., 1] = 0.01
+    plz[..., 0] = np.where(r.random(sh) < invalid, 100.0, 1.0)
+    nrm, fw = unit_normals(H, W, seed=5), np.full(sh + (3,), 0.5, np.float32)
+    mv = np.zeros(sh + (3,), np.float32)
+    mv[..., 0], mv[..., 1] = r.uniform(-2, 2, sh) / W, r.uniform(-2, 2, sh) / H
+    op, pop = ((r.random(sh + (1,)) < 0.97).astype(np.float32) for _ in range(2))
+    ins = [r.uniform(0, 2, sh + (d,)).astype(np.float32) for d in dims]
+    args = (mv, ins, lz, plz, nrm, nrm, fw, op, pop)
+    s_ref, o_ref = O.reproject(*args)
+    s, outs = ops.Reproject(to_dev(mv, dev), [to_dev(a, dev) for a in ins], *[to_dev(a, dev) for a in args[2:]])
+    assert np.array_equal(to_np(s), s_ref)
+    for g, rr in zip(outs, o_ref):
+        assert rel_l2(to_np(g), rr) <= 1e-6
