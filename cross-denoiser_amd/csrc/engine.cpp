@@ -3,11 +3,13 @@
 // One call advances every given slot (stream) by one frame. Each stage of train_step
 // (scripts/main.py:250-313) is ONE launch over all slots -- the frame-batch tile maps of the
 // kernels handle different resolutions in the same launch -- so n streams cost as many launches
-// as one: cross-regression (3), reprojection, erosion + screening, network forward (cnn5: layer 1,
-// then layers 2-5 in one row-streaming launch; the U-Net: 14 launches), fused filter + loss + backward, loss sums, network
-// backward (cnn5: 5 launches, the weight and data gradients of layers 2-5 fused; the
-// U-Net: 23 launches), one
-// weight-gradient reduction, Adam, pack.
+// as one (while the launches' tables hold them: the variance's 8 streams, the weight-gradient
+// reduction's 56 layers): variance, regression, reconstruction with the reprojection, erosion +
+// screening, network forward (cnn5: layer 1, then layers 2-5 in one row-streaming launch; the U-Net: 11
+// launches), fused filter + loss + backward, network backward (cnn5: 4 launches, the weight and data
+// gradients of layers 5-2 fused, layer 1's weight gradient in the last; the U-Net: 14 launches), one
+// weight-gradient reduction that also advances the Adam step counters, and Adam, which takes the loss
+// sums along and writes the packed fragments: 13 launches with cnn5, 32 with the U-Net.
 // Every slot owns its history, network, Adam moments and scratch; nothing is shared.
 #include <math.h>
 

@@ -845,11 +845,13 @@ static void sf_launch_split(const SfBatch &b, hipStream_t st)
 static int sf_own_tiles(const SfBatch &b) { return div_up(b.f[0].W, SF_T) * div_up(b.f[0].H, SF_T); }
 
 // Threads a pixel by the tiles of the launch, row groups by those of one image alone (an image's bits do not
-// depend on its batch). Measured at win 11, forward / band gradient in us a call: 256 tiles, one thread
-// 15.4 / 17.5, two 12.2 / 13.1, four 11.5 / 12.4; 480 tiles 20.0 / 21.4, 18.8 / 21.3, 20.9 / 22.5; from
-// 700 tiles on one thread is as fast as two, four are slower (1024 tiles: 32.8, 33.3, 40.0). One thread with its
-// rows in four groups instead of one: four images of 256 tiles 33.0 -> 34.0, sixteen 115 -> 118; the other windows
-// to 15 alike (win 3 24.6, win 7 54.0 -> 55.7, win 15 206 -> 211 for the sixteen).
+// depend on its batch). Kernel alone in us with one, two, four threads, forward (band gradient):
+//   256 tiles   win 3 3.8 4.0 4.2, win 7 8.3 7.0 6.7, win 11 15.2 11.8 10.9 (16.6 12.1 11.4), win 15 25.6 18.6 16.7
+//   484 tiles   win 3 4.4 4.7 5.2, win 7 10.2 9.8 11.8, win 11 18.6 18.3 20.5 (20.5 20.1 21.1), win 15 31.9 29.7 31.3
+//   1024 tiles  win 3 6.1 6.5 8.4, win 7 16.1 17.1 21.9, win 11 31.8 32.5 39.4 (36.1 35.3 40.8), win 15 58.0 54.5 60.6
+// (win 3 loses 0.4 us to the split where a call takes 17 on the host). One thread with its rows in four groups
+// instead of one: four images of 256 tiles at win 11 33.0 -> 34.0, sixteen 115 -> 118, at win 7 54.0 -> 55.7, at win
+// 15 206 -> 211.
 template <int HALF, int MODE>
 static void sf_launch(const SfBatch &b, hipStream_t st)
 {

@@ -573,7 +573,8 @@ __global__ __launch_bounds__(256) void crg_prep_tile(CrgBatch b)
 // second accumulation of the normal equations. Every factor of a tap's adjoint that only depends on the
 // center is taken out of the sum, e.g. sum gd_2 = beta_2 sum w g_acc: 28 sums for the reconstruction and
 // 22 for the regression side instead of all of g_d. One lane per (center, half) had 512 waves for the
-// whole chip at 512x512 and direct loads for every tap: 496 -> 63 us (VALU-bound now).
+// whole chip at 512x512 and direct loads for every tap: 496 -> 63 us (VALU-bound now; at four waves per SIMD it
+// spills five VGPRs, 24 B a lane).
 constexpr int CC_T = 4, CC_MAXPX = 29 * 29;
 __global__ __launch_bounds__(512, 4) void crg_center_tile(CrgBatch b)
 {

@@ -120,7 +120,8 @@ __device__ __forceinline__ uint32_t u_cvt2(float a, float b)
 // 28.3 -> 19.5 us for 66 MB, images -> 8 38.7 -> 34.0 us for 158 MB, 24 -> 8 and the head 50 -> 46 us
 // with only the even pixels of the upsampled source read), by staging latency and MFMA issue elsewhere
 // (48 -> 16 at half resolution 37.7 -> 20.4 us); registers for four waves per SIMD with one K
-// chunk, three with two, two with three chunks or two channel tiles.
+// chunk, three with two, two with three chunks or two channel tiles. 16 -> 32 spills 8 VGPRs (36 B a lane) at four
+// waves and 32 -> 32 four (20 B) at three; a scheduling barrier that removes the spills changed no time.
 constexpr int uconv_lds(int src, int ci, bool head)  // 16-bit elements
 {
     const int q = (src == UC_SRC_IMAGES ? 16 : ci) / 8;

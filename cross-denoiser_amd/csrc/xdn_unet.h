@@ -81,7 +81,7 @@ struct UwFrame {
 hipError_t launch_uwgrad_images(int n, const UwFrame *fr, hipStream_t st);  // images (15) x dY 8
 
 // The gradients of a 3x3 layer below the first: weights (wfr: input and dY) and data (cfr: dY into the input's
-// gradient), in one launch on small images.
+// gradient), in one launch.
 hipError_t launch_ubackward(int kind, int n, const UwFrame *wfr, const UcFrame *cfr, hipStream_t st);
 enum {
     UBW_8_8 = 0,  // layer 8 -> 8, data gradient masked
